@@ -272,7 +272,10 @@ struct KeysArgs {
   const uint32_t *plist;       // parents (node indices at level t); null: every node
   long long np;
   uint64_t *keys;              // by child index k * (P-1) + p - 1
-  uint32_t *k32, *v32;         // sort prefix and child index
+  uint32_t *k32, *v32;         // sort prefix and child index of every unmarked child, in child order
+  uint8_t *keep;               // by child: 1 unmarked, 0 marked
+  const unsigned long long *mask;  // per parent, bit p - 1: child p is a marked duplicate (null: none is)
+  const unsigned long long *off;   // per parent, the unmarked children of the parents before it (with mask)
 };
 
 // every child's coset key (src/tcount.cu:197-207): one wave per parent, the parent's F_p column in registers,
@@ -292,7 +295,9 @@ template <int NQ> __global__ __launch_bounds__(64) void k_keys(KeysArgs a) {
 #pragma unroll
     for (int r = 0; r < P; r++) v[r] = lane < P ? src[r * P + lane] : 0u;
     uint64_t mine = 0;
+    const uint64_t mask = a.mask ? a.mask[k] : 0ull;
     for (int p = 1; p <= G; p++) {
+      if ((mask >> (p - 1)) & 1) continue;       // a marked duplicate's key is never read
       const uint32_t *C = a.R.coef + (p - 1) * P;
       uint64_t lo = 0, hi = 0;
 #pragma unroll
@@ -306,11 +311,16 @@ template <int NQ> __global__ __launch_bounds__(64) void k_keys(KeysArgs a) {
       if (lane == p - 1) mine = s;
     }
     if (lane < G) {
-      const uint64_t key = coset_key(mine);
       const long long ch = k * G + lane;
-      a.keys[ch] = key;
-      a.k32[ch] = sort_prefix(key, inst);
-      a.v32[ch] = (uint32_t)ch;
+      const bool mk = (mask >> lane) & 1;
+      a.keep[ch] = mk ? 0 : 1;
+      if (!mk) {
+        const uint64_t key = coset_key(mine);
+        const long long x = a.mask ? (long long)a.off[k] + lane - __popcll(mask & ((1ull << lane) - 1)) : ch;
+        a.keys[ch] = key;
+        a.k32[x] = sort_prefix(key, inst);
+        a.v32[x] = (uint32_t)ch;
+      }
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -327,28 +337,82 @@ struct DedupeArgs {
   const unsigned long long *nruns;
   const uint64_t *keys;
   uint8_t *keep;               // by child; cleared for every child whose coset an earlier child holds
+  uint32_t *link;              // by child; set to that earlier child
   int *flags;                  // bit 1: a run held more than DMAXREP distinct cosets
   unsigned long long *stat;    // [0] children visited in runs, [1] exact comparisons, [2] duplicates
 };
 
-// A child (pa, p) whose parent is pa = (gp, q) with p < q and P_p, P_q commuting is the same matrix as the child
-// (pb, q) of pa's sibling pb = (gp, p): R(P_p) and R(P_q) commute.  pb precedes pa (siblings are ordered by
-// rotation, between them at most q - p - 1 others), so that child has the smaller index and this one is a
-// duplicate whenever pb is a node of the level (it may have been dropped as a duplicate or as a coset seen at a
-// lower level).  One lane per candidate position of pb.
-__device__ bool swap_duplicate(const Forest &F, const Rot &R, int t, uint32_t pa, int p, int lane) {
-  if (t < 1) return false;
-  const int q = F.rot[t][pa];
-  if (p >= q || ((R.anti[p - 1] >> q) & 1)) return false;
-  const uint32_t gp = F.par[t][pa];
-  const long long i = (long long)pa - 1 - lane;
-  const bool hit = lane < q - p && i >= 0 && F.par[t][i] == gp && F.rot[t][i] == p;
-  return __ballot(hit) != 0;
+constexpr uint32_t NO_NODE = 0xffffffffu;
+
+// Duplicates that rotations' commutation alone proves, before any key is formed.  When P_p and P_q commute,
+// peeling p and then q off a node g equals peeling q and then p.  With X and Y the nodes of the level that hold
+// the cosets of g's children q and p (peeling acts from the left, cosets are right cosets, so equal cosets have
+// equal children), child p of X and child q of Y are one coset: the one with the larger index is a duplicate.
+// Over all g of the level before and all commuting pairs this covers the equalities that commutation gives, also
+// where g's child is itself a duplicate of a node under another parent: on the 3-qubit table's fourth level
+// (8.13 million children) 2.45 of the 2.66 million duplicates, whose keys, sort and exact comparison (two 16 KB
+// matrices built in LDS) are left undone.  Measured there: comparisons 1.30 million -> 219 thousand, k_dedupe 68.9
+// -> 12.0 ms, k_keys 7.9 -> 6.7 ms, this kernel 0.2 ms.  A marked child always has an equal child of smaller index,
+// so the smallest child of a coset is never marked.
+struct MarkArgs {
+  const uint64_t *anti;
+  const uint32_t *cmap;        // the level before: node of the level that holds child k * G + p - 1, or NO_NODE
+  long long np;                // parents of the level before
+  const uint32_t *inv;         // node of the level -> its place among this growth's parents (null: the same)
+  unsigned long long *mask;    // per parent of this growth (zero at the start)
+  uint32_t *link;              // by child: itself, or an equal child of smaller index
+  int G;
+};
+
+// one wave per node g, lane q - 1 pairing its child q with every smaller p
+__global__ __launch_bounds__(64) void k_mark(MarkArgs a) {
+  const int lane = threadIdx.x, G = a.G, q = lane + 1;
+  for (long long k = blockIdx.x; k < a.np; k += gridDim.x) {
+    uint32_t x = lane < G ? a.cmap[k * G + lane] : NO_NODE;
+    if (a.inv && x != NO_NODE) x = a.inv[x];
+    for (int p = 1; p < G; p++) {
+      const uint32_t y = (uint32_t)__builtin_amdgcn_readlane((int)x, p - 1);
+      if (y == NO_NODE) continue;
+      if (lane >= p && x != NO_NODE && !((a.anti[p - 1] >> q) & 1)) {
+        const uint32_t c1 = x * (uint32_t)G + (uint32_t)(p - 1), c2 = y * (uint32_t)G + (uint32_t)(q - 1);
+        const bool first = c1 < c2;
+        atomicMin(&a.link[first ? c2 : c1], first ? c1 : c2);
+        atomicOr(&a.mask[first ? y : x], 1ull << (first ? q - 1 : p - 1));
+      }
+    }
+  }
+}
+
+// unmarked children per parent
+__global__ void k_unmarked(const unsigned long long *mask, long long np, int G, unsigned long long *cnt) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < np; i += (long long)gridDim.x * blockDim.x)
+    cnt[i] = (unsigned long long)(G - __popcll(mask[i]));
+}
+__global__ void k_iota_u32(uint32_t *p, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    p[i] = (uint32_t)i;
+}
+__global__ void k_fill_u32(uint32_t *p, long long n, uint32_t v) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = v;
+}
+// out[list[i]] = i
+__global__ void k_invert(const uint32_t *list, long long n, uint32_t *out) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    out[list[i]] = (uint32_t)i;
+}
+// every duplicate child takes the node of the child it leads to (links go to smaller indices and end at a child that
+// is its own link, whose entry is not written here)
+__global__ void k_resolve(const uint32_t *link, long long n, uint32_t *cmap) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    uint32_t c = link[i];
+    if (c == (uint32_t)i) continue;
+    for (uint32_t d = link[c]; d != c; d = link[c]) c = d;
+    cmap[i] = cmap[c];
+  }
 }
 
 // exact dedupe: within each run of equal prefixes (children in increasing index), the first child of every
-// exact coset stays (src/tcount.cu:327-360: the smallest index of each coset).  Commuting swaps of an earlier
-// child are marked without a comparison.
+// exact coset stays (src/tcount.cu:327-360: the smallest index of each coset).  Only unmarked children are sorted.
 template <int NQ> __global__ __launch_bounds__(64) void k_dedupe(DedupeArgs a) {
   constexpr int P = 1 << (2 * NQ), G = P - 1;
   __shared__ uint32_t A[P * P], B[P * P];
@@ -369,7 +433,8 @@ template <int NQ> __global__ __launch_bounds__(64) void k_dedupe(DedupeArgs a) {
       const uint32_t ch = a.v32[j];
       const uint64_t key = a.keys[ch];
       const uint32_t inst = inst_of(a.F, a.t, parent(ch));
-      bool dup = swap_duplicate(a.F, a.R, a.t, parent(ch), (int)(ch % G) + 1, lane), built = false;
+      bool dup = false, built = false;
+      uint32_t first = ch;
       uint64_t ka = 0;
       for (int q = 0; q < nrep && !dup; q++) {
         const uint32_t rc = rep[q];
@@ -383,12 +448,13 @@ template <int NQ> __global__ __launch_bounds__(64) void k_dedupe(DedupeArgs a) {
           bid = rc;
         }
         dup = same_cols<P>(A, ka, B, kb, lane);
+        first = rc;
         n_cmp++;
       }
       n_vis++;
       if (dup) {
         n_dup++;
-        if (lane == 0) a.keep[ch] = 0;
+        if (lane == 0) { a.keep[ch] = 0; a.link[ch] = first; }
       } else if (nrep < DMAXREP) {
         if (lane == 0) rep[nrep] = ch;
         nrep++;
@@ -747,6 +813,9 @@ struct Levels {
   std::vector<uint8_t *> rot;
   std::vector<uint64_t *> keys;
   std::vector<long long> count;
+  // the last growth's children -> nodes of the level it made (NO_NODE: none), and how many parents it had
+  uint32_t *cmap = nullptr;
+  long long cmap_np = 0;
   void release() {
     (void)chz::sync_owner();           // the blocks return to the cache: no kernel may still use them
     for (auto p : par) chz::dev_free(p);
@@ -754,6 +823,8 @@ struct Levels {
     for (auto p : rot) chz::dev_free(p);
     for (auto p : keys) chz::dev_free(p);
     for (size_t l = 1; l < mat.size(); l++) chz::dev_free(mat[l]);
+    chz::dev_free(cmap);
+    cmap = nullptr;
     par.clear(); inst.clear(); rot.clear(); keys.clear(); count.clear(); mat.clear();
   }
 };
@@ -786,9 +857,9 @@ struct chz_tc {
   long long nentries = 0;
   // work arrays
   chz::DBuf<uint64_t> ckeys;
-  chz::DBuf<uint32_t> sk[2], sv[2], runs, list, list2;
+  chz::DBuf<uint32_t> sk[2], sv[2], runs, list, list2, link, inv;
   chz::DBuf<uint8_t> keep, hit, fresh;
-  chz::DBuf<unsigned long long> cnt, bcount, hist, tmp;
+  chz::DBuf<unsigned long long> cnt, bcount, hist, tmp, mask, moff;
   chz::DBuf<int> flags;
   // measurement
   chz::EventLog ev;
@@ -865,9 +936,9 @@ struct GrowOut {
 
 // one level of growth of forest L (the table when table = true) from the nodes plist of level t (null: all np).
 // Children are keyed, sorted, deduplicated exactly, (table) filtered against the HBM table, and the survivors
-// become level t+1 (src/tcount.cu:327-395).
+// become level t+1 (src/tcount.cu:327-395).  last: no level grows from the new one.
 template <int NQ>
-static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long long np, bool table) {
+static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long long np, bool table, bool last) {
   constexpr int P = 1 << (2 * NQ), G = P - 1;
   GrowOut out;
   const long long nc = np * G;
@@ -882,32 +953,57 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
   c->flags.need(1);
   HIPCHK(hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
 
+  // duplicates by commutation, from the growth before
+  c->link.need(nc);
+  c->cnt.need(4);
+  hipLaunchKernelGGL(k_iota_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, c->link.p, nc);
+  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, c->cnt.p, 4ll, 0ull);
+  const bool marks = L.cmap != nullptr && np > 0;
+  long long nu = nc;                          // children not marked
+  if (marks) {
+    c->ev.begin(F_DEDUPE, c->stream);
+    c->mask.need(np);
+    c->moff.need(np + 1);
+    c->tmp.need(np / SC_TILE + 4);
+    hipLaunchKernelGGL(k_fill_u64, dim3(gridt(np)), dim3(256), 0, c->stream, c->mask.p, np, 0ull);
+    if (plist) {
+      c->inv.need(L.count[t]);
+      hipLaunchKernelGGL(k_fill_u32, dim3(gridt(L.count[t])), dim3(256), 0, c->stream, c->inv.p, L.count[t], NO_NODE);
+      hipLaunchKernelGGL(k_invert, dim3(gridt(np)), dim3(256), 0, c->stream, plist, np, c->inv.p);
+    }
+    MarkArgs ma{c->d_anti, L.cmap, L.cmap_np, plist ? c->inv.p : nullptr, c->mask.p, c->link.p, G};
+    hipLaunchKernelGGL(k_mark, dim3(grid1(L.cmap_np)), dim3(64), 0, c->stream, ma);
+    hipLaunchKernelGGL(k_unmarked, dim3(gridt(np)), dim3(256), 0, c->stream, c->mask.p, np, G, c->moff.p);
+    HIPCHK(scan_excl(c->moff.p, np, c->tmp.p, c->stream));
+    c->ev.end(c->stream);
+    unsigned long long tot = 0;
+    HIPCHK(hipMemcpyAsync(&tot, c->moff.p + np, 8, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    nu = (long long)tot;
+    chz::dev_free(L.cmap);                    // the marks that read it have run
+    L.cmap = nullptr;
+  }
+
   c->ev.begin(F_KEYS, c->stream);
-  KeysArgs ka{R, F, t, plist, np, c->ckeys.p, c->sk[0].p, c->sv[0].p};
+  KeysArgs ka{R, F, t, plist, np, c->ckeys.p, c->sk[0].p, c->sv[0].p, c->keep.p, marks ? c->mask.p : nullptr,
+              marks ? c->moff.p : nullptr};
   hipLaunchKernelGGL(k_keys<NQ>, dim3(grid1(np)), dim3(64), 0, c->stream, ka);
   c->ev.end(c->stream);
-  c->k_work[F_KEYS] += (double)nc * P * 2;
+  c->k_work[F_KEYS] += (double)nu * P * 2;
 
   c->ev.begin(F_SORT, c->stream);
-  sort_children(c, nc);
+  sort_children(c, nu);
   c->ev.end(c->stream);
-  c->k_work[F_SORT] += (double)nc * 8 * 4 * 2;
+  c->k_work[F_SORT] += (double)nu * 8 * 4 * 2;
 
   c->ev.begin(F_DEDUPE, c->stream);
-  c->runs.need(nc);
-  c->cnt.need(4);
-  HIPCHK(hipMemsetAsync(c->cnt.p, 0, 32, c->stream));
-  hipLaunchKernelGGL(k_fill_u8, dim3(gridt(nc)), dim3(256), 0, c->stream, c->keep.p, nc, (uint8_t)1);
-  hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nc / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p, nc,
+  c->runs.need(nu);
+  hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p, nu,
                      c->runs.p, c->cnt.p, nullptr);
-  unsigned long long nruns = 0;
-  HIPCHK(hipMemcpyAsync(&nruns, c->cnt.p, 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  if (nruns) {
-    DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nc, c->runs.p, c->cnt.p, c->ckeys.p, c->keep.p, c->flags.p,
-                  c->cnt.p + 1};
-    hipLaunchKernelGGL(k_dedupe<NQ>, dim3(grid1((long long)nruns)), dim3(64), 0, c->stream, da);
-  }
+  // blocks read the number of runs on the device
+  DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nu, c->runs.p, c->cnt.p, c->ckeys.p, c->keep.p, c->link.p,
+                c->flags.p, c->cnt.p + 1};
+  hipLaunchKernelGGL(k_dedupe<NQ>, dim3(grid1(nu / 2 + 1, 8192)), dim3(64), 0, c->stream, da);
   c->ev.end(c->stream);
 
   c->list.need(nc);
@@ -957,6 +1053,14 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
     hipLaunchKernelGGL(k_gather, dim3(gridt(nn)), dim3(256), 0, c->stream, ga);
     c->ev.end(c->stream);
   }
+  // where every child went, for the marks of the next growth
+  if (!last && nn) {
+    L.cmap = dalloc<uint32_t>(nc);
+    L.cmap_np = np;
+    hipLaunchKernelGGL(k_fill_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, L.cmap, nc, NO_NODE);
+    hipLaunchKernelGGL(k_invert, dim3(gridt(nn)), dim3(256), 0, c->stream, c->list.p, nn, L.cmap);
+    hipLaunchKernelGGL(k_resolve, dim3(gridt(nc)), dim3(256), 0, c->stream, c->link.p, nc, L.cmap);
+  }
   HIPCHK(hipMemcpyAsync(&out.flags, c->flags.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   unsigned long long st[4] = {0, 0, 0, 0};
   HIPCHK(hipMemcpyAsync(st, c->cnt.p, 32, hipMemcpyDeviceToHost, c->stream));
@@ -966,7 +1070,7 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
   c->dcount[0] += (double)st[0];
   c->dcount[1] += (double)st[1];
   c->dcount[2] += (double)st[2];
-  c->dcount[3] += (double)st[3];
+  c->dcount[3] += (double)st[3] + (double)(nc - nu);
   return out;
 }
 
@@ -1105,7 +1209,7 @@ template <int NQ> static void build_table(chz_tc *c) {
   for (int l = 1; l <= c->K; l++) {
     const double t0 = chz::now_s();
     const long long np = T.count[l - 1];
-    const GrowOut g = grow<NQ>(c, T, l - 1, nullptr, np, true);
+    const GrowOut g = grow<NQ>(c, T, l - 1, nullptr, np, true, l == c->K);
     if (g.flags & 2) { set_err("a dedupe run holds more distinct cosets than its buffer"); throw chz::DeviceError(); }
     table_insert_level(c, l);
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1117,6 +1221,8 @@ template <int NQ> static void build_table(chz_tc *c) {
   }
   // the table's nodes are replayed from the identity when a lookup needs them; drop materialised levels
   HIPCHK(hipStreamSynchronize(c->stream));
+  chz::dev_free(T.cmap);
+  T.cmap = nullptr;
   for (size_t l = 1; l < T.mat.size(); l++)
     if (T.mat[l]) { chz::dev_free(T.mat[l]); T.mat[l] = nullptr; }
 }
@@ -1188,7 +1294,7 @@ static void search_batch(chz_tc *c, std::vector<Inst> &ins, int maxt, chz_tc_res
         if (np) HIPCHK(hipMemcpyAsync(pl, c->list2.p, np * 4, hipMemcpyDeviceToDevice, c->stream));
         plist = pl;
       }
-      const GrowOut g = grow<NQ>(c, S, j - 1, plist, np, false);
+      const GrowOut g = grow<NQ>(c, S, j - 1, plist, np, false, j + c->Kt >= maxt);
       if (g.flags & 2) { set_err("a dedupe run holds more distinct cosets than its buffer"); throw chz::DeviceError(); }
       // per-instance counts of the new level
       const long long nn = S.count[j];

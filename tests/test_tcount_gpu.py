@@ -117,6 +117,33 @@ def test_random_two_qubit_targets_match_oracle(table2, tc_oracle):
         tc_oracle.orc_tc_free(h)
 
 
+@pytest.mark.parametrize("n,K,maxt", [(1, 0, 5), (1, 4, 8), (2, 0, 3), (2, 1, 5), (2, 2, 6), (2, 3, 8)])
+def test_shallow_tables_and_deep_searches_match_oracle(tc_oracle, n, K, maxt):
+    """tables of depth 0 to 3 leave the search several levels, in a batch whose targets finish at different ones:
+    level lines (children, cosets, new) and results equal the oracle's, which knows no commuting duplicates"""
+    specs = []
+    for seed in range(6):
+        k, circ = T.random_target(3000 + seed, n=n, kmin=0, kmax=min(maxt, 6),
+                                  clifford_words=lambda r: [(("h", "s")[r.below(2)], (r.below(n),)) for _ in range(5)]
+                                  + ([("cx", (0, 1))] if n > 1 else []))
+        specs.append(T.tspec_text(n, W.unitary(n, circ)))
+    table = T.CosetTable(specs[0], K=K)
+    buf = ctypes.create_string_buffer(1 << 16)
+    s0 = specs[0].encode()
+    h = tc_oracle.orc_tc_table(s0, len(s0), K, 0, buf, len(buf))
+    try:
+        assert strip_seconds("\n".join(table.table_lines())) == strip_seconds(buf.value.decode())
+        for spec, r in zip(specs, table.search(specs, maxt=maxt)):
+            raw = spec.encode()
+            rot = (ctypes.c_int * 64)()
+            rc = tc_oracle.orc_tc_search(h, raw, len(raw), maxt, buf, len(buf), rot)
+            assert rc == r["rc"]
+            assert strip_seconds("\n".join(r["lines"])) == strip_seconds(buf.value.decode())
+    finally:
+        tc_oracle.orc_tc_free(h)
+        table.close()
+
+
 def test_random_three_qubit_batch_verifies(table3):
     """16 seeded random three-qubit targets (T-count <= k by construction) in one batch: each decomposition is
     exact, no longer than k, and no single rotation can be dropped"""
