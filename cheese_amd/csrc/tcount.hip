@@ -472,6 +472,167 @@ template <int NQ> __global__ __launch_bounds__(64) void k_dedupe(DedupeArgs a) {
   }
 }
 
+// Members of the runs of equal prefixes: the sorted positions whose prefix equals the one before, appended in tiles
+// (a block scan places the tile's positions, one atomic reserves their slots; their order does not matter).
+__global__ __launch_bounds__(256) void k_run_members(const uint32_t *k, long long n, uint32_t *out,
+                                                     unsigned long long *count) {
+  __shared__ uint32_t s_wave[4];
+  __shared__ unsigned long long s_base;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const long long tile = 256ll * RH_ITEMS;
+  for (long long t0 = (long long)blockIdx.x * tile; t0 < n; t0 += (long long)gridDim.x * tile) {
+    uint32_t mask = 0;
+    for (int it = 0; it < RH_ITEMS; it++) {
+      const long long i = t0 + it * 256ll + tid;
+      if (i > 0 && i < n && k[i - 1] == k[i]) mask |= 1u << it;
+    }
+    const uint32_t c = (uint32_t)__popc(mask);
+    uint32_t x = c;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_up((int)x, d);
+      if (lane >= d) x += y;
+    }
+    if (lane == 63) s_wave[w] = x;
+    __syncthreads();
+    if (tid == 0) {
+      uint32_t tot = 0;
+      for (int j = 0; j < 4; j++) { const uint32_t v = s_wave[j]; s_wave[j] = tot; tot += v; }
+      s_base = tot ? atomicAdd(count, (unsigned long long)tot) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long pos = s_base + s_wave[w] + (x - c);
+    for (int it = 0; it < RH_ITEMS; it++)
+      if ((mask >> it) & 1u) out[pos++] = (uint32_t)(t0 + it * 256ll + tid);
+    __syncthreads();                                 // s_wave and s_base are reused by the next tile
+  }
+}
+
+// entry of the child (parent matrix src, rotation p) in row a of column c: rows that commute with P_p are the parent's
+struct ChildRows {
+  const uint32_t *src;
+  uint64_t anti, plus;
+  int p;
+};
+__device__ __forceinline__ uint32_t child_entry(const ChildRows &A, int a, uint32_t x, uint32_t y) {   // x, y: rows a, a ^ p
+  const uint32_t f = m31_rot(((A.plus >> a) & 1) ? m31_sub(x, y) : m31_add(x, y), 15);
+  return ((A.anti >> a) & 1) ? f : x;
+}
+__device__ __forceinline__ int m31_signed(uint32_t v) { return (int)(v > HALF ? v - MP : v); }
+
+// sort key of column `lane` of the child: a 58-bit hash that the column's sign does not change (a linear form of the
+// signed entries in 64 bits, or its negative) above the lane.  wl: lane r's weight of row r.  (Entries are multiples
+// of high powers of two, so a 32-bit form would keep few bits of the weights.)
+template <int P>
+__device__ __forceinline__ uint64_t child_col_key(const ChildRows &A, uint32_t wl, int lane) {
+  const int h = 31 - __clz(A.p), lowm = (1 << h) - 1, c = lane < P ? lane : 0;
+  long long sum = 0;
+#pragma unroll 8
+  for (int j = 0; j < P / 2; j++) {
+    const int a = ((j >> h) << (h + 1)) | (j & lowm), r = a ^ A.p;
+    const uint32_t x = A.src[a * P + c], y = A.src[r * P + c];
+    sum += (long long)__builtin_amdgcn_readlane((int)wl, a) * m31_signed(child_entry(A, a, x, y)) +
+           (long long)__builtin_amdgcn_readlane((int)wl, r) * m31_signed(child_entry(A, r, y, x));
+  }
+  const uint64_t k = (uint64_t)(sum < 0 ? -sum : sum) * 0x9e3779b97f4a7c15ull;
+  return lane < P ? (k & ~63ull) | (uint32_t)lane : ~0ull;
+}
+
+struct PairArgs {
+  Rot R;
+  const uint32_t *mat;         // the parents' level, materialised
+  const uint32_t *inst;        // instance of each parent (null: one instance)
+  const uint32_t *plist;
+  const uint32_t *k32, *v32;
+  long long n;
+  const uint32_t *members;     // sorted positions with the prefix of the one before
+  const unsigned long long *nmem;
+  const uint64_t *keys;
+  uint8_t *keep;
+  uint32_t *link;
+  uint32_t *runs;              // run starts left to k_dedupe (a run may appear more than once)
+  unsigned long long *nruns;
+  unsigned long long *stat;    // [0] runs, [1] children visited in them, [2] exact comparisons, [3] duplicates
+};
+
+// One wave per member: the member is compared with the first child of its run that has the same 64-bit key and
+// instance, which is never dropped here.  Columns are paired by sorting (hash, lane) and every pair is compared entry
+// by entry up to one sign, so a member found equal is a duplicate for certain.  A member that is not proven equal,
+// because its coset differs or its columns were paired wrongly (two with one hash), sends its run to k_dedupe, which
+// compares every member with every distinct coset of the run.
+// What bounded this work: k_dedupe walks a run's members one after another with two 16 KB matrices in LDS, which
+// leaves 5 waves to a CU.  Here a member is a wave of its own and the two children are formed row by row from their
+// parents, once for the columns' hashes and once, in paired order, for the comparison.  The 3-qubit table's
+// fourth level (219 thousand comparisons): 12.0 ms in k_dedupe, 4.4 ms here; no run is left open.
+template <int NQ> __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
+  constexpr int P = 1 << (2 * NQ), G = P - 1;
+  const int lane = threadIdx.x & 63;
+  const long long nm = (long long)*a.nmem;
+  const uint32_t wl = lane < P ? a.R.rv[lane] : 0u;
+  uint32_t n_run = 0, n_vis = 0, n_cmp = 0, n_dup = 0;
+  auto parent = [&](uint32_t ch) { return a.plist ? a.plist[ch / G] : ch / G; };
+  for (long long it = wave_index(); it < nm; it += (long long)gridDim.x * (blockDim.x >> 6)) {
+    const long long j = a.members[it];
+    const uint32_t kp = a.k32[j], ch = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.v32[j]);
+    const uint64_t key = a.keys[ch];
+    const uint32_t pa = (uint32_t)__builtin_amdgcn_readfirstlane((int)parent(ch));
+    const uint32_t inst = a.inst ? a.inst[pa] : 0u;
+    long long s = j - 1;                                   // the run's start: back over equal prefixes
+    for (;;) {
+      const long long x = s - lane;
+      const uint64_t same = __ballot(x >= 0 && a.k32[x] == kp);
+      if (same != ~0ull) { s -= __ffsll((long long)~same) - 1; break; }
+      s -= 64;
+    }
+    s++;
+    n_vis++;
+    if (s + 1 == j) { n_run++; n_vis++; }                  // the run's first member counts the run and its start
+    uint32_t first = ch;                                   // the run's first child of this key and instance
+    for (long long b = s; b < j; b += 64) {
+      const long long x = b + lane;
+      uint32_t o = 0;
+      bool hit = false;
+      if (x < j) {
+        o = a.v32[x];
+        hit = a.keys[o] == key && (a.inst ? a.inst[parent(o)] : 0u) == inst;
+      }
+      const uint64_t m = __ballot(hit);
+      if (m) { first = (uint32_t)__shfl((int)o, __ffsll((long long)m) - 1, 64); break; }
+    }
+    first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+    if (first == ch) continue;
+    n_cmp++;
+    const int qa = (int)(ch % G) + 1, qb = (int)(first % G) + 1;
+    const ChildRows A{a.mat + (size_t)pa * (P * P), a.R.anti[qa - 1], a.R.plus[qa - 1], qa};
+    const ChildRows B{a.mat + (size_t)parent(first) * (P * P), a.R.anti[qb - 1], a.R.plus[qb - 1], qb};
+    const uint64_t sa = bitonic64(child_col_key<P>(A, wl, lane), lane), sb = bitonic64(child_col_key<P>(B, wl, lane), lane);
+    bool equal = __ballot(((sa ^ sb) >> 6) != 0) == 0;
+    if (equal) {
+      const int ca = lane < P ? (int)(sa & 63) : 0, cb = lane < P ? (int)(sb & 63) : 0;
+      bool pos = true, neg = true;                         // this lane's pair is equal, equal up to the sign -1
+#pragma unroll 8
+      for (int r = 0; r < P; r++) {
+        const uint32_t x = child_entry(A, r, A.src[r * P + ca], A.src[(r ^ qa) * P + ca]);
+        const uint32_t y = child_entry(B, r, B.src[r * P + cb], B.src[(r ^ qb) * P + cb]);
+        pos &= x == y;
+        neg &= x == (y ? MP - y : 0u);
+      }
+      equal = __ballot(!pos && !neg) == 0;
+    }
+    if (equal) {
+      n_dup++;
+      if (lane == 0) { a.keep[ch] = 0; a.link[ch] = first; }
+    } else if (lane == 0) {
+      a.runs[atomicAdd(a.nruns, 1ull)] = (uint32_t)s;
+    }
+  }
+  if (lane == 0 && n_vis) {
+    atomicAdd(&a.stat[0], (unsigned long long)n_run);
+    atomicAdd(&a.stat[1], (unsigned long long)n_vis);
+    atomicAdd(&a.stat[2], (unsigned long long)n_cmp);
+    atomicAdd(&a.stat[3], (unsigned long long)n_dup);
+  }
+}
+
 struct MatArgs {
   Rot R;
   Forest F;                    // holds level t (par, rot) and a materialised level below it
@@ -955,9 +1116,9 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
 
   // duplicates by commutation, from the growth before
   c->link.need(nc);
-  c->cnt.need(4);
+  c->cnt.need(6);                             // runs, visited, compared, duplicates; run members; runs left open
   hipLaunchKernelGGL(k_iota_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, c->link.p, nc);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, c->cnt.p, 4ll, 0ull);
+  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, c->cnt.p, 6ll, 0ull);
   const bool marks = L.cmap != nullptr && np > 0;
   long long nu = nc;                          // children not marked
   if (marks) {
@@ -998,12 +1159,22 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
 
   c->ev.begin(F_DEDUPE, c->stream);
   c->runs.need(nu);
-  hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p, nu,
-                     c->runs.p, c->cnt.p, nullptr);
+  if (F.mat[t]) {
+    // each member of a run against the first child of its key; the runs this leaves open go to k_dedupe.  The
+    // sort's second buffers are free here.
+    hipLaunchKernelGGL(k_run_members, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p,
+                       nu, c->sk[1].p, c->cnt.p + 4);
+    PairArgs pa{R, F.mat[t], L.inst[t], plist, c->sk[0].p, c->sv[0].p, nu, c->sk[1].p, c->cnt.p + 4, c->ckeys.p,
+                c->keep.p, c->link.p, c->runs.p, c->cnt.p + 5, c->cnt.p};
+    hipLaunchKernelGGL(k_pairs<NQ>, dim3(grid1(nu / 4 + 1, 4096)), dim3(256), 0, c->stream, pa);
+  } else {
+    hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p,
+                       nu, c->runs.p, c->cnt.p, nullptr);
+  }
   // blocks read the number of runs on the device
-  DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nu, c->runs.p, c->cnt.p, c->ckeys.p, c->keep.p, c->link.p,
+  DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nu, c->runs.p, c->cnt.p + (F.mat[t] ? 5 : 0), c->ckeys.p, c->keep.p, c->link.p,
                 c->flags.p, c->cnt.p + 1};
-  hipLaunchKernelGGL(k_dedupe<NQ>, dim3(grid1(nu / 2 + 1, 8192)), dim3(64), 0, c->stream, da);
+  hipLaunchKernelGGL(k_dedupe<NQ>, dim3(grid1(nu / 2 + 1, F.mat[t] ? 512 : 8192)), dim3(64), 0, c->stream, da);
   c->ev.end(c->stream);
 
   c->list.need(nc);
