@@ -16,8 +16,8 @@
 // [-sqrt2^e, sqrt2^e]; for e <= 28 that bounds the integer x + 2^16 y strictly inside (-p/2, p/2), where the
 // residue determines it, and |x| < 2^15 then determines (x, y).  Two nodes whose exponents are <= 28 are
 // therefore equal exactly when their residues are.  The host checks the exponent bound before a run.
-//  * keys: a column hashes to (sum_r R[r] v_r)^2 (the square removes the column sign); the coset key is a mixed
-//    sum over columns (removes the column order).  A child's column hash is a fixed linear form of its
+//  * keys: a column hashes to sum_r R[r] v_r or its negative, whichever residue is smaller (removes the column
+//    sign); the coset key mixes the sums of two functions of it over the columns (removes the column order).  A child's column hash is a fixed linear form of its
 //    parent's column (coefficients per rotation, precomputed), so all P-1 children of a parent come from one
 //    parent column held in registers.
 //  * equality (dedupe and table hits, src/tcount.cu:174-188): columns are sign-normalised (the residue of the
@@ -76,18 +76,25 @@ __host__ __device__ __forceinline__ uint64_t tmix(uint64_t x) {
   x ^= x >> 32; x *= 0xd6e8feb86659fd93ull;
   return x ^ (x >> 32);
 }
-__device__ __forceinline__ uint64_t col_term(uint32_t g) { return tmix((uint64_t)g + 0x9e3779b97f4a7c15ull); }
-__host__ __device__ __forceinline__ uint64_t coset_key(uint64_t s) { return tmix(s ^ 0x632be59bd9b4e019ull); }
+// A column's share of the two 32-bit sums that a coset's key is mixed from; g is the column's linear form in F_p,
+// known up to its sign.  32-bit products: a key takes 64 of these, and 64-bit ones need three products each.
+struct KeySum { uint32_t lo, hi; };
+__device__ __forceinline__ KeySum col_term(uint32_t g) {
+  uint32_t x = min(g, MP - g);                 // (g = 0: 0)
+  x ^= x >> 16; x *= 0x7feb352du;
+  x ^= x >> 15;
+  uint32_t y = (x ^ 0x5bd1e995u) * 0x2c1b3c6du;
+  x *= 0x846ca68bu;
+  return KeySum{x ^ (x >> 16), y ^ (y >> 12)};
+}
+__device__ __forceinline__ uint64_t coset_key(KeySum s) {
+  return tmix(((uint64_t)s.hi << 32 | s.lo) ^ 0x632be59bd9b4e019ull);
+}
 // sort prefix: keys of different instances land in different runs
 __host__ __device__ __forceinline__ uint32_t sort_prefix(uint64_t key, uint32_t inst) {
   return (uint32_t)((key ^ ((uint64_t)inst * 0x9e3779b97f4a7c15ull)) >> 32);
 }
 
-__device__ __forceinline__ uint64_t wsum64(uint64_t v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
-  return v;
-}
 // rotation tables and hash coefficients on the device
 struct Rot {
   const uint64_t *anti;      // (P-1): bit a set when row a anticommutes with P_p (its partner is row a ^ p)
@@ -95,6 +102,7 @@ struct Rot {
   const uint32_t *coef;      // (P-1) x P: child column hash = sum_r coef[p][r] v_r over the parent's column
   const uint32_t *rv;        // P: column hash = sum_r rv[r] v_r
   const uint32_t *rw;        // P: second weights of the column hash used to pair columns
+  const uint32_t *limbs;     // n = 3: coef as the matrix cores' operand (k_keys_mfma)
 };
 
 // nodes of every level: level 0 node i is root i; a node at level t >= 1 is (par, rot)
@@ -259,8 +267,9 @@ template <int NQ> __global__ __launch_bounds__(64) void k_root_keys(RootKeyArgs 
         lo += (uint64_t)(k & 0xffffu) * v;
         hi += (uint64_t)(k >> 16) * v;
       }
-    const uint32_t h = m31_fold(lo, hi);
-    const uint64_t s = wsum64(lane < P ? col_term(m31_red((uint64_t)h * h)) : 0ull);
+    KeySum s = lane < P ? col_term(m31_fold(lo, hi)) : KeySum{0u, 0u};
+    s.lo = gsum<64>(s.lo);
+    s.hi = gsum<64>(s.hi);
     if (lane == 0) a.keys[i] = coset_key(s);
   }
 }
@@ -278,6 +287,20 @@ struct KeysArgs {
   const unsigned long long *off;   // per parent, the unmarked children of the parents before it (with mask)
 };
 
+// child `lane` + 1 of parent k: its keep flag and, unmarked, its key, sort prefix and place in the sort's input
+template <int G>
+__device__ __forceinline__ void put_key(const KeysArgs &a, long long k, int lane, uint64_t mask, uint32_t inst, KeySum s) {
+  const long long ch = k * G + lane;
+  const bool mk = (mask >> lane) & 1;
+  a.keep[ch] = mk ? 0 : 1;
+  if (mk) return;
+  const uint64_t key = coset_key(s);
+  const long long x = a.mask ? (long long)a.off[k] + lane - __popcll(mask & ((1ull << lane) - 1)) : ch;
+  a.keys[ch] = key;
+  a.k32[x] = sort_prefix(key, inst);
+  a.v32[x] = (uint32_t)ch;
+}
+
 // every child's coset key (src/tcount.cu:197-207): one wave per parent, the parent's F_p column in registers,
 // each child column hash a linear form of it
 template <int NQ> __global__ __launch_bounds__(64) void k_keys(KeysArgs a) {
@@ -294,7 +317,7 @@ template <int NQ> __global__ __launch_bounds__(64) void k_keys(KeysArgs a) {
     uint32_t v[P];
 #pragma unroll
     for (int r = 0; r < P; r++) v[r] = lane < P ? src[r * P + lane] : 0u;
-    uint64_t mine = 0;
+    KeySum mine{0u, 0u};
     const uint64_t mask = a.mask ? a.mask[k] : 0ull;
     for (int p = 1; p <= G; p++) {
       if ((mask >> (p - 1)) & 1) continue;       // a marked duplicate's key is never read
@@ -306,22 +329,106 @@ template <int NQ> __global__ __launch_bounds__(64) void k_keys(KeysArgs a) {
         lo += (uint64_t)(c & 0xffffu) * v[r];
         hi += (uint64_t)(c >> 16) * v[r];
       }
-      const uint32_t h = m31_fold(lo, hi);
-      const uint64_t s = wsum64(lane < P ? col_term(m31_red((uint64_t)h * h)) : 0ull);
+      KeySum s = lane < P ? col_term(m31_fold(lo, hi)) : KeySum{0u, 0u};
+      s.lo = gsum<64>(s.lo);
+      s.hi = gsum<64>(s.hi);
       if (lane == p - 1) mine = s;
     }
-    if (lane < G) {
-      const long long ch = k * G + lane;
-      const bool mk = (mask >> lane) & 1;
-      a.keep[ch] = mk ? 0 : 1;
-      if (!mk) {
-        const uint64_t key = coset_key(mine);
-        const long long x = a.mask ? (long long)a.off[k] + lane - __popcll(mask & ((1ull << lane) - 1)) : ch;
-        a.keys[ch] = key;
-        a.k32[x] = sort_prefix(key, inst);
-        a.v32[x] = (uint32_t)ch;
+    if (lane < G) put_key<G>(a, k, lane, mask, inst, mine);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// The same keys for n = 3 and materialised parents, on the matrix cores.  The column hashes of all children of a parent
+// are one product H = C V in F_p, C the 63 x 64 rotation coefficients (row 63 zero) and V the parent's 64 x 64 residues.
+// Both factors are split into four bytes (C, centred, into signed digits on the host; V's unsigned bytes b taken as b -
+// 128, whose constant share of a row of H is added back), so H is 16 integer products of bytes, summed exactly in 32
+// bits by weight 2^(8w): per accumulator at most four products of 64 terms below 2^14, and 2^31 = 1 in F_p folds the
+// seven weights into one residue.
+//  * columns may come in any order (the key sums over them): lane l & 15 takes columns 4 (l & 15) + 0..3, one 16-byte
+//    load per row, and the 64 dwords of its 16 rows become the four column tiles' byte operands by 4 x 4 transposes;
+//  * C's operand (16 KB) sits in LDS, one copy for the block's four waves.
+// On the vector unit a key took 128 64-bit multiply-adds per lane at a quarter of the rate, which bound k_keys: 6.7 ms
+// for the 129,087 parents of the 3-qubit table's fourth level.  256 MFMAs of 16 x 16 x 64 per parent replace them:
+// 0.87 ms, of which the parents' 2.1 GB take 0.45 at the rate of a large copy.  Two waves per SIMD hold the operands
+// without spilling (206 registers); one wave per SIMD took 1.24 ms.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+constexpr int CL_WORDS = 4 * 4 * 64 * 4 + 64;      // C's digits by row tile, digit and lane (16 bytes each), constants
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_keys_mfma(KeysArgs a) {
+  constexpr int P = 64, G = 63;
+  __shared__ __align__(16) uint32_t cl[CL_WORDS];
+  __shared__ KeySum sums[4][P];
+  for (int i = threadIdx.x; i < CL_WORDS / 4; i += 256) ((uint4 *)cl)[i] = ((const uint4 *)a.R.limbs)[i];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, kg = lane >> 4;
+  const uint32_t *const mat = a.F.mat[a.t];
+  for (long long k = wave_index(); k < a.np; k += (long long)gridDim.x * 4) {
+    const uint32_t node = a.plist ? a.plist[k] : (uint32_t)k;
+    const uint4 *src = (const uint4 *)(mat + (size_t)node * (P * P)) + kg * 16 * (P / 4) + (lane & 15);
+    uint4 v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = src[r * (P / 4)];
+    i32x4 bt[4][4];                                // column tile, byte
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) {
+        auto at = [&](int i) { return ct == 0 ? v[r + i].x : ct == 1 ? v[r + i].y : ct == 2 ? v[r + i].z : v[r + i].w; };
+        const uint32_t l01 = __builtin_amdgcn_perm(at(1), at(0), 0x05010400u), h01 = __builtin_amdgcn_perm(at(1), at(0), 0x07030602u);
+        const uint32_t l23 = __builtin_amdgcn_perm(at(3), at(2), 0x05010400u), h23 = __builtin_amdgcn_perm(at(3), at(2), 0x07030602u);
+        bt[ct][0][r / 4] = (int)(__builtin_amdgcn_perm(l23, l01, 0x05040100u) ^ 0x80808080u);
+        bt[ct][1][r / 4] = (int)(__builtin_amdgcn_perm(l23, l01, 0x07060302u) ^ 0x80808080u);
+        bt[ct][2][r / 4] = (int)(__builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u);
+        bt[ct][3][r / 4] = (int)(__builtin_amdgcn_perm(h23, h01, 0x07060302u) ^ 0x80808080u);
+      }
+#pragma unroll 1
+    for (int rt = 0; rt < 4; rt++) {
+      i32x4 ca[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) ca[i] = ((const i32x4 *)cl)[(rt * 4 + i) * 64 + lane];
+      const uint4 cst = ((const uint4 *)(cl + 4 * 4 * 64 * 4))[rt * 4 + kg];
+      KeySum s[4] = {};
+#pragma unroll
+      for (int ct = 0; ct < 4; ct++) {
+        i32x4 acc[7] = {};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[i], bt[ct][j], acc[i + j], 0, 0, 0);
+        // lane: column lane & 15 of the tile, rows 4 kg + e
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int x0 = acc[0][e] + (acc[1][e] << 8), x1 = acc[2][e] + (acc[3][e] << 8),
+                    x2 = acc[4][e] + (acc[5][e] << 8), x3 = acc[6][e];
+          // x0 + 2^16 x1 + 2^32 x2 + 2^48 x3 with 2^32 = 2, below 2^48 in magnitude; 2^18 p makes it positive
+          const long long T = (long long)x0 + 2ll * x2 + 65536ll * (x1 + 2 * x3) + ((long long)MP << 18) +
+                              (long long)(e == 0 ? cst.x : e == 1 ? cst.y : e == 2 ? cst.z : cst.w);
+          const uint32_t y = ((uint32_t)T & MP) + (uint32_t)((uint64_t)T >> 31);
+          const KeySum t = col_term(min(y, y - MP));
+          s[e].lo += t.lo;
+          s[e].hi += t.hi;
+        }
+      }
+      // sums over the 16 lanes of a row group
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        uint32_t *const q[2] = {&s[e].lo, &s[e].hi};
+#pragma unroll
+        for (int z = 0; z < 2; z++) {
+          uint32_t x = *q[z];
+          x += dpp32<DPP_QXOR1>(x);
+          x += dpp32<DPP_QXOR2>(x);
+          x += dpp32<DPP_HALF_MIRROR>(x);
+          x += dpp32<DPP_MIRROR>(x);
+          *q[z] = x;
+        }
+        if ((lane & 15) == e) sums[w][rt * 16 + kg * 4 + e] = s[e];
       }
     }
+    __builtin_amdgcn_wave_barrier();
+    if (lane < G) put_key<G>(a, k, lane, a.mask ? a.mask[k] : 0ull, inst_of(a.F, a.t, node), sums[w][lane]);
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -1006,7 +1113,7 @@ struct chz_tc {
   hipStream_t stream = nullptr;
   tcn::Spec spec;                            // the spec the table was built with (its rotation tables)
   uint64_t *d_anti = nullptr, *d_plus = nullptr;
-  uint32_t *d_coef = nullptr, *d_rv = nullptr, *d_rw = nullptr;
+  uint32_t *d_coef = nullptr, *d_rv = nullptr, *d_rw = nullptr, *d_limbs = nullptr;
   // table forest: one root, the identity
   tcn::Levels tab;
   uint32_t *d_troot_fp = nullptr;
@@ -1031,7 +1138,7 @@ struct chz_tc {
 
 namespace tcn {
 
-static Rot rot_of(const chz_tc *c) { return Rot{c->d_anti, c->d_plus, c->d_coef, c->d_rv, c->d_rw}; }
+static Rot rot_of(const chz_tc *c) { return Rot{c->d_anti, c->d_plus, c->d_coef, c->d_rv, c->d_rw, c->d_limbs}; }
 
 static Forest forest_of(const Levels &L) {
   Forest F{};
@@ -1148,7 +1255,10 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
   c->ev.begin(F_KEYS, c->stream);
   KeysArgs ka{R, F, t, plist, np, c->ckeys.p, c->sk[0].p, c->sv[0].p, c->keep.p, marks ? c->mask.p : nullptr,
               marks ? c->moff.p : nullptr};
-  hipLaunchKernelGGL(k_keys<NQ>, dim3(grid1(np)), dim3(64), 0, c->stream, ka);
+  if (NQ == 3 && F.mat[t])
+    hipLaunchKernelGGL(k_keys_mfma, dim3(grid1((np + 3) / 4, 2048)), dim3(256), 0, c->stream, ka);
+  else
+    hipLaunchKernelGGL(k_keys<NQ>, dim3(grid1(np)), dim3(64), 0, c->stream, ka);
   c->ev.end(c->stream);
   c->k_work[F_KEYS] += (double)nu * P * 2;
 
@@ -1312,6 +1422,28 @@ static void upload_rotations(chz_tc *c) {
         coef[p * P + a] = m31_rot(sb > 0 ? m31_sub(rv[a], rv[b]) : m31_add(rv[a], rv[b]), 15);
       }
     }
+  // coef as the operand of k_keys_mfma: row m = 16 rt + (l & 15), columns 16 (l >> 4) + 0..15, digit i of the centred
+  // coefficient per byte; then per row the share of V's 128s: 128 (1 + 2^8 + 2^16 + 2^24) sum_r coef[m][r]
+  if (P == 64) {
+    std::vector<uint32_t> lw(CL_WORDS, 0);
+    int8_t *b = (int8_t *)lw.data();
+    for (int m = 0; m < G; m++) {
+      uint32_t tot = 0;
+      for (int r = 0; r < P; r++) {
+        const uint32_t cf = coef[m * P + r];
+        tot = m31_add(tot, cf);
+        int64_t u = cf > HALF ? (int64_t)cf - MP : (int64_t)cf;
+        for (int i = 0; i < 4; i++) {
+          const int d = (int)(((u + 128) & 255) - 128);
+          u = (u - d) >> 8;
+          b[(((m / 16) * 4 + i) * 64 + (r / 16) * 16 + m % 16) * 16 + r % 16] = (int8_t)d;
+        }
+      }
+      lw[4 * 4 * 64 * 4 + m] = m31_red((uint64_t)tot * 0x80808080ull);
+    }
+    c->d_limbs = dalloc<uint32_t>(CL_WORDS);
+    chz::copy_sync(c->d_limbs, lw.data(), CL_WORDS * 4, hipMemcpyHostToDevice, c->stream);
+  }
   c->d_anti = dalloc<uint64_t>(G);
   c->d_plus = dalloc<uint64_t>(G);
   c->d_coef = dalloc<uint32_t>(G * P);
@@ -1702,7 +1834,7 @@ void chz_tc_free(chz_tc *c) {
   chz::StreamScope scope(c->stream);
   (void)chz::sync_owner();           // cached device blocks must be idle before they are reused
   c->tab.release();
-  void *ps[] = {c->d_anti, c->d_plus, c->d_coef, c->d_rv, c->d_rw, c->d_troot_fp, c->d_hkey, c->d_hval};
+  void *ps[] = {c->d_anti, c->d_plus, c->d_coef, c->d_rv, c->d_rw, c->d_limbs, c->d_troot_fp, c->d_hkey, c->d_hval};
   for (void *p : ps) chz::dev_free(p);
   c->ckeys.release();
   for (int i = 0; i < 2; i++) { c->sk[i].release(); c->sv[i].release(); }
