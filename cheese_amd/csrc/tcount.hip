@@ -614,35 +614,36 @@ __global__ __launch_bounds__(256) void k_run_members(const uint32_t *k, long lon
   }
 }
 
-// entry of the child (parent matrix src, rotation p) in row a of column c: rows that commute with P_p are the parent's
-struct ChildRows {
-  const uint32_t *src;
-  uint64_t anti, plus;
-  int p;
-};
-__device__ __forceinline__ uint32_t child_entry(const ChildRows &A, int a, uint32_t x, uint32_t y) {   // x, y: rows a, a ^ p
-  const uint32_t f = m31_rot(((A.plus >> a) & 1) ? m31_sub(x, y) : m31_add(x, y), 15);
-  return ((A.anti >> a) & 1) ? f : x;
-}
 __device__ __forceinline__ int m31_signed(uint32_t v) { return (int)(v > HALF ? v - MP : v); }
 
-// sort key of column `lane` of the child: a 58-bit hash that the column's sign does not change (a linear form of the
-// signed entries in 64 bits, or its negative) above the lane.  wl: lane r's weight of row r.  (Entries are multiples
-// of high powers of two, so a 32-bit form would keep few bits of the weights.)
+// rotation p peeled off M (LDS) in place as fp_peel does, and the sort key of column `lane` of the result: a 58-bit hash
+// that the column's sign does not change (a linear form of the signed entries in 64 bits, or its negative) above the
+// lane.  wl: lane r's weight of row r.  (Entries are multiples of high powers of two, so a 32-bit form would keep few
+// bits of the weights.)
 template <int P>
-__device__ __forceinline__ uint64_t child_col_key(const ChildRows &A, uint32_t wl, int lane) {
-  const int h = 31 - __clz(A.p), lowm = (1 << h) - 1, c = lane < P ? lane : 0;
+__device__ __forceinline__ uint64_t peel_col_key(uint32_t *M, const Rot &R, int p, uint32_t wl, int lane) {
+  const uint64_t anti = R.anti[p - 1], plus = R.plus[p - 1];
+  const int h = 31 - __clz(p), lowm = (1 << h) - 1, c = lane < P ? lane : 0;
   long long sum = 0;
 #pragma unroll 8
   for (int j = 0; j < P / 2; j++) {
-    const int a = ((j >> h) << (h + 1)) | (j & lowm), r = a ^ A.p;
-    const uint32_t x = A.src[a * P + c], y = A.src[r * P + c];
-    sum += (long long)__builtin_amdgcn_readlane((int)wl, a) * m31_signed(child_entry(A, a, x, y)) +
-           (long long)__builtin_amdgcn_readlane((int)wl, r) * m31_signed(child_entry(A, r, y, x));
+    const int a = ((j >> h) << (h + 1)) | (j & lowm), r = a ^ p;
+    uint32_t x = M[a * P + c], y = M[r * P + c];
+    if ((anti >> a) & 1) {
+      const uint32_t u = m31_rot(((plus >> a) & 1) ? m31_sub(x, y) : m31_add(x, y), 15);
+      y = m31_rot(((plus >> r) & 1) ? m31_sub(y, x) : m31_add(y, x), 15);
+      x = u;
+      if (lane < P) { M[a * P + c] = x; M[r * P + c] = y; }
+    }
+    sum += (long long)__builtin_amdgcn_readlane((int)wl, a) * m31_signed(x) +
+           (long long)__builtin_amdgcn_readlane((int)wl, r) * m31_signed(y);
   }
+  __builtin_amdgcn_wave_barrier();
   const uint64_t k = (uint64_t)(sum < 0 ? -sum : sum) * 0x9e3779b97f4a7c15ull;
   return lane < P ? (k & ~63ull) | (uint32_t)lane : ~0ull;
 }
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct PairArgs {
   Rot R;
@@ -667,17 +668,20 @@ struct PairArgs {
 // because its coset differs or its columns were paired wrongly (two with one hash), sends its run to k_dedupe, which
 // compares every member with every distinct coset of the run.
 // What bounded this work: k_dedupe walks a run's members one after another with two 16 KB matrices in LDS, which
-// leaves 5 waves to a CU.  Here a member is a wave of its own and the two children are formed row by row from their
-// parents, once for the columns' hashes and once, in paired order, for the comparison.  The 3-qubit table's
-// fourth level (219 thousand comparisons): 12.0 ms in k_dedupe, 4.4 ms here; no run is left open.
-template <int NQ> __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
-  constexpr int P = 1 << (2 * NQ), G = P - 1;
-  const int lane = threadIdx.x & 63;
+// leaves 5 waves to a CU.  Here a member is a wave of its own, both parents are read at once, and one LDS matrix serves
+// first the member, whose columns then move to registers, and then the other child (10 waves to a CU).  Forming the
+// children row by row from global memory instead, without LDS, reads every row several times from beyond the L2.
+// The 3-qubit table's fourth level (219 thousand comparisons): 12.0 ms in k_dedupe, 4.5 row by row, 2.2 here; no run is
+// left open.
+template <int NQ> __global__ __launch_bounds__(64) void k_pairs(PairArgs a) {
+  constexpr int P = 1 << (2 * NQ), G = P - 1, NV = P * P / 4, B = (NV + 63) / 64;
+  __shared__ __align__(16) uint32_t M[P * P];
+  const int lane = threadIdx.x;
   const long long nm = (long long)*a.nmem;
   const uint32_t wl = lane < P ? a.R.rv[lane] : 0u;
   uint32_t n_run = 0, n_vis = 0, n_cmp = 0, n_dup = 0;
   auto parent = [&](uint32_t ch) { return a.plist ? a.plist[ch / G] : ch / G; };
-  for (long long it = wave_index(); it < nm; it += (long long)gridDim.x * (blockDim.x >> 6)) {
+  for (long long it = blockIdx.x; it < nm; it += gridDim.x) {
     const long long j = a.members[it];
     const uint32_t kp = a.k32[j], ch = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.v32[j]);
     const uint64_t key = a.keys[ch];
@@ -708,23 +712,42 @@ template <int NQ> __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
     first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
     if (first == ch) continue;
     n_cmp++;
-    const int qa = (int)(ch % G) + 1, qb = (int)(first % G) + 1;
-    const ChildRows A{a.mat + (size_t)pa * (P * P), a.R.anti[qa - 1], a.R.plus[qa - 1], qa};
-    const ChildRows B{a.mat + (size_t)parent(first) * (P * P), a.R.anti[qb - 1], a.R.plus[qb - 1], qb};
-    const uint64_t sa = bitonic64(child_col_key<P>(A, wl, lane), lane), sb = bitonic64(child_col_key<P>(B, wl, lane), lane);
+    const u32x4 *const ga = (const u32x4 *)(a.mat + (size_t)pa * (P * P));
+    const u32x4 *const gb = (const u32x4 *)(a.mat + (size_t)parent(first) * (P * P));
+    u32x4 *const M4 = (u32x4 *)M;
+    u32x4 t[B], u[B];                                      // both parents, each read once
+#pragma unroll
+    for (int i = 0; i < B; i++) t[i] = ga[NV < 64 ? lane & (NV - 1) : i * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < B; i++) u[i] = gb[NV < 64 ? lane & (NV - 1) : i * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < B; i++) if (NV >= 64 || lane < NV) M4[i * 64 + lane] = t[i];
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t sa = bitonic64(peel_col_key<P>(M, a.R, (int)(ch % G) + 1, wl, lane), lane);
+    uint32_t v[P];                                         // the member's column `lane`
+#pragma unroll
+    for (int r = 0; r < P; r++) v[r] = M[r * P + (lane < P ? lane : 0)];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < B; i++) if (NV >= 64 || lane < NV) M4[i * 64 + lane] = u[i];
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t sb = bitonic64(peel_col_key<P>(M, a.R, (int)(first % G) + 1, wl, lane), lane);
     bool equal = __ballot(((sa ^ sb) >> 6) != 0) == 0;
     if (equal) {
-      const int ca = lane < P ? (int)(sa & 63) : 0, cb = lane < P ? (int)(sb & 63) : 0;
+      // the column that pairs with this lane's: sorted position i pairs columns sa & 63 and sb & 63 (lanes without a
+      // column hold all-ones keys behind the others and pair with themselves)
+      const int to = lane < P ? (int)(sa & 63) : lane, cb = lane < P ? (int)(sb & 63) : lane;
+      const int mine = __builtin_amdgcn_ds_permute(to << 2, cb);
       bool pos = true, neg = true;                         // this lane's pair is equal, equal up to the sign -1
-#pragma unroll 8
+#pragma unroll
       for (int r = 0; r < P; r++) {
-        const uint32_t x = child_entry(A, r, A.src[r * P + ca], A.src[(r ^ qa) * P + ca]);
-        const uint32_t y = child_entry(B, r, B.src[r * P + cb], B.src[(r ^ qb) * P + cb]);
-        pos &= x == y;
-        neg &= x == (y ? MP - y : 0u);
+        const uint32_t y = M[r * P + (mine & (P - 1))];
+        pos &= v[r] == y;
+        neg &= v[r] == (y ? MP - y : 0u);
       }
-      equal = __ballot(!pos && !neg) == 0;
+      equal = __ballot(lane < P && !pos && !neg) == 0;
     }
+    __builtin_amdgcn_wave_barrier();
     if (equal) {
       n_dup++;
       if (lane == 0) { a.keep[ch] = 0; a.link[ch] = first; }
@@ -1276,7 +1299,7 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
                        nu, c->sk[1].p, c->cnt.p + 4);
     PairArgs pa{R, F.mat[t], L.inst[t], plist, c->sk[0].p, c->sv[0].p, nu, c->sk[1].p, c->cnt.p + 4, c->ckeys.p,
                 c->keep.p, c->link.p, c->runs.p, c->cnt.p + 5, c->cnt.p};
-    hipLaunchKernelGGL(k_pairs<NQ>, dim3(grid1(nu / 4 + 1, 4096)), dim3(256), 0, c->stream, pa);
+    hipLaunchKernelGGL(k_pairs<NQ>, dim3(grid1(nu / 2 + 1, 16384)), dim3(64), 0, c->stream, pa);
   } else {
     hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p,
                        nu, c->runs.p, c->cnt.p, nullptr);
