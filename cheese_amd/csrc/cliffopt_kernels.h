@@ -66,20 +66,6 @@ __host__ __device__ inline uint64_t tinverse(uint64_t C, int n) {
   return D;
 }
 
-// distance of one tableau (scalar probe over the bucket layout), -1 when absent
-__device__ inline int find1(Table T, uint64_t key) {
-  uint64_t b = hmix(key) & T.bmask;
-  for (uint64_t guard = 0; guard <= T.bmask; guard++) {
-    for (int j = 0; j < 8; j++) {
-      const unsigned long long v = T.slot[b * 8 + j];
-      if (!v) return -1;
-      if ((v >> 8) == key) return (int)(v & 255);
-    }
-    b = (b + 1) & T.bmask;
-  }
-  return -1;
-}
-
 struct Cand { uint64_t K, Kinv; int qp, neg; };
 
 // element i (sorted order) is a placement for a T on qubit q: flag = q' + 1 where K Z_q' K^-1 = +-Z_q, else 0

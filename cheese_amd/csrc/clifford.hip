@@ -3,9 +3,12 @@
 // and optimal-word read-back.  Reference behaviour: src/clifford.cu:41-166 (tableaux, table, BFS),
 // :207-210 (batched find), :251-283 (BFS driver, group-order check), :344-372 (read-back).
 //
-// Table layout: 2^lg 64-bit slots, slot = tableau << 8 | distance, 0 = empty (no tableau is 0).  Slots are
-// grouped in buckets of 8 (one 64-byte sector); a group of 8 lanes probes a whole bucket per step, votes
-// for a match or an empty slot with a ballot, and claims the first empty slot with a 64-bit CAS.
+// Table layout.  A tableau is a symplectic matrix and a sign per row; a gate changes the matrix independently of the
+// signs and XORs the signs with a vector that depends on the matrix alone.  So the group is (symplectic matrices) x (sign
+// vectors): 1,451,520 x 64 at 3 qubits.  The matrices are numbered (in the order of their tableaux, by unranking), a
+// hash table of 2^22 8-byte slots maps a matrix to its number, and the distances of its 64 sign vectors are four 64-bit
+// planes, bit s of plane k being bit k of the distance of sign vector s (distances are at most 13).  78 MB instead of
+// 1.07 GB for a hash table of whole tableaux, which the 256 MB last-level cache holds.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -87,85 +90,241 @@ __host__ __device__ inline uint64_t hmix(uint64_t x) {
   return x ^ (x >> 33);
 }
 
+// bits 2n of every row: the signs
+__host__ __device__ inline uint64_t sign_mask(int n) {
+  uint64_t m = 0;
+  for (int i = 0; i < 2 * n; i++) m |= 1ull << (i * (2 * n + 1) + 2 * n);
+  return m;
+}
+// the rows' signs, row i in bit i
+__host__ __device__ inline uint32_t signs_of(uint64_t T, int n) {
+  uint32_t s = 0;
+  for (int i = 0; i < 2 * n; i++) s |= (uint32_t)((T >> (i * (2 * n + 1) + 2 * n)) & 1) << i;
+  return s;
+}
+
+constexpr int IDX_BITS = 21;       // matrix numbers; tableaux have at most 42 bits
+
 struct Table {
-  unsigned long long *slot;
-  uint64_t bmask;                  // buckets - 1
+  unsigned long long *slot;        // tableau without signs << 21 | number; 0 = empty (no tableau is 0)
+  uint32_t smask;                  // slots - 1
+  const ulonglong2 *planes;        // two per matrix: planes 0, 1 and 2, 3
+  int n;
 };
 
-// group of 8 lanes (l8 = lane & 7) probes for key; insert: claim an empty slot with distance d.
-// Returns the stored distance (>= 0), or -1 when absent (find) / -2 when this call inserted it.
-template <bool INSERT> __device__ inline int probe8(Table T, uint64_t key, int d, int l8) {
-  const int shift = __lane_id() & ~7;
-  uint64_t b = hmix(key) & T.bmask;
-  const unsigned long long want = (unsigned long long)((key << 8) | (uint64_t)d);
-  while (true) {
-    // while the table is being filled other CUs write it: read through to the coherent level so that a
-    // failed claim is never followed by the same stale view of the bucket
-    unsigned long long v = INSERT ? __hip_atomic_load(&T.slot[b * 8 + l8], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                  : T.slot[b * 8 + l8];
-    const uint64_t hit = (__ballot((v >> 8) == key && v != 0) >> shift) & 0xff;
-    if (hit) return (int)(__shfl(v, shift + __ffsll((long long)hit) - 1, 64) & 255);
-    uint64_t emp = (__ballot(v == 0) >> shift) & 0xff;
-    if (!emp) { b = (b + 1) & T.bmask; continue; }
-    if (!INSERT) return -1;
-    // the lowest empty slot: its lane tries to claim it, the group learns the outcome
-    const int e = __ffsll((long long)emp) - 1;
-    unsigned long long old = 0;
-    if (l8 == e) old = atomicCAS(&T.slot[b * 8 + e], 0ull, want);
-    old = __shfl(old, shift + e, 64);
-    if (old == 0) return -2;
-    if ((old >> 8) == key) return (int)(old & 255);
-    // another key took the slot: probe the same bucket again
+// number of the symplectic matrix with this sign-free tableau, -1 when it is none
+__device__ inline int find_sym(const Table &T, uint64_t key) {
+  for (uint32_t b = (uint32_t)hmix(key) & T.smask;; b = (b + 1) & T.smask) {
+    const unsigned long long v = T.slot[b];
+    if (!v) return -1;
+    if (v >> IDX_BITS == key) return (int)(v & ((1u << IDX_BITS) - 1));
   }
+}
+__device__ inline int plane_dist(ulonglong2 p, ulonglong2 q, uint32_t s) {
+  return (int)(((p.x >> s) & 1) | ((p.y >> s) & 1) << 1 | ((q.x >> s) & 1) << 2 | ((q.y >> s) & 1) << 3);
+}
+// distance of a tableau, -1 when it is none
+__device__ inline int find1(const Table &T, uint64_t key) {
+  const int i = find_sym(T, key & ~sign_mask(T.n));
+  return i < 0 ? -1 : plane_dist(T.planes[2 * i], T.planes[2 * i + 1], signs_of(key, T.n));
+}
+
+// ---- numbering.  A tableau's rows are chosen from the last to the first (the most significant first): row 2n - 1 any
+// nonzero vector, each further Z image a vector that commutes with those before it and is independent of them, each X
+// image a vector that anticommutes with its Z image and commutes with the other rows.  However the rows before it were
+// chosen, a row has the same number of choices (63, 30, 12, 8, 4, 2 at 3 qubits), so a mixed-radix number with a row's
+// choice, in increasing order of its vector, as digit lists the matrices in the order of their tableaux.  With the
+// row's sign above its choice in every digit the number lists all tableaux in order.
+template <int NQ> struct Num {
+  static constexpr int M = 2 * NQ;
+  static constexpr uint64_t FULL = M == 6 ? ~0ull : (1ull << (1 << M)) - 1;     // all vectors
+  // choices of the k-th row chosen (row M - 1 - k)
+  __host__ __device__ static constexpr uint32_t choices(int k) { return k < NQ ? (1u << (M - k)) - (1u << k) : 1u << (M - k); }
+  __host__ __device__ static constexpr long long matrices() {
+    long long t = 1;
+    for (int k = 0; k < M; k++) t *= choices(k);
+    return t;
+  }
+  static constexpr long long ORDER = matrices() << M;
+  // vectors (as bits of a mask) that anticommute with v
+  __host__ __device__ static uint64_t anti(uint32_t v) {
+    constexpr uint64_t B[6] = {0xaaaaaaaaaaaaaaaaull, 0xccccccccccccccccull, 0xf0f0f0f0f0f0f0f0ull,
+                               0xff00ff00ff00ff00ull, 0xffff0000ffff0000ull, 0xffffffff00000000ull};
+    uint64_t m = 0;
+#pragma unroll
+    for (int i = 0; i < M; i++)
+      if ((v >> ((i + NQ) % M)) & 1) m ^= B[i];
+    return m & FULL;
+  }
+  // the mask with bit v ^ d in place of bit v
+  __host__ __device__ static uint64_t shift(uint64_t m, uint32_t d) {
+    constexpr uint64_t L[6] = {0x5555555555555555ull, 0x3333333333333333ull, 0x0f0f0f0f0f0f0f0full,
+                               0x00ff00ff00ff00ffull, 0x0000ffff0000ffffull, 0x00000000ffffffffull};
+#pragma unroll
+    for (int i = 0; i < M; i++)
+      if ((d >> i) & 1) m = ((m >> (1 << i)) & L[i]) | ((m & L[i]) << (1 << i));
+    return m;
+  }
+  // the tableau whose k-th chosen row is choice r[k], row i signed by bit i of s
+  __host__ __device__ static uint64_t tableau(const uint32_t (&r)[M], uint32_t s) {
+    uint64_t an[M], span = 1, T = 0;
+#pragma unroll
+    for (int k = 0; k < M; k++) {
+      const int row = M - 1 - k;
+      uint64_t m = FULL;
+#pragma unroll
+      for (int j = 0; j < k; j++) m &= (M - 1 - j) == row + NQ ? an[j] : ~an[j];
+      if (k < NQ) m &= ~span;
+      for (uint32_t c = r[k]; c; c--) m &= m - 1;
+#ifdef __HIP_DEVICE_COMPILE__
+      const uint32_t v = (uint32_t)__ffsll((long long)m) - 1;
+#else
+      const uint32_t v = (uint32_t)__builtin_ctzll(m);
+#endif
+      an[k] = anti(v);
+      if (k < NQ) span |= shift(span, v);
+      T |= (uint64_t)(v | ((s >> row) & 1) << M) << (row * (M + 1));
+    }
+    return T;
+  }
+  // the i-th matrix's tableau, without signs
+  __host__ __device__ static uint64_t matrix(uint32_t i) {
+    uint32_t r[M];
+#pragma unroll
+    for (int k = M - 1; k >= 0; k--) { r[k] = i % choices(k); i /= choices(k); }
+    return tableau(r, 0);
+  }
+  // the i-th tableau
+  __host__ __device__ static uint64_t element(uint64_t i) {
+    uint32_t r[M], s = 0;
+#pragma unroll
+    for (int k = M - 1; k >= 0; k--) {
+      const uint32_t d = (uint32_t)(i % (2 * choices(k)));
+      i /= 2 * choices(k);
+      r[k] = d % choices(k);
+      s |= (d / choices(k)) << (M - 1 - k);
+    }
+    return tableau(r, s);
+  }
+};
+
+// ---- building the table.  Gates that change the matrix: H, S (Sdg with it) on each qubit, CX on each ordered pair.
+__host__ __device__ constexpr int sym_gates(int n) { return 2 * n + n * (n - 1); }
+
+template <int NQ> __global__ __launch_bounds__(256) void k_matrices(uint64_t *key, unsigned long long *slot, uint32_t smask) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= (uint32_t)Num<NQ>::matrices()) return;
+  const uint64_t T = Num<NQ>::matrix(i);
+  key[i] = T;
+  const unsigned long long v = (unsigned long long)T << IDX_BITS | i;
+  for (uint32_t b = (uint32_t)hmix(T) & smask;; b = (b + 1) & smask)
+    if (atomicCAS(&slot[b], 0ull, v) == 0ull) break;
+}
+
+// nb[g * count + i]: the matrix that matrix-changing gate g takes matrix i to (and from: each is its own inverse on the
+// matrices)
+template <int NQ> __global__ __launch_bounds__(256) void k_neighbours(Table T, const uint64_t *key, uint32_t *nb) {
+  constexpr uint32_t C = (uint32_t)Num<NQ>::matrices();
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= C) return;
+  const uint64_t t = key[i], sm = sign_mask(NQ);
+  int g = 0;
+#pragma unroll
+  for (int q = 0; q < NQ; q++)
+#pragma unroll
+    for (int k = 0; k < 2; k++, g++) nb[(size_t)g * C + i] = (uint32_t)find_sym(T, apply(t, NQ, k, q, 0) & ~sm);
+#pragma unroll
+  for (int x = 0; x < NQ; x++)
+#pragma unroll
+    for (int y = 0; y < NQ; y++)
+      if (x != y) { nb[(size_t)g * C + i] = (uint32_t)find_sym(T, apply(t, NQ, 5, x, y) & ~sm); g++; }
 }
 
 struct BfsArgs {
-  Gates G;
-  Table T;
-  const uint64_t *front;
-  long long nf;
-  uint64_t *next;
-  unsigned long long *cnt;          // [0] new elements, [1] capacity overflow
-  long long cap;
+  const uint64_t *key;
+  const uint32_t *nb;
+  const uint64_t *front;       // per matrix, the sign vectors at distance d - 1
+  uint64_t *next;              // those at distance d
+  uint64_t *seen;
+  ulonglong2 *planes;
+  unsigned long long *cnt;     // elements per distance
   int d;
 };
 
-constexpr int STAGE = 2048;
-
-// one BFS level: every (frontier element, gate) pair, 8 lanes per candidate; new tableaux are staged in LDS
-// and written out with one reservation per block
-__global__ __launch_bounds__(256) void k_bfs(BfsArgs a) {
-  __shared__ uint64_t buf[STAGE];
-  __shared__ unsigned int nbuf;
-  __shared__ unsigned long long base;
-  if (threadIdx.x == 0) nbuf = 0;
-  __syncthreads();
-  const int l8 = threadIdx.x & 7;
-  const long long total = a.nf * a.G.ng;
-  const long long groups = (long long)gridDim.x * (blockDim.x / 8);
-  const long long g0 = (long long)blockIdx.x * (blockDim.x / 8) + (threadIdx.x >> 3);
-  for (long long r0 = 0; r0 < total; r0 += groups) {
-    const long long c = r0 + g0;
-    if (c < total) {
-      const long long i = c / a.G.ng;
-      const int g = (int)(c % a.G.ng);
-      const uint64_t t = apply(a.front[i], a.G.n, a.G.k[g], a.G.a[g], a.G.b[g]);
-      if (probe8<true>(a.T, t, a.d, l8) == -2 && l8 == 0) buf[atomicAdd(&nbuf, 1u)] = t;
+// One level of the search, one thread per matrix: the sign vectors at distance d are those that a gate brings from a
+// matrix's sign vectors at distance d - 1, a set of 2^(2n) bits XOR-shifted by the gate's sign vector, less those seen
+// before.  Each (element, gate) pair is one bit of a 64-bit operation and each (matrix, gate) pair one gather from an
+// 11.6 MB array, where a hash table of whole tableaux took a probe of a random 128-byte line per pair: the 3-qubit
+// group (1.95 billion pairs) took 164 ms, all its levels here 0.84, numbering and neighbours 0.4 more.
+template <int NQ> __global__ __launch_bounds__(256) void k_bfs(BfsArgs a) {
+  constexpr uint32_t C = (uint32_t)Num<NQ>::matrices();
+  constexpr int M = 2 * NQ, RB = M + 1;
+  if (!a.cnt[a.d - 1]) return;                       // the level before is empty
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  uint64_t acc = 0, nx = 0;
+  if (i < C) {
+    const uint64_t t = a.key[i];
+    // column c of the matrix (x_0.. then z_0..), row r in bit r
+    uint32_t col[M];
+#pragma unroll
+    for (int c = 0; c < M; c++) {
+      col[c] = 0;
+#pragma unroll
+      for (int r = 0; r < M; r++) col[c] |= (uint32_t)((t >> (r * RB + c)) & 1) << r;
     }
-    __syncthreads();
-    if (nbuf > STAGE - 256 / 8 || r0 + groups >= total) {
-      if (threadIdx.x == 0) base = atomicAdd(&a.cnt[0], (unsigned long long)nbuf);
-      __syncthreads();
-      for (unsigned int j = threadIdx.x; j < nbuf; j += blockDim.x) {
-        const unsigned long long p = base + j;
-        if ((long long)p < a.cap) a.next[p] = buf[j];
-        else a.cnt[1] = 1;
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) nbuf = 0;
-      __syncthreads();
+    const uint64_t own = a.front[i];
+    int g = 0;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const uint32_t x = col[q], z = col[NQ + q];
+      if (own) acc |= Num<NQ>::shift(own, z) | Num<NQ>::shift(own, x);                       // X, Z
+      const uint64_t h = a.front[a.nb[(size_t)g++ * C + i]];
+      if (h) acc |= Num<NQ>::shift(h, x & z);                                                // H
+      const uint64_t p = a.front[a.nb[(size_t)g++ * C + i]];
+      if (p) acc |= Num<NQ>::shift(p, x & ~z) | Num<NQ>::shift(p, x & z);                     // S, Sdg
+    }
+#pragma unroll
+    for (int x = 0; x < NQ; x++)
+#pragma unroll
+      for (int y = 0; y < NQ; y++)
+        if (x != y) {
+          const uint64_t f = a.front[a.nb[(size_t)g++ * C + i]];
+          if (f) acc |= Num<NQ>::shift(f, col[x] & col[NQ + y] & ~(col[y] ^ col[NQ + x]));    // CX x -> y
+        }
+    const uint64_t s = a.seen[i];
+    nx = acc & ~s;
+    a.next[i] = nx;
+    if (nx) {
+      a.seen[i] = s | nx;
+      ulonglong2 p = a.planes[2 * i], q = a.planes[2 * i + 1];
+      if (a.d & 1) p.x |= nx;
+      if (a.d & 2) p.y |= nx;
+      if (a.d & 4) q.x |= nx;
+      if (a.d & 8) q.y |= nx;
+      a.planes[2 * i] = p;
+      a.planes[2 * i + 1] = q;
     }
   }
+  __shared__ uint32_t ws[4];
+  const uint32_t c = gsum<64>((uint32_t)__popcll(nx));
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t tot = ws[0] + ws[1] + ws[2] + ws[3];
+    if (tot) atomicAdd(&a.cnt[a.d], (unsigned long long)tot);
+  }
+}
+
+__global__ void k_fill_u64(unsigned long long *p, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = 0;
+}
+// the identity at distance 0
+__global__ void k_root(Table T, uint64_t id, uint64_t *front, uint64_t *seen, unsigned long long *cnt) {
+  if (blockIdx.x || threadIdx.x) return;
+  const int i = find_sym(T, id);
+  front[i] = 1;
+  seen[i] = 1;
+  cnt[0] = 1;
 }
 
 // tableaux of words (letters are gate-set indices, applied in order), one lane per word
@@ -180,17 +339,9 @@ __global__ void k_words(Gates G, const uint8_t *letters, const long long *offs, 
   }
 }
 
-// batched lookups: 8 lanes per query (src/clifford.cu:207-210)
+// batched lookups (src/clifford.cu:207-210), one lane per query
 __global__ __launch_bounds__(256) void k_find(Table T, const uint64_t *q, long long nq, int *out) {
-  const int l8 = threadIdx.x & 7;
-  const long long groups = (long long)gridDim.x * (blockDim.x / 8);
-  for (long long i0 = 0; i0 < nq; i0 += groups) {       // uniform trip count: every lane takes part in the ballots
-    const long long i = i0 + (long long)blockIdx.x * (blockDim.x / 8) + (threadIdx.x >> 3);
-    if (i < nq) {
-      const int d = probe8<false>(T, q[i], 0, l8);
-      if (l8 == 0) out[i] = d;
-    }
-  }
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nq; i += (long long)gridDim.x * 256) out[i] = find1(T, q[i]);
 }
 
 // optimal words: one wave per query; each step, lane g tests the predecessor through gate g (its distance
@@ -200,12 +351,7 @@ __global__ __launch_bounds__(64) void k_readback(Gates G, Table T, const uint64_
   const int lane = threadIdx.x;
   for (long long i = blockIdx.x; i < nq; i += gridDim.x) {
     uint64_t X = q[i];
-    // distance of the query: lanes 0..7 probe cooperatively
-    int d = -1;
-    {
-      const int dd = lane < 8 ? probe8<false>(T, X, 0, lane) : 0;
-      d = __shfl(dd, 0, 64);
-    }
+    const int d = find1(T, X);
     if (d < 0 || d > maxlen) { if (lane == 0) lens[i] = -1; continue; }
     if (lane == 0) lens[i] = d;
     for (int s = d; s > 0; s--) {
@@ -213,18 +359,7 @@ __global__ __launch_bounds__(64) void k_readback(Gates G, Table T, const uint64_
       bool ok = false;
       if (lane < G.ng) {
         pre = apply(X, G.n, inv_kind(G.k[lane]), G.a[lane], G.b[lane]);
-        // scalar linear probing of one key per lane over the same bucket layout
-        uint64_t b = hmix(pre) & T.bmask;
-        for (int guard = 0; guard < (1 << 20); guard++) {
-          bool done = false;
-          for (int j = 0; j < 8; j++) {
-            const unsigned long long v = T.slot[b * 8 + j];
-            if (!v) { done = true; break; }
-            if ((v >> 8) == pre) { ok = (int)(v & 255) == s - 1; done = true; break; }
-          }
-          if (done) break;
-          b = (b + 1) & T.bmask;
-        }
+        ok = find1(T, pre) == s - 1;
       }
       const uint64_t bal = __ballot(ok);
       const int g = bal ? __ffsll((long long)bal) - 1 : -1;
@@ -235,30 +370,10 @@ __global__ __launch_bounds__(64) void k_readback(Gates G, Table T, const uint64_
   }
 }
 
-// elements in a canonical order (sorted by tableau), so that seeded samples do not depend on where concurrent
-// inserts happened to place keys: occupied slots are compacted, then stably sorted by the low and then the high
-// 32 bits of the tableau
-struct FlagSlot {
-  const unsigned long long *s;
-  __device__ bool operator()(long long i) const { return s[i] != 0; }
-};
-__global__ void k_key_lo(const unsigned long long *slot, const uint32_t *idx, long long n, uint32_t *k, uint32_t *v) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    k[i] = (uint32_t)(slot[idx[i]] >> 8);
-    v[i] = (uint32_t)i;
-  }
-}
-__global__ void k_key_hi(const unsigned long long *slot, const uint32_t *idx, const uint32_t *perm, long long n,
-                         uint32_t *k, uint32_t *v) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    k[i] = (uint32_t)(slot[idx[perm[i]]] >> 40);
-    v[i] = perm[i];
-  }
-}
-__global__ void k_key_final(const unsigned long long *slot, const uint32_t *idx, const uint32_t *perm, long long n,
-                            uint64_t *out) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    out[i] = slot[idx[perm[i]]] >> 8;
+// every element, in the order of the tableaux
+template <int NQ> __global__ __launch_bounds__(256) void k_sorted(uint64_t *out) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < Num<NQ>::ORDER; i += (long long)gridDim.x * 256)
+    out[i] = Num<NQ>::element((uint64_t)i);
 }
 
 // seeded uniform elements: splitmix64 indices into the sorted element list
@@ -273,12 +388,19 @@ __global__ void k_sample(const uint64_t *sorted, long long order, unsigned long 
 }
 
 // order-independent digest: sum over entries of hmix-free mix of (tableau * 64 + distance), and the count
-__global__ __launch_bounds__(256) void k_digest(Table T, long long nslots, unsigned long long *out) {
+__global__ __launch_bounds__(256) void k_digest(Table T, const uint64_t *key, long long count, unsigned long long *out) {
   unsigned long long s = 0, c = 0;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nslots; i += (long long)gridDim.x * blockDim.x) {
-    const unsigned long long v = T.slot[i];
-    if (v) { uint64_t x = (v >> 8) * 64 + (v & 255); x ^= x >> 33; x *= 0xff51afd7ed558ccdull; x ^= x >> 33;
-             x *= 0xc4ceb9fe1a85ec53ull; x ^= x >> 33; s += x; c++; }
+  const int n = T.n, ns = 1 << (2 * n);
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (long long)gridDim.x * blockDim.x) {
+    const uint64_t t = key[i];
+    const ulonglong2 p = T.planes[2 * i], q = T.planes[2 * i + 1];
+    for (int v = 0; v < ns; v++) {
+      uint64_t w = t;
+      for (int r = 0; r < 2 * n; r++) w |= (uint64_t)((v >> r) & 1) << (r * (2 * n + 1) + 2 * n);
+      uint64_t x = w * 64 + (uint64_t)plane_dist(p, q, (uint32_t)v);
+      x ^= x >> 33; x *= 0xff51afd7ed558ccdull; x ^= x >> 33;
+      x *= 0xc4ceb9fe1a85ec53ull; x ^= x >> 33; s += x; c++;
+    }
   }
   for (int m = 1; m < 64; m <<= 1) { s += __shfl_xor(s, m, 64); c += __shfl_xor(c, m, 64); }
   if ((threadIdx.x & 63) == 0) { atomicAdd(&out[0], s); atomicAdd(&out[1], c); }
@@ -323,11 +445,12 @@ struct chz_cliff {
   uint64_t *scratch = nullptr;         // this device's chz_cl::scratch (its device address)
   chz_cl::Gates G{};
   chz_cl::Table T{};
-  long long nslots = 0;
+  void *block = nullptr;               // the table's arrays, one block
+  uint64_t *key = nullptr;             // sign-free tableaux of the matrices
+  long long count = 0;                 // matrices
   std::vector<long> levels;
   hipStream_t stream = nullptr;
   double build_ms = 0;
-  double probes = 0;
   uint64_t *sorted = nullptr;          // elements sorted by tableau (built on the first sample)
   long long order = 0;
 };
@@ -342,73 +465,87 @@ extern "C" {
 
 const char *chz_cliff_last_error(void) { return chz_cl::g_err.c_str(); }
 
-int chz_cliff_build(int n, int device, chz_cliff **out) {
-  chz::RelaxedCapture relaxed;
-  *out = nullptr;
-  if (n < 1 || n > 3) { chz_cl::g_err = "n must be 1..3"; return 3; }
-  chz_cliff *c = new chz_cliff();
-  c->n = n;
-  c->device = device;
-  c->G = chz_cl::gate_set(n);
-  const long long order = n == 1 ? 24 : n == 2 ? 11520 : 92897280;   // 2^(n^2+2n) prod_j (4^j - 1)
-  int lg = 6;
-  while ((1ll << lg) < order * 4 / 3) lg++;
-  c->nslots = 1ll << lg;
-  c->T.bmask = (uint64_t)(c->nslots / 8 - 1);
-  CLCHK(hipSetDevice(device));
-  if (const int rc = chz_cl::scratch_address(device, &c->scratch)) { delete c; return rc; }
-  CLCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  CLCHK(cl_malloc((void **)&c->T.slot, c->nslots * 8));
-  CLCHK(hipMemsetAsync(c->T.slot, 0, c->nslots * 8, c->stream));
-  const long long cap = std::max(1024ll, order / 2);
-  uint64_t *fa = nullptr, *fb = nullptr;
-  unsigned long long *cnt = nullptr;
-  CLCHK(cl_malloc((void **)&fa, cap * 8));
-  CLCHK(cl_malloc((void **)&fb, cap * 8));
-  CLCHK(cl_malloc((void **)&cnt, 16));
+}  // extern "C"
+
+// the table of c (its stream and n set); 0, 4 or 5
+template <int NQ> static int cliff_fill(chz_cliff *c) {
+  using namespace chz_cl;
+  constexpr long long C = Num<NQ>::matrices();
+  constexpr int MAXD = 15;                            // four planes
+  long long slots = 64;
+  while (slots < 2 * C) slots <<= 1;
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  // [slots | planes | keys], and for the build [seen | two frontiers | counts | neighbours]
+  const size_t o_pl = up(slots * 8), o_key = o_pl + up(C * 32), bytes = o_key + up(C * 8);
+  const size_t w_f0 = up(C * 8), w_f1 = 2 * w_f0, w_cnt = 3 * w_f0, w_nb = w_cnt + 256, wbytes = w_nb + up((size_t)sym_gates(NQ) * C * 4);
+  uint8_t *work = nullptr;
+  CLCHK(cl_malloc(&c->block, bytes));
+  CLCHK(cl_malloc((void **)&work, wbytes));
+  struct Guard { uint8_t *p; ~Guard() { (void)cl_free(p); } } guard{work};     // (hipFree waits for the device)
+  uint8_t *blk = (uint8_t *)c->block;
+  c->count = C;
+  c->key = (uint64_t *)(blk + o_key);
+  c->T = Table{(unsigned long long *)blk, (uint32_t)(slots - 1), (const ulonglong2 *)(blk + o_pl), NQ};
+  uint64_t *seen = (uint64_t *)work, *front[2] = {(uint64_t *)(work + w_f0), (uint64_t *)(work + w_f1)};
+  unsigned long long *cnt = (unsigned long long *)(work + w_cnt);
+  uint32_t *nb = (uint32_t *)(work + w_nb);
   hipEvent_t e0, e1;
   CLCHK(hipEventCreate(&e0));
   CLCHK(hipEventCreate(&e1));
   CLCHK(hipEventRecord(e0, c->stream));
-  // the identity takes its slot with distance 0
-  {
-    const uint64_t id = chz_cl::identity(n);
-    const unsigned long long w = (unsigned long long)(id << 8);
-    uint64_t b = chz_cl::hmix(id) & c->T.bmask;
-    CLCHK(hipMemcpyAsync(c->T.slot + b * 8, &w, 8, hipMemcpyHostToDevice, c->stream));
-    CLCHK(hipMemcpyAsync(fa, &id, 8, hipMemcpyHostToDevice, c->stream));
+  const dim3 grid((unsigned)((C + 255) / 256)), blockd(256);
+  hipLaunchKernelGGL(k_fill_u64, dim3(4096), blockd, 0, c->stream, (unsigned long long *)blk, (long long)(o_key / 8));
+  hipLaunchKernelGGL(k_fill_u64, dim3(4096), blockd, 0, c->stream, (unsigned long long *)work, (long long)(w_nb / 8));
+  hipLaunchKernelGGL(k_matrices<NQ>, grid, blockd, 0, c->stream, c->key, c->T.slot, c->T.smask);
+  hipLaunchKernelGGL(k_neighbours<NQ>, grid, blockd, 0, c->stream, c->T, c->key, nb);
+  hipLaunchKernelGGL(k_root, dim3(1), dim3(64), 0, c->stream, c->T, identity(NQ), front[0], seen, cnt);
+  // every level is queued at once: one after the last finds the level before it empty and ends
+  for (int d = 1; d <= MAXD; d++) {
+    const BfsArgs a{c->key, nb, front[(d - 1) & 1], front[d & 1], seen, (ulonglong2 *)(blk + o_pl), cnt, d};
+    hipLaunchKernelGGL(k_bfs<NQ>, grid, blockd, 0, c->stream, a);
   }
-  long long nf = 1, total = 1;
-  c->levels.assign(1, 1);
-  for (int d = 1; nf; d++) {
-    CLCHK(hipMemsetAsync(cnt, 0, 16, c->stream));
-    chz_cl::BfsArgs a{c->G, c->T, fa, nf, fb, cnt, cap, d};
-    const long long groups = nf * c->G.ng;
-    const int blocks = (int)std::min<long long>(std::max<long long>((groups + 31) / 32, 1), 8192);
-    hipLaunchKernelGGL(chz_cl::k_bfs, dim3(blocks), dim3(256), 0, c->stream, a);
-    unsigned long long h[2];
-    CLCHK(hipMemcpyAsync(h, cnt, 16, hipMemcpyDeviceToHost, c->stream));
-    CLCHK(hipStreamSynchronize(c->stream));
-    if (h[1]) { chz_cl::g_err = "frontier buffer too small"; return 4; }
-    c->probes += (double)groups;
-    nf = (long long)h[0];
-    total += nf;
-    if (nf) c->levels.push_back((long)nf);
-    std::swap(fa, fb);
-  }
+  CLCHK(hipGetLastError());
+  unsigned long long h[MAXD + 1];
+  CLCHK(hipMemcpyAsync(h, cnt, sizeof h, hipMemcpyDeviceToHost, c->stream));
   CLCHK(hipEventRecord(e1, c->stream));
-  CLCHK(hipEventSynchronize(e1));
+  CLCHK(hipStreamSynchronize(c->stream));
   float ms = 0;
   CLCHK(hipEventElapsedTime(&ms, e0, e1));
   c->build_ms = ms;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  (void)cl_free(fa);
-  (void)cl_free(fb);
-  (void)cl_free(cnt);
-  *out = c;
-  if (total != order) { chz_cl::g_err = "group order mismatch"; return 4; }   // src/clifford.cu:279-280
+  long long total = 0;
+  for (int d = 0; d <= MAXD && h[d]; d++) {
+    c->levels.push_back((long)h[d]);
+    total += (long long)h[d];
+  }
+  if (total != Num<NQ>::ORDER) { g_err = "group order mismatch"; return 4; }   // src/clifford.cu:279-280
   return 0;
+}
+
+extern "C" {
+
+int chz_cliff_build(int n, int device, chz_cliff **out) {
+  chz::RelaxedCapture relaxed;
+  *out = nullptr;
+  if (n < 1 || n > 3) { chz_cl::g_err = "n must be 1..3"; return 3; }
+  CLCHK(hipSetDevice(device));
+  uint64_t *scratch = nullptr;
+  if (const int rc = chz_cl::scratch_address(device, &scratch)) return rc;
+  chz_cliff *c = new chz_cliff();
+  c->n = n;
+  c->device = device;
+  c->scratch = scratch;
+  c->G = chz_cl::gate_set(n);
+  if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+    chz_cl::g_err = "HIP error: no stream";
+    delete c;
+    return 5;
+  }
+  const int rc = n == 1 ? cliff_fill<1>(c) : n == 2 ? cliff_fill<2>(c) : cliff_fill<3>(c);
+  if (rc == 5) { chz_cliff_free(c); return 5; }
+  *out = c;
+  return rc;
 }
 
 int chz_cliff_levels(const chz_cliff *c, long *counts, int maxd) {
@@ -426,7 +563,7 @@ int chz_cliff_digest(const chz_cliff *c, uint64_t *digest, long long *entries) {
   CLCHK(hipSetDevice(c->device));
   CLCHK(cl_malloc((void **)&d, 16));
   CLCHK(hipMemsetAsync(d, 0, 16, c->stream));
-  hipLaunchKernelGGL(chz_cl::k_digest, dim3(2048), dim3(256), 0, c->stream, c->T, c->nslots, d);
+  hipLaunchKernelGGL(chz_cl::k_digest, dim3(2048), dim3(256), 0, c->stream, c->T, c->key, c->count, d);
   CLCHK(hipMemcpyAsync(h, d, 16, hipMemcpyDeviceToHost, c->stream));
   CLCHK(hipStreamSynchronize(c->stream));
   (void)cl_free(d);
@@ -438,37 +575,14 @@ int chz_cliff_digest(const chz_cliff *c, uint64_t *digest, long long *entries) {
 // the sorted element list, built once
 static int cliff_sorted(chz_cliff *c) {
   if (c->sorted) return 0;
-  const long long ns = c->nslots;
-  const long long nb = (ns + CT_TILE - 1) / CT_TILE;
-  unsigned long long *bc = nullptr, *tmp = nullptr, *hist = nullptr;
-  uint32_t *idx = nullptr, *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
-  CLCHK(cl_malloc((void **)&bc, (nb + 1) * 8));
-  CLCHK(cl_malloc((void **)&tmp, (ns / SC_TILE + 8) * 8));
-  chz_cl::FlagSlot f{c->T.slot};
-  hipLaunchKernelGGL(k_flag_count<chz_cl::FlagSlot>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, f, ns, bc);
-  CLCHK(scan_excl(bc, nb, tmp, c->stream));
-  unsigned long long n = 0;
-  CLCHK(hipMemcpyAsync(&n, bc + nb, 8, hipMemcpyDeviceToHost, c->stream));
+  const long long n = c->count << (2 * c->n);
+  CLCHK(cl_malloc((void **)&c->sorted, n * 8));
+  const dim3 g((unsigned)std::min<long long>((n + 255) / 256, 16384)), b(256);
+  if (c->n == 1) hipLaunchKernelGGL(chz_cl::k_sorted<1>, g, b, 0, c->stream, c->sorted);
+  else if (c->n == 2) hipLaunchKernelGGL(chz_cl::k_sorted<2>, g, b, 0, c->stream, c->sorted);
+  else hipLaunchKernelGGL(chz_cl::k_sorted<3>, g, b, 0, c->stream, c->sorted);
   CLCHK(hipStreamSynchronize(c->stream));
-  const long long rb = ((long long)n + RS_TILE - 1) / RS_TILE;
-  CLCHK(cl_malloc((void **)&idx, std::max<unsigned long long>(n, 1) * 4));
-  CLCHK(cl_malloc((void **)&k0, std::max<unsigned long long>(n, 1) * 4));
-  CLCHK(cl_malloc((void **)&v0, std::max<unsigned long long>(n, 1) * 4));
-  CLCHK(cl_malloc((void **)&k1, std::max<unsigned long long>(n, 1) * 4));
-  CLCHK(cl_malloc((void **)&v1, std::max<unsigned long long>(n, 1) * 4));
-  CLCHK(cl_malloc((void **)&hist, (rb * 256 + 1) * 8));
-  CLCHK(cl_malloc((void **)&c->sorted, std::max<unsigned long long>(n, 1) * 8));
-  hipLaunchKernelGGL(k_scatter_idx<chz_cl::FlagSlot>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, f, ns, bc, idx);
-  const unsigned g = (unsigned)std::min<long long>(((long long)n + 255) / 256 + 1, 16384);
-  hipLaunchKernelGGL(chz_cl::k_key_lo, dim3(g), dim3(256), 0, c->stream, c->T.slot, idx, (long long)n, k0, v0);
-  CLCHK(radix_sort_pairs(k0, v0, k1, v1, (long long)n, hist, tmp, c->stream));
-  hipLaunchKernelGGL(chz_cl::k_key_hi, dim3(g), dim3(256), 0, c->stream, c->T.slot, idx, v0, (long long)n, k1, v1);
-  CLCHK(radix_sort_pairs(k1, v1, k0, v0, (long long)n, hist, tmp, c->stream));
-  hipLaunchKernelGGL(chz_cl::k_key_final, dim3(g), dim3(256), 0, c->stream, c->T.slot, idx, v1, (long long)n, c->sorted);
-  CLCHK(hipStreamSynchronize(c->stream));
-  c->order = (long long)n;
-  void *fr[] = {bc, tmp, hist, idx, k0, v0, k1, v1};
-  for (void *p : fr) (void)cl_free(p);
+  c->order = n;
   return 0;
 }
 
@@ -510,7 +624,7 @@ int chz_cliff_query_words(chz_cliff *c, const uint8_t *letters, const long long 
   CLCHK(hipEventRecord(e0, c->stream));
   hipLaunchKernelGGL(chz_cl::k_words, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
                      c->stream, c->G, dl, doff, nq, tab);
-  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 31) / 32 + 1, 8192)), dim3(256), 0,
+  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
                      c->stream, c->T, tab, nq, dd);
   CLCHK(hipEventRecord(e1, c->stream));
   CLCHK(hipMemcpyAsync(dist, dd, nq * 4, hipMemcpyDeviceToHost, c->stream));
@@ -544,7 +658,7 @@ int chz_cliff_query_words_noalloc(chz_cliff *c, const uint8_t *d_letters, const 
   hipStream_t st = stream ? (hipStream_t)stream : c->stream;
   hipLaunchKernelGGL(chz_cl::k_words, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
                      st, c->G, d_letters, d_offs, nq, c->scratch);
-  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 31) / 32 + 1, 8192)), dim3(256), 0,
+  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
                      st, c->T, c->scratch, nq, d_dist);
   CLCHK(hipGetLastError());
   if (!stream) CLCHK(hipStreamSynchronize(st));
@@ -589,7 +703,7 @@ void chz_cliff_free(chz_cliff *c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->T.slot) (void)cl_free(c->T.slot);
+  if (c->block) (void)cl_free(c->block);
   if (c->sorted) (void)cl_free(c->sorted);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
