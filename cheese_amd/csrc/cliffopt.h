@@ -1,6 +1,6 @@
 // Host side of `cliffopt JOB [--beam B]` (src/clifford.cu:285-385): the job file, the placements of every T gate
-// (in the table's sorted element order, so the search is deterministic), the beam over them, the final choice and
-// the optimal gate lists of the new segments.  Included by clifford.hip inside its extern "C" block.
+// (in the order of their tableaux, so the search is deterministic), the beam over them, the final choice and
+// the optimal gate lists of the new segments.  Included by clifford.hip.
 
 namespace {
 
@@ -42,86 +42,105 @@ int read_cliff_job(const char *text, size_t len, CliffJob &J, std::string &err) 
   return 0;
 }
 
-}  // namespace
-
-int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out, size_t cap) {
-  chz::RelaxedCapture relaxed;
+template <int NQ> int cliff_opt(chz_cliff *c, const CliffJob &J, int beam, double t0, char *out, size_t cap) {
   using chz_cl::Cand;
-  const double t0 = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
-  CliffJob J;
-  std::string err;
-  if (const int rc = read_cliff_job(job, len, J, err)) { chz_cl::g_err = err; return rc; }
-  if (J.n != c->n) { chz_cl::g_err = "the job's qubit count differs from the table's"; return 3; }
-  beam = std::max(1, std::min(chz_cl::TOPK - 1, beam));
-  const int n = J.n, t = (int)J.tq.size();
-  CLCHK(hipSetDevice(c->device));
-  if (const int rc = cliff_sorted(c)) return rc;
+  using Num = chz_cl::Num<NQ>;
+const int n = NQ, t = (int)J.tq.size();
   std::vector<uint64_t> D(t + 1);                             // segment tableaux
   for (int j = 0; j <= t; j++) {
     uint64_t X = chz_cl::identity(n);
     for (const auto &g : J.seg[j]) X = chz_cl::apply(X, n, g[0], g[1], g[2]);
     D[j] = X;
   }
-  // placements per qubit, in sorted element order (ordered compaction of the flags)
-  std::vector<Cand *> cands(n, nullptr);
-  std::vector<long long> ncand(n, 0);
   std::vector<void *> owned;
-  auto release = [&]() { for (void *p : owned) (void)cl_free(p); owned.clear(); };
+  struct Guard { std::vector<void *> &o; ~Guard() { for (void *p : o) (void)cl_free(p); } } guard{owned};
   auto dalloc = [&](size_t bytes) -> void * {
     void *p = nullptr;
     if (cl_malloc(&p, std::max<size_t>(bytes, 8)) != hipSuccess) return nullptr;
     owned.push_back(p);
     return p;
   };
+  // placements per qubit: the flagged signed Z images in order (candidate c is element zs[c / X_ALL] * X_ALL + c %
+  // X_ALL), their places, and the placements' matrices
+  struct Places { std::vector<uint32_t> zs; uint32_t *zpos = nullptr; chz_cl::PlaceMat *pm = nullptr; long long nm = 0; };
+  std::vector<Places> places(n);
+  constexpr int grid = 256;             // blocks of a beam step
+  uint64_t *d_left = (uint64_t *)dalloc(chz_cl::TOPK * 8);
+  int *d_cost = (int *)dalloc(chz_cl::TOPK * 4);
+  unsigned int *d_hist = (unsigned int *)dalloc(256 * 4);
+  unsigned long long *d_top = (unsigned long long *)dalloc((size_t)grid * chz_cl::TOPK * 8);
+  if (!d_left || !d_cost || !d_hist || !d_top) { chz_cl::g_err = "device memory"; return 5; }
+  long long most = 0;                   // rows of a step per state
   {
-    const long long ord = c->order, nb = (ord + CT_TILE - 1) / CT_TILE;
-    uint8_t *flag = (uint8_t *)dalloc(ord);
-    unsigned long long *bc = (unsigned long long *)dalloc((nb + 1) * 8);
-    unsigned long long *tmp = (unsigned long long *)dalloc((nb / SC_TILE + 8) * 8);
-    uint32_t *idx = (uint32_t *)dalloc(ord * 4);
-    if (!flag || !bc || !tmp || !idx) { release(); chz_cl::g_err = "device memory"; return 5; }
+    const long long nbs = (Num::Z_ALL + CT_TILE - 1) / CT_TILE, nbu = (Num::Z_SYM + CT_TILE - 1) / CT_TILE;
+    unsigned long long *bc = (unsigned long long *)dalloc((nbs + 1) * 8), *bu = (unsigned long long *)dalloc((nbu + 1) * 8);
+    unsigned long long *tmp = (unsigned long long *)dalloc((nbs / SC_TILE + 8) * 8);
+    uint32_t *zs = (uint32_t *)dalloc((size_t)Num::Z_ALL * 4), *zu = (uint32_t *)dalloc((size_t)Num::Z_SYM * 4);
+    if (!bc || !bu || !tmp || !zs || !zu) { chz_cl::g_err = "device memory"; return 5; }
     for (int q = 0; q < n; q++) {
       if (std::find(J.tq.begin(), J.tq.end(), q) == J.tq.end()) continue;
-      hipLaunchKernelGGL(chz_cl::k_cand_flags, dim3(4096), dim3(256), 0, c->stream, c->sorted, ord, n, q, flag);
-      const chz_cl::FlagNZ f{flag};
-      hipLaunchKernelGGL(k_flag_count<chz_cl::FlagNZ>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, f, ord, bc);
-      if (scan_excl(bc, nb, tmp, c->stream) != hipSuccess) { release(); chz_cl::g_err = "scan"; return 5; }
-      hipLaunchKernelGGL(k_scatter_idx<chz_cl::FlagNZ>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, f, ord, bc, idx);
-      unsigned long long nc = 0;
-      if (hipMemcpyAsync(&nc, bc + nb, 8, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-          hipStreamSynchronize(c->stream) != hipSuccess) { release(); chz_cl::g_err = "device error"; return 5; }
-      cands[q] = (Cand *)dalloc(std::max<unsigned long long>(nc, 1) * sizeof(Cand));
-      if (!cands[q]) { release(); chz_cl::g_err = "device memory"; return 5; }
-      ncand[q] = (long long)nc;
-      if (nc)
-        hipLaunchKernelGGL(chz_cl::k_cand_build, dim3((unsigned)std::min<unsigned long long>((nc + 255) / 256, 8192)), dim3(256),
-                           0, c->stream, c->sorted, idx, (long long)nc, flag, n, cands[q]);
+      Places &P = places[q];
+      const chz_cl::FlagZs<NQ> fs{q};
+      const chz_cl::FlagZ<NQ> fu{q};
+      P.zpos = (uint32_t *)dalloc((size_t)Num::Z_ALL * 4);
+      if (!P.zpos) { chz_cl::g_err = "device memory"; return 5; }
+      hipLaunchKernelGGL(k_flag_count<chz_cl::FlagZs<NQ>>, dim3((unsigned)nbs), dim3(CT_THREADS), 0, c->stream, fs,
+                         (long long)Num::Z_ALL, bc);
+      CLCHK(scan_excl(bc, nbs, tmp, c->stream));
+      hipLaunchKernelGGL(k_scatter_idx<chz_cl::FlagZs<NQ>>, dim3((unsigned)nbs), dim3(CT_THREADS), 0, c->stream, fs,
+                         (long long)Num::Z_ALL, bc, zs);
+      hipLaunchKernelGGL(chz_cl::k_invert, dim3(64), dim3(256), 0, c->stream, zs, bc + nbs, P.zpos);
+      hipLaunchKernelGGL(k_flag_count<chz_cl::FlagZ<NQ>>, dim3((unsigned)nbu), dim3(CT_THREADS), 0, c->stream, fu,
+                         (long long)Num::Z_SYM, bu);
+      CLCHK(scan_excl(bu, nbu, tmp, c->stream));
+      hipLaunchKernelGGL(k_scatter_idx<chz_cl::FlagZ<NQ>>, dim3((unsigned)nbu), dim3(CT_THREADS), 0, c->stream, fu,
+                         (long long)Num::Z_SYM, bu, zu);
+      unsigned long long ns = 0, nu = 0;
+      CLCHK(hipMemcpyAsync(&ns, bc + nbs, 8, hipMemcpyDeviceToHost, c->stream));
+      CLCHK(hipMemcpyAsync(&nu, bu + nbu, 8, hipMemcpyDeviceToHost, c->stream));
+      CLCHK(hipStreamSynchronize(c->stream));
+      P.nm = (long long)nu * Num::X_SYM;
+      P.zs.resize(ns);
+      P.pm = (chz_cl::PlaceMat *)dalloc((size_t)P.nm * sizeof(chz_cl::PlaceMat));
+      if (!P.pm) { chz_cl::g_err = "device memory"; return 5; }
+      if (ns) CLCHK(hipMemcpyAsync(P.zs.data(), zs, ns * 4, hipMemcpyDeviceToHost, c->stream));
+      if (P.nm)
+        hipLaunchKernelGGL(chz_cl::k_place<NQ>, dim3((unsigned)std::min<long long>((P.nm + 255) / 256, 4096)), dim3(256), 0,
+                           c->stream, zu, P.nm, q, P.pm);
+      CLCHK(hipStreamSynchronize(c->stream));
+      most = std::max(most, P.nm * 2);
     }
   }
+  uint8_t *d_low = (uint8_t *)dalloc((size_t)most * beam);
+  if (!d_low) { chz_cl::g_err = "device memory"; return 5; }
   // the beam over every T gate (src/clifford.cu:318-345)
-  const int grid = 4096;
-  uint64_t *d_K = (uint64_t *)dalloc(chz_cl::TOPK * 8);
-  int *d_cost = (int *)dalloc(chz_cl::TOPK * 4);
-  unsigned long long *d_top = (unsigned long long *)dalloc((size_t)grid * chz_cl::TOPK * 8);
-  if (!d_K || !d_cost || !d_top) { release(); chz_cl::g_err = "device memory"; return 5; }
   std::vector<std::vector<int>> parent(t), flips(t);
   std::vector<std::vector<Cand>> chosen(t);
   std::vector<uint64_t> hK(1, 0);
   std::vector<int> hcost(1, 0);
   for (int j = 0; j < t; j++) {
-    const int q = J.tq[j];
-    const long long nc = ncand[q], tot = (long long)hK.size() * nc * 2;
-    if (nc == 0) { release(); chz_cl::g_err = "no placement for a T gate"; return 4; }
-    CLCHK(hipMemcpyAsync(d_K, hK.data(), hK.size() * 8, hipMemcpyHostToDevice, c->stream));
-    CLCHK(hipMemcpyAsync(d_cost, hcost.data(), hcost.size() * 4, hipMemcpyHostToDevice, c->stream));
-    const int blocks = (int)std::min<long long>(grid, (tot + 255) / 256);
-    chz_cl::BeamArgs ba{c->T, n, d_K, d_cost, (int)hK.size(), j == 0, D[j], cands[q], nc, J.td[j], beam, d_top};
-    hipLaunchKernelGGL(chz_cl::k_beam, dim3(blocks), dim3(256), 0, c->stream, ba);
+    const int q = J.tq[j], nb = (int)hK.size();
+    const Places &P = places[q];
+    const long long nc = (long long)P.zs.size() * Num::X_ALL, tot = nb * nc * 2;
+    if (nc == 0) { chz_cl::g_err = "no placement for a T gate"; return 4; }
+    std::vector<uint64_t> left(nb);
+    for (int b = 0; b < nb; b++) left[b] = j == 0 ? D[0] : chz_cl::tcompose(hK[b], D[j], n);
+    CLCHK(hipMemcpyAsync(d_left, left.data(), nb * 8, hipMemcpyHostToDevice, c->stream));
+    CLCHK(hipMemcpyAsync(d_cost, hcost.data(), nb * 4, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(chz_cl::k_fill_u64, dim3(1), dim3(128), 0, c->stream, (unsigned long long *)d_hist, 128ll);
+    chz_cl::BeamArgs ba{c->T, d_left, d_cost, nb, *std::min_element(hcost.begin(), hcost.end()), P.pm, P.nm, P.zpos, d_low,
+                        d_hist, J.td[j], beam, d_top};
+    const long long rows = nb * P.nm * 2;
+    hipLaunchKernelGGL(chz_cl::k_beam_low<NQ>, dim3((unsigned)std::min<long long>((rows + 255) / 256, 4096)), dim3(256), 0,
+                       c->stream, ba);
+    const int blocks = (int)std::min<long long>(grid, (rows + 15) / 16);
+    hipLaunchKernelGGL(chz_cl::k_beam<NQ>, dim3(blocks), dim3(256), 0, c->stream, ba);
+    CLCHK(hipGetLastError());
     std::vector<unsigned long long> top((size_t)blocks * beam);
     CLCHK(hipMemcpyAsync(top.data(), d_top, top.size() * 8, hipMemcpyDeviceToHost, c->stream));
     CLCHK(hipStreamSynchronize(c->stream));
-    std::sort(top.begin(), top.end());
     const int keep = (int)std::min<long long>(beam, tot);
+    std::partial_sort(top.begin(), top.begin() + keep, top.end());
     parent[j].resize(keep);
     flips[j].resize(keep);
     chosen[j].resize(keep);
@@ -130,12 +149,12 @@ int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out
     for (int i = 0; i < keep; i++) {
       const int b = (int)((top[i] >> 32) & 0xff);
       const long long c2 = (long long)(top[i] & 0xffffffffull);
-      CLCHK(hipMemcpyAsync(&chosen[j][i], cands[q] + (c2 >> 1), sizeof(Cand), hipMemcpyDeviceToHost, c->stream));
+      const uint64_t cand = (uint64_t)(c2 >> 1);
+      chosen[j][i] = chz_cl::make_cand(Num::element((uint64_t)P.zs[cand / Num::X_ALL] * Num::X_ALL + cand % Num::X_ALL), n, q);
       parent[j][i] = b;
       flips[j][i] = (int)(c2 & 1);
       ncost[i] = (int)(top[i] >> 40);
     }
-    CLCHK(hipStreamSynchronize(c->stream));
     for (int i = 0; i < keep; i++) nk[i] = chosen[j][i].K;
     hK = nk;
     hcost = ncost;
@@ -144,9 +163,9 @@ int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out
   int best = 0, bestv = 1 << 30;
   if (t > 0) {
     int *d_fin = (int *)dalloc(chz_cl::TOPK * 4);
-    if (!d_fin) { release(); chz_cl::g_err = "device memory"; return 5; }
-    CLCHK(hipMemcpyAsync(d_K, hK.data(), hK.size() * 8, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(chz_cl::k_beam_final, dim3(((int)hK.size() + 63) / 64), dim3(64), 0, c->stream, c->T, n, d_K,
+    if (!d_fin) { chz_cl::g_err = "device memory"; return 5; }
+    CLCHK(hipMemcpyAsync(d_left, hK.data(), hK.size() * 8, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(chz_cl::k_beam_final, dim3(((int)hK.size() + 63) / 64), dim3(64), 0, c->stream, c->T, n, d_left,
                        (int)hK.size(), D[t], d_fin);
     std::vector<int> fin(hK.size());
     CLCHK(hipMemcpyAsync(fin.data(), d_fin, fin.size() * 4, hipMemcpyDeviceToHost, c->stream));
@@ -154,7 +173,6 @@ int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out
     for (size_t b = 0; b < hK.size(); b++)
       if (hcost[b] + fin[b] < bestv) { bestv = hcost[b] + fin[b]; best = (int)b; }
   }
-  release();
   std::vector<Cand> K(t);
   std::vector<int> flip(t), dag(t);
   for (int j = t - 1, b = best; j >= 0; j--) { K[j] = chosen[j][b]; flip[j] = flips[j][b]; b = parent[j][b]; }
@@ -202,4 +220,19 @@ int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out
   s.copy(out, s.size());
   out[s.size()] = 0;
   return 0;
+}
+
+}  // namespace
+
+extern "C" int chz_cliff_opt(chz_cliff *c, const char *job, size_t len, int beam, char *out, size_t cap) {
+  chz::RelaxedCapture relaxed;
+  const double t0 = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+  CliffJob J;
+  std::string err;
+  if (const int rc = read_cliff_job(job, len, J, err)) { chz_cl::g_err = err; return rc; }
+  if (J.n != c->n) { chz_cl::g_err = "the job's qubit count differs from the table's"; return 3; }
+  beam = std::max(1, std::min(chz_cl::TOPK - 1, beam));
+  CLCHK(hipSetDevice(c->device));
+  return J.n == 1 ? cliff_opt<1>(c, J, beam, t0, out, cap) : J.n == 2 ? cliff_opt<2>(c, J, beam, t0, out, cap)
+                                                                      : cliff_opt<3>(c, J, beam, t0, out, cap);
 }

@@ -109,6 +109,7 @@ struct Table {
   unsigned long long *slot;        // tableau without signs << 21 | number; 0 = empty (no tableau is 0)
   uint32_t smask;                  // slots - 1
   const ulonglong2 *planes;        // two per matrix: planes 0, 1 and 2, 3
+  const uint8_t *dmin;             // per matrix, the smallest distance of its sign vectors
   int n;
 };
 
@@ -187,6 +188,26 @@ template <int NQ> struct Num {
     }
     return T;
   }
+  // matrices and tableaux that share their Z images (the rows chosen first): numbers differ below these
+  __host__ __device__ static constexpr uint32_t x_matrices() {
+    uint32_t t = 1;
+    for (int k = NQ; k < M; k++) t *= choices(k);
+    return t;
+  }
+  static constexpr uint32_t X_SYM = x_matrices(), X_ALL = X_SYM << NQ;
+  static constexpr uint32_t Z_SYM = (uint32_t)(matrices() / X_SYM), Z_ALL = Z_SYM << NQ;
+  // the number, among all tableaux, of the i-th matrix with signs s
+  __host__ __device__ static uint64_t signed_number(uint32_t i, uint32_t s) {
+    uint64_t e = 0, scale = 1;
+#pragma unroll
+    for (int k = M - 1; k >= 0; k--) {
+      const uint32_t c = choices(k);
+      e += scale * (i % c + ((s >> (M - 1 - k)) & 1) * c);
+      scale *= 2 * c;
+      i /= c;
+    }
+    return e;
+  }
   // the i-th matrix's tableau, without signs
   __host__ __device__ static uint64_t matrix(uint32_t i) {
     uint32_t r[M];
@@ -247,6 +268,7 @@ struct BfsArgs {
   uint64_t *next;              // those at distance d
   uint64_t *seen;
   ulonglong2 *planes;
+  uint8_t *dmin;
   unsigned long long *cnt;     // elements per distance
   int d;
 };
@@ -296,6 +318,7 @@ template <int NQ> __global__ __launch_bounds__(256) void k_bfs(BfsArgs a) {
     a.next[i] = nx;
     if (nx) {
       a.seen[i] = s | nx;
+      if (!s) a.dmin[i] = (uint8_t)a.d;
       ulonglong2 p = a.planes[2 * i], q = a.planes[2 * i + 1];
       if (a.d & 1) p.x |= nx;
       if (a.d & 2) p.y |= nx;
@@ -370,20 +393,14 @@ __global__ __launch_bounds__(64) void k_readback(Gates G, Table T, const uint64_
   }
 }
 
-// every element, in the order of the tableaux
-template <int NQ> __global__ __launch_bounds__(256) void k_sorted(uint64_t *out) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < Num<NQ>::ORDER; i += (long long)gridDim.x * 256)
-    out[i] = Num<NQ>::element((uint64_t)i);
-}
-
-// seeded uniform elements: splitmix64 indices into the sorted element list
-__global__ void k_sample(const uint64_t *sorted, long long order, unsigned long long seed, long long n, uint64_t *out) {
+// seeded uniform elements: splitmix64 numbers of elements in the order of their tableaux
+template <int NQ> __global__ __launch_bounds__(256) void k_sample(unsigned long long seed, long long n, uint64_t *out) {
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
     uint64_t z = seed + (uint64_t)(i + 1) * 0x9e3779b97f4a7c15ull;
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
     z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
     z ^= z >> 31;
-    out[i] = sorted[z % (uint64_t)order];
+    out[i] = Num<NQ>::element(z % (uint64_t)Num<NQ>::ORDER);
   }
 }
 
@@ -451,8 +468,6 @@ struct chz_cliff {
   std::vector<long> levels;
   hipStream_t stream = nullptr;
   double build_ms = 0;
-  uint64_t *sorted = nullptr;          // elements sorted by tableau (built on the first sample)
-  long long order = 0;
 };
 
 #define CLCHK(x)                                                                         \
@@ -475,8 +490,8 @@ template <int NQ> static int cliff_fill(chz_cliff *c) {
   long long slots = 64;
   while (slots < 2 * C) slots <<= 1;
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  // [slots | planes | keys], and for the build [seen | two frontiers | counts | neighbours]
-  const size_t o_pl = up(slots * 8), o_key = o_pl + up(C * 32), bytes = o_key + up(C * 8);
+  // [slots | planes | smallest distances | keys], and for the build [seen | two frontiers | counts | neighbours]
+  const size_t o_pl = up(slots * 8), o_min = o_pl + up(C * 32), o_key = o_min + up(C), bytes = o_key + up(C * 8);
   const size_t w_f0 = up(C * 8), w_f1 = 2 * w_f0, w_cnt = 3 * w_f0, w_nb = w_cnt + 256, wbytes = w_nb + up((size_t)sym_gates(NQ) * C * 4);
   uint8_t *work = nullptr;
   CLCHK(cl_malloc(&c->block, bytes));
@@ -485,7 +500,7 @@ template <int NQ> static int cliff_fill(chz_cliff *c) {
   uint8_t *blk = (uint8_t *)c->block;
   c->count = C;
   c->key = (uint64_t *)(blk + o_key);
-  c->T = Table{(unsigned long long *)blk, (uint32_t)(slots - 1), (const ulonglong2 *)(blk + o_pl), NQ};
+  c->T = Table{(unsigned long long *)blk, (uint32_t)(slots - 1), (const ulonglong2 *)(blk + o_pl), blk + o_min, NQ};
   uint64_t *seen = (uint64_t *)work, *front[2] = {(uint64_t *)(work + w_f0), (uint64_t *)(work + w_f1)};
   unsigned long long *cnt = (unsigned long long *)(work + w_cnt);
   uint32_t *nb = (uint32_t *)(work + w_nb);
@@ -501,7 +516,7 @@ template <int NQ> static int cliff_fill(chz_cliff *c) {
   hipLaunchKernelGGL(k_root, dim3(1), dim3(64), 0, c->stream, c->T, identity(NQ), front[0], seen, cnt);
   // every level is queued at once: one after the last finds the level before it empty and ends
   for (int d = 1; d <= MAXD; d++) {
-    const BfsArgs a{c->key, nb, front[(d - 1) & 1], front[d & 1], seen, (ulonglong2 *)(blk + o_pl), cnt, d};
+    const BfsArgs a{c->key, nb, front[(d - 1) & 1], front[d & 1], seen, (ulonglong2 *)(blk + o_pl), blk + o_min, cnt, d};
     hipLaunchKernelGGL(k_bfs<NQ>, grid, blockd, 0, c->stream, a);
   }
   CLCHK(hipGetLastError());
@@ -572,29 +587,16 @@ int chz_cliff_digest(const chz_cliff *c, uint64_t *digest, long long *entries) {
   return 0;
 }
 
-// the sorted element list, built once
-static int cliff_sorted(chz_cliff *c) {
-  if (c->sorted) return 0;
-  const long long n = c->count << (2 * c->n);
-  CLCHK(cl_malloc((void **)&c->sorted, n * 8));
-  const dim3 g((unsigned)std::min<long long>((n + 255) / 256, 16384)), b(256);
-  if (c->n == 1) hipLaunchKernelGGL(chz_cl::k_sorted<1>, g, b, 0, c->stream, c->sorted);
-  else if (c->n == 2) hipLaunchKernelGGL(chz_cl::k_sorted<2>, g, b, 0, c->stream, c->sorted);
-  else hipLaunchKernelGGL(chz_cl::k_sorted<3>, g, b, 0, c->stream, c->sorted);
-  CLCHK(hipStreamSynchronize(c->stream));
-  c->order = n;
-  return 0;
-}
-
-// count uniformly random group elements (tableaux), seeded: uniform indices into the elements sorted by tableau
+// count uniformly random group elements (tableaux), seeded: uniform numbers in the order of the tableaux, so that
+// samples do not depend on anything but the seed
 int chz_cliff_sample(chz_cliff *c, uint64_t seed, long long count, uint64_t *tab) {
   CLCHK(hipSetDevice(c->device));
-  if (const int rc = cliff_sorted(c)) return rc;
-  if (c->order <= 0) { chz_cl::g_err = "empty table"; return 4; }
   uint64_t *d = nullptr;
   CLCHK(cl_malloc((void **)&d, std::max<long long>(count, 1) * 8));
-  hipLaunchKernelGGL(chz_cl::k_sample, dim3((unsigned)std::min<long long>((count + 255) / 256 + 1, 4096)), dim3(256), 0,
-                     c->stream, c->sorted, c->order, (unsigned long long)seed, count, d);
+  const dim3 g((unsigned)std::min<long long>((count + 255) / 256 + 1, 4096)), b(256);
+  if (c->n == 1) hipLaunchKernelGGL(chz_cl::k_sample<1>, g, b, 0, c->stream, (unsigned long long)seed, count, d);
+  else if (c->n == 2) hipLaunchKernelGGL(chz_cl::k_sample<2>, g, b, 0, c->stream, (unsigned long long)seed, count, d);
+  else hipLaunchKernelGGL(chz_cl::k_sample<3>, g, b, 0, c->stream, (unsigned long long)seed, count, d);
   CLCHK(hipMemcpyAsync(tab, d, count * 8, hipMemcpyDeviceToHost, c->stream));
   CLCHK(hipStreamSynchronize(c->stream));
   (void)cl_free(d);
@@ -697,16 +699,15 @@ int chz_cliff_readback(chz_cliff *c, const uint64_t *tab, long long nq, int maxl
   return 0;
 }
 
-#include "cliffopt.h"
-
 void chz_cliff_free(chz_cliff *c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->block) (void)cl_free(c->block);
-  if (c->sorted) (void)cl_free(c->sorted);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
 
 }  // extern "C"
+
+#include "cliffopt.h"

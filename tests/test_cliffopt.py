@@ -117,6 +117,30 @@ def test_hip_equals_oracle_two_qubits(oracle2, seed):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,t,beam", [(1, 1, 16), (1, 5, 255), (2, 1, 255), (2, 2, 1), (2, 4, 3), (2, 7, 255)])
+def test_hip_equals_oracle_over_beams(n, t, beam):
+    """beams of one state, more states than a step has items, and the widest: the same gates as the oracle, whose beam
+    costs every placement"""
+    L = ctypes.CDLL(os.path.join(ROOT, "oracle", "libclifford_oracle.so"))
+    L.orc_cliff_build.restype = ctypes.c_void_p
+    L.orc_cliff_opt.argtypes = [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_long, ctypes.c_int, ctypes.c_char_p,
+                                ctypes.c_long]
+    L.orc_cliff_free.argtypes = [ctypes.c_void_p]
+    if n == 1:
+        job = f"1 {t}\n" + "".join(f"0 {i % 2}\n" for i in range(t)) + "3 h 0 s 0 h 0\n" * t + "2 x 0 sdg 0\n"
+    else:
+        job, _ = CL.random_job(40 + t, n=n, t=t)
+    h = L.orc_cliff_build(n, 0)
+    table = CL.CliffordTable(n)
+    try:
+        want = oracle_opt(L, h, job, beam).strip().splitlines()
+        assert table.optimize(job, beam).strip().splitlines()[1:] == want[1:]
+    finally:
+        table.close()
+        L.orc_cliff_free(h)
+
+
+@pytest.mark.gpu
 def test_hip_three_qubits_equivalent_and_shorter():
     t = CL.CliffordTable(3)
     try:

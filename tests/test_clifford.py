@@ -96,3 +96,28 @@ def test_hip_table_identical_to_oracle(orc, n):
         assert w == list(out[:ln])
     orc.orc_cliff_free(h)
     T.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2])
+def test_samples_number_the_elements_in_tableau_order(n):
+    """a sample is the splitmix64 number modulo the group order among the tableaux in increasing order, which are listed
+    here by closure under the generators"""
+    T = clifford.CliffordTable(n)
+    try:
+        words = {T.tableau([]): []}
+        todo = list(words)
+        while todo:
+            t = todo.pop()
+            for g in range(T.ng):
+                w = words[t] + [g]
+                x = T.tableau(w)
+                if x not in words:
+                    words[x] = w
+                    todo.append(x)
+        order = sorted(words)
+        assert len(order) == ORDERS[n]
+        r = clifford.SplitMix64(99)
+        assert T.sample(99, 300) == [order[r.next() % len(order)] for _ in range(300)]
+    finally:
+        T.close()
