@@ -350,21 +350,92 @@ __global__ void k_root(Table T, uint64_t id, uint64_t *front, uint64_t *seen, un
   cnt[0] = 1;
 }
 
-// tableaux of words (letters are gate-set indices, applied in order), one lane per word
-__global__ void k_words(Gates G, const uint8_t *letters, const long long *offs, long long nq, uint64_t *tab) {
-  for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < nq; q += (long long)gridDim.x * blockDim.x) {
-    uint64_t T = identity(G.n);
-    for (long long j = offs[q]; j < offs[q + 1]; j++) {
-      const int g = letters[j];
-      T = apply(T, G.n, G.k[g], G.a[g], G.b[g]);
-    }
-    tab[q] = T;
-  }
+// ---- words.  A tableau's X images and its Z images are two words of n rows each; a gate acts on all rows of a word
+// at once.  A letter's gate is packed as its qubits and one flag per term of the update:
+enum { W_HS = 8, W_SDG, W_Z, W_X, W_CX, W_H, W_SZ };     // bits 0-3: a, 4-7: b; H or S, Sdg, Z, X, CX, H, S or Sdg
+static uint32_t pack_gate(int k, int a, int b) {
+  uint32_t f = (uint32_t)a | (uint32_t)b << 4;
+  if (k == 0) f |= 1u << W_HS | 1u << W_H;
+  else if (k == 1) f |= 1u << W_HS | 1u << W_SZ;
+  else if (k == 2) f |= 1u << W_SDG | 1u << W_SZ;
+  else if (k == 3) f |= 1u << W_X;
+  else if (k == 4) f |= 1u << W_Z;
+  else f |= 1u << W_CX;
+  return f;
+}
+struct WordGates { uint32_t g[32]; };
+static WordGates word_gates(const Gates &G) {
+  WordGates w{};
+  for (int i = 0; i < G.ng; i++) w.g[i] = pack_gate(G.k[i], G.a[i], G.b[i]);
+  return w;
+}
+template <int NQ> __device__ __forceinline__ uint32_t apply_rows(uint32_t w, uint32_t g) {
+  constexpr uint32_t M = NQ == 1 ? 1u : NQ == 2 ? 1u | 1u << 5 : 1u | 1u << 7 | 1u << 14;      // bit 0 of every row
+  auto on = [&](int bit) -> uint32_t { return (uint32_t)__builtin_amdgcn_sbfe((int)g, (unsigned)bit, 1u); };
+  const uint32_t a = g & 15u, b = (g >> 4) & 15u;
+  const uint32_t xa = w >> a & M, za = w >> (NQ + a) & M, xb = w >> b & M, zb = w >> (NQ + b) & M;
+  const uint32_t h = (xa ^ za) & on(W_H), xc = xa & on(W_CX);
+  const uint32_t sign = (xa & ((za & on(W_HS)) | (~za & on(W_SDG)) | on(W_Z))) | (za & on(W_X)) | (xc & zb & ~(xb ^ za));
+  return w ^ (sign << (2 * NQ)) ^ (h << a) ^ ((h ^ (xa & on(W_SZ)) ^ (zb & on(W_CX))) << (NQ + a)) ^ (xc << b);
 }
 
-// batched lookups (src/clifford.cu:207-210), one lane per query
-__global__ __launch_bounds__(256) void k_find(Table T, const uint64_t *q, long long nq, int *out) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nq; i += (long long)gridDim.x * 256) out[i] = find1(T, q[i]);
+// distances of words (letters are gate-set indices, applied in order; src/clifford.cu:207-210), one lane per word.  A
+// wave's letters are one range of memory: it is read as whole dwords into LDS, where the lanes pick their letters, when
+// it fits and the lanes' ranges lie in it; otherwise each lane reads its letters from global memory.
+// What bounded this: a serial chain per lane of byte loads from global memory, each letter's gate read from a per-lane
+// index into the kernel arguments and applied row by row in six divergent ways, then a second kernel for the look-ups:
+// 96 + 5 us for 1e5 words of 5 to 40 letters, 19 us here.
+constexpr int WORD_SPAN = 4096;        // bytes of letters per wave in LDS
+template <int NQ>
+__global__ __launch_bounds__(256) void k_query(Table T, WordGates G, const uint8_t *letters, const long long *offs, long long nq,
+                                               int *out) {
+  constexpr int HB = NQ * (2 * NQ + 1);      // bits of a word of n rows
+  __shared__ uint32_t stage[4][WORD_SPAN / 4], gate[32];
+  if (threadIdx.x < 32) gate[threadIdx.x] = G.g[threadIdx.x];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const uint64_t id = identity(NQ);
+  for (long long q0 = wave_index() * 64; q0 < nq; q0 += (long long)gridDim.x * 256) {
+    const long long q = q0 + lane, last = q0 + 64 < nq ? q0 + 64 : nq;
+    const long long beg = q < nq ? offs[q] : 0, end = q < nq ? offs[q + 1] : 0;
+    const long long lo = offs[q0], hi = offs[last];
+    // LDS byte i holds the letter at address base + i (base: lo rounded down to a dword)
+    const uintptr_t first = (uintptr_t)letters + (uintptr_t)lo, base = first & ~(uintptr_t)3, stop = (uintptr_t)letters + (uintptr_t)hi;
+    const bool staged = hi - lo <= WORD_SPAN - 4 && hi >= lo &&
+                        __ballot(q < nq && beg < end && (beg < lo || end > hi)) == 0;
+    uint32_t x = (uint32_t)(id & ((1ull << HB) - 1)), z = (uint32_t)(id >> HB);
+    if (staged) {
+      uint8_t *const s8 = (uint8_t *)stage[wv];
+      const uintptr_t d0 = (first + 3) & ~(uintptr_t)3, d1 = stop & ~(uintptr_t)3;      // whole dwords [d0, d1)
+      for (uintptr_t p = d0 + 4 * lane; p < d1; p += 256) stage[wv][(p - base) >> 2] = *(const uint32_t *)p;
+      // the bytes before and behind them, at most three each
+      if (lane < 3 && first + lane < d0 && first + lane < stop) s8[first + lane - base] = *(const uint8_t *)(first + lane);
+      if (lane >= 4 && lane < 7 && d1 >= d0 && d1 + (lane - 4) < stop) s8[d1 + (lane - 4) - base] = *(const uint8_t *)(d1 + (lane - 4));
+      __builtin_amdgcn_wave_barrier();
+      const int off = (int)((uintptr_t)letters + (uintptr_t)beg - base), len = beg < end ? (int)(end - beg) : 0;
+      for (int j = 0; j < len; j++) {
+        const uint32_t g = gate[s8[off + j] & 31];
+        x = apply_rows<NQ>(x, g);
+        z = apply_rows<NQ>(z, g);
+      }
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      for (long long j = beg; j < end; j++) {
+        const uint32_t g = gate[letters[j] & 31];
+        x = apply_rows<NQ>(x, g);
+        z = apply_rows<NQ>(z, g);
+      }
+    }
+    if (q < nq) out[q] = find1(T, (uint64_t)x | (uint64_t)z << HB);
+  }
+}
+static void launch_query(const Table &T, const Gates &G, const uint8_t *letters, const long long *offs, long long nq, int *out,
+                         hipStream_t s) {
+  const dim3 g((unsigned)std::min<long long>((nq + 255) / 256 + (nq == 0), 4096)), b(256);
+  const WordGates w = word_gates(G);
+  if (G.n == 1) hipLaunchKernelGGL(k_query<1>, g, b, 0, s, T, w, letters, offs, nq, out);
+  else if (G.n == 2) hipLaunchKernelGGL(k_query<2>, g, b, 0, s, T, w, letters, offs, nq, out);
+  else hipLaunchKernelGGL(k_query<3>, g, b, 0, s, T, w, letters, offs, nq, out);
 }
 
 // optimal words: one wave per query; each step, lane g tests the predecessor through gate g (its distance
@@ -430,36 +501,11 @@ static thread_local std::string g_err;
 }  // namespace chz_cl
 
 namespace chz_cl {
-
-// Fixed staging for chz_cliff_query_words_noalloc: the tableaux of up to kQueryScratch words, written by k_words
-// and read by k_find.  Each GPU the library runs on holds its own copy until the process ends.  Host code never
-// uses this name as an address: scratch_address() resolves each device's copy once, with that device current.
-constexpr long long kQueryScratch = 1ll << 20;
-__device__ __align__(256) uint64_t scratch[kQueryScratch];
-
-constexpr int kMaxDevices = 64;
-static std::mutex g_scratch_mu;
-static uint64_t *g_scratch_dev[kMaxDevices];
-
-// the device address of this device's scratch (the device must be current); 0 or 5 with g_err set
-static int scratch_address(int device, uint64_t **out) {
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (device < 0 || device >= kMaxDevices) { g_err = "device ordinal out of range"; return 3; }
-  if (!g_scratch_dev[device]) {
-    void *p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p) { g_err = std::string("hipGetSymbolAddress: ") + hipGetErrorString(e); return 5; }
-    g_scratch_dev[device] = (uint64_t *)p;
-  }
-  *out = g_scratch_dev[device];
-  return 0;
+constexpr long long kQueryScratch = 1ll << 20;      // most words of one chz_cliff_query_words_noalloc call
 }
-
-}  // namespace chz_cl
 
 struct chz_cliff {
   int n = 0, device = 0;
-  uint64_t *scratch = nullptr;         // this device's chz_cl::scratch (its device address)
   chz_cl::Gates G{};
   chz_cl::Table T{};
   void *block = nullptr;               // the table's arrays, one block
@@ -545,12 +591,9 @@ int chz_cliff_build(int n, int device, chz_cliff **out) {
   *out = nullptr;
   if (n < 1 || n > 3) { chz_cl::g_err = "n must be 1..3"; return 3; }
   CLCHK(hipSetDevice(device));
-  uint64_t *scratch = nullptr;
-  if (const int rc = chz_cl::scratch_address(device, &scratch)) return rc;
   chz_cliff *c = new chz_cliff();
   c->n = n;
   c->device = device;
-  c->scratch = scratch;
   c->G = chz_cl::gate_set(n);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     chz_cl::g_err = "HIP error: no stream";
@@ -612,11 +655,9 @@ int chz_cliff_query_words(chz_cliff *c, const uint8_t *letters, const long long 
   const long long nl = offs[nq];
   uint8_t *dl = nullptr;
   long long *doff = nullptr;
-  uint64_t *tab = nullptr;
   int *dd = nullptr;
   CLCHK(cl_malloc((void **)&dl, std::max<long long>(nl, 1)));
   CLCHK(cl_malloc((void **)&doff, (nq + 1) * 8));
-  CLCHK(cl_malloc((void **)&tab, std::max<long long>(nq, 1) * 8));
   CLCHK(cl_malloc((void **)&dd, std::max<long long>(nq, 1) * 4));
   CLCHK(hipMemcpyAsync(dl, letters, nl, hipMemcpyHostToDevice, c->stream));
   CLCHK(hipMemcpyAsync(doff, offs, (nq + 1) * 8, hipMemcpyHostToDevice, c->stream));
@@ -624,10 +665,7 @@ int chz_cliff_query_words(chz_cliff *c, const uint8_t *letters, const long long 
   CLCHK(hipEventCreate(&e0));
   CLCHK(hipEventCreate(&e1));
   CLCHK(hipEventRecord(e0, c->stream));
-  hipLaunchKernelGGL(chz_cl::k_words, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
-                     c->stream, c->G, dl, doff, nq, tab);
-  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
-                     c->stream, c->T, tab, nq, dd);
+  chz_cl::launch_query(c->T, c->G, dl, doff, nq, dd, c->stream);
   CLCHK(hipEventRecord(e1, c->stream));
   CLCHK(hipMemcpyAsync(dist, dd, nq * 4, hipMemcpyDeviceToHost, c->stream));
   CLCHK(hipStreamSynchronize(c->stream));
@@ -638,14 +676,12 @@ int chz_cliff_query_words(chz_cliff *c, const uint8_t *letters, const long long 
   (void)hipEventDestroy(e1);
   (void)cl_free(dl);
   (void)cl_free(doff);
-  (void)cl_free(tab);
   (void)cl_free(dd);
   return 0;
 }
 
-// chz_cliff_query_words with device buffers and no allocation: the tableaux are staged in this device's fixed
-// scratch (at most kQueryScratch words per call); the kernels go on `stream` (NULL: the table's own stream,
-// synchronised before returning).  Calls that overlap on one GPU share the scratch and race.
+// chz_cliff_query_words with device buffers and no allocation, at most kQueryScratch words per call; the kernel goes on
+// `stream` (NULL: the table's own stream, synchronised before returning).
 int chz_cliff_query_words_noalloc(chz_cliff *c, const uint8_t *d_letters, const long long *d_offs, long long nq,
                                   int *d_dist, void *stream) {
   if (nq < 0 || (nq > 0 && (!d_letters || !d_offs || !d_dist))) { chz_cl::g_err = "bad arguments"; return 3; }
@@ -658,10 +694,7 @@ int chz_cliff_query_words_noalloc(chz_cliff *c, const uint8_t *d_letters, const 
   chz::RelaxedCapture relaxed;
   CLCHK(hipSetDevice(c->device));
   hipStream_t st = stream ? (hipStream_t)stream : c->stream;
-  hipLaunchKernelGGL(chz_cl::k_words, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
-                     st, c->G, d_letters, d_offs, nq, c->scratch);
-  hipLaunchKernelGGL(chz_cl::k_find, dim3((unsigned)std::min<long long>((nq + 255) / 256 + 1, 4096)), dim3(256), 0,
-                     st, c->T, c->scratch, nq, d_dist);
+  chz_cl::launch_query(c->T, c->G, d_letters, d_offs, nq, d_dist, st);
   CLCHK(hipGetLastError());
   if (!stream) CLCHK(hipStreamSynchronize(st));
   return 0;

@@ -90,3 +90,32 @@ def test_noalloc_refuses_more_than_its_scratch(table):
     rc = fn(table.h, ctypes.c_void_p(8), ctypes.c_void_p(8), (1 << 20) + 1, ctypes.c_void_p(8), None)
     assert rc == 4
     assert "scratch" in CL._lib().chz_cliff_last_error().decode()
+
+
+@pytest.mark.parametrize("count,lengths,shift", [(1, (0,), 0), (63, (1, 2, 3), 1), (64, (0, 64), 2), (65, (63, 64), 3),
+                                                 (257, (0, 1, 5000), 1), (300, (5, 40), 0)])
+def test_noalloc_at_the_edges_of_the_staged_letters(count, lengths, shift):
+    """words of 0 letters, waves whose letters fill the LDS stage nearly to its last bytes and overflow it, letters that
+    start at any byte of a dword, partial waves: each distance equals the length of the word read back for its tableau"""
+    import random
+    rng = random.Random(count)
+    T = CL.CliffordTable(2)
+    hip = _Hip()
+    try:
+        words = [[rng.randrange(T.ng) for _ in range(lengths[i % len(lengths)])] for i in range(count)]
+        want = [len(w) for w in T.readback([T.tableau(w) for w in words], 32)]
+        assert T.query_words(words)[0] == want
+        flat = np.array([0] * shift + [g for w in words for g in w] + [0], dtype=np.uint8)
+        offs = np.zeros(count + 1, dtype=np.int64)
+        offs[1:] = np.cumsum([len(w) for w in words])
+        d_letters, d_offs = hip.upload(flat), hip.upload(offs)
+        d_dist = hip.upload(np.full(count, -7, dtype=np.int32))
+        at = ctypes.c_void_p(d_letters.value + shift)
+        print(f"noalloc query: {count} words of {lengths} letters at byte {shift}", flush=True)
+        assert _noalloc()(T.h, at, d_offs, count, d_dist, None) == 0
+        got = hip.download(d_dist, np.zeros(count, dtype=np.int32)).tolist()
+        for p in (d_letters, d_offs, d_dist):
+            hip.L.hipFree(p)
+        assert got == want
+    finally:
+        T.close()
