@@ -35,6 +35,8 @@ constexpr int TC_MAX = 8;                      // T-bound classes cached per par
 struct KSpec {                                 // device view of a spec (kernel argument)
   int n, G, depth, standard, lite, tdiv, gk, nsym, ncuts, have_table;
   int cx_mono;                                 // cx table non-decreasing in every cut need
+  int pre;                                     // bounds may settle a child before its residual is formed: the
+                                               // spec has bounds and they are 0 at the goal (the identity)
   int cxlds;                                   // the cx table fits the expansion kernel's LDS copy (CXL_MAX bytes)
   int ncx;                                     // cx table entries
   int ncd;                                     // distinct gate cdel values (0: more than CD_MAX)
@@ -164,19 +166,10 @@ __device__ __forceinline__ uint32_t fp_of(int4 v, const uint32_t *wm) {
   return s >= P_MOD ? s - P_MOD : s;
 }
 
-__device__ __forceinline__ int combine_bound(int h, int t, int c2, int supp) {   // src/cheese.cu:599-607
-  int best = 1 << 30;
-  const int hi = c2 > supp ? c2 : supp;
-  for (int c = c2; c <= hi; c++) {
-    const int one = (h + t > supp - 2 * c) ? h + t : supp - 2 * c;
-    if (c + one < best) best = c + one;
-  }
-  return best;
-}
-
-// The largest t with combine_bound(h, t, c2, supp) <= rem (negative: none), for rem >= 0.  The bound is at most
-// rem exactly when some c in [c2, max(c2, supp)] has c + h + t <= rem and supp - c <= rem; the smallest such c is
-// max(c2, supp - rem), which never exceeds max(c2, supp).
+// The bound of src/cheese.cu:599-607, the least over c in [c2, max(c2, supp)] of c + max(h + t, supp - 2c), as the
+// largest t for which it is at most rem (negative: none), for rem >= 0.  It is at most rem exactly when some c of the
+// range has c + h + t <= rem and supp - c <= rem; the smallest such c is max(c2, supp - rem), which never exceeds
+// max(c2, supp).
 __device__ __forceinline__ int t_budget(int h, int c2, int supp, int rem) {
   const int c = c2 > supp - rem ? c2 : supp - rem;
   return rem - h - c;

@@ -25,13 +25,14 @@ namespace chz {
 
 // ------------------------------------------------------------------------------------------------------
 // counters of one level (device): indices into a u64 array
-// C_EVAL children whose residual is formed, C_CHEAP through the structural bounds, C_CUTS cut ranks computed,
+// C_EVAL children past the windows, C_PRE those of them settled from the parent's bounds (the others' residuals are
+// formed), C_CHEAP through the structural bounds, C_CUTS cut ranks computed,
 // C_NEEDT T-bound evaluations (their f = 0 parts), C_KEYS class keys, C_TPASS flip-pair passes of the T bound: the
 // stage counts of the expansion's work model
 // C_M, C_NCC: the level's parents and children, written by the host with the level's control upload (read by the
 // kernels of a captured level step, whose launches are sized for a capacity)
 enum { C_W2 = 0, C_W3, C_DEAD, C_FOUND, C_ALIVE, C_OVF, C_NEEDT, C_FIRST, C_RUNS, C_REPOVF, C_KEPT, C_EVAL, C_SURV,
-       C_CHEAP, C_CUTS, C_KEYS, C_TPASS, C_M, C_NCC, C_N };
+       C_CHEAP, C_CUTS, C_KEYS, C_TPASS, C_PRE, C_M, C_NCC, C_N };
 // per-instance counters of one level (a batch carries several searches that share the spec's gate set)
 enum { IC_W2 = 0, IC_W3, IC_DEAD, IC_FOUND, IC_ALIVE, IC_OVF, IC_FIRST, IC_N };
 
@@ -69,6 +70,7 @@ template <int NQ> __device__ __forceinline__ GateHdr wuni(const GateHdr &h) {
                  wuni<NQ>(h.cls)};
 }
 constexpr int MAXG = 64;
+constexpr int PRE_SPLIT = 4;    // lane groups per parent up to which children are settled from the parent's bounds
 
 // The expansion kernel's LDS tables, built once per context on the host (build_level_tabs) and copied into LDS by
 // every block with coalesced 16-byte loads; built inside the kernel they cost each block scattered global loads,
@@ -80,6 +82,11 @@ struct LevelTabs {
   GateHdr shdr[MAXG];
   uint8_t spos[16 * 64];           // n = 3: position of entry e under symmetry y (y * 64 + e)
   uint8_t scx[CXL_MAX];            // the cx table when it fits (KSpec::cxlds)
+  // per candidate, for the bounds from the parent alone: bits 0-7 tdel, 8-10 qubits, 11-15 the most the sqrt2 exponent
+  // can fall (0 for a permutation of unit entries, which leaves divisibility by sqrt2 as it is, else the gate's own
+  // exponent), 16-23 cut-delta class, 24 an H (the exponent is read off the parent
+  // exactly), 25-31 1 + the T-bound class
+  uint32_t spre[MAXG];
   uint8_t scsrc[CSRC_MAX * 64];    // cut i's operator-Schmidt matrix: entry source of lane le (i * GS + le)
 };
 static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
@@ -113,7 +120,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   uint32_t *const tl = stally[threadIdx.x / GS];
   for (int i = le; i < 8; i += GS) tl[i] = 0;
   __builtin_amdgcn_wave_barrier();
-  uint32_t n_eval = 0, n_t = 0, n_cheap = 0, n_cuts = 0, n_keys = 0, n_tp = 0;
+  uint32_t n_eval = 0, n_pre = 0, n_t = 0, n_cheap = 0, n_cuts = 0, n_keys = 0, n_tp = 0;
   int cur = -1;
   auto flush = [&]() {
     __builtin_amdgcn_wave_barrier();
@@ -155,11 +162,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const int4 S = a.res[pi * E + le];
     const int pk = wuni<NQ>(a.pk[pi]), g1 = wuni<NQ>((int)a.g1[pi]), g2 = wuni<NQ>((int)a.g2[pi]);
     const uint32_t pbw = (uint32_t)wuni<NQ>((int)a.pb[pi]);
-    const bool small = gall<GS>(zmag(S) < (1u << 28));
+    const uint32_t mag = zmag(S);
+    const bool small = gall<GS>(mag < (1u << 28));
     // A search whose circuit is found at this level ends with it: its parents without a goal child (no
     // BW_GOAL) are passed over once their coefficients rule out an overflowing child.  Goal children come only
     // from BW_GOAL parents, so the level's found count, first circuit and overflow test are unchanged.
-    if (a.gflag && !(pbw & BW_GOAL) && wuni<NQ>((int)a.gflag[inst]) != 0 && gall<GS>(zmag(S) <= sp.maglim)) {
+    if (a.gflag && !(pbw & BW_GOAL) && wuni<NQ>((int)a.gflag[inst]) != 0 && gall<GS>(mag <= sp.maglim)) {
       for (int g = gbeg + le; g < gend; g += GS) a.status[pl * G + g] = ST_DEAD;
       continue;
     }
@@ -180,10 +188,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     // exact bound, else it is a lower bound (a transform stopped once the child was dead)
     uint64_t tc_val = 0;
     uint32_t tc_ok = 0, tc_ex = 0;
-    uint64_t w2m = 0, w3m = 0;
+    // Bounds from the parent alone, one candidate per lane: the child's sqrt2 exponent is at least the parent's less
+    // what the gate can take, its T bound and cut needs are bracketed as below, and a qubit the gate leaves alone
+    // stays as non-trivial as it is in the parent.  The bound combination grows with each of these, so a child that
+    // the lower ends put over its budget is dead, and its residual is not formed: on the Toffoli budget-12 proof 2.61
+    // of 5.71 million children past the windows still form one (3.12 without the T siblings below).  Only where no child
+    // can overflow (which would be reported) and the goal's own bounds are 0 (a goal child is never over its budget).
+    // On the budget-14 proof the expansion takes 111 ms instead of 139.  Where a parent's candidates are split over
+    // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.
+    const bool pre = sp.pre && gsplit <= PRE_SPLIT && gall<GS>(mag <= sp.maglim);
+    const bool tparent = (pbw & BW_TUNK) != BW_TUNK;
+    // H on qubit q pairs the columns c and c ^ 2^q as their sum and difference over sqrt2: the exponent rises by one,
+    // less one if sqrt2 divides every sum (the parities of a + c and b + d agree in each pair), less another if 2 does
+    // (every coefficient's parity agrees); it falls by no more than one
+    int he = 0;                                  // bits q, 4 + q: the first, the second holds for qubit q
+    if (pre) {
+      const uint64_t ba = gballot<GS>(S.x & 1), bb = gballot<GS>(S.y & 1), bc = gballot<GS>(S.z & 1), bd = gballot<GS>(S.w & 1);
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        auto differ = [&](uint64_t m) { return (m ^ (m >> (1 << q))) & pair_mask<NQ>(q); };
+        if (!(differ(ba ^ bc) | differ(bb ^ bd))) he |= 1 << q;
+        if (!(differ(ba) | differ(bb) | differ(bc) | differ(bd))) he |= 16 << q;
+      }
+    }
+    const int pq = pre && !sp.lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S))) : 0;
+    uint64_t w2m = 0, w3m = 0, dm = 0;
+    int lim = 1 << 30, tcl = -1;                 // n = 3: candidate `lane`'s largest T bound by these bounds; its T class
     for (int b0 = 0; b0 < G; b0 += GS) {
       const int g = b0 + le;
-      bool c2 = false, c3 = false;
+      bool c2 = false, c3 = false, dead = false;
       if (g < G && g1 != 255) {
         c2 = sp.bad2[g1 * G + g] != 0;
         if (g2 != 255) {
@@ -191,17 +224,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
           c3 = ((sp.bad3[tri >> 5] >> (tri & 31)) & 1) != 0;
         }
       }
+      if (pre && g < G) {
+        const uint32_t w = tb.spre[g];
+        const int td = (int)(w & 255u), Tp = (int)(pbw & BW_TUNK);
+        const int T = tparent && td != 255 && Tp > td ? Tp - td : 0;
+        const int gm = (int)((w >> 8) & 7u), hq = he >> (__ffs(gm) - 1);
+        const int kd = (w >> 24) & 1u ? pk + 1 - (hq & 1) - ((hq >> 4) & 1) : pk - (int)((w >> 11) & 31u), h = kd > 0 ? kd : 0;
+        const int c2lo = cdcache ? (int)((c2c >> (8 * ((w >> 16) & 255u))) & 0xff) : 0;
+        const int l = t_budget(h, c2lo, __popc(pq & ~gm), rem) * sp.tdiv;
+        dead = T > l;
+        if constexpr (NQ == 3) {
+          lim = l;
+          tcl = (int)(w >> 25) - 1;
+        }
+      }
       w2m |= gballot<GS>(c2) << b0;
       w3m |= gballot<GS>(c3) << b0;
+      dm |= gballot<GS>(dead) << b0;
     }
-    for (int g = gbeg; g < gend; g++) {
+    // (a split whose share of the candidates is empty has gbeg >= gend, and gbeg may lie beyond bit 63)
+    const uint64_t range = gbeg >= gend ? 0ull : (gend - gbeg < 64 ? (1ull << (gend - gbeg)) - 1 : ~0ull) << gbeg;
+    uint64_t todo = range & ~(w2m | w3m | dm);
+    w2m &= range;
+    w3m &= range & ~w2m;
+    dm &= range & ~w2m & ~w3m;
+    const uint32_t npre = (uint32_t)__popcll(dm);
+    n_eval += npre;
+    n_pre += npre;
+    // the settled children's status in one store per lane, their tallies at once
+    for (int b0 = 0; b0 < G; b0 += GS) {
+      const int g = b0 + le;
+      if (g < G && (((w2m | w3m | dm) >> g) & 1))
+        a.status[pl * G + g] = (w2m >> g) & 1 ? ST_W2 : (w3m >> g) & 1 ? ST_W3 : ST_DEAD;
+    }
+    if (le == 0) {
+      if (w2m) atomicAdd(&tl[ST_W2], (uint32_t)__popcll(w2m));
+      if (w3m) atomicAdd(&tl[ST_W3], (uint32_t)__popcll(w3m));
+      if (dm) atomicAdd(&tl[ST_DEAD], npre);
+    }
+    while (todo) {
+      const int g = wuni<NQ>(__ffsll((long long)todo) - 1);
+      todo &= todo - 1;
       const long long cc = pl * G + g;
-      uint8_t stt = 255;
-      if ((w2m >> g) & 1) stt = ST_W2;
-      else if ((w3m >> g) & 1) stt = ST_W3;
+      uint8_t stt;
       uint64_t key = 0;
       uint32_t bw = BW_TUNK;
-      if (stt == 255) {
+      {
         // child residual entry (r, c) = sum_m P[r][x_m] ginv[m][lc] (src/cheese.cu:146-174)
         const GateHdr h = wuni<NQ>(shdr[g]);
         int lc = (c >> h.q0) & 1;
@@ -272,7 +340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               // matrix exponent h.tdel (Clifford gates keep it), each cut need drops by at most h.cdel.  The
               // bound combination is monotone in T and in the cut bound, so the brackets settle most children
               // before the cut ranks and the T transform are computed.
-              const bool tpar = (pbw & BW_TUNK) != BW_TUNK && h.tdel != 255;
+              const bool tpar = tparent && h.tdel != 255;
               const int Tp = (int)(pbw & BW_TUNK);
               // a sibling of the same T-bound class already has its exact bound (it is this child's too) or a
               // lower bound
@@ -287,7 +355,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               const int c2lo = cdcache ? (int)((c2c >> (8 * (h.cls & 0xff))) & 0xff)
                                : !sp.lite && sp.cx_mono && (pbw & BW_CUTS) ? cx_lower(sp, scx, (pbw & BW_NEEDS) >> 8, (uint32_t)h.cdel)
                                : 0;
-              if (combine_bound(hh, (T + sp.tdiv - 1) / sp.tdiv, c2lo, supp) > rem) alive = false;
+              // alive exactly when T / tdiv, rounded up, is at most t_budget: T <= t_budget * tdiv
+              if (T > t_budget(hh, c2lo, supp, rem) * sp.tdiv) alive = false;
               else {
                 if (!sp.lite) {
                   uint32_t needs = (pbw & BW_NEEDS) >> 8;
@@ -296,9 +365,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                   c2 = wuni<NQ>(cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, needs));
                   bw = (needs << 8 & ~BW_CUTS) | (sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
                 }
-                if (combine_bound(hh, (T + sp.tdiv - 1) / sp.tdiv, c2, supp) > rem) alive = false;
-                else if (!texact && tpar && rem <= 1 &&
-                         combine_bound(hh, (Tp + h.tdel + sp.tdiv - 1) / sp.tdiv, c2, supp) <= rem) {
+                const int tmax = t_budget(hh, c2, supp, rem) * sp.tdiv;
+                if (T > tmax) alive = false;
+                else if (!texact && tpar && rem <= 1 && Tp + h.tdel <= tmax) {
                   // alive whatever the exact T; its children (budget 0) need no inherited T bound
                   alive = true;
                 } else if (!texact) {
@@ -307,7 +376,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                     // the f = 0 part, then the flip-pair passes (odd first) while the lower bound leaves the child
                     // alive: at T bound T it is alive exactly when T <= tmax
                     uint32_t np = 0;
-                    T = t_bound16s<NQ>(st, s, k, le, T, t_budget(hh, c2, supp, rem) * sp.tdiv, np, texact);
+                    T = t_bound16s<NQ>(st, s, k, le, T, tmax, np, texact);
                     n_tp += np;
                   } else {
                     T = t_bound_any<NQ>(s, k, le);
@@ -317,8 +386,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                     tc_val = (tc_val & ~(0xffull << (8 * tc))) | (uint64_t)T << (8 * tc);
                     tc_ok |= 1u << tc;
                     if (texact) tc_ex |= 1u << tc;
+                    // siblings of the class that this bound puts over their budget (by the parent's bounds) are dead
+                    if constexpr (NQ == 3) {
+                      const uint64_t sib = gballot<GS>(tcl == tc && T > lim) & todo;
+                      if (sib) {
+                        todo &= ~sib;
+                        if ((sib >> lane) & 1) a.status[pl * G + lane] = ST_DEAD;
+                        const uint32_t ns = (uint32_t)__popcll(sib);
+                        if (le == 0) atomicAdd(&tl[ST_DEAD], ns);
+                        n_eval += ns;
+                        n_pre += ns;
+                      }
+                    }
                   }
-                  alive = combine_bound(hh, (T + sp.tdiv - 1) / sp.tdiv, c2, supp) <= rem;
+                  alive = T <= tmax;
                 }
               }
               if (alive && texact && T < (int)BW_TUNK) bw = (bw & ~BW_TUNK) | (uint32_t)T;
@@ -347,8 +428,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     __builtin_amdgcn_wave_barrier();
   }
   flush();
-  if (le != 0) n_eval = n_t = n_cheap = n_cuts = n_keys = n_tp = 0;     // one copy per group
+  if (le != 0) n_eval = n_pre = n_t = n_cheap = n_cuts = n_keys = n_tp = 0;     // one copy per group
   n_eval = gsum<64>(n_eval);
+  n_pre = gsum<64>(n_pre);
   n_t = gsum<64>(n_t);
   n_cheap = gsum<64>(n_cheap);
   n_cuts = gsum<64>(n_cuts);
@@ -356,6 +438,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   n_tp = gsum<64>(n_tp);
   if (lane == 0) {
     if (n_eval) atomicAdd(&a.cnt[C_EVAL], (unsigned long long)n_eval);
+    if (n_pre) atomicAdd(&a.cnt[C_PRE], (unsigned long long)n_pre);
     if (n_t) atomicAdd(&a.cnt[C_NEEDT], (unsigned long long)n_t);
     if (n_cheap) atomicAdd(&a.cnt[C_CHEAP], (unsigned long long)n_cheap);
     if (n_cuts) atomicAdd(&a.cnt[C_CUTS], (unsigned long long)n_cuts);
@@ -870,7 +953,7 @@ static double expand_ops(const chz_ctx *c, int nq, const unsigned long long *hc)
   // class key per lane: two 32-bit entry hashes (about 16 ops each), then per symmetry one slot summand (a 24-bit
   // and two 32-bit products with their shifts and xors, 13 ops) and its two-word share of the 64-bit sums
   const double key = E * (2 * 16.0 + 15.0 * c->ks.nsym);
-  return (double)hc[C_EVAL] * child + (double)hc[C_CHEAP] * cheap + (double)hc[C_CUTS] * cut +
+  return (double)(hc[C_EVAL] - hc[C_PRE]) * child + (double)hc[C_CHEAP] * cheap + (double)hc[C_CUTS] * cut +
          (double)hc[C_NEEDT] * t_f0_ops(nq) + (double)hc[C_TPASS] * t_pass_ops(nq) + (double)hc[C_KEYS] * key;
 }
 
@@ -1505,6 +1588,11 @@ static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const
         if (nz != 1) kind = 1;
       }
     }
+    const int fall = kind == 2 ? 0 : std::min(31, std::max(0, s.gates[g].gk));
+    bool had = d.nq == 1 && d.unit && d.ik == 1 && s.gates[g].gk == 1;
+    for (int i = 0; had && i < 4; i++) had = d.ph[i] == 0 || d.ph[i] == 4;
+    T.spre[g] = (uint32_t)had << 24 | (uint32_t)(d.cls >> 8) << 25 | (uint32_t)std::min(255, d.tdel) | (uint32_t)(d.mask & 7) << 8 | (uint32_t)fall << 11 |
+                (uint32_t)(d.cls & 0xff) << 16;
     T.shdr[g] = GateHdr{d.nq, d.L, d.mask, d.ik, d.q[0], d.q[1], d.q[2], kind, d.tdel, d.cutloc, d.cdel, d.cls};
   }
   if (n == 3)
@@ -1651,6 +1739,12 @@ static void upload_spec(chz_ctx *c) {
   k.n = s.n; k.G = G; k.depth = c->depth; k.standard = s.standard; k.lite = s.lite; k.tdiv = s.tdiv;
   k.gk = s.gk; k.nsym = c->grp.size(); k.ncuts = (int)s.cutmask.size(); k.have_table = !s.cxtable.empty();
   for (int i = 0; i < k.ncuts; i++) { k.cutmask[i] = s.cutmask[i]; k.cutsize[i] = s.cutsize[i]; k.rad[i] = s.rad[i]; }
+  // the goal is the identity: exponent 0, T bound 0, rank-1 cuts, no support
+  k.pre = (s.standard || s.lite) && s.gk == 0 && s.tdiv > 0;
+  for (int i = 0; i < N * N; i++) {
+    const Zq &z = s.goal[i];
+    if (z.a != (i / N == i % N) || z.b || z.c || z.d) k.pre = 0;
+  }
   // a cut bound from lowered needs is a lower bound only if the table never decreases when a need grows
   k.cx_mono = 1;
   k.ncx = (int)s.cxtable.size();

@@ -123,22 +123,32 @@ template <int NQ> __host__ __device__ constexpr uint64_t offdiag_mask(int q) {
   return m;
 }
 
-// number of qubits the matrix acts on non-trivially (src/cheese.cu:305-319); b = group ballot of the nonzero
+// lanes whose column has bit q clear, as a group-local mask
+template <int NQ> __host__ __device__ constexpr uint64_t pair_mask(int q) {
+  constexpr int N = 1 << NQ, GS = N * N;
+  uint64_t m = 0;
+  for (int le = 0; le < GS; le++)
+    if (!((le >> q) & 1)) m |= 1ull << le;
+  return m;
+}
+
+// qubits the matrix acts on non-trivially (src/cheese.cu:305-319), as a mask; b = group ballot of the nonzero
 // entries.  A nonzero entry off the qubit's diagonal blocks settles that qubit without comparing blocks.
-template <int NQ> __device__ __forceinline__ int support(int4 s, int le, uint64_t b) {
+template <int NQ> __device__ __forceinline__ int support_mask(int4 s, int le, uint64_t b) {
   constexpr int N = 1 << NQ, GS = N * N;
   const int r = le >> NQ, c = le & (N - 1);
-  int cnt = 0;
+  int m = 0;
 #pragma unroll
   for (int q = 0; q < NQ; q++) {
-    if (b & offdiag_mask<NQ>(q)) { cnt++; continue; }
     const int bit = 1 << q;
+    if (b & offdiag_mask<NQ>(q)) { m |= bit; continue; }
     const int4 o = gxor<GS>(s, bit * N + bit);
     const bool viol = !((r | c) & bit) && !zeq(s, o);
-    cnt += gany<GS>(viol);
+    m |= gany<GS>(viol) ? bit : 0;
   }
-  return cnt;
+  return m;
 }
+template <int NQ> __device__ __forceinline__ int support(int4 s, int le, uint64_t b) { return __popc(support_mask<NQ>(s, le, b)); }
 
 __host__ __device__ inline int spread_bits(int v, int mask, int n) {   // bit j of v -> j-th set bit of mask
   int out = 0, j = 0;

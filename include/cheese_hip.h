@@ -104,9 +104,10 @@ enum { CHZ_FAM_EXPAND = 0, CHZ_FAM_COMPACT, CHZ_FAM_SORT, CHZ_FAM_DEDUPE, CHZ_FA
 unsigned chz_time_kernels(chz_ctx *ctx, unsigned families);
 
 /* Stage counts of the last run's expansion (no reference counterpart; for measurement), the factors of its work
- * model: out[0] residuals formed, [1] children through the structural bounds, [2] cut ranks computed, [3] T-bound
- * evaluations, [4] class keys, [5] flip-pair passes of the T-bound evaluations (0 to 2 each: a pass runs only while
- * the child is undecided).  out holds 6 values; returns 6. */
+ * model: out[0] children past the windows (residuals formed, or settled from the parent's bounds), [1] children
+ * through the structural bounds, [2] cut ranks computed, [3] T-bound evaluations, [4] class keys, [5] flip-pair passes
+ * of the T-bound evaluations (0 to 2 each: a pass runs only while the child is undecided).  out holds 6 values; returns
+ * 6. */
 int chz_expand_stages(const chz_ctx *ctx, double *out);
 
 /* Autotuner (no reference counterpart): times every candidate expansion schedule (occupancy variant x grid cap x
