@@ -36,6 +36,17 @@ enum { C_W2 = 0, C_W3, C_DEAD, C_FOUND, C_ALIVE, C_OVF, C_NEEDT, C_FIRST, C_RUNS
 // per-instance counters of one level (a batch carries several searches that share the spec's gate set)
 enum { IC_W2 = 0, IC_W3, IC_DEAD, IC_FOUND, IC_ALIVE, IC_OVF, IC_FIRST, IC_N };
 
+// The expansion's blocks add up their waves' counts in LDS and add them to the counters in the stripe of their block
+// number; the host sums the stripes.  With every wave adding its 13 counts (2 qubits: 31) to one set of counters, the
+// additions to one cache line, 2 to 4 ns each whatever the kernel did meanwhile, set the time of levels of up to some
+// ten thousand parents: a 2-qubit level of 28 thousand parents took 855 us, its next one without counts 58.  Expansion
+// of eight 2-qubit searches 12.9 -> 2.2 ms, of the budget-9 Toffoli proof 0.35 -> 0.17 ms.
+enum { SG_EVAL = 0, SG_PRE, SG_NEEDT, SG_CHEAP, SG_CUTS, SG_KEYS, SG_TPASS, SG_N = 8 };
+constexpr int NSTRIPE = 16;
+static int slot_stripes(int ns) { return std::max(1, std::min(NSTRIPE, 256 / ns)); }    // of the per-slot counters
+// words of the counters: [C_N | stage stripes | slot stripes]
+static size_t counter_words(int ns) { return (size_t)C_N + (size_t)NSTRIPE * SG_N + (size_t)slot_stripes(ns) * ns * IC_N; }
+
 struct ExpandArgs {
   const int4 *res;          // parents' residuals, E entries each
   const int *pk;            // parents' sqrt2 exponents
@@ -47,11 +58,12 @@ struct ExpandArgs {
   uint64_t *keys;           // [ncc] class keys of kept children
   uint32_t *info;           // [ncc] bound words of kept children
   const uint32_t *pb;       // parents' bound words
-  unsigned long long *cnt;  // global counters (stage counts C_EVAL, C_CHEAP, C_CUTS, C_NEEDT, C_KEYS, C_TPASS)
+  unsigned long long *stage;  // NSTRIPE stripes of the stage counts (ST_N each)
   const uint32_t *pinst;    // instance slot of every parent of the level (null: one instance, slot 0)
   const int *rem;           // per slot: gate budget left after this level's gate (depth - t)
   const uint8_t *keepi;     // per slot: this level's survivors become parents (t < depth)
-  unsigned long long *icnt; // per slot: IC_N counters
+  unsigned long long *icnt; // per slot: IC_N counters, in nstr stripes istride apart
+  int nstr, istride;
   int gsplit;               // a parent's candidates are split among this many lane groups (small levels)
   const unsigned long long *npd;   // parents read on the device (captured step; gsplit then from tw), or null
   int tw;                   // candidate-split threshold in waves (with npd)
@@ -122,19 +134,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   __builtin_amdgcn_wave_barrier();
   uint32_t n_eval = 0, n_pre = 0, n_t = 0, n_cheap = 0, n_cuts = 0, n_keys = 0, n_tp = 0;
   int cur = -1;
+  unsigned long long *const icnt = a.icnt + (size_t)(blockIdx.x & (unsigned)(a.nstr - 1)) * a.istride;
+  // the counter of a status value
+  auto slot_of = [](int st) {
+    return st == ST_W2 ? IC_W2 : st == ST_W3 ? IC_W3 : st == ST_DEAD ? IC_DEAD : st == ST_FOUND ? IC_FOUND : st == ST_OVF ? IC_OVF : IC_ALIVE;
+  };
   auto flush = [&]() {
     __builtin_amdgcn_wave_barrier();
-    if (le == 0 && cur >= 0) {
-      unsigned long long *ic = a.icnt + (size_t)cur * IC_N;
-      const uint32_t w2 = tl[ST_W2], w3 = tl[ST_W3], dead = tl[ST_DEAD], found = tl[ST_FOUND], ovf = tl[ST_OVF],
-                     alive = tl[ST_ALIVE];
-      if (w2) atomicAdd(&ic[IC_W2], (unsigned long long)w2);
-      if (w3) atomicAdd(&ic[IC_W3], (unsigned long long)w3);
-      if (dead) atomicAdd(&ic[IC_DEAD], (unsigned long long)dead);
-      if (found) atomicAdd(&ic[IC_FOUND], (unsigned long long)found);
-      if (ovf) atomicAdd(&ic[IC_OVF], (unsigned long long)ovf);
-      if (alive) atomicAdd(&ic[IC_ALIVE], (unsigned long long)alive);
-    }
+    if (le == 0 && cur >= 0)
+      for (int i = 0; i <= ST_OVF; i++)
+        if (const uint32_t v = tl[i]) atomicAdd(&icnt[(size_t)cur * IC_N + slot_of(i)], (unsigned long long)v);
     __builtin_amdgcn_wave_barrier();
     for (int i = le; i < 8; i += GS) tl[i] = 0;
     __builtin_amdgcn_wave_barrier();
@@ -422,28 +431,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         a.status[cc] = stt;
         if (stt == ST_ALIVE && keep) { a.keys[cc] = key; a.info[cc] = bw; }
         if (stt == ST_FOUND)
-          atomicMin(&a.icnt[(size_t)inst * IC_N + IC_FIRST], (unsigned long long)(a.off * G + cc));
+          atomicMin(&icnt[(size_t)inst * IC_N + IC_FIRST], (unsigned long long)(a.off * G + cc));
       }
     }
     __builtin_amdgcn_wave_barrier();
   }
+  // the block's counts: groups that ended in the first group's instance add up in LDS (a block's groups work on
+  // neighbouring parents, so nearly always all of them), the others add to the counters themselves
+  __shared__ uint32_t btally[8], bstage[SG_N];
+  __shared__ int binst;
+  if (threadIdx.x < 8) btally[threadIdx.x] = bstage[threadIdx.x] = 0;
+  if (threadIdx.x == 0) binst = cur;
+  __syncthreads();
+  if (le == 0 && cur >= 0 && cur == binst)
+    for (int i = 0; i <= ST_OVF; i++)
+      if (const uint32_t v = tl[i]) { atomicAdd(&btally[i], v); tl[i] = 0; }
   flush();
-  if (le != 0) n_eval = n_pre = n_t = n_cheap = n_cuts = n_keys = n_tp = 0;     // one copy per group
-  n_eval = gsum<64>(n_eval);
-  n_pre = gsum<64>(n_pre);
-  n_t = gsum<64>(n_t);
-  n_cheap = gsum<64>(n_cheap);
-  n_cuts = gsum<64>(n_cuts);
-  n_keys = gsum<64>(n_keys);
-  n_tp = gsum<64>(n_tp);
-  if (lane == 0) {
-    if (n_eval) atomicAdd(&a.cnt[C_EVAL], (unsigned long long)n_eval);
-    if (n_pre) atomicAdd(&a.cnt[C_PRE], (unsigned long long)n_pre);
-    if (n_t) atomicAdd(&a.cnt[C_NEEDT], (unsigned long long)n_t);
-    if (n_cheap) atomicAdd(&a.cnt[C_CHEAP], (unsigned long long)n_cheap);
-    if (n_cuts) atomicAdd(&a.cnt[C_CUTS], (unsigned long long)n_cuts);
-    if (n_keys) atomicAdd(&a.cnt[C_KEYS], (unsigned long long)n_keys);
-    if (n_tp) atomicAdd(&a.cnt[C_TPASS], (unsigned long long)n_tp);
+  if (le == 0) {
+    const uint32_t n[SG_N - 1] = {n_eval, n_pre, n_t, n_cheap, n_cuts, n_keys, n_tp};     // one copy per group
+#pragma unroll
+    for (int i = 0; i < SG_N - 1; i++) if (n[i]) atomicAdd(&bstage[i], n[i]);
+  }
+  __syncthreads();
+  if (threadIdx.x < 8) {
+    const int i = threadIdx.x;
+    if (i <= ST_OVF && btally[i]) atomicAdd(&icnt[(size_t)binst * IC_N + slot_of(i)], (unsigned long long)btally[i]);
+    if (bstage[i]) atomicAdd(&a.stage[(blockIdx.x & (NSTRIPE - 1)) * SG_N + i], (unsigned long long)bstage[i]);
   }
 }
 
@@ -517,10 +530,14 @@ __global__ __launch_bounds__(CT_THREADS) void k_scatter_alive_one(FlagAlive f, l
 }
 
 // searches that continue after this level: no circuit, no overflow, budget left (captured step)
-__global__ void k_active(const unsigned long long *icnt, const uint8_t *keepi, int nslots, uint8_t *active) {
+__global__ void k_active(const unsigned long long *icnt, int nstr, const uint8_t *keepi, int nslots, uint8_t *active) {
   for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nslots; s += gridDim.x * blockDim.x) {
-    const unsigned long long *x = icnt + (size_t)s * IC_N;
-    active[s] = !x[IC_FOUND] && !x[IC_OVF] && keepi[s];
+    bool on = keepi[s];
+    for (int j = 0; j < nstr; j++) {
+      const unsigned long long *x = icnt + ((size_t)j * nslots + s) * IC_N;
+      on = on && !x[IC_FOUND] && !x[IC_OVF];
+    }
+    active[s] = on;
   }
 }
 
@@ -850,9 +867,10 @@ struct chz_ctx {
   bool shared_steps = false;      // the batch has held more than one search at once (captured steps are used)
   std::vector<uint32_t> cdv;      // distinct cut-delta values of the spec's gates (bits 0-7 of DevGate::cls index them)
   // level control block, uploaded in one copy at the start of every level and read back in one copy:
-  // [cnt: C_N counters | icnt: per-slot IC_N counters | d_rem: per-slot budgets | d_keepi: per-slot keep flags]
+  // [cnt: C_N counters | stage stripes | icnt: stripes of per-slot IC_N counters | d_rem: per-slot budgets | d_keepi:
+  // per-slot keep flags]
   chz::DBuf<unsigned long long> ctl;
-  unsigned long long *cnt = nullptr, *icnt = nullptr;
+  unsigned long long *cnt = nullptr, *stage = nullptr, *icnt = nullptr;
   int *d_rem = nullptr;
   uint8_t *d_keepi = nullptr;
   chz::DBuf<uint8_t> d_active;
@@ -978,7 +996,23 @@ static void sort_pairs(chz_ctx *c, long long n) {
 }
 
 // bytes of the level control block for ns slots (its layout is the pinned staging area's)
-static size_t ctl_in_bytes(int ns) { return ((size_t)C_N + (size_t)ns * IC_N) * 8 + (size_t)ns * 4 + (size_t)ns; }
+static size_t ctl_in_bytes(int ns) { return counter_words(ns) * 8 + (size_t)ns * 4 + (size_t)ns; }
+
+// the counters read back (hc: counter_words), their stripes summed into hc's stage counts and the first slot stripe
+static void fold_counters(unsigned long long *hc, int ns) {
+  static const int at[SG_N - 1] = {C_EVAL, C_PRE, C_NEEDT, C_CHEAP, C_CUTS, C_KEYS, C_TPASS};
+  for (int i = 0; i < SG_N - 1; i++) {
+    hc[at[i]] = 0;
+    for (int j = 0; j < NSTRIPE; j++) hc[at[i]] += hc[C_N + j * SG_N + i];
+  }
+  unsigned long long *ic = hc + C_N + NSTRIPE * SG_N;
+  for (int j = 1; j < slot_stripes(ns); j++)
+    for (size_t x = 0; x < (size_t)ns * IC_N; x++) {
+      const unsigned long long v = ic[(size_t)j * ns * IC_N + x];
+      if (x % IC_N == IC_FIRST) ic[x] = std::min(ic[x], v);
+      else ic[x] += v;
+    }
+}
 
 // per-slot device arrays sized for `need` instance slots
 static void reserve_slots(chz_ctx *c, int need) {
@@ -987,8 +1021,9 @@ static void reserve_slots(chz_ctx *c, int need) {
   while (ns < need) ns *= 2;
   c->ctl.need((ctl_in_bytes(ns) + 7) / 8);
   c->cnt = c->ctl.p;
-  c->icnt = c->cnt + C_N;
-  c->d_rem = (int *)(c->icnt + (size_t)ns * IC_N);
+  c->stage = c->cnt + C_N;
+  c->icnt = c->stage + NSTRIPE * SG_N;
+  c->d_rem = (int *)(c->cnt + counter_words(ns));
   c->d_keepi = (uint8_t *)(c->d_rem + ns);
   c->d_active.need(ns);
   c->gflag.need(ns);
@@ -1103,7 +1138,7 @@ constexpr int STEP_BUCKET = 10;    // the schedule of the 1,024-parent bucket dr
 
 template <int NQ>
 static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long long *hc_in, unsigned long long *hc,
-                       unsigned long long *ic, unsigned long long *ptot, uint32_t *&tp, uint8_t *&tg) {
+                       unsigned long long *ptot, uint32_t *&tp, uint8_t *&tg) {
   constexpr int N = 1 << NQ, E = N * N, CPW = 64 / E;
   (void)N;
   const KSpec &ks = c->ks;
@@ -1142,8 +1177,8 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
     std::lock_guard<std::recursive_mutex> capture_lock(capture_mu());
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, 0, ncap, 0, 0,
-                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->cnt, pinst, c->d_rem, c->d_keepi,
-                  c->icnt, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
+                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
+                  c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cap * G + CPW - 1) / CPW, sc.cap));
     switch (sc.var) {
       case 0: hipLaunchKernelGGL((k_level<NQ, 4>), grid, dim3(256), 0, s, ks, ea, cap); break;
@@ -1167,7 +1202,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
     const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncap, c->surv_o.p, c->surv_key.p, c->runs.p, c->res[cur].p,
                         c->pk[cur].p, c->kept.p, c->cnt, pinst, dsurv};
     hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncap / CPW + 1, 4096)), dim3(256), 0, s, ks, da);
-    hipLaunchKernelGGL(k_active, dim3(1), dim3(256), 0, s, c->icnt, c->d_keepi, ns, c->d_active.p);
+    hipLaunchKernelGGL(k_active, dim3(1), dim3(256), 0, s, c->icnt, slot_stripes(ns), c->d_keepi, ns, c->d_active.p);
     const FlagKept fk{c->kept.p, c->surv_o.p, pinst, c->d_active.p, G};
     hipLaunchKernelGGL(k_flag_count<FlagKept>, dim3((unsigned)nbA), dim3(CT_THREADS), 0, s, fk, ncap, c->bcount.p, dsurv);
     hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, s, c->bcount.p, nbA);
@@ -1196,10 +1231,10 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   c->ev.begin(K_GATHER, c->stream);
   hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((ncap + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga);
   c->ev.end(c->stream);
-  HIPCHK(hipMemcpyAsync(hc, c->cnt, C_N * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(ic, c->icnt, (size_t)ns * IC_N * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipMemcpyAsync(ptot, c->bcount.p + nbA, 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  fold_counters(hc, ns);
   c->ev.flush(c->k_ms, c->k_launch);
   if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
   c->k_work[K_GATHER] += (double)*ptot * (E * 16.0 * 2.0 + 16.0);
@@ -1264,18 +1299,18 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   // in one copy), the kept total and the per-slot active flags
   const int ns = c->nslots;
   const size_t in_bytes = ctl_in_bytes(ns), o_out = (in_bytes + 63) & ~(size_t)63,
-               o_tot = o_out + ((size_t)C_N + (size_t)ns * IC_N) * 8, o_act = o_tot + 8;
+               o_tot = o_out + counter_words(ns) * 8, o_act = o_tot + 8;
   uint8_t *pin = c->pin.need(o_act + ns);
-  unsigned long long *hc_in = (unsigned long long *)pin, *ic_in = hc_in + C_N;
-  unsigned long long *hc = (unsigned long long *)(pin + o_out), *ic = hc + C_N;
+  unsigned long long *hc_in = (unsigned long long *)pin, *ic_in = hc_in + C_N + NSTRIPE * SG_N;
+  unsigned long long *hc = (unsigned long long *)(pin + o_out), *ic = hc + C_N + NSTRIPE * SG_N;
   unsigned long long *ptot = (unsigned long long *)(pin + o_tot);
-  int *rem = (int *)(ic_in + (size_t)ns * IC_N);
+  int *rem = (int *)(hc_in + counter_words(ns));
   uint8_t *keepi = (uint8_t *)(rem + ns), *active = pin + o_act;
-  for (int i = 0; i < C_N; i++) hc_in[i] = 0;
+  std::memset(hc_in, 0, counter_words(ns) * 8);
   for (int s = 0; s < ns; s++) {
     rem[s] = 0;
     keepi[s] = active[s] = 0;
-    for (int i = 0; i < IC_N; i++) ic_in[(size_t)s * IC_N + i] = i == IC_FIRST ? ~0ull : 0ull;
+    for (int j = 0; j < slot_stripes(ns); j++) ic_in[((size_t)j * ns + s) * IC_N + IC_FIRST] = ~0ull;
   }
   for (const BInst &b : c->binst)
     if (b.live) { rem[b.slot] = b.depth - (b.t + 1); keepi[b.slot] = b.t + 1 < b.depth; }
@@ -1295,7 +1330,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     for (int i = 0; i < C_N; i++) hc_in[i] = 0;
     hc_in[C_M] = (unsigned long long)m;
     hc_in[C_NCC] = (unsigned long long)(m * G);
-    step_graph<NQ>(c, cur, m, hc_in, hc, ic, ptot, tp, tg);
+    step_graph<NQ>(c, cur, m, hc_in, hc, ptot, tp, tg);
     nsurv = (long long)hc[C_SURV];
     distinct = (long long)*ptot;
     c->k_work[K_STEP] += expand_ops(c, NQ, hc) + (double)(m * G) + (double)nsurv * (24.0 + 16.0 + 4 * 20.0 + 9.0);
@@ -1324,8 +1359,8 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     const chz_ctx::Sched sc = c->tuning ? c->force : c->sched[bucket];
     const int gsplit = (int)std::max<long long>(1, std::min<long long>(G, ((long long)sc.tw * CPW + cm - 1) / cm));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, off, ncc, 0, 0,
-                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->cnt, pinst, c->d_rem, c->d_keepi,
-                  c->icnt, gsplit, nullptr, 0, c->goal_skip ? c->gflag.p : nullptr};
+                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
+                  c->icnt, slot_stripes(ns), ns * IC_N, gsplit, nullptr, 0, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cm * gsplit + CPW - 1) / CPW, sc.cap));
     hipEvent_t te0 = nullptr, te1 = nullptr;
     if (c->tuning) {
@@ -1362,8 +1397,9 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     c->ev.end(c->stream);
     c->k_work[K_COMPACT] += (double)ncc;
   }
-  HIPCHK(hipMemcpyAsync(hc, c->cnt, ((size_t)C_N + (size_t)ns * IC_N) * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  fold_counters(hc, ns);
   c->ev.flush(c->k_ms, c->k_launch);
   nsurv = (long long)hc[C_SURV];
   c->k_work[K_COMPACT] += (double)nsurv * 24.0;
