@@ -105,6 +105,24 @@ template <typename Op> __device__ __forceinline__ uint32_t wave_reduce32(uint32_
   return op(q[0], q[1]);
 }
 
+// v[lane ^ h] for a power of two h < 64 (lane ^ 4 as ^ 7 and ^ 3, lane ^ 8 as a rotation by half a row)
+__device__ __forceinline__ uint32_t wave_xor32(uint32_t v, int h) {
+  switch (h) {
+    case 1: return dpp32<DPP_QXOR1>(v);
+    case 2: return dpp32<DPP_QXOR2>(v);
+    case 4: return dpp32<0x1B>(dpp32<DPP_HALF_MIRROR>(v));
+    case 8: return dpp32<0x128>(v);
+    case 16: {
+      const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+      return __lane_id() & 16 ? p[0] : p[1];
+    }
+    default: {
+      const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      return __lane_id() & 32 ? p[0] : p[1];
+    }
+  }
+}
+
 template <int GS> __device__ __forceinline__ int4 gshfl(int4 v, int src) {
   return make_int4(__shfl(v.x, src, GS), __shfl(v.y, src, GS), __shfl(v.z, src, GS), __shfl(v.w, src, GS));
 }
@@ -154,8 +172,24 @@ __device__ __forceinline__ uint32_t mont_mul(uint32_t a, uint32_t b) {   // a < 
   const uint32_t r = (uint32_t)u;
   return r >= P_MOD ? r - P_MOD : r;
 }
+// a b + c d by one reduction; a, b, c, d < p
+__device__ __forceinline__ uint32_t mont_mul2(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  const uint64_t t = (uint64_t)a * b + (uint64_t)c * d;              // < 2 p^2 < 2^61
+  const uint32_t m = (uint32_t)t * P_NINV;
+  const uint32_t r = (uint32_t)((t + (uint64_t)m * P_MOD) >> 32);    // < 2 p^2 / 2^32 + p < 2 p
+  return r >= P_MOD ? r - P_MOD : r;
+}
 __device__ __forceinline__ uint32_t fp_sub(uint32_t a, uint32_t b) { return a >= b ? a - b : a + P_MOD - b; }
 __device__ __forceinline__ uint32_t fp_lift(int v) { return v < 0 ? (uint32_t)(v + 3 * (int64_t)P_MOD) : (uint32_t)v; }
+// image of a + b w + c w^2 + d w^3 in F_p, coefficients below p in magnitude: four products, one reduction
+__device__ __forceinline__ uint32_t fp_of_small(int4 v, const uint32_t *wm) {
+  auto lift = [](int x) { return (uint32_t)(x < 0 ? x + (int)P_MOD : x); };
+  const uint64_t t = (uint64_t)lift(v.x) * wm[0] + (uint64_t)lift(v.y) * wm[1] + (uint64_t)lift(v.z) * wm[2] +
+                     (uint64_t)lift(v.w) * wm[3];                    // < 4 p^2 < 2^62
+  const uint32_t m = (uint32_t)t * P_NINV;
+  const uint32_t r = (uint32_t)((t + (uint64_t)m * P_MOD) >> 32);    // < 4 p^2 / 2^32 + p < 2 p
+  return r >= P_MOD ? r - P_MOD : r;
+}
 // image of a + b w + c w^2 + d w^3 in F_p
 __device__ __forceinline__ uint32_t fp_of(int4 v, const uint32_t *wm) {
   uint32_t s = mont_mul(fp_lift(v.x), wm[0]) + mont_mul(fp_lift(v.y), wm[1]);

@@ -92,6 +92,7 @@ struct LevelTabs {
   // bits 0-2 source column x0, 3-5 power p0 of w, 6-8 x1, 9-11 p1, bit 12 two terms; bit 15: use the table loop
   uint16_t sdesc[MAXG * 64];
   GateHdr shdr[MAXG];
+  KeyTab kt;                       // n = 3: the class key's choice of symmetries
   uint8_t spos[16 * 64];           // n = 3: position of entry e under symmetry y (y * 64 + e)
   uint8_t scx[CXL_MAX];            // the cx table when it fits (KSpec::cxlds)
   // per candidate, for the bounds from the parent alone: bits 0-7 tdel, 8-10 qubits, 11-15 the most the sqrt2 exponent
@@ -102,6 +103,16 @@ struct LevelTabs {
   uint8_t scsrc[CSRC_MAX * 64];    // cut i's operator-Schmidt matrix: entry source of lane le (i * GS + le)
 };
 static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
+
+// the expansion's class key outside it: the tables read from their global copy
+template <int NQ> __device__ __forceinline__ uint64_t node_key(int4 s, int k, int le, const KSpec &sp) {
+  if constexpr (NQ == 3) {
+    const LevelTabs *t = (const LevelTabs *)sp.ktab;
+    return class_key3(s, k, le, t->spos, t->kt.adm, sp.cjm);
+  } else {
+    return class_key<NQ>(s, k, le, sp);
+  }
+}
 
 template <int NQ, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_level(KSpec sp, ExpandArgs a,
@@ -370,8 +381,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                 if (!sp.lite) {
                   uint32_t needs = (pbw & BW_NEEDS) >> 8;
                   const uint32_t keepc = (pbw & BW_CUTS) ? (uint32_t)h.loc : 0u;
-                  n_cuts += sp.ncuts - __popc(keepc & ((1u << sp.ncuts) - 1));
-                  c2 = wuni<NQ>(cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, needs));
+                  const bool stop = sp.cx_mono && sp.have_table && sp.ncuts <= BW_MAXCUTS && (pbw & BW_CUTS);
+                  const CutStop cst{stop, stop ? low_needs(sp, needs, (uint32_t)h.cdel) : 0u, T, hh, supp, rem};
+                  c2 = wuni<NQ>(cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts));
                   bw = (needs << 8 & ~BW_CUTS) | (sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
                 }
                 const int tmax = t_budget(hh, c2, supp, rem) * sp.tdiv;
@@ -416,7 +428,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
             if (alive && keep) {
               n_keys++;
               if constexpr (NQ == 3) {
-                key = sp.nsym <= 16 ? class_key3(s, k, lane, spos, cjm, sp.nsym) : class_key<NQ>(s, k, le, sp);
+                key = class_key3(s, k, lane, spos, tb.kt.adm, cjm);
               } else {
                 key = class_key<NQ>(s, k, le, sp);
               }
@@ -1631,9 +1643,25 @@ static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const
                 (uint32_t)(d.cls & 0xff) << 16;
     T.shdr[g] = GateHdr{d.nq, d.L, d.mask, d.ik, d.q[0], d.q[1], d.q[2], kind, d.tdel, d.cutloc, d.cdel, d.cls};
   }
-  if (n == 3)
+  if (n == 3) {
+    // per order of the qubits' sums, the symmetries that make it smallest: qubit q goes to place image(q)
+    for (int code = 0; code < 64; code++)
+      for (int cj = 0; cj < 2; cj++) {
+        int best = 1 << 30, score[16];
+        for (int y = 0; y < k.nsym; y++) {
+          score[y] = 0;
+          for (int q = 0; q < 3; q++) {
+            const int to = grp.bperm[y * 8 + (1 << q)] >> 1;      // 1, 2, 4 -> 0, 1, 2
+            score[y] |= ((code >> (2 * q)) & 3) << (4 - 2 * to);
+          }
+          if (grp.conj[y] == cj) best = std::min(best, score[y]);
+        }
+        for (int y = 0; y < k.nsym; y++)
+          if (grp.conj[y] == cj && score[y] == best) T.kt.adm[code] |= (uint16_t)(1u << y);
+      }
     for (int y = 0; y < 16 && y < k.nsym; y++)
       for (int e = 0; e < 64; e++) T.spos[y * 64 + e] = (uint8_t)(grp.bperm[y * 8 + (e >> 3)] * 8 + grp.bperm[y * 8 + (e & 7)]);
+  }
   if (k.cxlds && k.have_table)
     for (int i = 0; i < CXL_MAX && i < k.ncx; i++) T.scx[i] = (uint8_t)s.cxtable[i];
   for (int i = 0; i < CSRC_MAX * GS; i++) {

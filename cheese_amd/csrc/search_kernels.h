@@ -195,7 +195,7 @@ template <int NQ> __device__ __forceinline__ int cut_rank(uint32_t fp, int le, i
     const uint32_t fr = __shfl(v, (mrow << lgC) + pcol, GS);
     const uint32_t pr = __shfl(v, (prow << lgC) + mcol, GS);
     used |= 1 << prow;
-    if (mine && mrow != prow) v = fp_sub(mont_mul(v, pv), mont_mul(fr, pr));
+    if (mine && mrow != prow) v = mont_mul2(v, pv, fr, pr ? P_MOD - pr : 0u);      // v pv - fr pr
     rank++;
   }
   return rank;
@@ -217,27 +217,45 @@ __device__ __forceinline__ int cx_at(const KSpec &sp, const uint8_t *cxl, int id
   return sp.cxlds ? (int)cxl[idx] : sp.cxtable[idx];
 }
 
+// Bounds known before the cuts of a child: the smallest cut needs its parent leaves (packed as in the bound word) and
+// whether they may be used, its T bound's lower end, and the other arguments of the bound.  Once the needs found so far
+// and the smallest possible others put the child over its budget, the remaining ranks are left out (the value returned
+// is then that lower cut bound, and `needs` is not the child's).
+struct CutStop { bool on; uint32_t low; int T, h, supp, rem; };
+
 template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const KSpec &sp, const uint8_t *cxl,
-                                                          const uint8_t *csrc, uint32_t keepc, uint32_t &needs) {
+                                                          const uint8_t *csrc, uint32_t keepc, bool small, const CutStop &st,
+                                                          uint32_t &needs, uint32_t &ranks) {
   constexpr int GS = 1 << (2 * NQ);
   uint32_t fp = 0;
   bool have_fp = false;
-  int idx = 0, mult = 1, mx = 0;
+  int idx = 0, mult = 1, mx = 0, lo = 0;
   uint32_t out = 0;
+  int todo = sp.ncuts - __popc(keepc & ((1u << sp.ncuts) - 1));
+  if (st.on) {
+    int m = 1;
+    for (int i = 0; i < sp.ncuts; i++) { lo += (int)((st.low >> (3 * i)) & 7u) * m; m *= sp.rad[i]; }
+  }
   for (int i = 0; i < sp.ncuts; i++) {
     const int rad = sp.rad[i], sa = sp.cutsize[i];
     int need;
     if ((keepc >> i) & 1) need = (int)((needs >> (3 * i)) & 7u);
     else {
-      if (!have_fp) { fp = fp_of(s, sp.wm); have_fp = true; }
+      if (!have_fp) { fp = small ? fp_of_small(s, sp.wm) : fp_of(s, sp.wm); have_fp = true; }
       const int R = 1 << (2 * sa);
       int stop = R;
       if (rad >= 2 && rad - 2 < 30 && (1 << (rad - 2)) + 1 < stop) stop = (1 << (rad - 2)) + 1;
       const int src = i < CSRC_MAX ? (int)csrc[i * GS + le] : cut_source<NQ>(le, sp.cutmask[i], sa);
       const int rk = cut_rank<NQ>(fp, le, src, sa, stop);
+      ranks++;
       need = 0;
       while ((1 << need) < rk) need++;
       if (need > rad - 1) need = rad - 1;
+      if (st.on && --todo > 0) {
+        lo += (need - (int)((st.low >> (3 * i)) & 7u)) * mult;
+        const int c = cx_at(sp, cxl, lo);
+        if (st.T > t_budget(st.h, c, st.supp, st.rem) * sp.tdiv) return c;
+      }
     }
     if (i < BW_MAXCUTS) out |= (uint32_t)need << (3 * i);
     idx += need * mult;
@@ -246,6 +264,16 @@ template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const 
   }
   needs = out;
   return sp.have_table ? cx_at(sp, cxl, idx) : mx;
+}
+
+// the smallest needs a child can have: its parent's less its gate's deltas, packed
+__device__ __forceinline__ uint32_t low_needs(const KSpec &sp, uint32_t pneeds, uint32_t cdel) {
+  uint32_t out = 0;
+  for (int i = 0; i < sp.ncuts && i < BW_MAXCUTS; i++) {
+    const int dl = (int)((cdel >> (3 * i)) & 7u), nd = (int)((pneeds >> (3 * i)) & 7u) - dl;
+    out |= (uint32_t)(dl == 7 || nd < 0 ? 0 : nd) << (3 * i);
+  }
+  return out;
 }
 
 // Lower bound on a child's cut bound from its parent's packed needs: each need drops by at most the gate's
@@ -354,17 +382,17 @@ template <int NQ> __device__ __forceinline__ int t_bound16s(TStage st, int4 s, i
                                                              uint32_t &npass, bool &exact) {
   constexpr int E = 1 << (2 * NQ), H = E / 2, GS = E;
   const int top = 2 * (NQ + k);
-  // f = 0: |S[e]|^2 = r + y sqrt2 with r = a^2 + b^2 + c^2 + d^2, y = ab + bc + cd - da
-  uint32_t r = (uint32_t)(s.x * s.x + s.y * s.y + s.z * s.z + s.w * s.w);
-  uint32_t y = (uint32_t)(s.x * s.y + s.y * s.z + s.z * s.w - s.w * s.x);
+  // f = 0: |S[e]|^2 = r + y sqrt2 with r = a^2 + b^2 + c^2 + d^2, y = ab + bc + cd - da, as a pair mod 2^16
+  const u16x2 ab = pk(s.x, s.y), bc = pk(s.y, s.z), cd = pk(s.z, s.w), da = pk(s.w, -s.x);
+  u16x2 q0 = ab.xx * ab + bc.xx * bc + cd.xx * cd + da.xx * da;
 #pragma unroll
   for (int h = 1; h < GS; h <<= 1) {
-    const uint32_t ro = __shfl_xor(r, h, GS), yo = __shfl_xor(y, h, GS);
-    if (le & h) { r = ro - r; y = yo - y; } else { r = r + ro; y = y + yo; }
+    const u16x2 o = as16(NQ == 3 ? wave_xor32(bits(q0), h) : (uint32_t)__shfl_xor((int)bits(q0), h, GS));
+    q0 = q0 * as16(le & h ? 0xffffffffu : 0x00010001u) + o;
   }
   // group ORs are uniform over the group: read through readfirstlane (n = 3) they stay in scalar registers
-  const uint32_t accG = (uint32_t)wuni<NQ>((int)gor<GS>(r & 0xffffu));
-  const uint32_t accY = (uint32_t)wuni<NQ>((int)gor<GS>(y & 0xffffu));
+  const uint32_t acc0 = (uint32_t)wuni<NQ>((int)gor<GS>(bits(q0)));
+  const uint32_t accG = acc0 & 0xffffu, accY = acc0 >> 16;
   int v = 2 * ctz16(accG);
   const int vy = 1 + 2 * ctz16(accY);
   v = vy < v ? vy : v;
@@ -471,80 +499,50 @@ template <int NQ> __device__ __forceinline__ uint64_t class_key(int4 s, int k, i
   return best;
 }
 
-// ---- wave64 exchanges without the LDS crossbar (gfx950): permlane32/16 swaps and DPP row controls ----
-__device__ __forceinline__ uint64_t u64_of(uint32_t lo, uint32_t hi) { return (uint64_t)lo | ((uint64_t)hi << 32); }
-
-// lanes 0-31 receive a + a[lane ^ 32], lanes 32-63 receive b + b[lane ^ 32]: v_permlane32_swap exchanges the
-// upper half of its first operand with the lower half of its second
-__device__ __forceinline__ uint64_t rs32(uint64_t a, uint64_t b) {
-  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)a, (uint32_t)b, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(a >> 32), (uint32_t)(b >> 32), false, false);
-  return u64_of(lo[0], hi[0]) + u64_of(lo[1], hi[1]);
+// class_key for n = 3 (one matrix per wave64, whole wave active, at most 16 symmetries).  The group permutes qubits and
+// may conjugate, so most of its elements are ruled out before any image is hashed: sums over the entries that do not
+// depend on their places tell S from its conjugate, and for each qubit a sum over the entries off the qubit's diagonal
+// moves with the qubit.  Only the elements that bring the smaller of the two conjugates and the smallest order of the
+// qubits' sums are hashed; equal classes have the same images under these, so the smallest of their hashes is the same.
+// Hashing all twelve images of a 3-qubit default set took 410 vector instructions a key and a third of the expansion's
+// quarter-rate products; two or three sums and usually one image take about 130.
+//   spos[y * 64 + le]: position of entry le under symmetry y; cjm bit y: symmetry y conjugates; adm[order]: the
+//   symmetries that bring the qubits' sums into the smallest order, among those that conjugate and among the others,
+//   with `order` the number of smaller sums of each qubit in two bits (KeyTab)
+struct KeyTab { uint16_t adm[64]; };
+__host__ __device__ inline int key_order(uint32_t a, uint32_t b, uint32_t c) {
+  return ((b < a) + (c < a)) | ((a < b) + (c < b)) << 2 | ((a < c) + (b < c)) << 4;
 }
-// lanes with bit 4 clear receive a + a[lane ^ 16], the others b + b[lane ^ 16]: v_permlane16_swap exchanges
-// the odd 16-lane rows of its first operand with the even rows of its second
-__device__ __forceinline__ uint64_t rs16(uint64_t a, uint64_t b) {
-  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)a, (uint32_t)b, false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(a >> 32), (uint32_t)(b >> 32), false, false);
-  return u64_of(lo[0], hi[0]) + u64_of(lo[1], hi[1]);
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce32(v, [](uint32_t a, uint32_t b) { return a + b; }));
 }
-__device__ __forceinline__ uint64_t partner32(uint64_t x, int lane) {       // x[lane ^ 32]
-  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
-  return (lane & 32) ? u64_of(lo[0], hi[0]) : u64_of(lo[1], hi[1]);
-}
-__device__ __forceinline__ uint64_t partner16(uint64_t x, int lane) {       // x[lane ^ 16]
-  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
-  return (lane & 16) ? u64_of(lo[0], hi[0]) : u64_of(lo[1], hi[1]);
-}
-template <int CTRL> __device__ __forceinline__ uint64_t dpp64(uint64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xf, 0xf, false);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, false);
-  return u64_of(lo, hi);
-}
-
-// class_key for n = 3 (one matrix per wave64, whole wave active), at most 16 symmetries: the 16 per-lane
-// hashes are reduce-scattered over the wave (lane ^ 32, ^ 16 by permlane swaps; ^ 15, ^ 7 by DPP mirrors; then
-// sums over each quad), so lane L ends with the wave sum of slot (L >> 2) & 15; one mix per lane and a min over
-// lane bits 2-5 give the same key as class_key.  spos[y * 64 + le]: position of entry le under symmetry y (any
-// entry index for y >= nsym: those slots are hashed too, and their lanes are left out of the final min);
-// cjm bit y: symmetry y conjugates.  The conjugation bits are tested on a vector copy of cjm: tested on the
-// scalar they become 16 loop-invariant lane masks that the compiler hoists out of the child loop, where they
-// spill.
-__device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const uint8_t *spos, uint32_t cjm, int nsym) {
+__device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const uint8_t *spos, const uint16_t *adm, uint32_t cjm) {
   const uint32_t hv = entry_hash32(s), hc = entry_hash32(zconj(s));
-  uint32_t cjv = cjm;
-  asm volatile("" : "+v"(cjv));
-  auto slot = [&](int y) -> uint64_t { return slot64(((cjv >> y) & 1) ? hc : hv, (uint32_t)spos[y * 64 + lane] + 1); };
-  uint64_t h[8];      // slots y and y + 8 are combined as soon as they are hashed: 8 live values, not 16
-#pragma unroll
-  for (int j = 0; j < 8; j++) h[j] = rs32(slot(j), slot(j + 8));
-#pragma unroll
-  for (int j = 0; j < 4; j++) h[j] = rs16(h[j], h[j + 4]);
-  const bool b3 = lane & 8, b2 = lane & 4;
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const uint64_t send = b3 ? h[j] : h[j + 2], keep = b3 ? h[j + 2] : h[j];
-    h[j] = keep + dpp64<DPP_MIRROR>(send);
+  const int off = (lane >> 3) ^ (lane & 7);            // bit q: an entry off qubit q's diagonal
+  // 64 shares of 10 bits sum within 16 bits: two sums to a word
+  auto order = [&](uint32_t h) -> uint32_t {
+    const uint32_t x = h & 0x3ffu;
+    const uint32_t s01 = wave_sum((off & 1 ? x : 0u) | (off & 2 ? x << 16 : 0u)), s2 = wave_sum(off & 4 ? x : 0u);
+    return adm[key_order(s01 & 0xffffu, s01 >> 16, s2)];
+  };
+  uint32_t m;
+  if (!cjm) m = order(hv);
+  else {
+    const uint32_t t = wave_sum(hv >> 22 | (hc >> 22) << 16), tv = t & 0xffffu, tc = t >> 16;
+    m = 0;
+    if (tv <= tc) m |= order(hv) & ~cjm;
+    if (tv >= tc) m |= order(hc) & cjm;
   }
-  uint64_t x;
-  {
-    const uint64_t send = b2 ? h[0] : h[1], keep = b2 ? h[1] : h[0];
-    x = keep + dpp64<DPP_HALF_MIRROR>(send);
+  m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+  uint64_t best = ~0ull;
+  while (m) {
+    const int y = __ffs((int)m) - 1;
+    m &= m - 1;
+    const uint64_t x = slot64((cjm >> y) & 1 ? hc : hv, (uint32_t)spos[y * 64 + lane] + 1);
+    const uint64_t key = (uint64_t)wave_sum((uint32_t)(x >> 32)) << 32 | wave_sum((uint32_t)x);
+    best = key < best ? key : best;
   }
-  x += dpp64<DPP_QXOR1>(x);
-  x += dpp64<DPP_QXOR2>(x);
-  const int y = (lane >> 2) & 15;
-  uint64_t key = y < nsym ? mix64(x ^ ((uint64_t)(k + 1) * 0xc2b2ae3d27d4eb4full)) : ~0ull;
-  uint64_t o = dpp64<DPP_HALF_MIRROR>(key);
-  key = o < key ? o : key;
-  o = dpp64<DPP_MIRROR>(key);
-  key = o < key ? o : key;
-  o = partner16(key, lane);
-  key = o < key ? o : key;
-  o = partner32(key, lane);
-  return o < key ? o : key;
+  return mix64(best ^ ((uint64_t)(k + 1) * 0xc2b2ae3d27d4eb4full));
 }
 
 // exact: B = sigma(A) for some group element (src/cheese.cu:242-255)

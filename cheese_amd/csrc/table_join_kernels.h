@@ -43,7 +43,7 @@ template <int NQ> __global__ __launch_bounds__(256) void k_node_keys(KSpec sp, c
     const long long j = b + lane / GS;
     const bool in = j < m;
     const int4 s = in ? res[j * E + le] : make_int4(0, 0, 0, 0);
-    const uint64_t key = class_key<NQ>(s, in ? pk[j] : 0, le, sp);
+    const uint64_t key = node_key<NQ>(s, in ? pk[j] : 0, le, sp);
     if (in && le == 0) keys[j] = key;
   }
 }
@@ -174,7 +174,7 @@ template <int NQ> __global__ __launch_bounds__(256) void k_mitm_join(KSpec sp, G
       if (le == 0) { atomicAdd(ovf, 1ull); hashes[j] = 0; fwd[j] = -1; }
       continue;
     }
-    const uint64_t key = class_key<NQ>(K, kk, le, sp);
+    const uint64_t key = node_key<NQ>(K, kk, le, sp);
     const uint64_t stored = key | 1ull;
     uint64_t pos = gt_home(key, f.mask);
     bool any = false;
