@@ -108,7 +108,8 @@ static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
 template <int NQ> __device__ __forceinline__ uint64_t node_key(int4 s, int k, int le, const KSpec &sp) {
   if constexpr (NQ == 3) {
     const LevelTabs *t = (const LevelTabs *)sp.ktab;
-    return class_key3(s, k, le, t->spos, t->kt.adm, sp.cjm);
+    int image = 0;
+    return class_key3(s, k, le, t->spos, t->kt.adm, sp.cjm, image);
   } else {
     return class_key<NQ>(s, k, le, sp);
   }
@@ -428,7 +429,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
             if (alive && keep) {
               n_keys++;
               if constexpr (NQ == 3) {
-                key = class_key3(s, k, lane, spos, tb.kt.adm, cjm);
+                int image = 0;
+                key = class_key3(s, k, lane, spos, tb.kt.adm, cjm, image);
+                if (sp.ncuts <= BW_IMAGE_CUTS) bw |= (uint32_t)image << BW_IMAGE;
               } else {
                 key = class_key<NQ>(s, k, le, sp);
               }
@@ -577,6 +580,7 @@ struct DedupeArgs {
   const uint32_t *k, *v;          // sorted key prefixes and survivor ranks
   long long n;
   const uint64_t *surv_o, *surv_key;
+  const uint32_t *surv_bw;
   const uint32_t *runs;
   const int4 *res;                // parents' residuals
   const int *pk;
@@ -586,6 +590,17 @@ struct DedupeArgs {
   const unsigned long long *nd;   // survivors read on the device (captured step), or null
 };
 constexpr int MAXREP = 32, MAXSYM = 32;
+
+// the candidates' entry descriptors and exponents, copied into LDS by a block that forms children with child_terms
+struct ChildTab {
+  uint16_t desc[MAXG * 64];
+  uint8_t ik[MAXG];
+};
+__device__ __forceinline__ void load_child_tab(ChildTab &t, const KSpec &sp) {
+  const LevelTabs *g = (const LevelTabs *)sp.ktab;
+  for (int i = threadIdx.x; i < sp.G * 8; i += blockDim.x) ((uint4 *)t.desc)[i] = ((const uint4 *)g->sdesc)[i];
+  for (int i = threadIdx.x; i < sp.G; i += blockDim.x) t.ik[i] = (uint8_t)g->shdr[i].ik;
+}
 
 // value of lane q of the lane group (q uniform across the group)
 template <int GS> __device__ __forceinline__ uint32_t gget(uint32_t v, int q) {
@@ -597,15 +612,16 @@ template <int GS> __device__ __forceinline__ uint64_t gget64(uint64_t v, int q) 
 }
 
 template <int NQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NQ > 1 ? 6 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NQ > 1 ? 5 : 1)))
 void k_dedupe_runs(KSpec sp, DedupeArgs a) {
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
   constexpr int GPB = 256 / GS;     // groups per block
   __shared__ uint64_t rep_key[GPB][MAXREP], rep_o[GPB][MAXREP];
   __shared__ uint32_t rep_inst[GPB][MAXREP];
   __shared__ uint8_t spos[MAXSYM * E];
-  __shared__ int4 rep_res[GPB][2][E];     // the first two representatives' residuals
-  __shared__ int4 par_stage[GPB][E];      // the current member's parent residual
+  __shared__ int4 rep_img[GPB][2][E];     // images of the first two representatives' residuals (same_class_image)
+  __shared__ __align__(16) ChildTab ct;
+  load_child_tab(ct, sp);
   // the symmetry group's entry maps, staged once per block (the class test tries the elements in order)
   const int nsym = sp.nsym < MAXSYM ? sp.nsym : MAXSYM;
   const bool lds_sym = nsym == sp.nsym;
@@ -630,7 +646,11 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
     const uint32_t key = a.k[i0];
     int nrep = 0;
     // a run is almost always one class: its members are each rebuilt once and compared with the first
-    // representative, whose residual (and the second's) stays in LDS
+    // representative, of which (and of the second) an image stays in LDS.  A member's smallest image is known from its
+    // class key, so one comparison settles it where trying the group's elements in turn took six or seven; its
+    // entries come straight from its parent in global memory, the next member's on the way while it is compared.
+    // (The 22.4 million survivors of the Toffoli budget-14 proof: 20.4 ms with the members' parents staged in LDS,
+    // gate tables in global memory and the elements tried in turn, 12.3 here.)
     int ck0 = 0, ck1 = 0;
     // members in chunks of GS: lane le loads member j0 + le's rank, child, key, parent exponent and slot at once,
     // so each member then waits on one load (its parent's residual), issued while the member before it is
@@ -640,45 +660,46 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
       const bool in = jj < n && a.k[jj] == key;
       const uint64_t inb = gballot<GS>(in);
       const int nm = ~inb ? __ffsll((long long)~inb) - 1 : GS;     // members are contiguous from j0
-      uint32_t m_rank = 0, m_inst = 0;
+      uint32_t m_rank = 0, m_inst = 0, m_img = 0;
       uint64_t m_o = 0, m_key = 0;
       int m_pk = 0;
       if (le < nm) {
         m_rank = a.v[jj];
         m_o = a.surv_o[m_rank];
         m_key = a.surv_key[m_rank];
+        m_img = NQ == 3 && sp.ncuts <= BW_IMAGE_CUTS ? (a.surv_bw[m_rank] >> BW_IMAGE) & 15u : 0u;
         const long long pi = (long long)(m_o / G);
         m_pk = a.pk[pi];
         m_inst = a.pinst ? a.pinst[pi] : 0u;
       }
-      int4 nextv = make_int4(0, 0, 0, 0);
-      if (nm > 0) nextv = a.res[(long long)(gget64<GS>(m_o, 0) / G) * E + le];
+      auto terms = [&](int q) {
+        const uint64_t o = gget64<GS>(m_o, q);
+        return child_terms<NQ>(a.res + (long long)(o / G) * E, ct.desc[(int)(o % G) * 64 + le], le);
+      };
+      ChildTerms next{};
+      if (nm > 0) next = terms(0);
       for (int q = 0; q < nm; q++) {
         const uint32_t rank = gget<GS>(m_rank, q), inst = gget<GS>(m_inst, q);
         const uint64_t o = gget64<GS>(m_o, q), key64 = gget64<GS>(m_key, q);
-        const int pk = (int)gget<GS>((uint32_t)m_pk, q);
+        const int pk = (int)gget<GS>((uint32_t)m_pk, q), img = (int)gget<GS>(m_img, q);
         const int g = (int)(o % G);
-        __builtin_amdgcn_wave_barrier();
-        par_stage[grp][le] = nextv;
-        __builtin_amdgcn_wave_barrier();
-        if (q + 1 < nm) nextv = a.res[(long long)(gget64<GS>(m_o, q + 1) / G) * E + le];
+        const ChildTerms cur = next;
+        if (q + 1 < nm) next = terms(q + 1);
         int4 s;
         int ks;
-        make_child<NQ>(par_stage[grp], pk, sp.gates[g], le, s, ks);
+        if (!child_of<NQ>(cur, ct.desc[g * 64 + le], ct.ik[g], pk, s, ks))
+          make_child<NQ>(a.res + (long long)(o / G) * E, pk, sp.gates[g], le, s, ks);
         bool dup = false;
         for (int r = 0; r < nrep && !dup; r++) {
           if (rep_key[grp][r] != key64 || rep_inst[grp][r] != inst) continue;
           if (r < 2 && lds_sym) {
-            dup = same_class_rep<NQ>(s, ks, rep_res[grp][r], r ? ck1 : ck0, le, spos, cjm, nsym);
+            dup = same_class_image<NQ>(s, ks, rep_img[grp][r], r ? ck1 : ck0, img, le, spos, cjm, nsym);
           } else {
             int4 b;
             int kb;
-            if (r < 2) { b = rep_res[grp][r][le]; kb = r ? ck1 : ck0; }
-            else {
-              const uint64_t ro = rep_o[grp][r];
-              const long long rpi = (long long)(ro / G);
-              make_child<NQ>(a.res + rpi * E, a.pk[rpi], sp.gates[(int)(ro % G)], le, b, kb);
-            }
+            const uint64_t ro = rep_o[grp][r];
+            const long long rpi = (long long)(ro / G);
+            make_child<NQ>(a.res + rpi * E, a.pk[rpi], sp.gates[(int)(ro % G)], le, b, kb);
             dup = lds_sym ? same_class_lds<NQ>(s, ks, b, kb, le, spos, cjm, nsym) : same_class<NQ>(s, ks, b, kb, le, sp);
           }
         }
@@ -690,7 +711,7 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
             rep_inst[grp][nrep] = inst;
           }
           if (nrep < 2) {
-            rep_res[grp][nrep][le] = s;
+            rep_img[grp][nrep][spos[img * GS + le]] = (cjm >> img) & 1 ? zconj(s) : s;
             if (nrep == 0) ck0 = ks;
             else ck1 = ks;
           }
@@ -728,6 +749,8 @@ struct GatherArgs {
 // of a.tn consecutive kept nodes: one lane per node resolves the node's index chain (kept rank -> survivor ->
 // parent and gate) and writes its small fields, then the lane groups build the tile's residuals from the
 // parents, with the chain already in registers.
+// It is bound by memory (1 KB read and written per node at n = 3): 11.2 million nodes of the Toffoli budget-14 proof take
+// 5.9 ms, 4.9 at the rate of a large copy; 11.3 with gate tables and goal pre-images read from global memory per node.
 template <int NQ>
 __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
@@ -736,33 +759,53 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
   const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
   const long long nk = dev_n(a.nk, a.nkd);
   const int tn = a.tn;
+  __shared__ __align__(16) ChildTab ct;
+  load_child_tab(ct, sp);
+  __syncthreads();
+  // goal pre-images, one candidate per lane (n = 3: every candidate)
+  const int xgk = NQ == 3 && a.gflag && lane < sp.G ? sp.xgk[lane] : -1;
+  const uint64_t xgm = NQ == 3 && a.gflag && lane < sp.G ? sp.xgm[lane] : 0ull;
+  const uint32_t bwkeep = NQ == 3 && sp.ncuts <= BW_IMAGE_CUTS ? ~(15u << BW_IMAGE) : ~0u;
   for (long long tb = wave * tn; tb < nk; tb += nwaves * tn) {
     const long long pl = tb + lane;
     uint32_t pi_l = 0, bw_l = 0;
-    int g_l = 0, gp_l = 255;
+    int g_l = 0, gp_l = 255, pk_l = 0;
     if (lane < tn && pl < nk) {
       const uint32_t kid = a.kidx[pl];
       const uint64_t o = a.surv_o[kid];
       pi_l = (uint32_t)(o / (uint64_t)sp.G);
       g_l = (int)(o % (uint64_t)sp.G);
-      bw_l = a.surv_bw[kid];
+      bw_l = a.surv_bw[kid] & bwkeep;
       gp_l = a.g1[pi_l];
+      pk_l = a.pk[pi_l];
       a.g1_next[pl] = (uint8_t)g_l;
       a.g2_next[pl] = (uint8_t)gp_l;
       a.tree_par[pl] = pi_l;
       a.tree_gate[pl] = (uint8_t)g_l;
       a.inst_next[pl] = a.pinst ? a.pinst[pi_l] : 0u;
     }
+    // a node's parent entries are on the way while the node before it is finished
+    auto terms = [&](int src) {
+      const uint32_t pi = (uint32_t)__shfl((int)pi_l, src);
+      const int g = __shfl(g_l, src);
+      ChildTerms t{};
+      if (src < tn && tb + src < nk) t = child_terms<NQ>(a.res + (long long)pi * E, ct.desc[g * 64 + le], le);
+      return t;
+    };
+    ChildTerms next = terms(slot);
     for (int j = 0; j < tn; j += CPW) {
       const int src = j + slot;
       const long long pi = (long long)(uint32_t)__shfl((int)pi_l, src);
-      const int g = __shfl(g_l, src), gp = __shfl(gp_l, src);
+      const int g = __shfl(g_l, src), gp = __shfl(gp_l, src), pk = __shfl(pk_l, src);
       const uint32_t bwp = (uint32_t)__shfl((int)bw_l, src);
       const long long p = tb + src;
+      const ChildTerms cur = next;
+      if (j + CPW < tn) next = terms(j + CPW + slot);
       if (src >= tn || p >= nk) continue;
       int4 s;
       int k;
-      make_child<NQ>(a.res + pi * E, a.pk[pi], sp.gates[g], le, s, k);
+      if (!child_of<NQ>(cur, ct.desc[g * 64 + le], ct.ik[g], pk, s, k))
+        make_child<NQ>(a.res + pi * E, pk, sp.gates[g], le, s, k);
       a.res_next[p * E + le] = s;
       // goal child: the node equals the pre-image of a candidate its windows allow.  One lane per candidate
       // filters by exponent and nonzero pattern; the few that pass are compared exactly.
@@ -771,7 +814,8 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
         const uint64_t nzb = gballot<GS>(!zzero(s));
         for (int b0 = 0; b0 < sp.G && !adj; b0 += GS) {
           const int x = b0 + le;
-          uint64_t cm = gballot<GS>(x < sp.G && sp.xgk[x] == k && sp.xgm[x] == nzb);
+          uint64_t cm = NQ == 3 ? gballot<GS>(xgk == k && xgm == nzb)
+                                : gballot<GS>(x < sp.G && sp.xgk[x] == k && sp.xgm[x] == nzb);
           while (cm && !adj) {
             const int xx = b0 + __builtin_ctzll(cm);
             cm &= cm - 1;
@@ -1211,7 +1255,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
                        0);
     hipLaunchKernelGGL(k_run_starts, dim3(grid_for(ncap / (64 * RH_ITEMS) + 1)), dim3(256), 0, s, c->sk[0].p, ncap,
                        c->runs.p, c->cnt + C_RUNS, dsurv);
-    const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncap, c->surv_o.p, c->surv_key.p, c->runs.p, c->res[cur].p,
+    const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncap, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p, c->res[cur].p,
                         c->pk[cur].p, c->kept.p, c->cnt, pinst, dsurv};
     hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncap / CPW + 1, 4096)), dim3(256), 0, s, ks, da);
     hipLaunchKernelGGL(k_active, dim3(1), dim3(256), 0, s, c->icnt, slot_stripes(ns), c->d_keepi, ns, c->d_active.p);
@@ -1448,7 +1492,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       gflag_clear = true;
       hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nsurv / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream,
                          c->sk[0].p, nsurv, c->runs.p, c->cnt + C_RUNS, nullptr);
-      const DedupeArgs da{c->sk[0].p, c->sv[0].p, nsurv, c->surv_o.p, c->surv_key.p, c->runs.p,
+      const DedupeArgs da{c->sk[0].p, c->sv[0].p, nsurv, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p,
                           c->res[cur].p, c->pk[cur].p, c->kept.p, c->cnt, pinst, nullptr};
       hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(nsurv / CPW + 1, 4096)), dim3(256), 0, c->stream, ks, da);
       c->ev.end(c->stream);

@@ -90,6 +90,32 @@ __device__ __forceinline__ bool make_child(const int4 *__restrict__ par, int pk,
   return true;
 }
 
+// Children of unit gates with at most two terms per column and parents below 2^28 (all others: make_child), in two parts:
+// the parent entries a lane needs, by its entry descriptor (LevelTabs::sdesc), and the child entry from them.  The
+// loads of several children can then be in flight together.  par: the parent's entries in global memory.
+struct ChildTerms { int4 a, b; };
+template <int NQ> __device__ __forceinline__ ChildTerms child_terms(const int4 *__restrict__ par, uint32_t desc, int le) {
+  constexpr int N = 1 << NQ;
+  const int4 *row = par + (le >> NQ) * N;
+  ChildTerms t;
+  t.a = row[desc & 7];
+  t.b = desc & 0x1000u ? row[(desc >> 6) & 7] : make_int4(0, 0, 0, 0);
+  return t;
+}
+// false when the parent's entries are too large for the rotations, or the gate is none of these
+template <int NQ> __device__ __forceinline__ bool child_of(ChildTerms t, uint32_t desc, int ik, int pk, int4 &s, int &k) {
+  constexpr int GS = 1 << (2 * NQ);
+  if (!gall<GS>(!(desc & 0x8000u) && (zmag(t.a) | zmag(t.b)) < (1u << 28))) return false;
+  s = zrot(t.a, (desc >> 3) & 7);
+  if (desc & 0x1000u) {
+    const int4 u = zrot(t.b, (desc >> 9) & 7);
+    s.x += u.x; s.y += u.y; s.z += u.z; s.w += u.w;
+  }
+  k = pk + ik;
+  while (k > 0 && gall<GS>(zhalf(s))) { s = zdown(s); k--; }
+  return true;
+}
+
 // 2 if the matrix is monomial with a column permutation that is not affine over GF(2) (src/cheese.cu:321-338);
 // b = group ballot of the nonzero entries
 template <int NQ> __device__ __forceinline__ int h_struct(uint64_t b) {
@@ -207,6 +233,9 @@ template <int NQ> __device__ __forceinline__ int cut_rank(uint32_t fp, int le, i
 // change and computes the rest.
 constexpr uint32_t BW_TUNK = 0xffu, BW_CUTS = 1u << 31, BW_GOAL = 1u << 30, BW_NEEDS = 0x1fffff00u;
 constexpr int BW_MAXCUTS = 7;
+// A survivor's word carries the symmetry of its class key's image (class_key3) in bits 24-27 until the gather, where the
+// spec has at most BW_IMAGE_CUTS cuts.
+constexpr int BW_IMAGE = 24, BW_IMAGE_CUTS = 5;
 
 // CX/CZ lower bound from the cut ranks and the ILP table (src/cheese.cu:585-597).  Cuts in `keepc` take the
 // need packed in `needs` (the parent's: the gate acts on one side of them, so the rank is unchanged); the
@@ -509,6 +538,8 @@ template <int NQ> __device__ __forceinline__ uint64_t class_key(int4 s, int k, i
 //   spos[y * 64 + le]: position of entry le under symmetry y; cjm bit y: symmetry y conjugates; adm[order]: the
 //   symmetries that bring the qubits' sums into the smallest order, among those that conjugate and among the others,
 //   with `order` the number of smaller sums of each qubit in two bits (KeyTab)
+// image: the symmetry whose image has the smallest hash; matrices of one class have that image in common, so the dedupe
+// compares two of them by it.
 struct KeyTab { uint16_t adm[64]; };
 __host__ __device__ inline int key_order(uint32_t a, uint32_t b, uint32_t c) {
   return ((b < a) + (c < a)) | ((a < b) + (c < b)) << 2 | ((a < c) + (b < c)) << 4;
@@ -516,7 +547,8 @@ __host__ __device__ inline int key_order(uint32_t a, uint32_t b, uint32_t c) {
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce32(v, [](uint32_t a, uint32_t b) { return a + b; }));
 }
-__device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const uint8_t *spos, const uint16_t *adm, uint32_t cjm) {
+__device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const uint8_t *spos, const uint16_t *adm, uint32_t cjm,
+                                               int &image) {
   const uint32_t hv = entry_hash32(s), hc = entry_hash32(zconj(s));
   const int off = (lane >> 3) ^ (lane & 7);            // bit q: an entry off qubit q's diagonal
   // 64 shares of 10 bits sum within 16 bits: two sums to a word
@@ -540,7 +572,7 @@ __device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const ui
     m &= m - 1;
     const uint64_t x = slot64((cjm >> y) & 1 ? hc : hv, (uint32_t)spos[y * 64 + lane] + 1);
     const uint64_t key = (uint64_t)wave_sum((uint32_t)(x >> 32)) << 32 | wave_sum((uint32_t)x);
-    best = key < best ? key : best;
+    if (key < best || best == ~0ull) { best = key; image = y; }
   }
   return mix64(best ^ ((uint64_t)(k + 1) * 0xc2b2ae3d27d4eb4full));
 }
@@ -561,17 +593,18 @@ template <int NQ> __device__ __forceinline__ bool same_class_lds(int4 a, int ka,
   return false;
 }
 
-// the same test against a residual held in LDS (rep: E entries), read through the staged maps
-template <int NQ> __device__ __forceinline__ bool same_class_rep(int4 a, int ka, const int4 *rep, int kb, int le,
-                                                                const uint8_t *spos, uint32_t cjm, int nsym) {
+// the same test of b against the image of a representative held in LDS (rep: sigma_y(A) for some group element y, E
+// entries): b is of A's class exactly when some group element takes it to that image.  `first` is tried before the
+// others: the symmetry of b's own smallest image, which is nearly always the one
+template <int NQ> __device__ __forceinline__ bool same_class_image(int4 b, int kb, const int4 *rep, int krep, int first, int le,
+                                                                  const uint8_t *spos, uint32_t cjm, int nsym) {
   constexpr int GS = (1 << NQ) * (1 << NQ);
-  if (ka != kb) return false;
-  const int4 ac = zconj(a);
-  for (int y = 0; y < nsym; y++) {
-    const int4 bv = rep[spos[y * GS + le]];
-    const int4 av = (cjm >> y) & 1 ? ac : a;
-    if (gall<GS>(zeq(av, bv))) return true;
-  }
+  if (kb != krep) return false;
+  const int4 bc = zconj(b);
+  auto hit = [&](int y) { return gall<GS>(zeq((cjm >> y) & 1 ? bc : b, rep[spos[y * GS + le]])); };
+  if (hit(first)) return true;
+  for (int y = 0; y < nsym; y++)
+    if (y != first && hit(y)) return true;
   return false;
 }
 
