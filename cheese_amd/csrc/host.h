@@ -73,14 +73,20 @@ inline hipError_t sync_owner() {
 
 // Process-wide cache of device blocks by (device, size class): contexts opened and closed one after another
 // (one search per context, as the command line does) reuse memory instead of paying hipMalloc/hipFree each time.
-// Size classes are 2^k rounded up to a quarter step (at most 25 % slack).  A block enters the cache only when no
-// kernel can still use it: after a device synchronisation on growth, and from closed contexts whose stream has
-// finished.  At most kMaxCached bytes stay cached; the rest is freed.
+// Size classes are 2^k rounded up to a quarter step (at most 25 % slack); a request takes the smallest cached block
+// that holds it and is at most twice its size.  A block enters the cache only when no kernel can still use it: after a
+// device synchronisation on growth, and from closed contexts whose stream has finished.  At most kMaxCached bytes stay
+// cached, the ones given back last: a full cache frees its oldest blocks for the one that comes in.  (Freeing the
+// incoming block instead leaves a process that closed a few large contexts with a cache of sizes nobody asks for, and
+// every later context pays hipMalloc and hipFree for all of its buffers: the budget-13 proof with a 6-gate table, 28 ms
+// a call, took 123 ms after budget-14 proofs, and its first call 1.26 s instead of 25 ms.)
 struct DevPool {
   static constexpr size_t kMaxCached = 16ull << 30;
+  struct Block { void *p; uint64_t seq; };
   std::mutex mu;
-  std::multimap<std::pair<int, size_t>, void *> free_blocks;
+  std::multimap<std::pair<int, size_t>, Block> free_blocks;
   size_t cached = 0;
+  uint64_t seq = 0;
   static size_t size_class(size_t b) {
     if (b <= 256) return 256;
     int lg = 63 - __builtin_clzll((unsigned long long)b);
@@ -90,17 +96,19 @@ struct DevPool {
   void *get(size_t bytes, size_t &got) {
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
-    got = size_class(bytes);
+    const size_t want = size_class(bytes);
     {
       std::lock_guard<std::mutex> g(mu);
-      auto it = free_blocks.find({dev, got});
-      if (it != free_blocks.end()) {
-        void *p = it->second;
+      auto it = free_blocks.lower_bound({dev, want});
+      if (it != free_blocks.end() && it->first.first == dev && it->first.second <= 2 * want) {
+        void *p = it->second.p;
+        got = it->first.second;
         free_blocks.erase(it);
         cached -= got;
         return p;
       }
     }
+    got = want;
     void *p = nullptr;
     std::lock_guard<std::recursive_mutex> cg(capture_mu());
     if (hipMalloc(&p, got) != hipSuccess) {
@@ -114,16 +122,23 @@ struct DevPool {
     if (!p) return;
     int dev = 0;
     std::lock_guard<std::recursive_mutex> cg(capture_mu());
-    if (hipGetDevice(&dev) != hipSuccess) { (void)hipFree(p); return; }
+    if (hipGetDevice(&dev) != hipSuccess || got > kMaxCached) { (void)hipFree(p); return; }
     std::lock_guard<std::mutex> g(mu);
-    if (cached + got > kMaxCached) { (void)hipFree(p); return; }
-    free_blocks.insert({{dev, got}, p});
+    while (cached + got > kMaxCached) {
+      auto old = free_blocks.begin();
+      for (auto it = free_blocks.begin(); it != free_blocks.end(); ++it)
+        if (it->second.seq < old->second.seq) old = it;
+      (void)hipFree(old->second.p);
+      cached -= old->first.second;
+      free_blocks.erase(old);
+    }
+    free_blocks.insert({{dev, got}, {p, seq++}});
     cached += got;
   }
   void trim() {
     std::lock_guard<std::recursive_mutex> cg(capture_mu());
     std::lock_guard<std::mutex> g(mu);
-    for (auto &kv : free_blocks) (void)hipFree(kv.second);
+    for (auto &kv : free_blocks) (void)hipFree(kv.second.p);
     free_blocks.clear();
     cached = 0;
   }
