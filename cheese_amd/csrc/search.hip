@@ -74,13 +74,6 @@ struct ExpandArgs {
 // residual in LDS and walks all G candidates: windows, child residual, overflow, goal, cheap bounds, T bound
 // (mod 2^16, one lane per flip pair, when n + k <= 16; else mod 2^32 / 2^64, one lane per entry) and the
 // class key of a kept child.  Writes the status byte (and key) of every child of the chunk.
-// kind: 0 general, 1 unit entries, 2 unit permutation; tdel, loc, cdel: DevGate::tdel, ::cutloc, ::cdel
-struct GateHdr { int nq, L, mask, ik, q0, q1, q2, kind, tdel, loc, cdel, cls; };
-template <int NQ> __device__ __forceinline__ GateHdr wuni(const GateHdr &h) {
-  return GateHdr{wuni<NQ>(h.nq), wuni<NQ>(h.L), wuni<NQ>(h.mask), wuni<NQ>(h.ik), wuni<NQ>(h.q0), wuni<NQ>(h.q1),
-                 wuni<NQ>(h.q2), wuni<NQ>(h.kind), wuni<NQ>(h.tdel), wuni<NQ>(h.loc), wuni<NQ>(h.cdel),
-                 wuni<NQ>(h.cls)};
-}
 constexpr int MAXG = 64;
 constexpr int PRE_SPLIT = 4;    // lane groups per parent up to which children are settled from the parent's bounds
 
@@ -88,26 +81,56 @@ constexpr int PRE_SPLIT = 4;    // lane groups per parent up to which children a
 // every block with coalesced 16-byte loads; built inside the kernel they cost each block scattered global loads,
 // which small levels (one parent per wave) cannot amortise.
 struct LevelTabs {
-  // per candidate and entry (g * 64 + e), the child entry's terms for unit gates with at most two per column:
-  // bits 0-2 source column x0, 3-5 power p0 of w, 6-8 x1, 9-11 p1, bit 12 two terms; bit 15: use the table loop
-  uint16_t sdesc[MAXG * 64];
-  GateHdr shdr[MAXG];
+  // per candidate and entry (g * 64 + e), the child entry's terms for unit gates with at most two per column (Parent):
+  // bits 0-5 ring word of the first term in its row, 6 its sign, 7-12 and 13 the second, 14 two terms
+  uint16_t term[MAXG * 64];
+  // per candidate: x: bits 0-7 tdel (at most 255), 8-10 qubits, 11-15 the most the sqrt2 exponent can fall (0 for a
+  // permutation of unit entries, which leaves divisibility by sqrt2 as it is, else the gate's own exponent), 16 an H
+  // (the exponent is read off the parent exactly), 24-31 1 + the T-bound class; y: DevGate::cdel; z: DevGate::ik;
+  // w: bit 0 the terms above form its children, 1 a permutation of unit entries, 8-23 DevGate::cutloc
+  uint4 head[MAXG];
   KeyTab kt;                       // n = 3: the class key's choice of symmetries
   uint8_t spos[16 * 64];           // n = 3: position of entry e under symmetry y (y * 64 + e)
   uint8_t scx[CXL_MAX];            // the cx table when it fits (KSpec::cxlds)
-  // per candidate, for the bounds from the parent alone: bits 0-7 tdel, 8-10 qubits, 11-15 the most the sqrt2 exponent
-  // can fall (0 for a permutation of unit entries, which leaves divisibility by sqrt2 as it is, else the gate's own
-  // exponent), 16-23 cut-delta class, 24 an H (the exponent is read off the parent
-  // exactly), 25-31 1 + the T-bound class
-  uint32_t spre[MAXG];
   uint8_t scsrc[CSRC_MAX * 64];    // cut i's operator-Schmidt matrix: entry source of lane le (i * GS + le)
 };
+// the table in device memory: the part above, then what the dedupe and the gather copy
+// sdesc: bits 0-2 source column x0, 3-5 power p0 of w, 6-8 x1, 9-11 p1, bit 12 two terms; bit 15: use the table loop
+struct SpecTabs {
+  LevelTabs level;
+  uint16_t sdesc[MAXG * 64];
+};
 static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
+
+// A parent's residual in LDS: each entry a + b w + c w^2 + d w^3 as the seven words -b, -c, -d, a, b, c, d, of which the
+// four from word 3 - p on are the entry times w^p (w^4 = -1), for p up to 3; a sign gives the other powers.  A child's
+// term is then two two-word reads, where rotating a coefficient vector in registers took some 30 instructions.  The odd
+// stride keeps the lanes of a row on different banks.
+constexpr int RING = 7;
+template <int NQ> struct Parent {
+  int *e;                          // the group's entries
+  int c;                           // this lane's column
+  const int *row;                  // this lane's row of entries
+  __device__ __forceinline__ void put(int le, int4 v) const {
+    int *w = e + le * RING;
+    w[0] = (int)(0u - (uint32_t)v.y); w[1] = (int)(0u - (uint32_t)v.z); w[2] = (int)(0u - (uint32_t)v.w);
+    w[3] = v.x; w[4] = v.y; w[5] = v.z; w[6] = v.w;
+  }
+  __device__ __forceinline__ int4 entry(int i) const {
+    const int *w = e + i * RING + 3;
+    return make_int4(w[0], w[1], w[2], w[3]);
+  }
+  // the entry and turn at `word` of this lane's row
+  __device__ __forceinline__ int4 turned(uint32_t word) const {
+    const int *w = row + word;
+    return make_int4(w[0], w[1], w[2], w[3]);
+  }
+};
 
 // the expansion's class key outside it: the tables read from their global copy
 template <int NQ> __device__ __forceinline__ uint64_t node_key(int4 s, int k, int le, const KSpec &sp) {
   if constexpr (NQ == 3) {
-    const LevelTabs *t = (const LevelTabs *)sp.ktab;
+    const LevelTabs *t = &((const SpecTabs *)sp.ktab)->level;
     int image = 0;
     return class_key3(s, k, le, t->spos, t->kt.adm, sp.cjm, image);
   } else {
@@ -121,18 +144,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
   __shared__ uint2 stage_x[TS_STRIDE];
   __shared__ uint4 stage_p[2 * TS_STRIDE];
-  __shared__ int4 spar[256];                   // each group's parent residual
+  __shared__ int spar[256 * RING];             // each group's parent residual (Parent)
   __shared__ __align__(16) LevelTabs tb;
   for (int i = threadIdx.x; i < (int)(sizeof(LevelTabs) / 16); i += blockDim.x) ((uint4 *)&tb)[i] = sp.ktab[i];
-  const uint16_t *const sdesc = tb.sdesc;
-  const GateHdr *const shdr = tb.shdr;
   const uint8_t *const spos = tb.spos, *const scx = tb.scx, *const scsrc = tb.scsrc;
   const uint32_t cjm = NQ == 3 ? sp.cjm : 0u;
   __syncthreads();
   const int lane = threadIdx.x & 63, le = lane & (GS - 1), slot = lane / GS;
   const int r = le >> NQ, c = le & (N - 1);
   const TStage st{stage_x + (threadIdx.x & ~(GS - 1)), stage_p + (threadIdx.x & ~(GS - 1))};
-  int4 *P = spar + (threadIdx.x & ~(GS - 1));
+  const Parent<NQ> P{spar + (threadIdx.x & ~(GS - 1)) * RING, c, spar + ((threadIdx.x & ~(GS - 1)) + r * N) * RING};
   const long long wave = wave_index();
   const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
   const int G = sp.G;
@@ -171,9 +192,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   for (long long base = wave * CPW; base < nitems; base += nwaves * CPW) {
     const long long item = base + slot;
     if (item >= nitems) continue;
-    // the 64-bit division runs on the vector unit; readfirstlane keeps the parent and the candidate range (the
-    // child loop's bounds) scalar for n = 3
-    const long long pl = wuni64<NQ>(item / gsplit);
+    // readfirstlane keeps the parent and the candidate range (the child loop's bounds) scalar for n = 3; the 64-bit
+    // division, some 150 instructions, is only for split parents
+    const long long pl = wuni64<NQ>(gsplit == 1 ? item : item / gsplit);
     const int gbeg = wuni<NQ>((int)(item - pl * gsplit) * cs), gend = gbeg + cs < G ? gbeg + cs : G;
     const long long pi = a.off + pl;
     const int inst = wuni<NQ>(a.pinst ? (int)a.pinst[pi] : 0);
@@ -193,18 +214,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
       continue;
     }
     __builtin_amdgcn_wave_barrier();
-    P[le] = S;
+    P.put(le, S);
     __builtin_amdgcn_wave_barrier();
-    // window cuts of every candidate of this parent, one candidate per lane, as two bit masks: the candidate
-    // loop then tests bits instead of waiting on a table load per child
-    // lower cut bound of each cut-delta class (one per parent instead of one per child)
-    const bool cdcache = !sp.lite && sp.cx_mono && (pbw & BW_CUTS) && sp.ncd > 0;
-    uint64_t c2c = 0;
-    if (cdcache)
-      for (int j = 0; j < sp.ncd; j++) {
-        const int v = cx_lower(sp, scx, (pbw & BW_NEEDS) >> 8, sp.cdv[j]);
-        c2c |= (uint64_t)(v < 255 ? v : 255) << (8 * j);
-      }
+    // a child's cut needs can be bounded from its parent's
+    const bool cutlow = !sp.lite && sp.cx_mono && (pbw & BW_CUTS);
+    const uint32_t pneeds = (pbw & BW_NEEDS) >> 8;
     // T bounds of this parent's children per T-bound class: tc_ok bit set when one is known, tc_ex when it is the
     // exact bound, else it is a lower bound (a transform stopped once the child was dead)
     uint64_t tc_val = 0;
@@ -232,9 +246,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         if (!(differ(ba) | differ(bb) | differ(bc) | differ(bd))) he |= 16 << q;
       }
     }
-    const int pq = pre && !sp.lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S))) : 0;
+    const int pq = !sp.lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S)), N - 1) : 0;
     uint64_t w2m = 0, w3m = 0, dm = 0;
     int lim = 1 << 30, tcl = -1;                 // n = 3: candidate `lane`'s largest T bound by these bounds; its T class
+    CutLow cl{0, 0, 0};                          // n = 3: candidate `lane`'s least cut needs
+    // window cuts of every candidate of this parent, one candidate per lane, as two bit masks: the candidate
+    // loop then tests bits instead of waiting on a table load per child
     for (int b0 = 0; b0 < G; b0 += GS) {
       const int g = b0 + le;
       bool c2 = false, c3 = false, dead = false;
@@ -245,18 +262,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
           c3 = ((sp.bad3[tri >> 5] >> (tri & 31)) & 1) != 0;
         }
       }
-      if (pre && g < G) {
-        const uint32_t w = tb.spre[g];
-        const int td = (int)(w & 255u), Tp = (int)(pbw & BW_TUNK);
-        const int T = tparent && td != 255 && Tp > td ? Tp - td : 0;
-        const int gm = (int)((w >> 8) & 7u), hq = he >> (__ffs(gm) - 1);
-        const int kd = (w >> 24) & 1u ? pk + 1 - (hq & 1) - ((hq >> 4) & 1) : pk - (int)((w >> 11) & 31u), h = kd > 0 ? kd : 0;
-        const int c2lo = cdcache ? (int)((c2c >> (8 * ((w >> 16) & 255u))) & 0xff) : 0;
-        const int l = t_budget(h, c2lo, __popc(pq & ~gm), rem) * sp.tdiv;
-        dead = T > l;
-        if constexpr (NQ == 3) {
-          lim = l;
-          tcl = (int)(w >> 25) - 1;
+      if ((pre || (NQ == 3 && cutlow)) && g < G) {
+        const uint4 hd = tb.head[g];
+        const CutLow lo = cutlow ? cut_low(sp, scx, pneeds, hd.y) : CutLow{0, 0, 0};
+        if constexpr (NQ == 3) cl = lo;
+        if (pre) {
+          const uint32_t w = hd.x;
+          const int td = (int)(w & 255u), Tp = (int)(pbw & BW_TUNK);
+          const int T = tparent && td != 255 && Tp > td ? Tp - td : 0;
+          const int gm = (int)((w >> 8) & 7u), hq = he >> (__ffs(gm) - 1);
+          const int kd = (w >> 16) & 1u ? pk + 1 - (hq & 1) - ((hq >> 4) & 1) : pk - (int)((w >> 11) & 31u), h = kd > 0 ? kd : 0;
+          const int l = t_budget(h, lo.c2, __popc(pq & ~gm), rem) * sp.tdiv;
+          dead = T > l;
+          if constexpr (NQ == 3) {
+            lim = l;
+            tcl = (int)(w >> 24) - 1;
+          }
         }
       }
       w2m |= gballot<GS>(c2) << b0;
@@ -265,86 +286,82 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     // (a split whose share of the candidates is empty has gbeg >= gend, and gbeg may lie beyond bit 63)
     const uint64_t range = gbeg >= gend ? 0ull : (gend - gbeg < 64 ? (1ull << (gend - gbeg)) - 1 : ~0ull) << gbeg;
-    uint64_t todo = range & ~(w2m | w3m | dm);
     w2m &= range;
     w3m &= range & ~w2m;
-    dm &= range & ~w2m & ~w3m;
-    const uint32_t npre = (uint32_t)__popcll(dm);
-    n_eval += npre;
-    n_pre += npre;
-    // the settled children's status in one store per lane, their tallies at once
-    for (int b0 = 0; b0 < G; b0 += GS) {
-      const int g = b0 + le;
-      if (g < G && (((w2m | w3m | dm) >> g) & 1))
-        a.status[pl * G + g] = (w2m >> g) & 1 ? ST_W2 : (w3m >> g) & 1 ? ST_W3 : ST_DEAD;
-    }
-    if (le == 0) {
-      if (w2m) atomicAdd(&tl[ST_W2], (uint32_t)__popcll(w2m));
-      if (w3m) atomicAdd(&tl[ST_W3], (uint32_t)__popcll(w3m));
-      if (dm) atomicAdd(&tl[ST_DEAD], npre);
-    }
+    const uint64_t evalm = range & ~w2m & ~w3m;
+    dm &= evalm;
+    uint64_t todo = evalm & ~dm, alivem = 0, foundm = 0, ovfm = 0;      // status of the children that are formed: else dead
+    n_pre += (uint32_t)__popcll(dm);
     while (todo) {
       const int g = wuni<NQ>(__ffsll((long long)todo) - 1);
       todo &= todo - 1;
-      const long long cc = pl * G + g;
       uint8_t stt;
       uint64_t key = 0;
       uint32_t bw = BW_TUNK;
       {
         // child residual entry (r, c) = sum_m P[r][x_m] ginv[m][lc] (src/cheese.cu:146-174)
-        const GateHdr h = wuni<NQ>(shdr[g]);
-        int lc = (c >> h.q0) & 1;
-        if (h.nq > 1) lc |= ((c >> h.q1) & 1) << 1;
-        if (h.nq > 2) lc |= ((c >> h.q2) & 1) << 2;
-        const int cb = c & ~h.mask;
-        const int8_t *ph = sp.gates[g].ph;    // table loop only: gates with more than two terms per column
+        const uint4 hv = tb.head[g];
+        const uint32_t hx = (uint32_t)wuni<NQ>((int)hv.x), hw = (uint32_t)wuni<NQ>((int)hv.w);
         int4 s;
         bool of = false;
-        const uint32_t desc = sdesc[g * 64 + le];
-        if (h.kind && small && !(desc & 0x8000u)) {
-          s = zrot(P[r * N + (desc & 7)], (desc >> 3) & 7);
-          if (desc & 0x1000u) {
-            const int4 t = zrot(P[r * N + ((desc >> 6) & 7)], (desc >> 9) & 7);
-            s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
+        int k = pk + wuni<NQ>((int)hv.z);
+        const bool fast = (hw & 1u) && small;
+        if (fast) {
+          const uint32_t d = tb.term[g * 64 + le];
+          const int4 u = P.turned(d & 63u);
+          const int m0 = -(int)((d >> 6) & 1u);
+          if (hw & 2u) s = make_int4((u.x ^ m0) - m0, (u.y ^ m0) - m0, (u.z ^ m0) - m0, (u.w ^ m0) - m0);
+          else {
+            int4 v = P.turned((d >> 7) & 63u);
+            const int m1 = -(int)((d >> 13) & 1u), on = -(int)((d >> 14) & 1u), o = -m0 - m1;
+            v = make_int4(v.x & on, v.y & on, v.z & on, v.w & on);
+            s = make_int4((u.x ^ m0) + ((v.x ^ m1) + o), (u.y ^ m0) + ((v.y ^ m1) + o), (u.z ^ m0) + ((v.z ^ m1) + o),
+                          (u.w ^ m0) + ((v.w ^ m1) + o));
           }
-        } else if (h.kind && small) {
-          int4 acc = make_int4(0, 0, 0, 0);
-          for (int m = 0; m < h.L; m++) {
-            const int p = ph[m * h.L + lc];
-            if (p < 0) continue;
-            int x = cb | ((m & 1) << h.q0);
-            if (h.nq > 1) x |= ((m >> 1) & 1) << h.q1;
-            if (h.nq > 2) x |= ((m >> 2) & 1) << h.q2;
-            const int4 t = zrot(P[r * N + x], p);
-            acc.x += t.x; acc.y += t.y; acc.z += t.z; acc.w += t.w;
-            if (h.kind == 2) break;
-          }
-          s = acc;
         } else {
           const DevGate &dg = sp.gates[g];
-          long long va = 0, vb = 0, vc = 0, vd = 0;
-          for (int m = 0; m < h.L; m++) {
-            const int4 gm = dg.inv[m * h.L + lc];
-            if (zzero(gm)) continue;
-            int x = cb | ((m & 1) << h.q0);
-            if (h.nq > 1) x |= ((m >> 1) & 1) << h.q1;
-            if (h.nq > 2) x |= ((m >> 2) & 1) << h.q2;
-            const int4 v = P[r * N + x];
-            va += (long long)v.x * gm.x - (long long)v.y * gm.w - (long long)v.z * gm.z - (long long)v.w * gm.y;
-            vb += (long long)v.x * gm.y + (long long)v.y * gm.x - (long long)v.z * gm.w - (long long)v.w * gm.z;
-            vc += (long long)v.x * gm.z + (long long)v.y * gm.y + (long long)v.z * gm.x - (long long)v.w * gm.w;
-            vd += (long long)v.x * gm.w + (long long)v.y * gm.z + (long long)v.z * gm.y + (long long)v.w * gm.x;
+          int lc = (c >> dg.q[0]) & 1;
+          if (dg.nq > 1) lc |= ((c >> dg.q[1]) & 1) << 1;
+          if (dg.nq > 2) lc |= ((c >> dg.q[2]) & 1) << 2;
+          const int cb = c & ~dg.mask;
+          auto source = [&](int m) {
+            int x = cb | ((m & 1) << dg.q[0]);
+            if (dg.nq > 1) x |= ((m >> 1) & 1) << dg.q[1];
+            if (dg.nq > 2) x |= ((m >> 2) & 1) << dg.q[2];
+            return P.entry(r * N + x);
+          };
+          if (dg.unit && small) {
+            int4 acc = make_int4(0, 0, 0, 0);
+            for (int m = 0; m < dg.L; m++) {
+              const int p = dg.ph[m * dg.L + lc];
+              if (p < 0) continue;
+              const int4 t = zrot(source(m), p);
+              acc.x += t.x; acc.y += t.y; acc.z += t.z; acc.w += t.w;
+            }
+            s = acc;
+          } else {
+            long long va = 0, vb = 0, vc = 0, vd = 0;
+            for (int m = 0; m < dg.L; m++) {
+              const int4 gm = dg.inv[m * dg.L + lc];
+              if (zzero(gm)) continue;
+              const int4 v = source(m);
+              va += (long long)v.x * gm.x - (long long)v.y * gm.w - (long long)v.z * gm.z - (long long)v.w * gm.y;
+              vb += (long long)v.x * gm.y + (long long)v.y * gm.x - (long long)v.z * gm.w - (long long)v.w * gm.z;
+              vc += (long long)v.x * gm.z + (long long)v.y * gm.y + (long long)v.z * gm.x - (long long)v.w * gm.w;
+              vd += (long long)v.x * gm.w + (long long)v.y * gm.z + (long long)v.z * gm.y + (long long)v.w * gm.x;
+            }
+            of = va != (int)va || vb != (int)vb || vc != (int)vc || vd != (int)vd;
+            s = make_int4((int)va, (int)vb, (int)vc, (int)vd);
           }
-          of = va != (int)va || vb != (int)vb || vc != (int)vc || vd != (int)vd;
-          s = make_int4((int)va, (int)vb, (int)vc, (int)vd);
         }
-        int k = pk + h.ik;
-        n_eval++;
-        if (gany<GS>(of)) stt = ST_OVF;
+        if (!fast && gany<GS>(of)) stt = ST_OVF;
         else {
-          while (k > 0 && gall<GS>(zhalf(s))) { s = zdown(s); k--; }
+          // parents that are children themselves are normalised, which a permutation of unit entries leaves them
+          if (!(g1 != 255 && fast && (hw & 2u) && k == pk))
+            while (k > 0 && gall<GS>(zhalf(s))) { s = zdown(s); k--; }
+          const uint64_t nzb = gballot<GS>(!zzero(s));
           // the goal's entries are read only for a child with the goal's exponent and nonzero pattern
-          if (k == sp.gk && gballot<GS>(!zzero(s)) == sp.goalnz && gall<GS>(zeq(s, sp.goal[le]))) stt = ST_FOUND;
+          if (k == sp.gk && nzb == sp.goalnz && gall<GS>(zeq(s, sp.goal[le]))) stt = ST_FOUND;
           else {
             bool alive = true;
             if (sp.standard || sp.lite) {
@@ -352,44 +369,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               if (sp.lite) hh = k;
               else {
                 n_cheap++;
-                const uint64_t nzb = gballot<GS>(!zzero(s));
-                const int hs = h_struct<NQ>(nzb);
+                const int hs = h_struct<NQ>(nzb), gm = (int)((hx >> 8) & 7u);
                 hh = k > hs ? k : hs;
-                supp = support<NQ>(s, le, nzb);
+                supp = __popc((pq & ~gm) | support_mask<NQ>(s, le, nzb, gm));
               }
               // Bracket the child's bounds from its parent's: the T bound moves by at most the gate's transfer-
-              // matrix exponent h.tdel (Clifford gates keep it), each cut need drops by at most h.cdel.  The
+              // matrix exponent tdel (Clifford gates keep it), each cut need drops by at most its cdel.  The
               // bound combination is monotone in T and in the cut bound, so the brackets settle most children
               // before the cut ranks and the T transform are computed.
-              const bool tpar = tparent && h.tdel != 255;
+              const int tdel = (int)(hx & 255u);
+              const bool tpar = tparent && tdel != 255;
               const int Tp = (int)(pbw & BW_TUNK);
               // a sibling of the same T-bound class already has its exact bound (it is this child's too) or a
               // lower bound
-              const int tc = (h.cls >> 8) - 1;
+              const int tc = (int)(hx >> 24) - 1;
               const bool tcached = tc >= 0 && ((tc_ok >> tc) & 1);
               const int tcv = tcached ? (int)((tc_val >> (8 * tc)) & 0xff) : 0;
               const bool tcex = tcached && ((tc_ex >> tc) & 1);
-              const bool tknown = (tpar && h.tdel == 0) || tcex;
-              const int Tbr = tpar ? (Tp > h.tdel ? Tp - h.tdel : 0) : 0;
+              const bool tknown = (tpar && tdel == 0) || tcex;
+              const int Tbr = tpar ? (Tp > tdel ? Tp - tdel : 0) : 0;
               int T = tcex ? tcv : (Tbr > tcv ? Tbr : tcv);    // exact if tknown, else a lower bound
               bool texact = tknown;
-              const int c2lo = cdcache ? (int)((c2c >> (8 * (h.cls & 0xff))) & 0xff)
-                               : !sp.lite && sp.cx_mono && (pbw & BW_CUTS) ? cx_lower(sp, scx, (pbw & BW_NEEDS) >> 8, (uint32_t)h.cdel)
-                               : 0;
+              CutLow lo{0, 0, 0};
+              if (cutlow) {
+                if constexpr (NQ == 3) lo = CutLow{gget<GS>(cl.low, g), (int)gget<GS>((uint32_t)cl.idx, g), (int)gget<GS>((uint32_t)cl.c2, g)};
+                else lo = cut_low(sp, scx, pneeds, hv.y);
+              }
               // alive exactly when T / tdiv, rounded up, is at most t_budget: T <= t_budget * tdiv
-              if (T > t_budget(hh, c2lo, supp, rem) * sp.tdiv) alive = false;
+              if (T > t_budget(hh, lo.c2, supp, rem) * sp.tdiv) alive = false;
               else {
                 if (!sp.lite) {
-                  uint32_t needs = (pbw & BW_NEEDS) >> 8;
-                  const uint32_t keepc = (pbw & BW_CUTS) ? (uint32_t)h.loc : 0u;
-                  const bool stop = sp.cx_mono && sp.have_table && sp.ncuts <= BW_MAXCUTS && (pbw & BW_CUTS);
-                  const CutStop cst{stop, stop ? low_needs(sp, needs, (uint32_t)h.cdel) : 0u, T, hh, supp, rem};
+                  uint32_t needs = pneeds;
+                  const uint32_t keepc = (pbw & BW_CUTS) ? hw >> 8 : 0u;
+                  const CutStop cst{cutlow && sp.have_table, lo.low, lo.idx, T, hh, supp, rem};
                   c2 = wuni<NQ>(cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts));
                   bw = (needs << 8 & ~BW_CUTS) | (sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
                 }
                 const int tmax = t_budget(hh, c2, supp, rem) * sp.tdiv;
                 if (T > tmax) alive = false;
-                else if (!texact && tpar && rem <= 1 && Tp + h.tdel <= tmax) {
+                else if (!texact && tpar && rem <= 1 && Tp + tdel <= tmax) {
                   // alive whatever the exact T; its children (budget 0) need no inherited T bound
                   alive = true;
                 } else if (!texact) {
@@ -413,11 +431,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                       const uint64_t sib = gballot<GS>(tcl == tc && T > lim) & todo;
                       if (sib) {
                         todo &= ~sib;
-                        if ((sib >> lane) & 1) a.status[pl * G + lane] = ST_DEAD;
-                        const uint32_t ns = (uint32_t)__popcll(sib);
-                        if (le == 0) atomicAdd(&tl[ST_DEAD], ns);
-                        n_eval += ns;
-                        n_pre += ns;
+                        n_pre += (uint32_t)__popcll(sib);
                       }
                     }
                   }
@@ -441,12 +455,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
           }
         }
       }
-      if (le == 0) {
-        atomicAdd(&tl[stt], 1u);
-        a.status[cc] = stt;
-        if (stt == ST_ALIVE && keep) { a.keys[cc] = key; a.info[cc] = bw; }
-        if (stt == ST_FOUND)
-          atomicMin(&icnt[(size_t)inst * IC_N + IC_FIRST], (unsigned long long)(a.off * G + cc));
+      const uint64_t me = 1ull << g;
+      if (stt == ST_ALIVE) alivem |= me;
+      if (stt == ST_FOUND) foundm |= me;
+      if (stt == ST_OVF) ovfm |= me;
+      if (stt == ST_ALIVE && keep && le == 0) { a.keys[pl * G + g] = key; a.info[pl * G + g] = bw; }
+    }
+    // the children's status, one candidate per lane, and their tallies
+    for (int b0 = 0; b0 < G; b0 += GS) {
+      const int g = b0 + le;
+      if (g < G && ((range >> g) & 1))
+        a.status[pl * G + g] = (w2m >> g) & 1      ? ST_W2
+                               : (w3m >> g) & 1    ? ST_W3
+                               : (alivem >> g) & 1 ? ST_ALIVE
+                               : (foundm >> g) & 1 ? ST_FOUND
+                               : (ovfm >> g) & 1   ? ST_OVF
+                                                   : ST_DEAD;
+    }
+    n_eval += (uint32_t)__popcll(evalm);
+    if (le == 0) {
+      if (w2m) atomicAdd(&tl[ST_W2], (uint32_t)__popcll(w2m));
+      if (w3m) atomicAdd(&tl[ST_W3], (uint32_t)__popcll(w3m));
+      if (alivem) atomicAdd(&tl[ST_ALIVE], (uint32_t)__popcll(alivem));
+      const uint64_t dead = evalm & ~(alivem | foundm | ovfm);
+      if (dead) atomicAdd(&tl[ST_DEAD], (uint32_t)__popcll(dead));
+      if (ovfm) atomicAdd(&tl[ST_OVF], (uint32_t)__popcll(ovfm));
+      if (foundm) {
+        atomicAdd(&tl[ST_FOUND], (uint32_t)__popcll(foundm));
+        atomicMin(&icnt[(size_t)inst * IC_N + IC_FIRST],
+                  (unsigned long long)((a.off + pl) * G + __ffsll((long long)foundm) - 1));
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -597,18 +634,9 @@ struct ChildTab {
   uint8_t ik[MAXG];
 };
 __device__ __forceinline__ void load_child_tab(ChildTab &t, const KSpec &sp) {
-  const LevelTabs *g = (const LevelTabs *)sp.ktab;
+  const SpecTabs *g = (const SpecTabs *)sp.ktab;
   for (int i = threadIdx.x; i < sp.G * 8; i += blockDim.x) ((uint4 *)t.desc)[i] = ((const uint4 *)g->sdesc)[i];
-  for (int i = threadIdx.x; i < sp.G; i += blockDim.x) t.ik[i] = (uint8_t)g->shdr[i].ik;
-}
-
-// value of lane q of the lane group (q uniform across the group)
-template <int GS> __device__ __forceinline__ uint32_t gget(uint32_t v, int q) {
-  if constexpr (GS == 64) return (uint32_t)__builtin_amdgcn_readlane((int)v, q);
-  else return (uint32_t)__shfl((int)v, q, GS);
-}
-template <int GS> __device__ __forceinline__ uint64_t gget64(uint64_t v, int q) {
-  return (uint64_t)gget<GS>((uint32_t)v, q) | ((uint64_t)gget<GS>((uint32_t)(v >> 32), q) << 32);
+  for (int i = threadIdx.x; i < sp.G; i += blockDim.x) t.ik[i] = (uint8_t)g->level.head[i].z;
 }
 
 template <int NQ>
@@ -921,7 +949,6 @@ struct chz_ctx {
   long long m = 0;             // nodes in the current frontier (buffer cur)
   int cur = 0, gstep = -1, nslots = 0;
   bool shared_steps = false;      // the batch has held more than one search at once (captured steps are used)
-  std::vector<uint32_t> cdv;      // distinct cut-delta values of the spec's gates (bits 0-7 of DevGate::cls index them)
   // level control block, uploaded in one copy at the start of every level and read back in one copy:
   // [cnt: C_N counters | stage stripes | icnt: stripes of per-slot IC_N counters | d_rem: per-slot budgets | d_keepi:
   // per-slot keep flags]
@@ -1646,12 +1673,14 @@ template <int NQ> static void batch_step(chz_ctx *c) {
 
 // LevelTabs for a spec: the term descriptors and headers of its candidates, its symmetries' entry positions (n = 3),
 // its cx table (when it fits) and the entry sources of its cut matrices
-static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const KSpec &k, const chz::SymGroup &grp,
+static void build_level_tabs(SpecTabs &TS, const std::vector<DevGate> &dg, const KSpec &k, const chz::SymGroup &grp,
                              const HostSpec &s) {
-  std::memset(&T, 0, sizeof T);
+  std::memset(&TS, 0, sizeof TS);
+  LevelTabs &T = TS.level;
   const int n = k.n, N = 1 << n, GS = N * N;
   for (int g = 0; g < k.G; g++) {
     const DevGate &d = dg[g];
+    bool terms = true;
     for (int e = 0; e < GS; e++) {
       const int ec = e & (N - 1);
       int lc = (ec >> d.q[0]) & 1;
@@ -1659,6 +1688,7 @@ static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const
       if (d.nq > 2) lc |= ((ec >> d.q[2]) & 1) << 2;
       const int cb = ec & ~d.mask;
       uint32_t desc = 0;
+      uint32_t ring = 0;
       int nt = 0;
       for (int m = 0; d.unit && m < d.L; m++) {
         const int p = d.ph[m * d.L + lc];
@@ -1666,10 +1696,15 @@ static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const
         int x = cb | ((m & 1) << d.q[0]);
         if (d.nq > 1) x |= ((m >> 1) & 1) << d.q[1];
         if (d.nq > 2) x |= ((m >> 2) & 1) << d.q[2];
-        if (nt < 2) desc |= (uint32_t)(x | (p << 3)) << (6 * nt);
+        if (nt < 2) {
+          desc |= (uint32_t)(x | (p << 3)) << (6 * nt);
+          ring |= (uint32_t)(x * RING + 3 - (p & 3) | (p >> 2 & 1) << 6) << (7 * nt);
+        }
         nt++;
       }
-      T.sdesc[g * 64 + e] = (uint16_t)(!d.unit || nt == 0 || nt > 2 ? 0x8000u : nt == 2 ? desc | 0x1000u : desc);
+      T.term[g * 64 + e] = (uint16_t)(ring | (nt == 2 ? 0x4000u : 0u));
+      terms = terms && d.unit && nt >= 1 && nt <= 2;
+      TS.sdesc[g * 64 + e] = (uint16_t)(!d.unit || nt == 0 || nt > 2 ? 0x8000u : nt == 2 ? desc | 0x1000u : desc);
     }
     int kind = 0;
     if (d.unit) {
@@ -1683,9 +1718,10 @@ static void build_level_tabs(LevelTabs &T, const std::vector<DevGate> &dg, const
     const int fall = kind == 2 ? 0 : std::min(31, std::max(0, s.gates[g].gk));
     bool had = d.nq == 1 && d.unit && d.ik == 1 && s.gates[g].gk == 1;
     for (int i = 0; had && i < 4; i++) had = d.ph[i] == 0 || d.ph[i] == 4;
-    T.spre[g] = (uint32_t)had << 24 | (uint32_t)(d.cls >> 8) << 25 | (uint32_t)std::min(255, d.tdel) | (uint32_t)(d.mask & 7) << 8 | (uint32_t)fall << 11 |
-                (uint32_t)(d.cls & 0xff) << 16;
-    T.shdr[g] = GateHdr{d.nq, d.L, d.mask, d.ik, d.q[0], d.q[1], d.q[2], kind, d.tdel, d.cutloc, d.cdel, d.cls};
+    T.head[g] = make_uint4((uint32_t)std::min(255, d.tdel) | (uint32_t)(d.mask & 7) << 8 | (uint32_t)fall << 11 |
+                               (uint32_t)had << 16 | (uint32_t)d.cls << 24,
+                           (uint32_t)d.cdel, (uint32_t)d.ik,
+                           (uint32_t)terms | (uint32_t)(kind == 2) << 1 | (uint32_t)(d.cutloc & 0xffff) << 8);
   }
   if (n == 3) {
     // per order of the qubits' sums, the symmetries that make it smallest: qubit q goes to place image(q)
@@ -1761,16 +1797,6 @@ static void upload_spec(chz_ctx *c) {
       }
   }
   c->avg_terms = columns > 0 ? terms / columns : 1.0;
-  // cut-delta classes: the lower cut bound of a child depends on its parent and on its gate's cdel only, so the
-  // expansion computes it once per parent and class
-  std::vector<uint32_t> cdv;
-  for (DevGate &d : dg) {
-    size_t j = 0;
-    while (j < cdv.size() && cdv[j] != (uint32_t)d.cdel) j++;
-    if (j == cdv.size()) cdv.push_back((uint32_t)d.cdel);
-    d.cls = (int)j;
-  }
-  c->cdv = cdv;
   // T-bound classes: non-Clifford candidates whose children always have equal T bounds (same_t_bound), so a
   // parent's expansion computes the bound once per class
   {
@@ -1785,7 +1811,7 @@ static void upload_spec(chz_ctx *c) {
       for (int m : mem) cls[m] = ncls;
       ncls++;
     }
-    for (int g = 0; g < G; g++) dg[g].cls |= (cls[g] + 1) << 8;
+    for (int g = 0; g < G; g++) dg[g].cls = cls[g] + 1;
   }
   std::vector<int4> goal(N * N);
   for (int i = 0; i < N * N; i++) goal[i] = make_int4((int)s.goal[i].a, (int)s.goal[i].b, (int)s.goal[i].c, (int)s.goal[i].d);
@@ -1856,8 +1882,8 @@ static void upload_spec(chz_ctx *c) {
   // a cut bound from lowered needs is a lower bound only if the table never decreases when a need grows
   k.cx_mono = 1;
   k.ncx = (int)s.cxtable.size();
-  k.ncd = c->cdv.size() <= (size_t)CD_MAX ? (int)c->cdv.size() : 0;
-  for (int j = 0; j < k.ncd; j++) k.cdv[j] = c->cdv[j];
+  k.cut1 = k.ncuts <= std::min(CSRC_MAX, BW_MAXCUTS);
+  for (int i = 0; i < k.ncuts; i++) k.cut1 = k.cut1 && k.cutsize[i] == 1 && k.rad[i] == 3 && k.n > 1;
   k.cxlds = s.cxtable.size() <= (size_t)CXL_MAX;
   for (int v : s.cxtable) if (v < 0 || v > 255) k.cxlds = 0;
   if (k.have_table) {
@@ -1892,10 +1918,10 @@ static void upload_spec(chz_ctx *c) {
   k.maglim = (uint32_t)(0x7fffffffull / gmax);
   k.cjm = 0;
   for (int y = 0; y < k.nsym && y < 16; y++) k.cjm |= (uint32_t)(c->grp.conj[y] != 0) << y;
-  std::vector<LevelTabs> tabs(1);
+  std::vector<SpecTabs> tabs(1);
   build_level_tabs(tabs[0], dg, k, c->grp, s);
-  c->ktab.need(sizeof(LevelTabs));
-  chz::copy_sync(c->ktab.p, tabs.data(), sizeof(LevelTabs), hipMemcpyHostToDevice, c->stream);
+  c->ktab.need(sizeof(SpecTabs));
+  chz::copy_sync(c->ktab.p, tabs.data(), sizeof(SpecTabs), hipMemcpyHostToDevice, c->stream);
   k.ktab = (const uint4 *)c->ktab.p;
 }
 

@@ -19,6 +19,15 @@ template <int NQ> __device__ __forceinline__ long long wuni64(long long v) {
   else return v;
 }
 
+// value of lane q of the lane group (q uniform across the group)
+template <int GS> __device__ __forceinline__ uint32_t gget(uint32_t v, int q) {
+  if constexpr (GS == 64) return (uint32_t)__builtin_amdgcn_readlane((int)v, q);
+  else return (uint32_t)__shfl((int)v, q, GS);
+}
+template <int GS> __device__ __forceinline__ uint64_t gget64(uint64_t v, int q) {
+  return (uint64_t)gget<GS>((uint32_t)v, q) | ((uint64_t)gget<GS>((uint32_t)(v >> 32), q) << 32);
+}
+
 enum : uint8_t { ST_DEAD = 0, ST_ALIVE = 1, ST_FOUND = 2, ST_W2 = 3, ST_W3 = 4, ST_OVF = 6 };
 constexpr uint32_t INFO_NOBOUND = 1u << 31;    // spec without bounds: every child is kept
 
@@ -120,6 +129,7 @@ template <int NQ> __device__ __forceinline__ bool child_of(ChildTerms t, uint32_
 // b = group ballot of the nonzero entries
 template <int NQ> __device__ __forceinline__ int h_struct(uint64_t b) {
   constexpr int N = 1 << NQ;
+  if (__popcll(b) != N) return 0;
   uint64_t col0 = 0;
 #pragma unroll
   for (int r = 0; r < N; r++) col0 |= 1ull << (r * N);
@@ -160,13 +170,15 @@ template <int NQ> __host__ __device__ constexpr uint64_t pair_mask(int q) {
 
 // qubits the matrix acts on non-trivially (src/cheese.cu:305-319), as a mask; b = group ballot of the nonzero
 // entries.  A nonzero entry off the qubit's diagonal blocks settles that qubit without comparing blocks.
-template <int NQ> __device__ __forceinline__ int support_mask(int4 s, int le, uint64_t b) {
+// Only the qubits in `ask` are looked at: a gate leaves the others as trivial or not as they were in the parent.
+template <int NQ> __device__ __forceinline__ int support_mask(int4 s, int le, uint64_t b, int ask) {
   constexpr int N = 1 << NQ, GS = N * N;
   const int r = le >> NQ, c = le & (N - 1);
   int m = 0;
 #pragma unroll
   for (int q = 0; q < NQ; q++) {
     const int bit = 1 << q;
+    if (!(ask & bit)) continue;
     if (b & offdiag_mask<NQ>(q)) { m |= bit; continue; }
     const int4 o = gxor<GS>(s, bit * N + bit);
     const bool viol = !((r | c) & bit) && !zeq(s, o);
@@ -174,7 +186,6 @@ template <int NQ> __device__ __forceinline__ int support_mask(int4 s, int le, ui
   }
   return m;
 }
-template <int NQ> __device__ __forceinline__ int support(int4 s, int le, uint64_t b) { return __popc(support_mask<NQ>(s, le, b)); }
 
 __host__ __device__ inline int spread_bits(int v, int mask, int n) {   // bit j of v -> j-th set bit of mask
   int out = 0, j = 0;
@@ -246,40 +257,82 @@ __device__ __forceinline__ int cx_at(const KSpec &sp, const uint8_t *cxl, int id
   return sp.cxlds ? (int)cxl[idx] : sp.cxtable[idx];
 }
 
-// Bounds known before the cuts of a child: the smallest cut needs its parent leaves (packed as in the bound word) and
-// whether they may be used, its T bound's lower end, and the other arguments of the bound.  Once the needs found so far
-// and the smallest possible others put the child over its budget, the remaining ranks are left out (the value returned
-// is then that lower cut bound, and `needs` is not the child's).
-struct CutStop { bool on; uint32_t low; int T, h, supp, rem; };
+// The least a child's cuts can need, from its parent's packed needs: each need drops by at most the gate's per-cut delta
+// (operator-Schmidt ranks multiply; 7: by any amount).  low: the needs, packed; idx: their place in the cx table; c2: the
+// cut bound there, a lower bound on the child's since the table is non-decreasing in every need.
+struct CutLow { uint32_t low; int idx, c2; };
+__device__ __forceinline__ CutLow cut_low(const KSpec &sp, const uint8_t *cxl, uint32_t pneeds, uint32_t cdel) {
+  CutLow o{0, 0, 0};
+  int mult = 1, mx = 0;
+  for (int i = 0; i < sp.ncuts; i++) {
+    const int dl = (int)((cdel >> (3 * i)) & 7u);
+    int nd = (int)((pneeds >> (3 * i)) & 7u) - dl;
+    nd = dl == 7 || nd < 0 ? 0 : nd;
+    o.low |= (uint32_t)nd << (3 * i);
+    o.idx += nd * mult;
+    mult *= sp.rad[i];
+    if (nd > mx) mx = nd;
+  }
+  o.c2 = sp.have_table ? cx_at(sp, cxl, o.idx) : mx;
+  return o;
+}
+
+// Bounds known before the cuts of a child: the smallest cut needs its parent leaves (CutLow) and whether they may be
+// used, its T bound's lower end, and the other arguments of the bound.  Once the needs found so far and the smallest
+// possible others put the child over its budget, the remaining ranks are left out (the value returned is then that lower
+// cut bound, and `needs` is not the child's).
+struct CutStop { bool on; uint32_t low; int lo, T, h, supp, rem; };
+
+// The need of a cut of one qubit, whose rank is clipped at 3: 0, 1 or 2 for a rank of at most 1, 2 or more.  v: the
+// operator-Schmidt matrix, 4 rows of 4^(n - 1) lanes, in F_p.  v pv - fr pr is zero in the pivot's row and column by
+// itself, so no row needs to be masked, and two eliminations decide.
+template <int NQ> __device__ __forceinline__ int cut_need1(uint32_t v, int le) {
+  constexpr int GS = 1 << (2 * NQ), C = GS / 4;
+  int need = 0;
+#pragma unroll
+  for (int step = 0; step < 2; step++) {
+    const uint64_t bb = gballot<GS>(v != 0);
+    if (!bb) return need;
+    need = step;
+    const int p = __ffsll((long long)bb) - 1;
+    const uint32_t pv = gget<GS>(v, p);
+    const uint32_t fr = __shfl(v, (le & ~(C - 1)) | (p & (C - 1)), GS);
+    const uint32_t pr = __shfl(v, (p & ~(C - 1)) | (le & (C - 1)), GS);
+    v = mont_mul2(v, pv, fr, pr ? P_MOD - pr : 0u);
+  }
+  return gany<GS>(v != 0) ? 2 : need;
+}
+
+// need of cut i of a matrix with the F_p image fp
+template <int NQ> __device__ __forceinline__ int cut_need(uint32_t fp, int le, const KSpec &sp, const uint8_t *csrc, int i) {
+  constexpr int GS = 1 << (2 * NQ);
+  if (sp.cut1) return cut_need1<NQ>((uint32_t)__shfl(fp, (int)csrc[i * GS + le], GS), le);
+  const int rad = sp.rad[i], sa = sp.cutsize[i];
+  const int R = 1 << (2 * sa);
+  int stop = R;
+  if (rad >= 2 && rad - 2 < 30 && (1 << (rad - 2)) + 1 < stop) stop = (1 << (rad - 2)) + 1;
+  const int src = i < CSRC_MAX ? (int)csrc[i * GS + le] : cut_source<NQ>(le, sp.cutmask[i], sa);
+  const int rk = cut_rank<NQ>(fp, le, src, sa, stop);
+  int need = 0;
+  while ((1 << need) < rk) need++;
+  return need > rad - 1 ? rad - 1 : need;
+}
 
 template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const KSpec &sp, const uint8_t *cxl,
                                                           const uint8_t *csrc, uint32_t keepc, bool small, const CutStop &st,
                                                           uint32_t &needs, uint32_t &ranks) {
-  constexpr int GS = 1 << (2 * NQ);
   uint32_t fp = 0;
   bool have_fp = false;
-  int idx = 0, mult = 1, mx = 0, lo = 0;
+  int idx = 0, mult = 1, mx = 0, lo = st.lo;
   uint32_t out = 0;
   int todo = sp.ncuts - __popc(keepc & ((1u << sp.ncuts) - 1));
-  if (st.on) {
-    int m = 1;
-    for (int i = 0; i < sp.ncuts; i++) { lo += (int)((st.low >> (3 * i)) & 7u) * m; m *= sp.rad[i]; }
-  }
   for (int i = 0; i < sp.ncuts; i++) {
-    const int rad = sp.rad[i], sa = sp.cutsize[i];
     int need;
     if ((keepc >> i) & 1) need = (int)((needs >> (3 * i)) & 7u);
     else {
       if (!have_fp) { fp = small ? fp_of_small(s, sp.wm) : fp_of(s, sp.wm); have_fp = true; }
-      const int R = 1 << (2 * sa);
-      int stop = R;
-      if (rad >= 2 && rad - 2 < 30 && (1 << (rad - 2)) + 1 < stop) stop = (1 << (rad - 2)) + 1;
-      const int src = i < CSRC_MAX ? (int)csrc[i * GS + le] : cut_source<NQ>(le, sp.cutmask[i], sa);
-      const int rk = cut_rank<NQ>(fp, le, src, sa, stop);
+      need = cut_need<NQ>(fp, le, sp, csrc, i);
       ranks++;
-      need = 0;
-      while ((1 << need) < rk) need++;
-      if (need > rad - 1) need = rad - 1;
       if (st.on && --todo > 0) {
         lo += (need - (int)((st.low >> (3 * i)) & 7u)) * mult;
         const int c = cx_at(sp, cxl, lo);
@@ -288,35 +341,10 @@ template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const 
     }
     if (i < BW_MAXCUTS) out |= (uint32_t)need << (3 * i);
     idx += need * mult;
-    mult *= rad;
+    mult *= sp.cut1 ? 3 : sp.rad[i];
     if (need > mx) mx = need;
   }
   needs = out;
-  return sp.have_table ? cx_at(sp, cxl, idx) : mx;
-}
-
-// the smallest needs a child can have: its parent's less its gate's deltas, packed
-__device__ __forceinline__ uint32_t low_needs(const KSpec &sp, uint32_t pneeds, uint32_t cdel) {
-  uint32_t out = 0;
-  for (int i = 0; i < sp.ncuts && i < BW_MAXCUTS; i++) {
-    const int dl = (int)((cdel >> (3 * i)) & 7u), nd = (int)((pneeds >> (3 * i)) & 7u) - dl;
-    out |= (uint32_t)(dl == 7 || nd < 0 ? 0 : nd) << (3 * i);
-  }
-  return out;
-}
-
-// Lower bound on a child's cut bound from its parent's packed needs: each need drops by at most the gate's
-// per-cut delta (operator-Schmidt ranks multiply), and the table is non-decreasing in every need.
-__device__ __forceinline__ int cx_lower(const KSpec &sp, const uint8_t *cxl, uint32_t pneeds, uint32_t cdel) {
-  int idx = 0, mult = 1, mx = 0;
-  for (int i = 0; i < sp.ncuts; i++) {
-    const int dl = (int)((cdel >> (3 * i)) & 7u);
-    int nd = (int)((pneeds >> (3 * i)) & 7u) - dl;
-    nd = dl == 7 || nd < 0 ? 0 : nd;
-    idx += nd * mult;
-    mult *= sp.rad[i];
-    if (nd > mx) mx = nd;
-  }
   return sp.have_table ? cx_at(sp, cxl, idx) : mx;
 }
 
