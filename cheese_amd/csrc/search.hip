@@ -142,8 +142,7 @@ template <int NQ, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_level(KSpec sp, ExpandArgs a,
                                                                                          long long np) {
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
-  __shared__ uint2 stage_x[TS_STRIDE];
-  __shared__ uint4 stage_p[2 * TS_STRIDE];
+  __shared__ __align__(1024) uint4 stage[2 * TS_STRIDE];
   __shared__ int spar[256 * RING];             // each group's parent residual (Parent)
   __shared__ __align__(16) LevelTabs tb;
   for (int i = threadIdx.x; i < (int)(sizeof(LevelTabs) / 16); i += blockDim.x) ((uint4 *)&tb)[i] = sp.ktab[i];
@@ -152,7 +151,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   __syncthreads();
   const int lane = threadIdx.x & 63, le = lane & (GS - 1), slot = lane / GS;
   const int r = le >> NQ, c = le & (N - 1);
-  const TStage st{stage_x + (threadIdx.x & ~(GS - 1)), stage_p + (threadIdx.x & ~(GS - 1))};
+  const TStage st{(char *)stage, (threadIdx.x & ~(GS - 1)) << 4};
   const Parent<NQ> P{spar + (threadIdx.x & ~(GS - 1)) * RING, c, spar + ((threadIdx.x & ~(GS - 1)) + r * N) * RING};
   const long long wave = wave_index();
   const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;

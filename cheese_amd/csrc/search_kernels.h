@@ -388,25 +388,25 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u16x2 pk(int lo, int hi) { u16x2 r; r.x = (unsigned short)lo; r.y = (unsigned short)hi; return r; }
 __device__ __forceinline__ uint32_t bits(u16x2 v) { return (uint32_t)v.x | ((uint32_t)v.y << 16); }
 
-// Per-entry operands of the packed transform, staged in LDS by the lane owning entry e, one array per field
-// (a group's entries are read at a stride of 8 bytes, free of bank conflicts): x[e] = (a, b | c, d) of S[e] mod
-// 2^16, and p[pass * TS_STRIDE + e] the four packed multipliers of conj(S[e]) = (a, -d, -c, -b) for a pass (one
-// 128-bit read per entry and pass).  With
-// Q = S[x] conj(S[e]) = (Qa, Qb, Qc, Qd) the transform needs only Qa, Qc and Qb -+ Qd (below), in two passes:
+// Per-entry operands of the packed transform, staged in LDS by the lane owning entry e, 16 bytes each: x[e] =
+// (a, b | c, d) of S[e] mod 2^16, and p[e] the four packed multipliers of conj(S[e]) = (a, -d, -c, -b) for the pass at
+// hand.  With Q = S[x] conj(S[e]) = (Qa, Qb, Qc, Qd) the transform needs only Qa, Qc and Qb -+ Qd (below), in two passes:
 //   (Qa | Qc)           = xa (a | -c)    + xb (b | -d)    + xc (c | a)     + xd (d | b)
 //   (Qb - Qd | Qb + Qd) = xa (b-d | -b-d) + xb (a+c | a-c) + xc (b+d | b-d) + xd (c-a | c+a)
 constexpr int TS_STRIDE = 256;      // entries per field: one per thread of a block
 struct TStage {
-  uint2 *x;
-  uint4 *p;
+  char *lds;                        // a block's p[TS_STRIDE], then its x[TS_STRIDE], aligned to a wave's share
+  uint32_t group;                   // byte offset of this group's first entry in either
 };
 
-template <int NQ> __device__ __forceinline__ void t_stage(TStage st, int4 s, int le) {
+template <int NQ> __device__ __forceinline__ void t_stage_x(TStage st, int4 s, int le) {
+  *(uint2 *)(st.lds + 16 * TS_STRIDE + (st.group | (uint32_t)le << 4)) = make_uint2(bits(pk(s.x, s.y)), bits(pk(s.z, s.w)));
+}
+template <int NQ> __device__ __forceinline__ void t_stage_p(TStage st, int4 s, int le, int pass) {
   const int a = s.x, b = s.y, c = s.z, d = s.w;
-  st.x[le] = make_uint2(bits(pk(a, b)), bits(pk(c, d)));
-  st.p[le] = make_uint4(bits(pk(a, -c)), bits(pk(b, -d)), bits(pk(c, a)), bits(pk(d, b)));
-  st.p[TS_STRIDE + le] = make_uint4(bits(pk(b - d, -b - d)), bits(pk(a + c, a - c)), bits(pk(b + d, b - d)),
-                                    bits(pk(c - a, c + a)));
+  const uint4 p = pass ? make_uint4(bits(pk(b - d, -b - d)), bits(pk(a + c, a - c)), bits(pk(b + d, b - d)), bits(pk(c - a, c + a)))
+                       : make_uint4(bits(pk(a, -c)), bits(pk(b, -d)), bits(pk(c, a)), bits(pk(d, b)));
+  *(uint4 *)(st.lds + (st.group | (uint32_t)le << 4)) = p;
 }
 
 __device__ __forceinline__ u16x2 as16(uint32_t v) { u16x2 r; r.x = (unsigned short)v; r.y = (unsigned short)(v >> 16); return r; }
@@ -445,7 +445,12 @@ template <int NQ> __device__ __forceinline__ int t_bound16s(TStage st, int4 s, i
 #pragma unroll
   for (int h = 1; h < GS; h <<= 1) {
     const u16x2 o = as16(NQ == 3 ? wave_xor32(bits(q0), h) : (uint32_t)__shfl_xor((int)bits(q0), h, GS));
-    q0 = q0 * as16(le & h ? 0xffffffffu : 0x00010001u) + o;
+    // the lanes with bit h set, as a constant mask: compared per lane, the six factors stayed in registers across the
+    // child loop and were spilled
+    uint64_t hm = 0;
+#pragma unroll
+    for (int l = 0; l < 64; l++) hm |= (uint64_t)((l & h) != 0) << l;
+    q0 = q0 * as16(__builtin_amdgcn_inverse_ballot_w64(hm) ? 0xffffffffu : 0x00010001u) + o;
   }
   // group ORs are uniform over the group: read through readfirstlane (n = 3) they stay in scalar registers
   const uint32_t acc0 = (uint32_t)wuni<NQ>((int)gor<GS>(bits(q0)));
@@ -457,33 +462,39 @@ template <int NQ> __device__ __forceinline__ int t_bound16s(TStage st, int4 s, i
   exact = v <= 1;
   if (exact || T > tmax) return T;
   __builtin_amdgcn_wave_barrier();
-  t_stage<NQ>(st, s, le);
-  __builtin_amdgcn_wave_barrier();
+  t_stage_x<NQ>(st, s, le);
   // lane f of the group handles flip pair f (lane 0 repeats f = 1; OR-accumulation is idempotent)
   int f = le == 0 ? 1 : le;
-  // keep the per-lane LDS address arithmetic inside the child loop: hoisted, its 64 addresses would
-  // halve the kernel's occupancy
+  // keep the per-lane LDS address arithmetic inside the child loop: hoisted, it would cost the kernel occupancy
   asm volatile("" : "+v"(f));
   const int j = 31 - __clz(f);
-  const int lowm = (1 << j) - 1;
+  // entry e of R number i, as byte offsets: bit b of i is bit b of e below j and bit b + 1 from there on.  In the order
+  // of a Gray code one XOR leads from an entry to the next and one from e to e ^ f (two thirds of the instructions that
+  // inserting the zero bit takes)
+  uint32_t vb[2 * NQ - 1];
+#pragma unroll
+  for (int b = 0; b < 2 * NQ - 1; b++) vb[b] = (b >= j ? 32u : 16u) << b;
+  const uint32_t fo = (uint32_t)f << 4;
 #pragma unroll 1
   for (int pass = 1; pass >= 0; pass--) {
-    const uint4 *pm = st.p + pass * TS_STRIDE;
+    __builtin_amdgcn_wave_barrier();
+    t_stage_p<NQ>(st, s, le, pass);
+    __builtin_amdgcn_wave_barrier();
     // the addresses below depend on a value the compiler cannot see through, so they are formed per pass
     // instead of being hoisted out of the pass loop (64 more live registers)
-    int fp = f, lm = lowm;
-    asm volatile("" : "+v"(fp), "+v"(lm));
+    uint32_t at = st.group;
+    asm volatile("" : "+v"(at));
     u16x2 q[H];
 #pragma unroll
-    for (int i = 0; i < H; i++) {
-      const int e = ((i & ~lm) << 1) | (i & lm);         // i with a 0 inserted at bit j
-      const uint2 xv = st.x[e ^ fp];
+    for (int t = 0; t < H; t++) {
+      if (t) at ^= vb[t & 1 ? 0 : t & 2 ? 1 : t & 4 ? 2 : t & 8 ? 3 : 4];
+      const uint2 xv = *(const uint2 *)(st.lds + 16 * TS_STRIDE + (at ^ fo));
+      const uint4 m = *(const uint4 *)(st.lds + at);
       const u16x2 x01 = as16(xv.x), x23 = as16(xv.y);
-      const uint4 m = pm[e];
-      q[i] = x01.xx * as16(m.x) + x01.yy * as16(m.y) + x23.xx * as16(m.z) + x23.yy * as16(m.w);
+      q[t ^ (t >> 1)] = x01.xx * as16(m.x) + x01.yy * as16(m.y) + x23.xx * as16(m.z) + x23.yy * as16(m.w);
     }
 #pragma unroll
-    for (int h = 1; h < H; h <<= 1)
+    for (int h = 1; h < H / 2; h <<= 1)
 #pragma unroll
       for (int i = 0; i < H; i++)
         if (!(i & h)) {
@@ -491,9 +502,17 @@ template <int NQ> __device__ __forceinline__ int t_bound16s(TStage st, int4 s, i
           q[i] = u + w;
           q[i | h] = u - w;
         }
-    uint32_t o = 0;
+    // The last step's sums and differences are wanted for the lowest bit set in any of them: where v2(u) and v2(w)
+    // differ it is the lower one, which is the lowest bit of u ^ w; where they agree exactly one of u + w, u - w has
+    // valuation v2(u) + 1, the lowest bit of 2 (u & w), and u ^ w has none below it
+    uint32_t ox = 0, oa = 0;
 #pragma unroll
-    for (int i = 0; i < H; i++) o |= bits(q[i]);
+    for (int i = 0; i < H / 2; i++) {
+      const uint32_t u = bits(q[i]), w = bits(q[i | H / 2]);
+      ox |= u ^ w;
+      oa |= u & w;
+    }
+    const uint32_t o = ox | (oa << 1 & 0xfffefffeu);
     const uint32_t acc = (uint32_t)wuni<NQ>((int)gor<GS>((o & 0xffffu) | (o >> 16)));
     npass++;
     const int vp = (pass ? 1 : 2) + 2 * ctz16(acc);    // pass 1: 1 + 2 v2 of (b - d | b + d); pass 0: 2 + 2 v2 of (a | c)
