@@ -102,6 +102,29 @@ template <typename Op> __device__ __forceinline__ uint32_t wave_reduce32(uint32_
   return op(q[0], q[1]);
 }
 
+// The same for an operation with identity 0, as a wave-uniform value: two row broadcasts instead of the swaps leave the
+// total in lane 63 (six vector instructions and a readlane, where the all-reduce and a readfirstlane take thirteen).
+// row_bcast15 brings lane 15 of a row to the next one, here to rows 1 and 3, row_bcast31 lane 31 to rows 2 and 3.
+template <typename Op> __device__ __forceinline__ uint32_t wave_total32(uint32_t v, Op op) {
+  v = op(v, dpp32<DPP_QXOR1>(v));
+  v = op(v, dpp32<DPP_QXOR2>(v));
+  v = op(v, dpp32<DPP_HALF_MIRROR>(v));
+  v = op(v, dpp32<DPP_MIRROR>(v));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// the same for groups of 16 lanes (a DPP row) and 4, in every lane of the group
+template <int GS, typename Op> __device__ __forceinline__ uint32_t row_total32(uint32_t v, Op op) {
+  v = op(v, dpp32<DPP_QXOR1>(v));
+  v = op(v, dpp32<DPP_QXOR2>(v));
+  if constexpr (GS == 16) {
+    v = op(v, dpp32<DPP_HALF_MIRROR>(v));
+    v = op(v, dpp32<DPP_MIRROR>(v));
+  }
+  return v;
+}
+
 // v[lane ^ h] for a power of two h < 64 (lane ^ 4 as ^ 7 and ^ 3, lane ^ 8 as a rotation by half a row)
 __device__ __forceinline__ uint32_t wave_xor32(uint32_t v, int h) {
   switch (h) {
@@ -128,7 +151,9 @@ template <int GS> __device__ __forceinline__ int4 gxor(int4 v, int m) {
 }
 template <int GS, typename T> __device__ __forceinline__ T gsum(T v) {
   if constexpr (GS == 64 && sizeof(T) == 4) {
-    return (T)wave_reduce32((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
+    return (T)wave_total32((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
+  } else if constexpr (GS < 64 && sizeof(T) == 4) {
+    return (T)row_total32<GS>((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
   } else {
 #pragma unroll
     for (int m = 1; m < GS; m <<= 1) v += __shfl_xor(v, m, GS);
@@ -137,10 +162,12 @@ template <int GS, typename T> __device__ __forceinline__ T gsum(T v) {
 }
 template <int GS, typename T> __device__ __forceinline__ T gor(T v) {
   if constexpr (GS == 64 && sizeof(T) == 4) {
-    return (T)wave_reduce32((uint32_t)v, [](uint32_t a, uint32_t b) { return a | b; });
+    return (T)wave_total32((uint32_t)v, [](uint32_t a, uint32_t b) { return a | b; });
   } else if constexpr (GS == 64 && sizeof(T) == 8) {
     const auto o = [](uint32_t a, uint32_t b) { return a | b; };
-    return (T)(((uint64_t)wave_reduce32((uint32_t)((uint64_t)v >> 32), o) << 32) | wave_reduce32((uint32_t)v, o));
+    return (T)(((uint64_t)wave_total32((uint32_t)((uint64_t)v >> 32), o) << 32) | wave_total32((uint32_t)v, o));
+  } else if constexpr (GS < 64 && sizeof(T) == 4) {
+    return (T)row_total32<GS>((uint32_t)v, [](uint32_t a, uint32_t b) { return a | b; });
   } else {
 #pragma unroll
     for (int m = 1; m < GS; m <<= 1) v |= __shfl_xor(v, m, GS);

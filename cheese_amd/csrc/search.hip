@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                   uint32_t needs = pneeds;
                   const uint32_t keepc = (pbw & BW_CUTS) ? hw >> 8 : 0u;
                   const CutStop cst{cutlow && sp.have_table, lo.low, lo.idx, T, hh, supp, rem};
-                  c2 = wuni<NQ>(cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts));
+                  c2 = cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts);
                   bw = (needs << 8 & ~BW_CUTS) | (sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
                 }
                 const int tmax = t_budget(hh, c2, supp, rem) * sp.tdiv;
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                     T = t_bound16s<NQ>(st, s, k, le, T, tmax, np, texact);
                     n_tp += np;
                   } else {
-                    T = t_bound_any<NQ>(s, k, le);
+                    T = wuni<NQ>(t_bound_any<NQ>(s, k, le));
                     texact = true;
                   }
                   if (tc >= 0 && T < 255 && (texact || !tcached || T > tcv)) {

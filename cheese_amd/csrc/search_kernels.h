@@ -335,7 +335,7 @@ template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const 
       ranks++;
       if (st.on && --todo > 0) {
         lo += (need - (int)((st.low >> (3 * i)) & 7u)) * mult;
-        const int c = cx_at(sp, cxl, lo);
+        const int c = wuni<NQ>(cx_at(sp, cxl, lo));
         if (st.T > t_budget(st.h, c, st.supp, st.rem) * sp.tdiv) return c;
       }
     }
@@ -345,7 +345,7 @@ template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const 
     if (need > mx) mx = need;
   }
   needs = out;
-  return sp.have_table ? cx_at(sp, cxl, idx) : mx;
+  return sp.have_table ? wuni<NQ>(cx_at(sp, cxl, idx)) : mx;
 }
 
 // T lower bound: max over Pauli pairs of 2(n+k) - v(X_ab), all X_ab by one 2-D Walsh-Hadamard transform
@@ -529,33 +529,23 @@ template <int NQ> __device__ __forceinline__ int t_bound_any(int4 s, int k, int 
   return 2 * (NQ + k) <= 64 ? t_bound<NQ, uint32_t>(s, k, le) : t_bound<NQ, unsigned long long>(s, k, le);
 }
 
-// 32-bit hash of one entry's four coefficients.  A multiply moves information only towards the high bits, so
-// each round folds the high half back down before the next coefficient enters; without that, entries with small
-// coefficients collide far more often than a random function would.
+// 32-bit hash of one entry's four coefficients and of its conjugate's: linear forms with 24-bit products (full rate; a
+// 32-bit product runs at a quarter of it), folded once.  Entries that collide differ by a vector of the forms' lattice,
+// whose shortest ones have coefficients of some 2^8; the summands below are not linear in them.  Coefficients of more
+// than 24 bits enter by their low 24.
 __device__ __forceinline__ uint32_t entry_hash32(int4 v) {
-  uint32_t h = (uint32_t)v.x * 0x9e3779b1u + (uint32_t)v.y;
-  h ^= h >> 15;
-  h = h * 0x85ebca77u + (uint32_t)v.z;
-  h ^= h >> 13;
-  h = h * 0xc2b2ae3du + (uint32_t)v.w;
-  h ^= h >> 16;
-  h *= 0x27d4eb2fu;
+  const uint32_t h = (uint32_t)(__mul24(v.x, 0x5e3779) + __mul24(v.y, 0x3ebca7) + __mul24(v.z, 0x72b2ae) + __mul24(v.w, 0x27d4eb));
   return h ^ (h >> 15);
 }
-// the 64-bit summand of an entry hash at position pos (1..64): two independent one-multiply mixes of the pair.
-// 32-bit multiplies run at a quarter of the VALU rate and 64-bit ones take four of them, so the summand costs
-// two where a 64-bit mix costs eight; the sum over the entries still differs between two matrices unless their
-// differing entries' hashes collide (2^-32 per entry) or the 64-bit sums do.
+__device__ __forceinline__ uint32_t entry_hash32_conj(int4 v) {
+  const uint32_t h = (uint32_t)(__mul24(v.x, 0x5e3779) + __mul24(v.w, -0x3ebca7) + __mul24(v.z, -0x72b2ae) + __mul24(v.y, -0x27d4eb));
+  return h ^ (h >> 15);
+}
+// The 64-bit summand of an entry hash at position pos (1..64): a square of the two mixed, one product at a quarter of
+// the rate where two mixes took two.  Its halves are summed apart.
 __device__ __forceinline__ uint64_t slot64(uint32_t h, uint32_t pos) {
   const uint32_t x = h ^ __umul24(pos, 0x9e3779u);
-  uint32_t lo = x ^ (x >> 16);
-  lo *= 0x7feb352du;
-  lo ^= lo >> 15;
-  uint32_t hi = x ^ 0x5bd1e995u;
-  hi ^= hi >> 15;
-  hi *= 0x2c1b3c6du;
-  hi ^= hi >> 12;
-  return ((uint64_t)hi << 32) | lo;
+  return (uint64_t)x * (x ^ 0x5bd1e995u);
 }
 
 // class key: the smallest over the symmetry group of an entry-sum hash of sigma(S); equal classes give
@@ -563,13 +553,13 @@ __device__ __forceinline__ uint64_t slot64(uint32_t h, uint32_t pos) {
 template <int NQ> __device__ __forceinline__ uint64_t class_key(int4 s, int k, int le, const KSpec &sp) {
   constexpr int N = 1 << NQ, GS = N * N;
   const int r = le >> NQ, c = le & (N - 1);
-  const uint32_t hv = entry_hash32(s), hc = entry_hash32(zconj(s));
+  const uint32_t hv = entry_hash32(s), hc = entry_hash32_conj(s);
   uint64_t best = ~0ull;
   for (int y = 0; y < sp.nsym; y++) {
     const uint8_t *pm = sp.symperm + y * N;
     const uint32_t pos = (uint32_t)(pm[r] * N + pm[c]) + 1;
     const uint64_t h = slot64(sp.symconj[y] ? hc : hv, pos);
-    const uint64_t key = mix64(gsum<GS>(h) ^ ((uint64_t)(k + 1) * 0xc2b2ae3d27d4eb4full));
+    const uint64_t key = mix64(((uint64_t)gsum<GS>((uint32_t)(h >> 32)) << 32 | gsum<GS>((uint32_t)h)) ^ ((uint64_t)(k + 1) * 0xc2b2ae3d27d4eb4full));
     best = key < best ? key : best;
   }
   return best;
@@ -592,11 +582,11 @@ __host__ __device__ inline int key_order(uint32_t a, uint32_t b, uint32_t c) {
   return ((b < a) + (c < a)) | ((a < b) + (c < b)) << 2 | ((a < c) + (b < c)) << 4;
 }
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce32(v, [](uint32_t a, uint32_t b) { return a + b; }));
+  return wave_total32(v, [](uint32_t a, uint32_t b) { return a + b; });
 }
 __device__ __forceinline__ uint64_t class_key3(int4 s, int k, int lane, const uint8_t *spos, const uint16_t *adm, uint32_t cjm,
                                                int &image) {
-  const uint32_t hv = entry_hash32(s), hc = entry_hash32(zconj(s));
+  const uint32_t hv = entry_hash32(s), hc = entry_hash32_conj(s);
   const int off = (lane >> 3) ^ (lane & 7);            // bit q: an entry off qubit q's diagonal
   // 64 shares of 10 bits sum within 16 bits: two sums to a word
   auto order = [&](uint32_t h) -> uint32_t {
