@@ -2011,20 +2011,22 @@ int chz_open(const char *spec_text, size_t len, const chz_opts *opts, chz_ctx **
   // symmetry classes: not with --mitm, whose join compares exact residuals (src/cheese.cu:1786)
   c->grp = chz::build_symmetry(c->hs, o.sym != 0 && !o.mitm);
   if (o.table < 0 || o.table > CHZ_DMAX) { chz::set_err("--table K outside 0..48"); return 3; }
-  // default occupancy: 5 waves per SIMD fits the n = 3 kernel's registers; smaller groups spill there, so 4
+  // default occupancy: groups of less than a wave spill above 4 waves per SIMD
   if (c->hs.n < 3)
     for (auto &sc : c->sched) sc.var = 0;
   else
     // n = 3 defaults per level-size bucket (log2 of the parents in a launch), from the autotuner's winners on the
-    // Toffoli budget-12 and budget-13 proofs on MI355X: up to 32K parents run at 4 waves per SIMD (the variant with
-    // the most registers), below 8K parents with a parent's candidates split over lane groups down to about 2,048
-    // groups per launch, 8K-32K in two lane groups per parent; mid-size levels want fewer blocks, the largest more
+    // Toffoli proofs of budgets 9 to 14 on MI355X.  The expansion is bound by instruction issue, with waits on LDS and on
+    // the parents' loads between: from 4K parents on 6 waves per SIMD (80 registers) win, budget-13 levels of a million
+    // parents take 4.7 ms instead of 5.4 with 5.  Below, the waves have a parent or less each, and it is the longest
+    // chain that counts: a parent's candidates are split over lane groups, up to 512 parents down to one or two
+    // candidates each at the variant with the most registers
     for (int b = 0; b < (int)(sizeof c->sched / sizeof c->sched[0]); b++) {
       chz_ctx::Sched &sc = c->sched[b];
-      if (b == 13 || b == 14) { sc.var = 0; sc.cap = 4096; sc.tw = 16384; }
-      else if (b <= 12) { sc.var = 0; sc.tw = 2048; }
-      else if (b >= 15 && b <= 17) sc.cap = 4096;
-      else if (b >= 19) sc.cap = 16384;
+      if (b <= 8) { sc.var = 0; sc.tw = 16384; }
+      else if (b <= 11) { sc.var = 1; sc.tw = 8192; }
+      else if (b <= 14) { sc.var = 2; sc.cap = 4096; sc.tw = b == 12 ? 8192 : 16384; }
+      else { sc.var = 2; sc.cap = b == 15 ? 8192 : 16384; }
     }
   try {
     c->device = o.device;
