@@ -21,18 +21,23 @@ __device__ __forceinline__ long long dev_n(long long n, const unsigned long long
   return nd ? (long long)*nd : n;
 }
 
+// this thread's flags of a tile: bit i for item t0 + i * CT_THREADS + thread (all items' loads in flight together)
+template <typename F> __device__ __forceinline__ uint32_t tile_flags(F f, long long t0, long long n) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < CT_ITEMS; i++) {
+    const long long x = t0 + (long long)i * CT_THREADS + threadIdx.x;
+    if (x < n && f(x)) m |= 1u << i;
+  }
+  return m;
+}
+
 template <typename F>
 __global__ __launch_bounds__(CT_THREADS) void k_flag_count(F f, long long n, unsigned long long *bcount,
                                                            const unsigned long long *nd = nullptr) {
   n = dev_n(n, nd);
-  const long long t0 = (long long)blockIdx.x * CT_TILE;
-  int c = 0;
-  for (int i = 0; i < CT_ITEMS; i++) {
-    const long long x = t0 + (long long)i * CT_THREADS + threadIdx.x;
-    if (x < n && f(x)) c++;
-  }
-  __shared__ int ws[CT_THREADS / 64];
-  c = gsum<64>(c);
+  __shared__ uint32_t ws[CT_THREADS / 64];
+  const uint32_t c = gsum<64>((uint32_t)__popc(tile_flags(f, (long long)blockIdx.x * CT_TILE, n)));
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = c;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -72,52 +77,79 @@ __global__ __launch_bounds__(1024) void k_scan_one_block(unsigned long long *v, 
   if (threadIdx.x == 0) v[n] = carry;
 }
 
-// block-wide exclusive scan of one flag per thread, in thread order; returns the block total
-__device__ __forceinline__ int block_flag_scan(bool flag, int &excl, int *ws) {
+// write(x, position) for the flagged items of the tile at t0, in order, positions from pos0; returns their number.  One
+// scan over the (item, wave) counts places the whole tile: with a block scan per item, a tile's 32 barriers were most of
+// a small level's compaction (15 us for 6 tiles).
+template <typename F, typename W>
+__device__ __forceinline__ uint32_t tile_compact(F f, long long t0, long long n, unsigned long long pos0, W write) {
+  constexpr int NW = CT_THREADS / 64;
+  static_assert(CT_ITEMS * NW == 64, "the counts are scanned by one wave");
+  __shared__ uint32_t ws[65];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t b = __ballot(flag);
-  const int below = __popcll(b & ((1ull << lane) - 1));
-  if (lane == 0) ws[w] = __popcll(b);
+  const uint32_t m = tile_flags(f, t0, n);
+#pragma unroll
+  for (int i = 0; i < CT_ITEMS; i++) {
+    const uint64_t b = __ballot((m >> i) & 1u);
+    if (lane == 0) ws[i * NW + w] = (uint32_t)__popcll(b);
+  }
   __syncthreads();
-  int off = 0, tot = 0;
-  for (int k = 0; k < CT_THREADS / 64; k++) { if (k < w) off += ws[k]; tot += ws[k]; }
+  if (threadIdx.x < 64) {
+    const uint32_t v = ws[lane];
+    uint32_t inc = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t y = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += y;
+    }
+    ws[lane] = inc - v;
+    if (lane == 63) ws[64] = inc;
+  }
   __syncthreads();
-  excl = off + below;
-  return tot;
+#pragma unroll
+  for (int i = 0; i < CT_ITEMS; i++) {
+    const bool fl = (m >> i) & 1u;
+    const uint64_t b = __ballot(fl);
+    if (fl) write(t0 + (long long)i * CT_THREADS + threadIdx.x, pos0 + ws[i * NW + w] + __popcll(b & ((1ull << lane) - 1)));
+  }
+  return ws[64];
 }
 
-// flagged positions -> ordered index list (kept survivor ranks, children needing the T bound)
+// Sum of v[0..n) over a block of CT_THREADS threads: the tiles before a block's own, where the counts of at most
+// CT_DIRECT tiles are not scanned by a launch of its own (each block reads up to 4 KB from L2; a scan and a total took
+// two launches of 4 to 5 us)
+constexpr long long CT_DIRECT = 512;
+__device__ __forceinline__ unsigned long long tile_offset(const unsigned long long *v, long long n) {
+  __shared__ uint32_t ts[CT_THREADS / 64];
+  uint32_t s = 0;
+  for (long long i = threadIdx.x; i < n; i += CT_THREADS) s += (uint32_t)v[i];
+  s = gsum<64>(s);
+  if ((threadIdx.x & 63) == 0) ts[threadIdx.x >> 6] = s;
+  __syncthreads();
+  unsigned long long o = 0;
+  for (int w = 0; w < CT_THREADS / 64; w++) o += ts[w];
+  return o;
+}
+
+// flagged positions -> ordered index list (kept survivor ranks, children needing the T bound).  boff: the tiles' offsets,
+// or with tot their counts, the total then going to *tot
 template <typename F>
 __global__ __launch_bounds__(CT_THREADS) void k_scatter_idx(F f, long long n, const unsigned long long *boff,
-                                                            uint32_t *out, const unsigned long long *nd = nullptr) {
+                                                            uint32_t *out, const unsigned long long *nd = nullptr,
+                                                            unsigned long long *tot = nullptr) {
   n = dev_n(n, nd);
-  __shared__ int ws[CT_THREADS / 64];
-  const long long t0 = (long long)blockIdx.x * CT_TILE;
-  long long pos = (long long)boff[blockIdx.x];
-  for (int i = 0; i < CT_ITEMS; i++) {
-    const long long x = t0 + (long long)i * CT_THREADS + threadIdx.x;
-    const bool fl = x < n && f(x);
-    int ex;
-    const int tot = block_flag_scan(fl, ex, ws);
-    if (fl) out[pos + ex] = (uint32_t)x;
-    pos += tot;
-  }
+  const unsigned long long pos = tot ? tile_offset(boff, blockIdx.x) : boff[blockIdx.x];
+  const uint32_t c = tile_compact(f, (long long)blockIdx.x * CT_TILE, n, pos,
+                                  [&](long long x, unsigned long long p) { out[p] = (uint32_t)x; });
+  if (tot && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *tot = pos + c;
 }
 
 // one tile (n <= CT_TILE) in one launch: flagged positions -> ordered index list, total written to *tot
 template <typename F>
-__global__ __launch_bounds__(CT_THREADS) void k_compact_one(F f, long long n, uint32_t *out, unsigned long long *tot) {
-  __shared__ int ws[CT_THREADS / 64];
-  long long pos = 0;
-  for (int i = 0; i < CT_ITEMS; i++) {
-    const long long x = (long long)i * CT_THREADS + threadIdx.x;
-    const bool fl = x < n && f(x);
-    int ex;
-    const int t = block_flag_scan(fl, ex, ws);
-    if (fl) out[pos + ex] = (uint32_t)x;
-    pos += t;
-  }
-  if (threadIdx.x == 0) *tot = (unsigned long long)pos;
+__global__ __launch_bounds__(CT_THREADS) void k_compact_one(F f, long long n, uint32_t *out, unsigned long long *tot,
+                                                            const unsigned long long *nd = nullptr) {
+  n = dev_n(n, nd);
+  const uint32_t c = tile_compact(f, 0, n, 0, [&](long long x, unsigned long long p) { out[p] = (uint32_t)x; });
+  if (threadIdx.x == 0) *tot = c;
 }
 
 // run starts (a position whose key differs from the one before and equals the one after), appended in tiles:
@@ -163,33 +195,84 @@ __attribute__((unused)) __global__ __launch_bounds__(256) void k_run_starts(cons
 }
 
 // ------------------------------------------------------------------------------------------------------
-// small sorts in one launch: n <= SS_MAX (key prefix, rank) pairs as 64-bit composites (prefix << 32 | rank,
-// all distinct) by a bitonic network in LDS.  Ascending composites are the stable order of the prefixes, so the
-// result is the radix sort's.
-constexpr int SS_MAX = 4096;
-__attribute__((unused)) __global__ __launch_bounds__(1024) void k_sort_small(const uint64_t *key, long long n,
-                                                                           uint32_t *kout, uint32_t *vout) {
-  __shared__ uint64_t s[SS_MAX];
+// Key prefixes that a sort of n survivors looks at, in passes of 8 bits: the sort only has to bring equal keys
+// together, in order of their ranks, and keys that agree in a shorter prefix are told apart by the run's own comparison
+// of whole keys.  At these lines a position's run holds another class with a chance of at most a quarter.
+static inline int sort_passes(long long n) { return n <= (1 << 14) ? 2 : n <= (1 << 22) ? 3 : 4; }
+__host__ __device__ inline uint32_t sort_prefix(uint64_t key, int passes) {
+  return (uint32_t)(key >> 32) & (passes >= 4 ? 0xffffffffu : (1u << (8 * passes)) - 1);
+}
+
+// small sorts in one launch: n <= SS_MAX survivors by the low 16 bits of their prefixes, stable, two 8-bit passes in LDS
+// (4096 survivors by a bitonic network of 64-bit composites: 55 us, here 11)
+constexpr int SS_MAX = 4096, SS_THREADS = 1024;
+__attribute__((unused)) __global__ __launch_bounds__(SS_THREADS) void k_sort_small(const uint64_t *key, long long n,
+                                                                                 uint32_t *kout, uint32_t *vout,
+                                                                                 const unsigned long long *nd) {
+  constexpr int NW = SS_THREADS / 64;
+  __shared__ uint32_t buf[2][SS_MAX];            // prefix << 12 | rank
+  __shared__ uint16_t wc[NW][256];
+  __shared__ uint32_t base[256], ws[4];
+  n = dev_n(n, nd);
   if (n > SS_MAX) return;                  // callers take the radix sort beyond one block's LDS
-  int np = 1;
-  while (np < n) np <<= 1;
-  for (int i = threadIdx.x; i < np; i += blockDim.x)
-    s[i] = i < n ? ((key[i] >> 32) << 32) | (uint64_t)i : ~0ull;
-  __syncthreads();
-  for (int k = 2; k <= np; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = threadIdx.x; i < np; i += blockDim.x) {
-        const int l = i ^ j;
-        if (l > i) {
-          const uint64_t a = s[i], b = s[l];
-          if ((a > b) == ((i & k) == 0)) { s[i] = b; s[l] = a; }
-        }
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  for (int i = tid; i < n; i += SS_THREADS) buf[0][i] = sort_prefix(key[i], 2) << 12 | (uint32_t)i;
+  for (int pass = 0; pass < 2; pass++) {
+    const uint32_t *in = buf[pass];
+    uint32_t *out = buf[pass ^ 1];
+    const int shift = 12 + 8 * pass;
+    if (tid < 256) base[tid] = 0;
+    for (int k = tid; k < NW * 256; k += SS_THREADS) (&wc[0][0])[k] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += SS_THREADS) atomicAdd(&base[(in[i] >> shift) & 255], 1u);
+    __syncthreads();
+    // exclusive scan of the 256 digit counts
+    uint32_t inc = 0, own = 0;
+    if (tid < 256) {
+      own = inc = base[tid];
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += y;
+      }
+      if (lane == 63) ws[w] = inc;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      for (int k = 0; k < w; k++) inc += ws[k];
+      base[tid] = inc - own;
+    }
+    __syncthreads();
+    for (int r0 = 0; r0 < n; r0 += SS_THREADS) {
+      const int i = r0 + tid;
+      const bool valid = i < n;
+      const uint32_t v = valid ? in[i] : 0u;
+      const int dg = (int)(v >> shift) & 255;
+      uint64_t peers = __ballot(valid);
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        const uint64_t bb = __ballot((dg >> b) & 1);
+        peers &= ((dg >> b) & 1) ? bb : ~bb;
+      }
+      const int rank = __popcll(peers & ((1ull << lane) - 1));
+      if (valid && rank == 0) wc[w][dg] = (uint16_t)__popcll(peers);
+      __syncthreads();
+      // the waves' counts of a digit become their start positions, the digit's base moves on
+      if (tid < 256) {
+        uint32_t o = base[tid];
+        for (int k = 0; k < NW; k++) { const uint32_t c = wc[k][tid]; wc[k][tid] = (uint16_t)o; o += c; }
+        base[tid] = o;
       }
       __syncthreads();
+      if (valid) out[wc[w][dg] + rank] = v;
+      __syncthreads();
+      for (int k = tid; k < NW * 256; k += SS_THREADS) (&wc[0][0])[k] = 0;
+      __syncthreads();
     }
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    kout[i] = (uint32_t)(s[i] >> 32);
-    vout[i] = (uint32_t)s[i];
+  }
+  for (int i = tid; i < n; i += SS_THREADS) {
+    kout[i] = buf[0][i] >> 12;
+    vout[i] = buf[0][i] & 0xfffu;
   }
 }
 
@@ -380,27 +463,28 @@ static inline hipError_t scan_excl(unsigned long long *v, long long n, unsigned 
   return hipMemcpyAsync(v + n, tmp + nt, sizeof(unsigned long long), hipMemcpyDeviceToDevice, s);
 }
 
-// stable sort of n (u32 key, u32 value) pairs, 4 passes of 8 bits: (k0, v0) -> (k0, v0) through (k1, v1).
+// stable sort of n (u32 key, u32 value) pairs by the low 8 * passes bits: (k0, v0) -> (k0, v0) through (k1, v1); an odd
+// number of passes starts from (k1, v1).
 // hist holds at least 256 * ceil(n / RS_TILE) + 1 entries, tmp what scan_excl needs for that many.
 // With nd the count is read on the device and n is the capacity the launches are sized for.
 static inline hipError_t radix_sort_pairs(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, long long n,
                                           unsigned long long *hist, unsigned long long *tmp, hipStream_t s,
-                                          const unsigned long long *nd = nullptr) {
-  if (n <= 1) return hipSuccess;
+                                          const unsigned long long *nd = nullptr, int passes = 4) {
+  if (n < 1 || (n == 1 && passes % 2 == 0)) return hipSuccess;
   const long long nb = (n + RS_TILE - 1) / RS_TILE;
   uint32_t *ks[2] = {k0, k1}, *vs[2] = {v0, v1};
   if (nb <= RS_DIRECT_MAX) {
     uint32_t *cnt = reinterpret_cast<uint32_t *>(hist);     // nb * 256 counts fit the histogram's space
-    for (int pass = 0; pass < 4; pass++) {
-      const int a = pass & 1, b = a ^ 1;
+    for (int pass = 0; pass < passes; pass++) {
+      const int a = (pass + passes) & 1, b = a ^ 1;
       hipLaunchKernelGGL(k_radix_count, dim3((unsigned)nb), dim3(RS_THREADS), 0, s, ks[a], n, pass * 8, cnt, nd);
       hipLaunchKernelGGL(k_radix_scatter_direct, dim3((unsigned)nb), dim3(RS_THREADS), 0, s, ks[a], vs[a], n,
                          pass * 8, cnt, nb, ks[b], vs[b], nd);
     }
     return hipGetLastError();
   }
-  for (int pass = 0; pass < 4; pass++) {
-    const int a = pass & 1, b = a ^ 1;
+  for (int pass = 0; pass < passes; pass++) {
+    const int a = (pass + passes) & 1, b = a ^ 1;
     hipLaunchKernelGGL(k_radix_hist, dim3((unsigned)nb), dim3(RS_THREADS), 0, s, ks[a], n, pass * 8, hist, nb, nd);
     hipError_t e = scan_excl(hist, nb * 256, tmp, s);
     if (e != hipSuccess) return e;

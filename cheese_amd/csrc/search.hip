@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
       if (g < G && ((range >> g) & 1))
         a.status[pl * G + g] = (w2m >> g) & 1      ? ST_W2
                                : (w3m >> g) & 1    ? ST_W3
-                               : (alivem >> g) & 1 ? ST_ALIVE
+                               : (alivem >> g) & 1 ? (keep ? ST_ALIVE : ST_LAST)
                                : (foundm >> g) & 1 ? ST_FOUND
                                : (ovfm >> g) & 1   ? ST_OVF
                                                    : ST_DEAD;
@@ -513,83 +513,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 
 struct FlagAlive {      // survivors of a chunk that become parents, in child order
   const uint8_t *status;
-  const uint32_t *pinst;
-  const uint8_t *keepi;
-  long long off;          // first parent of the chunk
-  int G;
-  __device__ bool operator()(long long i) const {
-    return status[i] == ST_ALIVE && keepi[pinst ? pinst[off + i / G] : 0] != 0;
-  }
+  __device__ bool operator()(long long i) const { return status[i] == ST_ALIVE; }
 };
-struct FlagKept {       // kept survivors of instances still searching
+struct FlagKept {       // kept survivors (k_fill_kept leaves out those of searches that ended)
   const uint8_t *kept;
-  const uint64_t *surv_o;
-  const uint32_t *pinst;
-  const uint8_t *active;
-  int G;
-  __device__ bool operator()(long long i) const {
-    return kept[i] != 0 && active[pinst ? pinst[surv_o[i] / (uint64_t)G] : 0] != 0;
-  }
+  __device__ bool operator()(long long i) const { return kept[i] != 0; }
 };
 
-// survivors of a chunk -> level survivor list (child index in the level, class key)
-__global__ __launch_bounds__(CT_THREADS) void k_scatter_alive(FlagAlive f, long long n, const unsigned long long *boff,
-                                                              const uint64_t *keys, long long child0,
-                                                              const unsigned long long *out0, uint64_t *surv_o,
-                                                              uint64_t *surv_key, const uint32_t *info,
-                                                              uint32_t *surv_bw, const unsigned long long *nd) {
+// Survivors of a chunk -> level survivor list (child index in the level, class key, bound word).  boff: the tiles' offsets
+// from the survivors *out0 of the chunks before; with tot the tiles' counts, the chunk being the level's only one, and
+// the total goes to *tot.  boff null: one tile.
+struct AliveOut {
+  const uint64_t *keys;
+  const uint32_t *info;
+  long long child0;
+  uint64_t *surv_o, *surv_key;
+  uint32_t *surv_bw;
+};
+__global__ __launch_bounds__(CT_THREADS) void k_scatter_alive(FlagAlive f, long long n, const unsigned long long *boff, AliveOut o,
+                                                              const unsigned long long *out0, unsigned long long *tot,
+                                                              const unsigned long long *nd) {
   n = dev_n(n, nd);
-  __shared__ int ws[CT_THREADS / 64];
-  const long long t0 = (long long)blockIdx.x * CT_TILE;
-  long long pos = (long long)*out0 + (long long)boff[blockIdx.x];
-  for (int i = 0; i < CT_ITEMS; i++) {
-    const long long x = t0 + (long long)i * CT_THREADS + threadIdx.x;
-    const bool fl = x < n && f(x);
-    int ex;
-    const int tot = block_flag_scan(fl, ex, ws);
-    if (fl) {
-      surv_o[pos + ex] = (uint64_t)(child0 + x);
-      surv_key[pos + ex] = keys[x];
-      surv_bw[pos + ex] = info[x];
-    }
-    pos += tot;
-  }
-}
-
-// the same for a chunk of one tile (n <= CT_TILE) in one launch: the level's survivor count *out0 is read at the
-// start and advanced at the end
-__global__ __launch_bounds__(CT_THREADS) void k_scatter_alive_one(FlagAlive f, long long n, const uint64_t *keys,
-                                                                  long long child0, unsigned long long *out0,
-                                                                  uint64_t *surv_o, uint64_t *surv_key,
-                                                                  const uint32_t *info, uint32_t *surv_bw) {
-  __shared__ int ws[CT_THREADS / 64];
-  const long long p0 = (long long)*out0;
-  long long pos = p0;
-  for (int i = 0; i < CT_ITEMS; i++) {
-    const long long x = (long long)i * CT_THREADS + threadIdx.x;
-    const bool fl = x < n && f(x);
-    int ex;
-    const int tot = block_flag_scan(fl, ex, ws);
-    if (fl) {
-      surv_o[pos + ex] = (uint64_t)(child0 + x);
-      surv_key[pos + ex] = keys[x];
-      surv_bw[pos + ex] = info[x];
-    }
-    pos += tot;
-  }
-  if (threadIdx.x == 0) *out0 = (unsigned long long)pos;
-}
-
-// searches that continue after this level: no circuit, no overflow, budget left (captured step)
-__global__ void k_active(const unsigned long long *icnt, int nstr, const uint8_t *keepi, int nslots, uint8_t *active) {
-  for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nslots; s += gridDim.x * blockDim.x) {
-    bool on = keepi[s];
-    for (int j = 0; j < nstr; j++) {
-      const unsigned long long *x = icnt + ((size_t)j * nslots + s) * IC_N;
-      on = on && !x[IC_FOUND] && !x[IC_OVF];
-    }
-    active[s] = on;
-  }
+  const unsigned long long pos = !boff ? 0 : tot ? tile_offset(boff, blockIdx.x) : *out0 + boff[blockIdx.x];
+  const uint32_t c = tile_compact(f, (long long)blockIdx.x * CT_TILE, n, pos, [&](long long x, unsigned long long p) {
+    o.surv_o[p] = (uint64_t)(o.child0 + x);
+    o.surv_key[p] = o.keys[x];
+    o.surv_bw[p] = o.info[x];
+  });
+  if (tot && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *tot = pos + c;
 }
 
 // the level's survivor count grows by a chunk's total (the scan's last entry)
@@ -601,15 +552,45 @@ __global__ void k_add_total(unsigned long long *acc, const unsigned long long *t
 // segmented dedupe over the sorted survivors: runs of equal 32-bit key prefix are partitioned into exact
 // classes, keeping the smallest survivor rank (= lexicographically first prefix) of each class
 // (src/cheese.cu:1334-1343, :1046-1065)
-// every survivor starts kept (a sequential fill: setting kept[v[i]] here would scatter byte writes over the array)
-// (it runs after the level's expansion has read the goal flags, before the gather sets them for the next level:
-// gflag, when given, is cleared here)
-__global__ void k_fill_kept(uint8_t *kept, long long n, const unsigned long long *nd, uint32_t *gflag, int ns) {
+// Every survivor of a search that continues after this level (no circuit, no overflow) starts kept: a sequential fill;
+// setting kept[v[i]] in the dedupe would scatter byte writes over the array.  (It runs after the level's expansion has read
+// the goal flags, before the gather sets them for the next level: gflag, when given, is cleared here.)
+struct ActiveArgs {
+  const unsigned long long *icnt;   // the expansion's per-slot counters, in nstr stripes
+  int nstr, ns, G;
+  const uint64_t *surv_o;
+  const uint32_t *pinst;
+};
+constexpr int ACT_LDS = 1024;       // slots whose state a block keeps in LDS; beyond it is read per survivor
+__device__ __forceinline__ bool slot_ended(const ActiveArgs &a, int s) {
+  unsigned long long x = 0;
+  for (int j = 0; j < a.nstr; j++) {
+    const unsigned long long *c = a.icnt + ((size_t)j * a.ns + s) * IC_N;
+    x |= c[IC_FOUND] | c[IC_OVF];
+  }
+  return x != 0;
+}
+__global__ __launch_bounds__(256) void k_fill_kept(uint8_t *kept, long long n, const unsigned long long *nd, ActiveArgs a,
+                                                   uint32_t *gflag) {
+  __shared__ uint32_t ended[ACT_LDS];
   n = dev_n(n, nd);
+  const bool lds = a.ns <= ACT_LDS;
+  if (lds) {
+    for (int s = threadIdx.x; s < a.ns; s += blockDim.x) ended[s] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < a.ns * a.nstr; i += blockDim.x) {
+      const unsigned long long *c = a.icnt + (size_t)i * IC_N;
+      if (c[IC_FOUND] | c[IC_OVF]) atomicOr(&ended[i % a.ns], 1u);
+    }
+    __syncthreads();
+  }
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long long)gridDim.x * blockDim.x;
-  for (long long i = i0; i < n; i += stride) kept[i] = 1;
+  for (long long i = i0; i < n; i += stride) {
+    const int s = (int)a.pinst[a.surv_o[i] / (uint64_t)a.G];
+    kept[i] = !(lds ? ended[s] != 0 : slot_ended(a, s));
+  }
   if (gflag)
-    for (long long i = i0; i < ns; i += stride) gflag[i] = 0u;
+    for (long long i = i0; i < a.ns; i += stride) gflag[i] = 0u;
 }
 
 struct DedupeArgs {
@@ -703,15 +684,28 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
         const uint64_t o = gget64<GS>(m_o, q);
         return child_terms<NQ>(a.res + (long long)(o / G) * E, ct.desc[(int)(o % G) * 64 + le], le);
       };
+      // a run that ends in this chunk: only members that share their whole key with another one are looked at (the sort
+      // brings together what agrees in part of it)
+      uint64_t left = nm < 64 ? (1ull << nm) - 1 : ~0ull;
+      if (j0 == i0 && nm < GS) {
+        uint64_t shared = 0;
+        for (int q = 0; q < nm; q++) {
+          const uint64_t same = gballot<GS>(le < nm && m_key == gget64<GS>(m_key, q));
+          if (same & (same - 1)) shared |= 1ull << q;
+        }
+        left = shared;
+      }
       ChildTerms next{};
-      if (nm > 0) next = terms(0);
-      for (int q = 0; q < nm; q++) {
+      if (left) next = terms(__ffsll((long long)left) - 1);
+      while (left) {
+        const int q = __ffsll((long long)left) - 1;
+        left &= left - 1;
         const uint32_t rank = gget<GS>(m_rank, q), inst = gget<GS>(m_inst, q);
         const uint64_t o = gget64<GS>(m_o, q), key64 = gget64<GS>(m_key, q);
         const int pk = (int)gget<GS>((uint32_t)m_pk, q), img = (int)gget<GS>(m_img, q);
         const int g = (int)(o % G);
         const ChildTerms cur = next;
-        if (q + 1 < nm) next = terms(q + 1);
+        if (left) next = terms(__ffsll((long long)left) - 1);
         int4 s;
         int ks;
         if (!child_of<NQ>(cur, ct.desc[g * 64 + le], ct.ik[g], pk, s, ks))
@@ -874,12 +868,12 @@ template <int NQ> static int gather_tile(long long nk) {
 }
 
 
-// 64-bit class keys -> sortable 32-bit prefixes and survivor ranks
-__global__ void k_init_sort(const uint64_t *key, long long n, uint32_t *k32, uint32_t *v32,
+// 64-bit class keys -> sortable prefixes and survivor ranks
+__global__ void k_init_sort(const uint64_t *key, long long n, int passes, uint32_t *k32, uint32_t *v32,
                             const unsigned long long *nd) {
   n = dev_n(n, nd);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    k32[i] = (uint32_t)(key[i] >> 32);
+    k32[i] = sort_prefix(key[i], passes);
     v32[i] = (uint32_t)i;
   }
 }
@@ -955,7 +949,6 @@ struct chz_ctx {
   unsigned long long *cnt = nullptr, *stage = nullptr, *icnt = nullptr;
   int *d_rem = nullptr;
   uint8_t *d_keepi = nullptr;
-  chz::DBuf<uint8_t> d_active;
   chz::DBuf<uint32_t> gflag;        // per slot: a node of the current frontier has a goal child
   chz::DBuf<unsigned long long> scan_tmp;
   chz::Pinned pin;                  // staging of the per-level control transfers
@@ -1069,12 +1062,51 @@ __global__ void k_carry_tree(uint32_t *tp, uint8_t *tg, long long n, long long f
   }
 }
 
-// stable sort of (key prefix, rank) pairs of n survivors; the result lands in sk[0]/sv[0]
-static void sort_pairs(chz_ctx *c, long long n) {
+// (key prefix, rank) pairs of the survivors in sk[0]/sv[0], equal prefixes together in order of rank.  nd: their number
+// is read on the device, n bounds it.
+static void sort_survivors(chz_ctx *c, long long n, const unsigned long long *nd, hipStream_t s) {
+  for (int b = 0; b < 2; b++) { c->sk[b].need(n); c->sv[b].need(n); }
+  if (n <= SS_MAX) {
+    hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(SS_THREADS), 0, s, c->surv_key.p, n, c->sk[0].p, c->sv[0].p, nd);
+    return;
+  }
+  const int passes = sort_passes(n), from = passes & 1;
   const long long nb = (n + RS_TILE - 1) / RS_TILE;
   c->hist.need((size_t)nb * 256 + 1);
   c->scan_tmp.need((size_t)nb * 256 / SC_TILE + 4);
-  HIPCHK(radix_sort_pairs(c->sk[0].p, c->sv[0].p, c->sk[1].p, c->sv[1].p, n, c->hist.p, c->scan_tmp.p, c->stream));
+  hipLaunchKernelGGL(k_init_sort, dim3(grid_for(n / 64 + 1)), dim3(256), 0, s, c->surv_key.p, n, passes, c->sk[from].p,
+                     c->sv[from].p, nd);
+  HIPCHK(radix_sort_pairs(c->sk[0].p, c->sv[0].p, c->sk[1].p, c->sv[1].p, n, c->hist.p, c->scan_tmp.p, s, nd, passes));
+}
+
+// the survivors of the level's only chunk, in order, their number in C_SURV
+static void compact_alive(chz_ctx *c, const FlagAlive &fa, long long ncc, const AliveOut &ao, const unsigned long long *dncc,
+                          hipStream_t s) {
+  const long long nb = (ncc + CT_TILE - 1) / CT_TILE;
+  if (nb > 1)
+    hipLaunchKernelGGL(k_flag_count<FlagAlive>, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fa, ncc, c->bcount.p, dncc);
+  hipLaunchKernelGGL(k_scatter_alive, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fa, ncc, nb > 1 ? c->bcount.p : nullptr, ao,
+                     nullptr, c->cnt + C_SURV, dncc);
+}
+
+// the kept survivors' ranks in kidx, their number in C_KEPT
+static void compact_kept(chz_ctx *c, long long n, const unsigned long long *nd, hipStream_t s) {
+  const long long nb = (n + CT_TILE - 1) / CT_TILE;
+  const FlagKept fk{c->kept.p};
+  if (nb == 1) {
+    hipLaunchKernelGGL(k_compact_one<FlagKept>, dim3(1), dim3(CT_THREADS), 0, s, fk, n, c->kidx.p, c->cnt + C_KEPT, nd);
+    return;
+  }
+  hipLaunchKernelGGL(k_flag_count<FlagKept>, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fk, n, c->bcount.p, nd);
+  if (nb <= CT_DIRECT) {
+    hipLaunchKernelGGL(k_scatter_idx<FlagKept>, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fk, n, c->bcount.p, c->kidx.p, nd,
+                       c->cnt + C_KEPT);
+    return;
+  }
+  hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, s, c->bcount.p, nb);
+  hipLaunchKernelGGL(k_scatter_idx<FlagKept>, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fk, n, c->bcount.p, c->kidx.p, nd,
+                     nullptr);
+  hipLaunchKernelGGL(k_add_total, dim3(1), dim3(64), 0, s, c->cnt + C_KEPT, c->bcount.p + nb);
 }
 
 // bytes of the level control block for ns slots (its layout is the pinned staging area's)
@@ -1107,7 +1139,6 @@ static void reserve_slots(chz_ctx *c, int need) {
   c->icnt = c->stage + NSTRIPE * SG_N;
   c->d_rem = (int *)(c->cnt + counter_words(ns));
   c->d_keepi = (uint8_t *)(c->d_rem + ns);
-  c->d_active.need(ns);
   c->gflag.need(ns);
   HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)ns * 4, c->stream));   // fresh slots: no goal child known
   c->d_lo.need(ns);
@@ -1199,6 +1230,44 @@ static void prune_tree(chz_ctx *c) {
   }
 }
 
+// A level of one chunk from its expansion's statuses to the kept survivors' ranks without the host: survivors, sort, exact
+// dedupe, kept ranks, launched for ncc children (dncc: their number on the device) and reading the sizes that come out
+// on the way from the counters.  The buffers hold ncc entries.
+template <int NQ>
+static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long long *dncc, uint32_t *gflag, hipStream_t s) {
+  constexpr int CPW = 64 >> (2 * NQ);
+  const unsigned long long *nd = c->cnt + C_SURV;
+  const uint32_t *pinst = c->finst[cur].p;
+  const AliveOut ao{c->keys.p, c->info.p, 0, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
+  compact_alive(c, FlagAlive{c->status.p}, ncc, ao, dncc, s);
+  sort_survivors(c, ncc, nd, s);
+  const ActiveArgs aa{c->icnt, slot_stripes(c->nslots), c->nslots, c->ks.G, c->surv_o.p, pinst};
+  hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(ncc / 256 + 1, 256)), dim3(256), 0, s, c->kept.p, ncc, nd, aa, gflag);
+  hipLaunchKernelGGL(k_run_starts, dim3(grid_for(ncc / (64 * RH_ITEMS) + 1)), dim3(256), 0, s, c->sk[0].p, ncc, c->runs.p,
+                     c->cnt + C_RUNS, nd);
+  const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncc, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p, c->res[cur].p,
+                      c->pk[cur].p, c->kept.p, c->cnt, pinst, nd};
+  hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncc / CPW / 8 + 1, 1024)), dim3(256), 0, s, c->ks, da);
+  compact_kept(c, ncc, nd, s);
+}
+
+// the buffers of level_tail and of a gather behind it for ncc children, and the tree level of mx nodes
+template <int NQ>
+static void level_room(chz_ctx *c, int nxt, long long ncc, long long mx, uint32_t *&tp, uint8_t *&tg) {
+  constexpr int E = 1 << (2 * NQ);
+  const long long nbA = (ncc + CT_TILE - 1) / CT_TILE, nbS = (ncc + RS_TILE - 1) / RS_TILE;
+  c->status.need(ncc); c->keys.need(ncc); c->info.need(ncc);
+  c->bcount.need(nbA + 1);
+  c->surv_o.need(ncc); c->surv_key.need(ncc); c->surv_bw.need(ncc);
+  c->kept.need(ncc); c->kidx.need(ncc); c->runs.need(ncc);
+  for (int b = 0; b < 2; b++) { c->sk[b].need(ncc); c->sv[b].need(ncc); }
+  c->hist.need((size_t)nbS * 256 + 1);
+  c->scan_tmp.need((size_t)nbS * 256 / SC_TILE + 4);
+  c->res[nxt].need((size_t)mx * E); c->pk[nxt].need(mx); c->g1[nxt].need(mx); c->g2[nxt].need(mx);
+  c->pb[nxt].need(mx); c->finst[nxt].need(mx);
+  tree_alloc(c, mx, tp, tg);
+}
+
 // Captured level step for levels of at most STEP_CAP parents: expansion, survivor compaction, radix sort, exact
 // dedupe, the searches' continue flags and the kept compaction, in one graph built once per frontier parity with
 // launches sized for the capacity; every kernel reads the level's sizes from the counters the host uploads
@@ -1220,24 +1289,14 @@ constexpr int STEP_BUCKET = 10;    // the schedule of the 1,024-parent bucket dr
 
 template <int NQ>
 static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long long *hc_in, unsigned long long *hc,
-                       unsigned long long *ptot, uint32_t *&tp, uint8_t *&tg) {
+                       uint32_t *&tp, uint8_t *&tg) {
   constexpr int N = 1 << NQ, E = N * N, CPW = 64 / E;
   (void)N;
   const KSpec &ks = c->ks;
   const int G = ks.G, nxt = cur ^ 1, ns = c->nslots;
   const long long cap = STEP_CAP, ncap = cap * G;
-  const long long nbA = (ncap + CT_TILE - 1) / CT_TILE, nbS = (ncap + RS_TILE - 1) / RS_TILE;
   const long long mx = ncap + (long long)c->pending.size();
-  c->status.need(ncap); c->keys.need(ncap); c->info.need(ncap);
-  c->bcount.need(nbA + 1);
-  c->surv_o.need(ncap); c->surv_key.need(ncap); c->surv_bw.need(ncap);
-  c->kept.need(ncap); c->kidx.need(ncap); c->runs.need(ncap);
-  for (int b = 0; b < 2; b++) { c->sk[b].need(ncap); c->sv[b].need(ncap); }
-  c->hist.need((size_t)nbS * 256 + 1);
-  c->scan_tmp.need((size_t)nbS * 256 / SC_TILE + 4);
-  c->res[nxt].need((size_t)mx * E); c->pk[nxt].need(mx); c->g1[nxt].need(mx); c->g2[nxt].need(mx);
-  c->pb[nxt].need(mx); c->finst[nxt].need(mx);
-  tree_alloc(c, mx, tp, tg);
+  level_room<NQ>(c, nxt, ncap, mx, tp, tg);
   const chz_ctx::Sched sc = c->sched[STEP_BUCKET];
   const uint32_t *pinst = c->finst[cur].p;
   const std::vector<uintptr_t> key = {
@@ -1247,12 +1306,12 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       (uintptr_t)c->bcount.p, (uintptr_t)c->surv_o.p, (uintptr_t)c->surv_key.p, (uintptr_t)c->surv_bw.p,
       (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->runs.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
       (uintptr_t)c->sv[0].p, (uintptr_t)c->sv[1].p, (uintptr_t)c->hist.p, (uintptr_t)c->scan_tmp.p,
-      (uintptr_t)c->d_active.p, (uintptr_t)c->gflag.p, (uintptr_t)ns, (uintptr_t)sc.var, (uintptr_t)sc.cap,
+      (uintptr_t)c->gflag.p, (uintptr_t)ns, (uintptr_t)sc.var, (uintptr_t)sc.cap,
       (uintptr_t)sc.tw};
   chz_ctx::StepGraph &sg = c->sgraph[cur];
   if (!sg.exec || sg.key != key) {
     if (sg.exec) { HIPCHK(hipGraphExecDestroy(sg.exec)); sg.exec = nullptr; }
-    const unsigned long long *dm = c->cnt + C_M, *dncc = c->cnt + C_NCC, *dsurv = c->cnt + C_SURV;
+    const unsigned long long *dm = c->cnt + C_M, *dncc = c->cnt + C_NCC;
     hipStream_t s = c->stream;
     hipGraph_t graph = nullptr;
     // no device-wide or allocating HIP call from another thread while this stream is captured (capture_mu)
@@ -1267,30 +1326,8 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       case 2: hipLaunchKernelGGL((k_level<NQ, 6>), grid, dim3(256), 0, s, ks, ea, cap); break;
       default: hipLaunchKernelGGL((k_level<NQ, 5>), grid, dim3(256), 0, s, ks, ea, cap); break;
     }
-    const FlagAlive fa{c->status.p, pinst, c->d_keepi, 0, G};
-    hipLaunchKernelGGL(k_flag_count<FlagAlive>, dim3((unsigned)nbA), dim3(CT_THREADS), 0, s, fa, ncap, c->bcount.p, dncc);
-    hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, s, c->bcount.p, nbA);
-    hipLaunchKernelGGL(k_scatter_alive, dim3((unsigned)nbA), dim3(CT_THREADS), 0, s, fa, ncap, c->bcount.p, c->keys.p,
-                       0ll, c->cnt + C_SURV, c->surv_o.p, c->surv_key.p, c->info.p, c->surv_bw.p, dncc);
-    hipLaunchKernelGGL(k_add_total, dim3(1), dim3(64), 0, s, c->cnt + C_SURV, c->bcount.p + nbA);
-    hipLaunchKernelGGL(k_init_sort, dim3(grid_for(ncap / 64 + 1)), dim3(256), 0, s, c->surv_key.p, ncap, c->sk[0].p,
-                       c->sv[0].p, dsurv);
-    hipError_t e = radix_sort_pairs(c->sk[0].p, c->sv[0].p, c->sk[1].p, c->sv[1].p, ncap, c->hist.p, c->scan_tmp.p, s,
-                                    dsurv);
-    hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(ncap / 256 + 1)), dim3(256), 0, s, c->kept.p, ncap, dsurv, nullptr,
-                       0);
-    hipLaunchKernelGGL(k_run_starts, dim3(grid_for(ncap / (64 * RH_ITEMS) + 1)), dim3(256), 0, s, c->sk[0].p, ncap,
-                       c->runs.p, c->cnt + C_RUNS, dsurv);
-    const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncap, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p, c->res[cur].p,
-                        c->pk[cur].p, c->kept.p, c->cnt, pinst, dsurv};
-    hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncap / CPW + 1, 4096)), dim3(256), 0, s, ks, da);
-    hipLaunchKernelGGL(k_active, dim3(1), dim3(256), 0, s, c->icnt, slot_stripes(ns), c->d_keepi, ns, c->d_active.p);
-    const FlagKept fk{c->kept.p, c->surv_o.p, pinst, c->d_active.p, G};
-    hipLaunchKernelGGL(k_flag_count<FlagKept>, dim3((unsigned)nbA), dim3(CT_THREADS), 0, s, fk, ncap, c->bcount.p, dsurv);
-    hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, s, c->bcount.p, nbA);
-    hipLaunchKernelGGL(k_scatter_idx<FlagKept>, dim3((unsigned)nbA), dim3(CT_THREADS), 0, s, fk, ncap, c->bcount.p,
-                       c->kidx.p, dsurv);
-    if (e == hipSuccess) e = hipGetLastError();
+    level_tail<NQ>(c, cur, ncap, dncc, nullptr, s);
+    hipError_t e = hipGetLastError();
     const hipError_t ec = hipStreamEndCapture(s, &graph);
     if (e == hipSuccess) e = ec;
     if (e == hipSuccess) e = hipGraphInstantiate(&sg.exec, graph, nullptr, nullptr, 0);
@@ -1308,18 +1345,17 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   c->ev.end(c->stream);
   const GatherArgs ga{c->kidx.p, ncap, c->surv_o.p, c->res[cur].p, c->pk[cur].p, c->g1[cur].p,
                       c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tp, tg, pinst, c->finst[nxt].p,
-                      c->surv_bw.p, c->pb[nxt].p, c->bcount.p + nbA, c->goal_skip ? c->gflag.p : nullptr, CPW};
+                      c->surv_bw.p, c->pb[nxt].p, c->cnt + C_KEPT, c->goal_skip ? c->gflag.p : nullptr, CPW};
   HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)ns * 4, c->stream));   // the graph's expansion has read them
   c->ev.begin(K_GATHER, c->stream);
   hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((ncap + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga);
   c->ev.end(c->stream);
   HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(ptot, c->bcount.p + nbA, 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   fold_counters(hc, ns);
   c->ev.flush(c->k_ms, c->k_launch);
   if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
-  c->k_work[K_GATHER] += (double)*ptot * (E * 16.0 * 2.0 + 16.0);
+  c->k_work[K_GATHER] += (double)hc[C_KEPT] * (E * 16.0 * 2.0 + 16.0);
 }
 
 // One level of every live search of the batch (src/cheese.cu:1249-1377 per search): expansion in chunks,
@@ -1381,11 +1417,10 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   // in one copy), the kept total and the per-slot active flags
   const int ns = c->nslots;
   const size_t in_bytes = ctl_in_bytes(ns), o_out = (in_bytes + 63) & ~(size_t)63,
-               o_tot = o_out + counter_words(ns) * 8, o_act = o_tot + 8;
+               o_act = o_out + counter_words(ns) * 8;
   uint8_t *pin = c->pin.need(o_act + ns);
   unsigned long long *hc_in = (unsigned long long *)pin, *ic_in = hc_in + C_N + NSTRIPE * SG_N;
   unsigned long long *hc = (unsigned long long *)(pin + o_out), *ic = hc + C_N + NSTRIPE * SG_N;
-  unsigned long long *ptot = (unsigned long long *)(pin + o_tot);
   int *rem = (int *)(hc_in + counter_words(ns));
   uint8_t *keepi = (uint8_t *)(rem + ns), *active = pin + o_act;
   std::memset(hc_in, 0, counter_words(ns) * 8);
@@ -1412,9 +1447,9 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     for (int i = 0; i < C_N; i++) hc_in[i] = 0;
     hc_in[C_M] = (unsigned long long)m;
     hc_in[C_NCC] = (unsigned long long)(m * G);
-    step_graph<NQ>(c, cur, m, hc_in, hc, ptot, tp, tg);
+    step_graph<NQ>(c, cur, m, hc_in, hc, tp, tg);
     nsurv = (long long)hc[C_SURV];
-    distinct = (long long)*ptot;
+    distinct = (long long)hc[C_KEPT];
     c->k_work[K_STEP] += expand_ops(c, NQ, hc) + (double)(m * G) + (double)nsurv * (24.0 + 16.0 + 4 * 20.0 + 9.0);
     static const int stage_ctr[6] = {C_EVAL, C_CHEAP, C_CUTS, C_NEEDT, C_KEYS, C_TPASS};
     for (int i = 0; i < 6; i++) c->k_stage[i] += (double)hc[stage_ctr[i]];
@@ -1462,18 +1497,16 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       c->tune_ev.push_back({bucket, {te0, te1}});
     }
     const long long nb = (ncc + CT_TILE - 1) / CT_TILE;
-    const FlagAlive fa{c->status.p, pinst, c->d_keepi, off, G};
+    const FlagAlive fa{c->status.p};
+    const AliveOut ao{c->keys.p, c->info.p, off * G, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
     c->ev.begin(K_COMPACT, c->stream);
-    if (nb == 1) {   // one tile: count, place and advance the survivor count in one launch
-      hipLaunchKernelGGL(k_scatter_alive_one, dim3(1), dim3(CT_THREADS), 0, c->stream, fa, ncc, c->keys.p, off * G,
-                         c->cnt + C_SURV, c->surv_o.p, c->surv_key.p, c->info.p, c->surv_bw.p);
-    } else {
+    if (ncc <= CT_DIRECT * CT_TILE && ma <= chunk) compact_alive(c, fa, ncc, ao, nullptr, c->stream);
+    else {
       hipLaunchKernelGGL(k_flag_count<FlagAlive>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, fa, ncc,
                          c->bcount.p);
       hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, c->stream, c->bcount.p, nb);
-      hipLaunchKernelGGL(k_scatter_alive, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, fa, ncc, c->bcount.p,
-                         c->keys.p, off * G, c->cnt + C_SURV, c->surv_o.p, c->surv_key.p, c->info.p, c->surv_bw.p,
-                         nullptr);
+      hipLaunchKernelGGL(k_scatter_alive, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, fa, ncc, c->bcount.p, ao,
+                         c->cnt + C_SURV, nullptr, nullptr);
       hipLaunchKernelGGL(k_add_total, dim3(1), dim3(64), 0, c->stream, c->cnt + C_SURV, c->bcount.p + nb);
     }
     c->ev.end(c->stream);
@@ -1494,28 +1527,20 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       const unsigned long long *x = &ic[(size_t)b.slot * IC_N];
       active[b.slot] = !x[IC_FOUND] && !x[IC_OVF] && keepi[b.slot];
     }
-  HIPCHK(hipMemcpyAsync(c->d_active.p, active, ns, hipMemcpyHostToDevice, c->stream));
   if (nsurv > 0) {
     c->kept.need(nsurv);
     c->kidx.need(nsurv);
+    const ActiveArgs aa{c->icnt, slot_stripes(ns), ns, G, c->surv_o.p, pinst};
+    gflag_clear = true;
     if (c->opts.dedupe && nsurv > 1) {
-      for (int bb = 0; bb < 2; bb++) { c->sk[bb].need(nsurv); c->sv[bb].need(nsurv); }
       c->runs.need(nsurv);
       c->ev.begin(K_SORT, c->stream);
-      if (nsurv <= SS_MAX) {
-        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(1024), 0, c->stream, c->surv_key.p, nsurv, c->sk[0].p,
-                           c->sv[0].p);
-      } else {
-        hipLaunchKernelGGL(k_init_sort, dim3(grid_for(nsurv / 64 + 1)), dim3(256), 0, c->stream, c->surv_key.p,
-                           nsurv, c->sk[0].p, c->sv[0].p, nullptr);
-        sort_pairs(c, nsurv);
-      }
+      sort_survivors(c, nsurv, nullptr, c->stream);
       c->ev.end(c->stream);
       c->k_work[K_SORT] += (double)nsurv * (16.0 + 4 * (4.0 + 16.0));
       c->ev.begin(K_DEDUPE, c->stream);
       hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(nsurv / 256 + 1)), dim3(256), 0, c->stream, c->kept.p, nsurv,
-                         nullptr, c->gflag.p, ns);
-      gflag_clear = true;
+                         nullptr, aa, c->gflag.p);
       hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nsurv / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream,
                          c->sk[0].p, nsurv, c->runs.p, c->cnt + C_RUNS, nullptr);
       const DedupeArgs da{c->sk[0].p, c->sv[0].p, nsurv, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p,
@@ -1524,7 +1549,8 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       c->ev.end(c->stream);
       c->k_work[K_DEDUPE] += (double)nsurv * 9.0;
     } else {
-      HIPCHK(hipMemsetAsync(c->kept.p, 1, nsurv, c->stream));
+      hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(nsurv / 256 + 1)), dim3(256), 0, c->stream, c->kept.p, nsurv,
+                         nullptr, aa, c->gflag.p);
     }
     if (c->gt_filter)      // a table build: classes already in the table (lower levels) are dropped
       hipLaunchKernelGGL(k_gt_filter<NQ>, dim3(grid_for(nsurv / CPW + 1)), dim3(256), 0, c->stream, ks,
@@ -1532,24 +1558,13 @@ template <int NQ> static void batch_step(chz_ctx *c) {
                          c->kept.p);
     const long long nb = (nsurv + CT_TILE - 1) / CT_TILE;
     c->bcount.need(nb + 1);
-    const FlagKept fk{c->kept.p, c->surv_o.p, pinst, c->d_active.p, G};
     c->ev.begin(K_COMPACT, c->stream);
-    if (nb == 1) {
-      hipLaunchKernelGGL(k_compact_one<FlagKept>, dim3(1), dim3(CT_THREADS), 0, c->stream, fk, nsurv, c->kidx.p,
-                         c->bcount.p + nb);
-    } else {
-      hipLaunchKernelGGL(k_flag_count<FlagKept>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, fk, nsurv,
-                         c->bcount.p);
-      hipLaunchKernelGGL(k_scan_one_block, dim3(1), dim3(1024), 0, c->stream, c->bcount.p, nb);
-      hipLaunchKernelGGL(k_scatter_idx<FlagKept>, dim3((unsigned)nb), dim3(CT_THREADS), 0, c->stream, fk, nsurv,
-                         c->bcount.p, c->kidx.p);
-    }
+    compact_kept(c, nsurv, nullptr, c->stream);
     c->ev.end(c->stream);
-    HIPCHK(hipMemcpyAsync(ptot, c->bcount.p + nb, 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(hc, c->cnt, C_N * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
-    distinct = (long long)*ptot;
+    distinct = (long long)hc[C_KEPT];
   }
   }   // normal path
   // next frontier: kept children, then the searches admitted since the last step.  The goal flags describe the
@@ -2332,7 +2347,7 @@ void chz_close(chz_ctx *c) {
     c->pb[b].release();
     c->sk[b].release(); c->sv[b].release();
   }
-  c->finst[0].release(); c->finst[1].release(); c->ctl.release(); c->d_active.release(); c->gflag.release();
+  c->finst[0].release(); c->finst[1].release(); c->ctl.release(); c->gflag.release();
   c->scan_tmp.release(); c->d_lo.release(); c->d_hi.release();
   c->pin.release();
   for (auto &g : c->sgraph) if (g.exec) { (void)hipGraphExecDestroy(g.exec); g.exec = nullptr; }

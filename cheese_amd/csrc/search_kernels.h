@@ -28,7 +28,8 @@ template <int GS> __device__ __forceinline__ uint64_t gget64(uint64_t v, int q) 
   return (uint64_t)gget<GS>((uint32_t)v, q) | ((uint64_t)gget<GS>((uint32_t)(v >> 32), q) << 32);
 }
 
-enum : uint8_t { ST_DEAD = 0, ST_ALIVE = 1, ST_FOUND = 2, ST_W2 = 3, ST_W3 = 4, ST_OVF = 6 };
+// ST_LAST: alive at its search's last level, so no parent of the next one (tallied as alive)
+enum : uint8_t { ST_DEAD = 0, ST_ALIVE = 1, ST_FOUND = 2, ST_W2 = 3, ST_W3 = 4, ST_OVF = 6, ST_LAST = 7 };
 constexpr uint32_t INFO_NOBOUND = 1u << 31;    // spec without bounds: every child is kept
 
 // x * w^p for a coefficient vector of int32 values (entries below 2^28 in magnitude: no overflow)
