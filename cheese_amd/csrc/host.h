@@ -51,11 +51,21 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&prev); }
 };
 
+// Blocks that buffers of a context outgrew while its stream may still use them, given back once it has synchronised for
+// another reason: a search on a new context grows some twenty buffers level by level, and a synchronisation for each
+// cost it 0.2 ms
+using Retired = std::vector<std::pair<void *, size_t>>;
+inline Retired *&retire_list() { static thread_local Retired *l = nullptr; return l; }
+
 struct StreamScope {
   hipStream_t prev;
+  Retired *prev_list;
   RelaxedCapture relaxed;
-  explicit StreamScope(hipStream_t s) : prev(owner_stream()) { owner_stream() = s; }
-  ~StreamScope() { owner_stream() = prev; }
+  explicit StreamScope(hipStream_t s, Retired *list = nullptr) : prev(owner_stream()), prev_list(retire_list()) {
+    owner_stream() = s;
+    retire_list() = list;
+  }
+  ~StreamScope() { owner_stream() = prev; retire_list() = prev_list; }
 };
 // a synchronous copy on the context's own stream (a copy on the legacy default stream would depend on every
 // blocking stream, which is not allowed while another thread captures one)
@@ -176,6 +186,12 @@ inline void dev_free(void *p) {
   dev_pool().put(p, got);
 }
 
+// the outgrown blocks of a context whose stream has synchronised
+inline void settle(Retired &list) {
+  for (auto &b : list) dev_pool().put(b.first, b.second);
+  list.clear();
+}
+
 template <typename T> struct DBuf {     // grow-only device array on the block cache
   T *p = nullptr;
   size_t cap = 0, bytes = 0;
@@ -183,11 +199,23 @@ template <typename T> struct DBuf {     // grow-only device array on the block c
     if (n <= cap) return;
     const size_t c = std::max<size_t>(std::max<size_t>(n, cap + cap / 2), 1);
     size_t got = 0;
-    T *np = (T *)dev_pool().get(c * sizeof(T), got);
+    T *np = nullptr;
+    Retired *list = owner_stream() ? retire_list() : nullptr;
+    try {
+      np = (T *)dev_pool().get(c * sizeof(T), got);
+    } catch (DeviceError &) {
+      if (!list || list->empty()) throw;
+      HIPCHK(sync_owner());                 // the outgrown blocks are memory too
+      settle(*list);
+      np = (T *)dev_pool().get(c * sizeof(T), got);
+    }
     if (p) {
       // kernels already queued may still read the old block
-      HIPCHK(sync_owner());
-      dev_pool().put(p, bytes);
+      if (list) list->push_back({p, bytes});
+      else {
+        HIPCHK(sync_owner());
+        dev_pool().put(p, bytes);
+      }
     }
     p = np;
     bytes = got;

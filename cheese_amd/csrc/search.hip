@@ -44,8 +44,9 @@ enum { IC_W2 = 0, IC_W3, IC_DEAD, IC_FOUND, IC_ALIVE, IC_OVF, IC_FIRST, IC_N };
 enum { SG_EVAL = 0, SG_PRE, SG_NEEDT, SG_CHEAP, SG_CUTS, SG_KEYS, SG_TPASS, SG_N = 8 };
 constexpr int NSTRIPE = 16;
 static int slot_stripes(int ns) { return std::max(1, std::min(NSTRIPE, 256 / ns)); }    // of the per-slot counters
-// words of the counters: [C_N | stage stripes | slot stripes]
-static size_t counter_words(int ns) { return (size_t)C_N + (size_t)NSTRIPE * SG_N + (size_t)slot_stripes(ns) * ns * IC_N; }
+// words of the counters: [C_N | stage stripes | slot stripes | slot bounds]
+static size_t bounds_at(int ns) { return (size_t)C_N + (size_t)NSTRIPE * SG_N + (size_t)slot_stripes(ns) * ns * IC_N; }
+static size_t counter_words(int ns) { return bounds_at(ns) + 2 * (size_t)ns; }
 
 struct ExpandArgs {
   const int4 *res;          // parents' residuals, E entries each
@@ -943,19 +944,21 @@ struct chz_ctx {
   int cur = 0, gstep = -1, nslots = 0;
   bool shared_steps = false;      // the batch has held more than one search at once (captured steps are used)
   // level control block, uploaded in one copy at the start of every level and read back in one copy:
-  // [cnt: C_N counters | stage stripes | icnt: stripes of per-slot IC_N counters | d_rem: per-slot budgets | d_keepi:
-  // per-slot keep flags]
+  // [cnt: C_N counters | stage stripes | icnt: stripes of per-slot IC_N counters | slo, shi: each slot's nodes in the next
+  // frontier | d_rem: per-slot budgets | d_keepi: per-slot keep flags]
   chz::DBuf<unsigned long long> ctl;
   unsigned long long *cnt = nullptr, *stage = nullptr, *icnt = nullptr;
+  long long *slo = nullptr, *shi = nullptr;
   int *d_rem = nullptr;
   uint8_t *d_keepi = nullptr;
   chz::DBuf<uint32_t> gflag;        // per slot: a node of the current frontier has a goal child
   chz::DBuf<unsigned long long> scan_tmp;
   chz::Pinned pin;                  // staging of the per-level control transfers
+  chz::Pinned pin_io;               // what kernels read and write on the host: admitted roots, walked circuits
+  chz::Retired retired;             // outgrown buffers, given back when the stream has synchronised
   // captured level steps (one per frontier parity) and the buffer addresses and schedule they were captured with
   struct StepGraph { hipGraphExec_t exec = nullptr; std::vector<uintptr_t> key; };
   StepGraph sgraph[2];
-  chz::DBuf<long long> d_lo, d_hi;
   // expansion schedule per level-size bucket (log2 of the chunk's parents): occupancy variant, grid cap in
   // blocks, candidate-split threshold in waves; chosen by chz_tune, defaults otherwise
   struct Sched { int var = 1, cap = 8192, tw = 4096; };
@@ -1137,65 +1140,72 @@ static void reserve_slots(chz_ctx *c, int need) {
   c->cnt = c->ctl.p;
   c->stage = c->cnt + C_N;
   c->icnt = c->stage + NSTRIPE * SG_N;
+  c->slo = (long long *)(c->cnt + bounds_at(ns));
+  c->shi = c->slo + ns;
   c->d_rem = (int *)(c->cnt + counter_words(ns));
   c->d_keepi = (uint8_t *)(c->d_rem + ns);
   c->gflag.need(ns);
   HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)ns * 4, c->stream));   // fresh slots: no goal child known
-  c->d_lo.need(ns);
-  c->d_hi.need(ns);
   c->nslots = ns;
 }
 
-// nodes of every slot in frontier buffer `b` of m nodes (nodes are contiguous per instance)
-__global__ void k_slot_bounds(const uint32_t *inst, long long n, long long *lo, long long *hi) {
+// the nodes [lo, hi) of every slot in a frontier of n nodes (contiguous per slot; a slot without nodes keeps the zeros of
+// the level's control upload)
+__global__ void k_slot_bounds(const uint32_t *inst, long long n, const unsigned long long *nd, long long *lo, long long *hi) {
+  n = dev_n(n, nd);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
     const uint32_t s = inst[i];
     if (i == 0 || inst[i - 1] != s) lo[s] = i;
     if (i == n - 1 || inst[i + 1] != s) hi[s] = i + 1;
   }
 }
-__global__ void k_fill_ll(long long *p, long long n, long long v) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = v;
+
+// admitted roots from the host's memory into the frontier behind its first `at` nodes
+struct RootArgs {
+  const int4 *u;             // nr matrices of E entries
+  const int *k, *slot;
+  long long nr, at;
+  int4 *res;
+  int *pk;
+  uint8_t *g1, *g2, *tg;
+  uint32_t *finst, *pb, *tp;
+  uint32_t *gflag;           // goal flags of ns slots to clear (a frontier of roots only), or null
+  int ns;
+};
+template <int E> __global__ void k_put_roots(RootArgs a) {
+  const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < a.nr * E; i += stride) a.res[a.at * E + i] = a.u[i];
+  for (long long i = i0; i < a.nr; i += stride) {
+    const long long x = a.at + i;
+    a.pk[x] = a.k[i];
+    a.g1[x] = a.g2[x] = a.tg[x] = 255;
+    a.finst[x] = (uint32_t)a.slot[i];
+    a.pb[x] = BW_TUNK;
+    a.tp[x] = NO_PARENT;
+  }
+  if (a.gflag)
+    for (long long i = i0; i < a.ns; i += stride) a.gflag[i] = 0u;
 }
 
-static std::vector<long long> slot_counts(chz_ctx *c, const uint32_t *inst, long long m) {
-  std::vector<long long> out(c->nslots);
-  // (called after the level's control transfers completed: the staging area is free)
-  long long *lo = (long long *)c->pin.need((size_t)c->nslots * 16), *hi = lo + c->nslots;
-  hipLaunchKernelGGL(k_fill_ll, dim3(16), dim3(256), 0, c->stream, c->d_lo.p, (long long)c->nslots, 0ll);
-  hipLaunchKernelGGL(k_fill_ll, dim3(16), dim3(256), 0, c->stream, c->d_hi.p, (long long)c->nslots, 0ll);
-  if (m) hipLaunchKernelGGL(k_slot_bounds, dim3(grid_for(m / 64 + 1)), dim3(256), 0, c->stream, inst, m, c->d_lo.p, c->d_hi.p);
-  HIPCHK(hipMemcpyAsync(lo, c->d_lo.p, c->nslots * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(hi, c->d_hi.p, c->nslots * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  for (int s = 0; s < c->nslots; s++) out[s] = hi[s] - lo[s];
-  return out;
-}
-
-// the next frontier: `distinct` gathered children (already in buffer nxt) followed by the admitted roots
+// the next frontier: `distinct` gathered children (already in buffer nxt) followed by the admitted roots, which one kernel
+// reads from host memory (eight copies and a synchronisation took longer than a small search's first two levels; what the
+// kernel reads is written again only after the level's synchronisation)
 template <int NQ> static void append_roots(chz_ctx *c, int nxt, long long distinct, uint32_t *tp, uint8_t *tg) {
   constexpr int E = 1 << (2 * NQ);
   const long long nr = (long long)c->pending.size();
   if (!nr) return;
-  std::vector<int4> res(nr * E);
-  std::vector<int> pk(nr);
-  std::vector<uint8_t> none(nr, 255);
-  std::vector<uint32_t> slot(nr), np(nr, NO_PARENT), bw(nr, BW_TUNK);
+  int4 *u = (int4 *)c->pin_io.need((size_t)nr * (E * sizeof(int4) + 8));
+  int *k = (int *)(u + nr * E), *slot = k + nr;
   for (long long i = 0; i < nr; i++) {
     const Pending &q = c->pending[i];
-    for (int e = 0; e < E; e++) res[i * E + e] = q.U[e];
-    pk[i] = q.k;
-    slot[i] = (uint32_t)c->binst[q.inst].slot;
+    std::copy(q.U.begin(), q.U.end(), u + i * E);
+    k[i] = q.k;
+    slot[i] = c->binst[q.inst].slot;
   }
-  HIPCHK(hipMemcpyAsync(c->res[nxt].p + distinct * E, res.data(), nr * E * sizeof(int4), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->pk[nxt].p + distinct, pk.data(), nr * 4, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->g1[nxt].p + distinct, none.data(), nr, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->g2[nxt].p + distinct, none.data(), nr, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->finst[nxt].p + distinct, slot.data(), nr * 4, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(c->pb[nxt].p + distinct, bw.data(), nr * 4, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(tp + distinct, np.data(), nr * 4, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(tg + distinct, none.data(), nr, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  const RootArgs ra{u, k, slot, nr, distinct, c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tg,
+                    c->finst[nxt].p, c->pb[nxt].p, tp, c->m ? nullptr : c->gflag.p, c->nslots};
+  hipLaunchKernelGGL(k_put_roots<E>, dim3(grid_for(nr * E / 64 + 1, 1024)), dim3(256), 0, c->stream, ra);
+  HIPCHK(hipGetLastError());
   for (long long i = 0; i < nr; i++) {
     c->binst[c->pending[i].inst].root_step = c->gstep + 1;
     c->forder.push_back(c->pending[i].inst);
@@ -1203,21 +1213,65 @@ template <int NQ> static void append_roots(chz_ctx *c, int nxt, long long distin
   c->pending.clear();
 }
 
-// the lexicographically first circuit of a FOUND child: gate of the child, then the tree walked up to the root
-static void walk_circuit(chz_ctx *c, unsigned long long o, int G, std::vector<int> &seq) {
-  seq.clear();
-  seq.push_back((int)(o % G));
-  uint32_t i = (uint32_t)(o / G);
-  for (int s = c->gstep; s >= 0; s--) {
-    uint32_t par;
-    uint8_t g;
-    chz::copy_sync(&par, c->tree_par[s] + i, 4, hipMemcpyDeviceToHost, c->stream);
-    if (par == NO_PARENT) break;
-    chz::copy_sync(&g, c->tree_gate[s] + i, 1, hipMemcpyDeviceToHost, c->stream);
-    if (g != CARRY_GATE) seq.push_back(g);     // a level the search waited through
-    i = par;
+// The lexicographically first circuit of FOUND children: the child's gate, then the tree walked up to the root, one
+// thread a search, WALK levels a launch (a copy and a synchronisation for every step of a walk took 0.3 ms for 12 gates)
+constexpr int WALK = 32, WALK_MAX = 64;
+struct WalkState { uint32_t i; int n, done; uint8_t g[WALK_MAX + 4]; };
+struct WalkArgs {
+  const uint32_t *par[WALK];     // levels from the highest down
+  const uint8_t *gate[WALK];
+  int levels, n;
+  WalkState *w;                  // host memory
+};
+__global__ void k_walk(WalkArgs a) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= a.n || a.w[q].done) return;
+  uint32_t i = a.w[q].i;
+  int n = a.w[q].n, done = 0;
+  for (int s = 0; s < a.levels && !done; s++) {
+    const uint32_t par = a.par[s][i];
+    const uint8_t g = a.gate[s][i];
+    if (par == NO_PARENT) done = 1;
+    else {
+      if (g != CARRY_GATE && n < WALK_MAX) a.w[q].g[n++] = g;     // else a level the search waited through
+      i = par;
+    }
   }
-  std::reverse(seq.begin(), seq.end());
+  a.w[q].i = i;
+  a.w[q].n = n;
+  a.w[q].done = done;
+}
+// at[j]: FOUND child of the instance from[j]
+static void walk_circuits(chz_ctx *c, const std::vector<unsigned long long> &at, const std::vector<int> &from, int G,
+                          std::vector<std::vector<int>> &seq) {
+  const int n = (int)at.size();
+  seq.assign(n, {});
+  if (!n) return;
+  WalkState *w = (WalkState *)c->pin_io.need((size_t)n * sizeof(WalkState));
+  int lo = c->gstep;
+  for (int q = 0; q < n; q++) {
+    w[q].i = (uint32_t)(at[q] / G);
+    w[q].n = 1;
+    w[q].done = 0;
+    w[q].g[0] = (uint8_t)(at[q] % G);
+    lo = std::min(lo, c->binst[from[q]].root_step);
+  }
+  for (int s = c->gstep; s >= lo; s -= WALK) {
+    WalkArgs a{};
+    a.n = n;
+    a.w = w;
+    for (a.levels = 0; a.levels < WALK && s - a.levels >= lo; a.levels++) {
+      a.par[a.levels] = c->tree_par[s - a.levels];
+      a.gate[a.levels] = c->tree_gate[s - a.levels];
+    }
+    hipLaunchKernelGGL(k_walk, dim3((n + 63) / 64), dim3(64), 0, c->stream, a);
+  }
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(c->stream));
+  for (int q = 0; q < n; q++) {
+    seq[q].assign(w[q].g, w[q].g + w[q].n);
+    std::reverse(seq[q].begin(), seq[q].end());
+  }
 }
 
 // tree levels no live search can reach any more
@@ -1234,13 +1288,21 @@ static void prune_tree(chz_ctx *c) {
 // dedupe, kept ranks, launched for ncc children (dncc: their number on the device) and reading the sizes that come out
 // on the way from the counters.  The buffers hold ncc entries.
 template <int NQ>
-static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long long *dncc, uint32_t *gflag, hipStream_t s) {
+static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long long *dncc, uint32_t *gflag, bool timed,
+                       hipStream_t s) {
   constexpr int CPW = 64 >> (2 * NQ);
   const unsigned long long *nd = c->cnt + C_SURV;
   const uint32_t *pinst = c->finst[cur].p;
   const AliveOut ao{c->keys.p, c->info.p, 0, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
+  auto begin = [&](int fam) { if (timed) c->ev.begin(fam, s); };
+  auto end = [&]() { if (timed) c->ev.end(s); };
+  begin(K_COMPACT);
   compact_alive(c, FlagAlive{c->status.p}, ncc, ao, dncc, s);
+  end();
+  begin(K_SORT);
   sort_survivors(c, ncc, nd, s);
+  end();
+  begin(K_DEDUPE);
   const ActiveArgs aa{c->icnt, slot_stripes(c->nslots), c->nslots, c->ks.G, c->surv_o.p, pinst};
   hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(ncc / 256 + 1, 256)), dim3(256), 0, s, c->kept.p, ncc, nd, aa, gflag);
   hipLaunchKernelGGL(k_run_starts, dim3(grid_for(ncc / (64 * RH_ITEMS) + 1)), dim3(256), 0, s, c->sk[0].p, ncc, c->runs.p,
@@ -1248,7 +1310,10 @@ static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long l
   const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncc, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p, c->res[cur].p,
                       c->pk[cur].p, c->kept.p, c->cnt, pinst, nd};
   hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncc / CPW / 8 + 1, 1024)), dim3(256), 0, s, c->ks, da);
+  end();
+  begin(K_COMPACT);
   compact_kept(c, ncc, nd, s);
+  end();
 }
 
 // the buffers of level_tail and of a gather behind it for ncc children, and the tree level of mx nodes
@@ -1285,6 +1350,7 @@ constexpr long long STEP_CAP = 1024;
 // budget 9: 0.86 ms against 1.00 ms with captured steps, budget 12: 8.34 ms against 8.44 ms), while in the server
 // they lower the latency tail.
 constexpr bool kStepGraphs = true;
+constexpr long long ONCE_NCC = 1 << 16;
 constexpr int STEP_BUCKET = 10;    // the schedule of the 1,024-parent bucket drives the captured expansion
 
 template <int NQ>
@@ -1326,7 +1392,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       case 2: hipLaunchKernelGGL((k_level<NQ, 6>), grid, dim3(256), 0, s, ks, ea, cap); break;
       default: hipLaunchKernelGGL((k_level<NQ, 5>), grid, dim3(256), 0, s, ks, ea, cap); break;
     }
-    level_tail<NQ>(c, cur, ncap, dncc, nullptr, s);
+    level_tail<NQ>(c, cur, ncap, dncc, nullptr, false, s);
     hipError_t e = hipGetLastError();
     const hipError_t ec = hipStreamEndCapture(s, &graph);
     if (e == hipSuccess) e = ec;
@@ -1367,7 +1433,6 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   const int G = ks.G;
   if (c->m == 0 && c->pending.empty()) return;
   if (c->m == 0) {   // a frontier of roots only
-    if (c->nslots) HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)c->nslots * 4, c->stream));
     const long long nr = (long long)c->pending.size();
     const int nxt = c->cur ^ 1;
     c->res[nxt].need(nr * E); c->pk[nxt].need(nr); c->g1[nxt].need(nr); c->g2[nxt].need(nr); c->finst[nxt].need(nr);
@@ -1383,8 +1448,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     c->gstep++;
     c->cur = nxt;
     c->m = nr;
-    const std::vector<long long> cnts = slot_counts(c, c->finst[c->cur].p, c->m);
-    for (BInst &b : c->binst) if (b.live) b.nodes = cnts[b.slot];
+    for (BInst &b : c->binst) if (b.live) b.nodes = 1;
   }
   const double tl = now_s();
   const int cur = c->cur;
@@ -1437,6 +1501,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   const int nxt = cur ^ 1;
   long long nsurv = 0, distinct = 0;
   bool gflag_clear = false;          // the goal flags were cleared by this level's kept fill
+  bool once = false, counted = false;
   uint32_t *tp = nullptr;
   uint8_t *tg = nullptr;
   // small levels run as one captured graph (expansion through kept compaction) plus the gather: one
@@ -1459,7 +1524,13 @@ template <int NQ> static void batch_step(chz_ctx *c) {
         active[b.slot] = !x[IC_FOUND] && !x[IC_OVF] && keepi[b.slot];
       }
   } else {
+  const bool alone = c->pending.empty() && chz_batch_live(c) == 1;
+  // levels of few children need the host for nothing between their expansion and the next frontier: launched for all
+  // children of the level, with one synchronisation and one copy at the end
+  once = !c->tuning && !c->gt_filter && c->opts.dedupe && c->pending.empty() && ma == m && ma <= chunk && ma * G <= ONCE_NCC;
   const long long maxcc = std::min<long long>(chunk, std::max<long long>(ma, 1)) * G;
+  if (once) level_room<NQ>(c, nxt, maxcc, maxcc, tp, tg);
+
   c->status.need(maxcc);
   c->info.need(maxcc);
   c->keys.need(maxcc);
@@ -1497,6 +1568,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       c->tune_ev.push_back({bucket, {te0, te1}});
     }
     const long long nb = (ncc + CT_TILE - 1) / CT_TILE;
+    if (once) break;
     const FlagAlive fa{c->status.p};
     const AliveOut ao{c->keys.p, c->info.p, off * G, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
     c->ev.begin(K_COMPACT, c->stream);
@@ -1511,6 +1583,21 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     }
     c->ev.end(c->stream);
     c->k_work[K_COMPACT] += (double)ncc;
+  }
+  if (once) {
+    level_tail<NQ>(c, cur, maxcc, nullptr, c->gflag.p, true, c->stream);
+    gflag_clear = true;
+    const GatherArgs ga{c->kidx.p, maxcc, c->surv_o.p, c->res[cur].p, c->pk[cur].p, c->g1[cur].p,
+                        c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tp, tg, pinst, c->finst[nxt].p,
+                        c->surv_bw.p, c->pb[nxt].p, c->cnt + C_KEPT, c->goal_skip ? c->gflag.p : nullptr, CPW};
+    c->ev.begin(K_GATHER, c->stream);
+    hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((maxcc / 4 + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga);
+    c->ev.end(c->stream);
+    if (!alone) {
+      hipLaunchKernelGGL(k_slot_bounds, dim3(grid_for(maxcc / 256 + 1, 256)), dim3(256), 0, c->stream, c->finst[nxt].p, maxcc,
+                         c->cnt + C_KEPT, c->slo, c->shi);
+      counted = true;
+    }
   }
   HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -1527,7 +1614,15 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       const unsigned long long *x = &ic[(size_t)b.slot * IC_N];
       active[b.slot] = !x[IC_FOUND] && !x[IC_OVF] && keepi[b.slot];
     }
-  if (nsurv > 0) {
+  settle(c->retired);
+  if (once) {
+    if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
+    distinct = (long long)hc[C_KEPT];
+    c->k_work[K_COMPACT] += (double)(m * G);
+    c->k_work[K_SORT] += (double)nsurv * (16.0 + 4 * (4.0 + 16.0));
+    c->k_work[K_DEDUPE] += (double)nsurv * 9.0;
+    c->k_work[K_GATHER] += (double)distinct * (E * 16.0 * 2.0 + 16.0);
+  } else if (nsurv > 0) {
     c->kept.need(nsurv);
     c->kidx.need(nsurv);
     const ActiveArgs aa{c->icnt, slot_stripes(ns), ns, G, c->surv_o.p, pinst};
@@ -1569,18 +1664,19 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   }   // normal path
   // next frontier: kept children, then the searches admitted since the last step.  The goal flags describe the
   // frontier being expanded until here; the gather sets them for the next one.
+  const bool gathered = graphed || once;      // the next frontier's children are in place
   if (!graphed && !gflag_clear) HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)ns * 4, c->stream));
   const long long ncarry = m - ma;            // nodes of the searches that waited
   const long long mn = distinct + ncarry + (long long)c->pending.size();
   std::vector<long long> cnts(c->nslots, 0);
   if (mn) {
-    if (!graphed) {
+    if (!gathered) {
       c->res[nxt].need((size_t)mn * E); c->pk[nxt].need(mn); c->g1[nxt].need(mn); c->g2[nxt].need(mn);
       c->pb[nxt].need(mn);
       c->finst[nxt].need(mn);
       tree_alloc(c, mn, tp, tg);
     }
-    if (distinct && !graphed) {
+    if (distinct && !gathered) {
       const GatherArgs ga{c->kidx.p, distinct, c->surv_o.p, c->res[cur].p, c->pk[cur].p, c->g1[cur].p,
                           c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tp, tg, pinst, c->finst[nxt].p,
                           c->surv_bw.p, c->pb[nxt].p, nullptr, c->goal_skip ? c->gflag.p : nullptr,
@@ -1617,15 +1713,35 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     if (single) {   // one search: its nodes are the whole frontier (its kernel times are read next step)
       for (const BInst &b : c->binst) if (b.live) cnts[b.slot] = mn;
     } else {
-      cnts = slot_counts(c, c->finst[nxt].p, mn);
+      const long long *lo = (const long long *)(hc + bounds_at(ns));
+      if (!counted) {
+        hipLaunchKernelGGL(k_slot_bounds, dim3(grid_for(mn / 64 + 1)), dim3(256), 0, c->stream, c->finst[nxt].p, mn, nullptr,
+                           c->slo, c->shi);
+        HIPCHK(hipMemcpyAsync(hc + bounds_at(ns), c->slo, (size_t)ns * 16, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        settle(c->retired);
+      }
+      for (int x = 0; x < ns; x++) cnts[x] = lo[ns + x] - lo[x];
       c->ev.flush(c->k_ms, c->k_launch);
     }
   } else {
-    if (graphed && tp) c->tree_free.push_back(tp);     // the level's tree block holds no node
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (gathered && tp) c->tree_free.push_back(tp);    // the level's tree block holds no node
+    if (!once) HIPCHK(hipStreamSynchronize(c->stream));
     c->ev.flush(c->k_ms, c->k_launch);
   }
   // events of this level, per search
+  std::vector<unsigned long long> found_at;
+  std::vector<int> found_by;
+  std::vector<std::vector<int>> found_seq;
+  for (size_t bi = 0; bi < c->binst.size(); bi++) {
+    const BInst &b = c->binst[bi];
+    if (!b.live || b.root_step > c->gstep || (bi < carried.size() && carried[bi])) continue;
+    const unsigned long long *x = &ic[(size_t)b.slot * IC_N];
+    if (x[IC_OVF] || !x[IC_FOUND]) continue;
+    found_at.push_back(x[IC_FIRST]);
+    found_by.push_back((int)bi);
+  }
+  walk_circuits(c, found_at, found_by, G, found_seq);
   const double now = now_s();
   for (size_t bi = 0; bi < c->binst.size(); bi++) {
     BInst &b = c->binst[bi];
@@ -1640,8 +1756,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       evn.result.seconds = now - b.t0;
       set_err("residual coefficients exceed the storage type (int32)");
     } else if (x[IC_FOUND]) {
-      std::vector<int> seq;
-      walk_circuit(c, x[IC_FIRST], G, seq);
+      const std::vector<int> &seq = found_seq[std::find(found_by.begin(), found_by.end(), (int)bi) - found_by.begin()];
       evn.kind = 1;
       evn.result.rc = 0;
       evn.result.len = (int)seq.size();
@@ -2047,7 +2162,7 @@ int chz_open(const char *spec_text, size_t len, const chz_opts *opts, chz_ctx **
     c->device = o.device;
     HIPCHK(hipSetDevice(o.device));
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    chz::StreamScope scope(c->stream);
+    chz::StreamScope scope(c->stream, &c->retired);
     chz::upload_spec(c.get());
   } catch (chz::DeviceError &) {
     return 5;
@@ -2069,7 +2184,7 @@ int chz_run(chz_ctx *c, chz_level_cb cb, void *user, chz_result *out) {
   if (c->opts.mitm || c->opts.table > 0) {   // --mitm takes precedence, as in the reference (src/cheese.cu:1803)
     try {
       HIPCHK(hipSetDevice(c->device));
-      chz::StreamScope scope(c->stream);
+      chz::StreamScope scope(c->stream, &c->retired);
       switch (c->hs.n) {
         case 1: return c->opts.mitm ? chz::run_mitm<1>(c, cb, user, res) : chz::run_table<1>(c, cb, user, res);
         case 2: return c->opts.mitm ? chz::run_mitm<2>(c, cb, user, res) : chz::run_table<2>(c, cb, user, res);
@@ -2166,7 +2281,7 @@ int chz_batch_add(chz_ctx *c, const char *spec_text, size_t len, int depth, int 
 int chz_batch_step(chz_ctx *c) {
   try {
     HIPCHK(hipSetDevice(c->device));
-    chz::StreamScope scope(c->stream);
+    chz::StreamScope scope(c->stream, &c->retired);
     switch (c->hs.n) {
       case 1: chz::batch_step<1>(c); break;
       case 2: chz::batch_step<2>(c); break;
@@ -2188,7 +2303,7 @@ long long chz_batch_frontier(chz_ctx *c, long long max, long long stride, int *p
   long long n = 0;
   try {
     HIPCHK(hipSetDevice(c->device));
-    chz::StreamScope scope(c->stream);
+    chz::StreamScope scope(c->stream, &c->retired);
     HIPCHK(hipStreamSynchronize(c->stream));
     std::vector<int> seq;
     for (long long j = 0; j < c->m && n < max; j += stride, n++) {
@@ -2348,8 +2463,10 @@ void chz_close(chz_ctx *c) {
     c->sk[b].release(); c->sv[b].release();
   }
   c->finst[0].release(); c->finst[1].release(); c->ctl.release(); c->gflag.release();
-  c->scan_tmp.release(); c->d_lo.release(); c->d_hi.release();
+  c->scan_tmp.release();
+  chz::settle(c->retired);
   c->pin.release();
+  c->pin_io.release();
   for (auto &g : c->sgraph) if (g.exec) { (void)hipGraphExecDestroy(g.exec); g.exec = nullptr; }
   c->status.release(); c->kept.release(); c->keys.release(); c->surv_o.release(); c->surv_key.release();
   c->surv_bw.release();

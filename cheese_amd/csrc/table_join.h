@@ -69,7 +69,7 @@ static chz_ctx *aux_context(const chz_ctx *c, const HostSpec &hs, int depth) {
   a->device = c->device;
   for (int b = 0; b < 32; b++) a->sched[b] = c->sched[b];
   HIPCHK(hipStreamCreateWithFlags(&a->stream, hipStreamNonBlocking));
-  StreamScope scope(a->stream);
+  StreamScope scope(a->stream, &a->retired);
   upload_spec(a.get());
   return a.release();
 }
@@ -91,7 +91,7 @@ template <int NQ> static void gt_build(chz_ctx *c, int K, chz_level_cb cb, void 
     t->ks.gk = -1;                              // no residual has exponent -1: no goal
     t->goal_skip = false;
     t->nogoal = true;
-    StreamScope scope(t->stream);
+    StreamScope scope(t->stream, &t->retired);
     {   // level 0: the identity's class
       DBuf<int4> r0;
       DBuf<int> k0;
@@ -305,7 +305,7 @@ template <int NQ> static int run_mitm(chz_ctx *c, chz_level_cb cb, void *user, c
   auto finish = [&](int rc) {
     batch_clear(c);
     {
-      StreamScope sb(bk->stream);
+      StreamScope sb(bk->stream, &bk->retired);
       batch_clear(bk);
       for (auto &l : blev) { l->res.release(); l->pk.release(); }
       chz_close(bk);
@@ -316,7 +316,7 @@ template <int NQ> static int run_mitm(chz_ctx *c, chz_level_cb cb, void *user, c
   try {
     if (const int rc = batch_add_parsed(c, hs, D, 0)) return finish(rc);
     {
-      StreamScope sb(bk->stream);
+      StreamScope sb(bk->stream, &bk->retired);
       if (const int rc = batch_add_parsed(bk, hb, D, 0)) return finish(rc);
     }
     int a = 0, b = 0;
@@ -325,7 +325,7 @@ template <int NQ> static int run_mitm(chz_ctx *c, chz_level_cb cb, void *user, c
     while (a + b < D) {
       const bool fwd = bdead || nfa <= nbb;
       chz_ctx *x = fwd ? c : bk;
-      StreamScope sx(x->stream);
+      StreamScope sx(x->stream, &x->retired);
       batch_step<NQ>(x);
       bool dead = false;
       while (!x->events.empty()) {
@@ -382,7 +382,7 @@ template <int NQ> static int run_mitm(chz_ctx *c, chz_level_cb cb, void *user, c
       res->seconds = now_s() - t0;
       return 1;
     }
-    StreamScope sc(c->stream);
+    StreamScope sc(c->stream, &c->retired);
     const long long nf = c->m;                        // forward level a (a >= 1: the forward side moves first)
     gt_add_level<NQ>(c->ks, F, c->res[c->cur].p, c->pk[c->cur].p, nullptr, nullptr, nf, c->stream);
     DBuf<int4> dU;
