@@ -79,12 +79,14 @@ __global__ __launch_bounds__(1024) void k_scan_one_block(unsigned long long *v, 
 
 // write(x, position) for the flagged items of the tile at t0, in order, positions from pos0; returns their number.  One
 // scan over the (item, wave) counts places the whole tile: with a block scan per item, a tile's 32 barriers were most of
-// a small level's compaction (15 us for 6 tiles).
+// a small level's compaction (15 us for 6 tiles).  The items' offsets go through LDS, so that the writes, a few items a
+// thread, have their loads in flight together.
 template <typename F, typename W>
 __device__ __forceinline__ uint32_t tile_compact(F f, long long t0, long long n, unsigned long long pos0, W write) {
   constexpr int NW = CT_THREADS / 64;
   static_assert(CT_ITEMS * NW == 64, "the counts are scanned by one wave");
   __shared__ uint32_t ws[65];
+  __shared__ uint16_t at[CT_TILE];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint32_t m = tile_flags(f, t0, n);
 #pragma unroll
@@ -109,9 +111,12 @@ __device__ __forceinline__ uint32_t tile_compact(F f, long long t0, long long n,
   for (int i = 0; i < CT_ITEMS; i++) {
     const bool fl = (m >> i) & 1u;
     const uint64_t b = __ballot(fl);
-    if (fl) write(t0 + (long long)i * CT_THREADS + threadIdx.x, pos0 + ws[i * NW + w] + __popcll(b & ((1ull << lane) - 1)));
+    if (fl) at[ws[i * NW + w] + __popcll(b & ((1ull << lane) - 1))] = (uint16_t)(i * CT_THREADS + threadIdx.x);
   }
-  return ws[64];
+  __syncthreads();
+  const uint32_t c = ws[64];
+  for (uint32_t j = threadIdx.x; j < c; j += CT_THREADS) write(t0 + at[j], pos0 + j);
+  return c;
 }
 
 // Sum of v[0..n) over a block of CT_THREADS threads: the tiles before a block's own, where the counts of at most
@@ -165,13 +170,12 @@ __attribute__((unused)) __global__ __launch_bounds__(256) void k_run_starts(cons
   const long long tile = 256ll * RH_ITEMS;
   for (long long t0 = (long long)blockIdx.x * tile; t0 < n; t0 += (long long)gridDim.x * tile) {
     uint32_t mask = 0;
+    // (indices clamped, not branched on: all loads are in flight together)
+#pragma unroll
     for (int it = 0; it < RH_ITEMS; it++) {
-      const long long i = t0 + it * 256ll + tid;
-      if (i < n) {
-        const uint32_t ki = k[i];
-        const bool head = i == 0 || k[i - 1] != ki;
-        if (head && i + 1 < n && k[i + 1] == ki) mask |= 1u << it;
-      }
+      const long long i = t0 + it * 256ll + tid, x = i < n ? i : n - 1;
+      const uint32_t ki = k[x], kp = k[x > 0 ? x - 1 : 0], kn = k[x + 1 < n ? x + 1 : x];
+      if (i < n && (i == 0 || kp != ki) && i + 1 < n && kn == ki) mask |= 1u << it;
     }
     const uint32_t c = (uint32_t)__popc(mask);
     uint32_t x = c;                                  // inclusive scan of the starts over the wave
@@ -277,61 +281,82 @@ __attribute__((unused)) __global__ __launch_bounds__(SS_THREADS) void k_sort_sma
 }
 
 // ------------------------------------------------------------------------------------------------------
-// LSD radix sort of (u32 key, u32 value) pairs, 8-bit digits, stable: tiles of 256 threads x 8 rounds
-constexpr int RS_THREADS = 256, RS_ROUNDS = 8, RS_TILE = RS_THREADS * RS_ROUNDS;
+// LSD radix sort of (u32 key, u32 value) pairs, 8-bit digits, stable: tiles of 1024 threads x 2 rounds.  (With 256 threads
+// x 8 rounds a tile's scatter was a chain of 24 barriers, which is what a sort of a few tiles takes: 12 us, here 7.)
+constexpr int RS_THREADS = 1024, RS_ROUNDS = 2, RS_TILE = RS_THREADS * RS_ROUNDS;
+
+// counts of this tile's digits in h (256, shared)
+__device__ __forceinline__ void radix_tile_counts(const uint32_t *keys, long long n, int shift, unsigned int *h) {
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
+  __syncthreads();
+  const long long t0 = (long long)blockIdx.x * RS_TILE;
+#pragma unroll
+  for (int r = 0; r < RS_ROUNDS; r++) {
+    const long long x = t0 + (long long)r * RS_THREADS + threadIdx.x;
+    if (x < n) atomicAdd(&h[(keys[x] >> shift) & 255], 1u);
+  }
+  __syncthreads();
+}
 
 __global__ __launch_bounds__(RS_THREADS) void k_radix_hist(const uint32_t *keys, long long n, int shift,
                                                            unsigned long long *hist, long long nblocks,
                                                            const unsigned long long *nd = nullptr) {
   n = dev_n(n, nd);
   __shared__ unsigned int h[256];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  const long long t0 = (long long)blockIdx.x * RS_TILE;
-  for (int r = 0; r < RS_ROUNDS; r++) {
-    const long long x = t0 + (long long)r * RS_THREADS + threadIdx.x;
-    if (x < n) atomicAdd(&h[(keys[x] >> shift) & 255], 1u);
-  }
-  __syncthreads();
-  hist[(long long)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+  radix_tile_counts(keys, n, shift, h);
+  if (threadIdx.x < 256) hist[(long long)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
 // this block's tile of (key, value) pairs placed from base[d], the first output position of digit d for the tile
 // (shared; advanced as the rounds go)
 __device__ __forceinline__ void radix_scatter_tile(const uint32_t *kin, const uint32_t *vin, long long n, int shift,
                                                    unsigned long long *base, uint32_t *kout, uint32_t *vout) {
-  __shared__ unsigned int wc[RS_THREADS / 64][256];
+  constexpr int NW = RS_THREADS / 64;
+  __shared__ uint16_t wc[RS_ROUNDS][NW][256];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  for (int k = 0; k < RS_THREADS / 64; k++) wc[k][tid] = 0;
-  __syncthreads();
+  for (int k = tid; k < RS_ROUNDS * NW * 128; k += RS_THREADS) ((uint32_t *)wc)[k] = 0;
   const long long t0 = (long long)blockIdx.x * RS_TILE;
+  uint32_t key[RS_ROUNDS], val[RS_ROUNDS];
+  int rank[RS_ROUNDS];
+#pragma unroll
   for (int r = 0; r < RS_ROUNDS; r++) {
     const long long x = t0 + (long long)r * RS_THREADS + tid;
-    const bool valid = x < n;
-    const uint32_t key = valid ? kin[x] : 0u;
-    const uint32_t val = valid ? vin[x] : 0u;
-    const int dg = (key >> shift) & 255;
+    key[r] = x < n ? kin[x] : 0u;
+    val[r] = x < n ? vin[x] : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ROUNDS; r++) {
+    const bool valid = t0 + (long long)r * RS_THREADS + tid < n;
+    const int dg = (key[r] >> shift) & 255;
     uint64_t peers = __ballot(valid);
 #pragma unroll
     for (int b = 0; b < 8; b++) {
       const uint64_t bb = __ballot((dg >> b) & 1);
       peers &= ((dg >> b) & 1) ? bb : ~bb;
     }
-    const int rank = __popcll(peers & ((1ull << lane) - 1));
-    if (valid && rank == 0) wc[w][dg] = __popcll(peers);
-    __syncthreads();
-    unsigned int before = 0;
-    if (valid) for (int k = 0; k < w; k++) before += wc[k][dg];
-    if (valid) {
-      const unsigned long long p = base[dg] + before + rank;
-      kout[p] = key;
-      vout[p] = val;
+    rank[r] = __popcll(peers & ((1ull << lane) - 1));
+    if (valid && rank[r] == 0) wc[r][w][dg] = (uint16_t)__popcll(peers);
+  }
+  __syncthreads();
+  // the (round, wave) counts of a digit become offsets from its base
+  if (tid < 256) {
+    uint32_t o = 0;
+    for (int k = 0; k < RS_ROUNDS * NW; k++) {
+      uint16_t &c = (&wc[0][0][0])[k * 256 + tid];
+      const uint32_t v = c;
+      c = (uint16_t)o;
+      o += v;
     }
-    __syncthreads();
-    unsigned int tot = 0;
-    for (int k = 0; k < RS_THREADS / 64; k++) { tot += wc[k][tid]; wc[k][tid] = 0; }
-    base[tid] += tot;
-    __syncthreads();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ROUNDS; r++) {
+    if (t0 + (long long)r * RS_THREADS + tid >= n) continue;
+    const int dg = (key[r] >> shift) & 255;
+    const unsigned long long p = base[dg] + wc[r][w][dg] + rank[r];
+    kout[p] = key[r];
+    vout[p] = val[r];
   }
 }
 
@@ -341,7 +366,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(const uint32_t *ki
                                                               const unsigned long long *nd = nullptr) {
   n = dev_n(n, nd);
   __shared__ unsigned long long base[256];
-  base[threadIdx.x] = hist[(long long)threadIdx.x * nblocks + blockIdx.x];
+  if (threadIdx.x < 256) base[threadIdx.x] = hist[(long long)threadIdx.x * nblocks + blockIdx.x];
   radix_scatter_tile(kin, vin, n, shift, base, kout, vout);
 }
 
@@ -355,15 +380,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_count(const uint32_t *keys
                                                             uint32_t *cnt, const unsigned long long *nd = nullptr) {
   n = dev_n(n, nd);
   __shared__ unsigned int h[256];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  const long long t0 = (long long)blockIdx.x * RS_TILE;
-  for (int r = 0; r < RS_ROUNDS; r++) {
-    const long long x = t0 + (long long)r * RS_THREADS + threadIdx.x;
-    if (x < n) atomicAdd(&h[(keys[x] >> shift) & 255], 1u);
-  }
-  __syncthreads();
-  cnt[(long long)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+  radix_tile_counts(keys, n, shift, h);
+  if (threadIdx.x < 256) cnt[(long long)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
 }
 
 __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter_direct(const uint32_t *kin, const uint32_t *vin,
@@ -372,38 +390,47 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter_direct(const uint3
                                                                      uint32_t *vout,
                                                                      const unsigned long long *nd = nullptr) {
   n = dev_n(n, nd);
+  // the tiles that hold no element place nothing (launches sized for a capacity)
+  if ((long long)blockIdx.x * RS_TILE >= n) return;
+  const long long used = (n + RS_TILE - 1) / RS_TILE;
+  if (used < nblocks) nblocks = used;
+  constexpr int Q = RS_THREADS / 256;
   __shared__ unsigned long long base[256];
-  __shared__ unsigned long long wsum[RS_THREADS / 64];
-  const int d = threadIdx.x, lane = d & 63, w = d >> 6;
-  // digit d: its count over all tiles and over the tiles before this one (coalesced rows of 256 counts)
-  unsigned long long tot = 0, below = 0;
+  __shared__ uint32_t stot[Q][256], sbel[Q][256];
+  __shared__ uint32_t wsum[4];
+  const int d = threadIdx.x & 255, qq = threadIdx.x >> 8, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  // digit d: its count over all tiles and over the tiles before this one (coalesced rows of 256 counts), every Q-th tile
+  uint32_t tot = 0, below = 0;
   const long long me = blockIdx.x;
-  long long t = 0;
-  for (; t + 4 <= nblocks; t += 4) {
-    const uint32_t c0 = cnt[t * 256 + d], c1 = cnt[(t + 1) * 256 + d], c2 = cnt[(t + 2) * 256 + d],
-                   c3 = cnt[(t + 3) * 256 + d];
-    tot += (unsigned long long)c0 + c1 + c2 + c3;
-    below += (t < me ? c0 : 0u) + (t + 1 < me ? c1 : 0u) + (t + 2 < me ? c2 : 0u) + (t + 3 < me ? c3 : 0u);
-  }
-  for (; t < nblocks; t++) {
+#pragma unroll 4
+  for (long long t = qq; t < nblocks; t += Q) {
     const uint32_t c = cnt[t * 256 + d];
     tot += c;
-    if (t < me) below += c;
+    below += t < me ? c : 0u;
   }
+  stot[qq][d] = tot;
+  sbel[qq][d] = below;
+  __syncthreads();
   // exclusive scan of the digit totals over the 256 digits
-  unsigned long long inc = tot;
+  uint32_t inc = 0;
+  if (threadIdx.x < 256) {
+    tot = below = 0;
+    for (int k = 0; k < Q; k++) { tot += stot[k][d]; below += sbel[k][d]; }
+    inc = tot;
 #pragma unroll
-  for (int k = 1; k < 64; k <<= 1) {
-    const unsigned long long y = __shfl_up(inc, k, 64);
-    if (lane >= k) inc += y;
+    for (int k = 1; k < 64; k <<= 1) {
+      const uint32_t y = __shfl_up(inc, k, 64);
+      if (lane >= k) inc += y;
+    }
+    if (lane == 63) wsum[w] = inc;
   }
-  if (lane == 63) wsum[w] = inc;
   __syncthreads();
-  unsigned long long off = 0;
-  for (int k = 0; k < w; k++) off += wsum[k];
-  base[d] = off + inc - tot + below;
-  __syncthreads();
-  radix_scatter_tile(kin, vin, n, shift, base, kout, vout);
+  if (threadIdx.x < 256) {
+    uint32_t off = 0;
+    for (int k = 0; k < w; k++) off += wsum[k];
+    base[d] = (unsigned long long)off + inc - tot + below;
+  }
+  radix_scatter_tile(kin, vin, n, shift, base, kout, vout);     // (its first barrier orders base)
 }
 
 

@@ -1350,7 +1350,9 @@ constexpr long long STEP_CAP = 1024;
 // budget 9: 0.86 ms against 1.00 ms with captured steps, budget 12: 8.34 ms against 8.44 ms), while in the server
 // they lower the latency tail.
 constexpr bool kStepGraphs = true;
-constexpr long long ONCE_NCC = 1 << 16;
+// Levels launched for all their children at once (below): their next frontier's room, E entries a child, is bounded by
+// this many bytes (64K children of 3 qubits, 256K of 2)
+constexpr long long ONCE_BYTES = 64ll << 20;
 constexpr int STEP_BUCKET = 10;    // the schedule of the 1,024-parent bucket drives the captured expansion
 
 template <int NQ>
@@ -1527,7 +1529,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   const bool alone = c->pending.empty() && chz_batch_live(c) == 1;
   // levels of few children need the host for nothing between their expansion and the next frontier: launched for all
   // children of the level, with one synchronisation and one copy at the end
-  once = !c->tuning && !c->gt_filter && c->opts.dedupe && c->pending.empty() && ma == m && ma <= chunk && ma * G <= ONCE_NCC;
+  once = !c->tuning && !c->gt_filter && c->opts.dedupe && c->pending.empty() && ma == m && ma <= chunk && ma * G * E * 16 <= ONCE_BYTES;
   const long long maxcc = std::min<long long>(chunk, std::max<long long>(ma, 1)) * G;
   if (once) level_room<NQ>(c, nxt, maxcc, maxcc, tp, tg);
 
