@@ -39,7 +39,6 @@ struct KSpec {                                 // device view of a spec (kernel 
   int ncx;                                     // cx table entries
   int cut1;                                    // every cut is of one qubit with radix 3, and CSRC_MAX hold them all
   int cutmask[16], cutsize[16], rad[16];
-  uint32_t wm[4];                              // Montgomery constants w^i * 2^32 mod p, i = 0..3
   const DevGate *gates;
   const uint8_t *bad2;                         // G x G
   const uint32_t *bad3;                        // bits over G^3
@@ -205,22 +204,37 @@ __device__ __forceinline__ uint32_t mont_mul2(uint32_t a, uint32_t b, uint32_t c
 }
 __device__ __forceinline__ uint32_t fp_sub(uint32_t a, uint32_t b) { return a >= b ? a - b : a + P_MOD - b; }
 __device__ __forceinline__ uint32_t fp_lift(int v) { return v < 0 ? (uint32_t)(v + 3 * (int64_t)P_MOD) : (uint32_t)v; }
+// Montgomery images of w^i, i = 0..3: w = 3^((p - 1) / 8) mod p, times 2^32
+struct FpW { uint32_t m[4]; };
+constexpr FpW fp_w() {
+  uint64_t w = 1, b = 3, e = (P_MOD - 1) / 8, x = (1ull << 32) % P_MOD;
+  while (e) {
+    if (e & 1) w = w * b % P_MOD;
+    b = b * b % P_MOD;
+    e >>= 1;
+  }
+  FpW o{};
+  for (int i = 0; i < 4; i++) { o.m[i] = (uint32_t)x; x = x * w % P_MOD; }
+  return o;
+}
 // image of a + b w + c w^2 + d w^3 in F_p, coefficients below p in magnitude: four products, one reduction
-__device__ __forceinline__ uint32_t fp_of_small(int4 v, const uint32_t *wm) {
+__device__ __forceinline__ uint32_t fp_of_small(int4 v) {
+  constexpr FpW wm = fp_w();
   auto lift = [](int x) { return (uint32_t)(x < 0 ? x + (int)P_MOD : x); };
-  const uint64_t t = (uint64_t)lift(v.x) * wm[0] + (uint64_t)lift(v.y) * wm[1] + (uint64_t)lift(v.z) * wm[2] +
-                     (uint64_t)lift(v.w) * wm[3];                    // < 4 p^2 < 2^62
+  const uint64_t t = (uint64_t)lift(v.x) * wm.m[0] + (uint64_t)lift(v.y) * wm.m[1] + (uint64_t)lift(v.z) * wm.m[2] +
+                     (uint64_t)lift(v.w) * wm.m[3];                    // < 4 p^2 < 2^62
   const uint32_t m = (uint32_t)t * P_NINV;
   const uint32_t r = (uint32_t)((t + (uint64_t)m * P_MOD) >> 32);    // < 4 p^2 / 2^32 + p < 2 p
   return r >= P_MOD ? r - P_MOD : r;
 }
 // image of a + b w + c w^2 + d w^3 in F_p
-__device__ __forceinline__ uint32_t fp_of(int4 v, const uint32_t *wm) {
-  uint32_t s = mont_mul(fp_lift(v.x), wm[0]) + mont_mul(fp_lift(v.y), wm[1]);
+__device__ __forceinline__ uint32_t fp_of(int4 v) {
+  constexpr FpW wm = fp_w();
+  uint32_t s = mont_mul(fp_lift(v.x), wm.m[0]) + mont_mul(fp_lift(v.y), wm.m[1]);
   s = s >= P_MOD ? s - P_MOD : s;
-  s += mont_mul(fp_lift(v.z), wm[2]);
+  s += mont_mul(fp_lift(v.z), wm.m[2]);
   s = s >= P_MOD ? s - P_MOD : s;
-  s += mont_mul(fp_lift(v.w), wm[3]);
+  s += mont_mul(fp_lift(v.w), wm.m[3]);
   return s >= P_MOD ? s - P_MOD : s;
 }
 

@@ -108,6 +108,12 @@ static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
 // term is then two two-word reads, where rotating a coefficient vector in registers took some 30 instructions.  The odd
 // stride keeps the lanes of a row on different banks.
 constexpr int RING = 7;
+// the identity's nonzero entries
+template <int NQ> __host__ __device__ constexpr uint64_t ident_mask() {
+  uint64_t m = 0;
+  for (int i = 0; i < 1 << NQ; i++) m |= 1ull << (i * (1 << NQ) + i);
+  return m;
+}
 template <int NQ> struct Parent {
   int *e;                          // the group's entries
   int c;                           // this lane's column
@@ -139,7 +145,11 @@ template <int NQ> __device__ __forceinline__ uint64_t node_key(int4 s, int k, in
   }
 }
 
-template <int NQ, int WPE>
+// STD: the kernel of the specs and levels that std_level accepts (bounds on, the identity as the goal, one table of
+// one-qubit cuts in LDS, unit gates of at most two terms a column, coefficients and exponents that no child of the level
+// can take out of the fast forms).  It leaves out every other form; carried along, they cost the child loop registers,
+// spilled scalars and branches (budget-14 proof 104.4 ms without this kernel, 86.4 with it).
+template <int NQ, int WPE, bool STD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_level(KSpec sp, ExpandArgs a,
                                                                                          long long np) {
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
@@ -157,6 +167,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   const long long wave = wave_index();
   const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
   const int G = sp.G;
+  const bool lite = !STD && sp.lite, bounds = STD || sp.standard || sp.lite;
   // per-instance status tallies: one LDS counter per status value and group, bumped by the group's leader lane
   // and flushed when the group's instance changes (32-bit: one wave's share of a launch is far below 2^32
   // children).  Held in registers they cost two vector or scalar instructions per tally and child, and the
@@ -204,12 +215,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const int4 S = a.res[pi * E + le];
     const int pk = wuni<NQ>(a.pk[pi]), g1 = wuni<NQ>((int)a.g1[pi]), g2 = wuni<NQ>((int)a.g2[pi]);
     const uint32_t pbw = (uint32_t)wuni<NQ>((int)a.pb[pi]);
-    const uint32_t mag = zmag(S);
-    const bool small = gall<GS>(mag < (1u << 28));
+    const uint32_t mag = STD ? 0u : zmag(S);
+    const bool small = STD || gall<GS>(mag < (1u << 28));
     // A search whose circuit is found at this level ends with it: its parents without a goal child (no
     // BW_GOAL) are passed over once their coefficients rule out an overflowing child.  Goal children come only
     // from BW_GOAL parents, so the level's found count, first circuit and overflow test are unchanged.
-    if (a.gflag && !(pbw & BW_GOAL) && wuni<NQ>((int)a.gflag[inst]) != 0 && gall<GS>(mag <= sp.maglim)) {
+    if (a.gflag && !(pbw & BW_GOAL) && wuni<NQ>((int)a.gflag[inst]) != 0 && (STD || gall<GS>(mag <= sp.maglim))) {
       for (int g = gbeg + le; g < gend; g += GS) a.status[pl * G + g] = ST_DEAD;
       continue;
     }
@@ -217,7 +228,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     P.put(le, S);
     __builtin_amdgcn_wave_barrier();
     // a child's cut needs can be bounded from its parent's
-    const bool cutlow = !sp.lite && sp.cx_mono && (pbw & BW_CUTS);
+    const bool cutlow = !lite && (STD || sp.cx_mono) && (pbw & BW_CUTS);
     const uint32_t pneeds = (pbw & BW_NEEDS) >> 8;
     // T bounds of this parent's children per T-bound class: tc_ok bit set when one is known, tc_ex when it is the
     // exact bound, else it is a lower bound (a transform stopped once the child was dead)
@@ -231,7 +242,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     // can overflow (which would be reported) and the goal's own bounds are 0 (a goal child is never over its budget).
     // On the budget-14 proof the expansion takes 111 ms instead of 139.  Where a parent's candidates are split over
     // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.
-    const bool pre = sp.pre && gsplit <= PRE_SPLIT && gall<GS>(mag <= sp.maglim);
+    const bool pre = gsplit <= PRE_SPLIT && (STD || (sp.pre && gall<GS>(mag <= sp.maglim)));
     const bool tparent = (pbw & BW_TUNK) != BW_TUNK;
     // H on qubit q pairs the columns c and c ^ 2^q as their sum and difference over sqrt2: the exponent rises by one,
     // less one if sqrt2 divides every sum (the parities of a + c and b + d agree in each pair), less another if 2 does
@@ -246,7 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         if (!(differ(ba) | differ(bb) | differ(bc) | differ(bd))) he |= 16 << q;
       }
     }
-    const int pq = !sp.lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S)), N - 1) : 0;
+    const int pq = !lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S)), N - 1) : 0;
     uint64_t w2m = 0, w3m = 0, dm = 0;
     int lim = 1 << 30, tcl = -1;                 // n = 3: candidate `lane`'s largest T bound by these bounds; its T class
     CutLow cl{0, 0, 0};                          // n = 3: candidate `lane`'s least cut needs
@@ -264,7 +275,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
       }
       if ((pre || (NQ == 3 && cutlow)) && g < G) {
         const uint4 hd = tb.head[g];
-        const CutLow lo = cutlow ? cut_low(sp, scx, pneeds, hd.y) : CutLow{0, 0, 0};
+        const CutLow lo = cutlow ? cut_low<NQ, STD>(sp, scx, pneeds, hd.y) : CutLow{0, 0, 0};
         if constexpr (NQ == 3) cl = lo;
         if (pre) {
           const uint32_t w = hd.x;
@@ -290,8 +301,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     w3m &= range & ~w2m;
     const uint64_t evalm = range & ~w2m & ~w3m;
     dm &= evalm;
-    uint64_t todo = evalm & ~dm, alivem = 0, foundm = 0, ovfm = 0;      // status of the children that are formed: else dead
-    n_pre += (uint32_t)__popcll(dm);
+    uint64_t todo = evalm & ~dm, alivem = 0, rarem = 0;      // children alive; found or overflowed (their status is written)
+    uint32_t settled = (uint32_t)__popcll(dm);
+    // n = 3: the status of candidate `lane` as far as the windows decide it
+    int wst = ST_DEAD;
+    const uint32_t nw2 = (uint32_t)__popcll(w2m), nw3 = (uint32_t)__popcll(w3m), nev = (uint32_t)__popcll(evalm);
+    if constexpr (NQ == 3) wst = (w2m >> lane) & 1 ? ST_W2 : (w3m >> lane) & 1 ? ST_W3 : ST_DEAD;
     while (todo) {
       const int g = wuni<NQ>(__ffsll((long long)todo) - 1);
       todo &= todo - 1;
@@ -305,7 +320,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         int4 s;
         bool of = false;
         int k = pk + wuni<NQ>((int)hv.z);
-        const bool fast = (hw & 1u) && small;
+        const bool fast = STD || ((hw & 1u) && small);
         if (fast) {
           const uint32_t d = tb.term[g * 64 + le];
           const int4 u = P.turned(d & 63u);
@@ -361,14 +376,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
             while (k > 0 && gall<GS>(zhalf(s))) { s = zdown(s); k--; }
           const uint64_t nzb = gballot<GS>(!zzero(s));
           // the goal's entries are read only for a child with the goal's exponent and nonzero pattern
-          if (k == sp.gk && nzb == sp.goalnz && gall<GS>(zeq(s, sp.goal[le]))) stt = ST_FOUND;
+          if (STD ? k == 0 && nzb == ident_mask<NQ>() && gall<GS>(s.x == (r == c) && !(s.y | s.z | s.w))
+                  : k == sp.gk && nzb == sp.goalnz && gall<GS>(zeq(s, sp.goal[le])))
+            stt = ST_FOUND;
           else {
             bool alive = true;
-            if (sp.standard || sp.lite) {
+            if (bounds) {
               int hh, supp = 0, c2 = 0;
-              if (sp.lite) hh = k;
+              if (lite) hh = k;
               else {
-                n_cheap++;
                 const int hs = h_struct<NQ>(nzb), gm = (int)((hx >> 8) & 7u);
                 hh = k > hs ? k : hs;
                 supp = __popc((pq & ~gm) | support_mask<NQ>(s, le, nzb, gm));
@@ -393,17 +409,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               CutLow lo{0, 0, 0};
               if (cutlow) {
                 if constexpr (NQ == 3) lo = CutLow{gget<GS>(cl.low, g), (int)gget<GS>((uint32_t)cl.idx, g), (int)gget<GS>((uint32_t)cl.c2, g)};
-                else lo = cut_low(sp, scx, pneeds, hv.y);
+                else lo = cut_low<NQ, STD>(sp, scx, pneeds, hv.y);
               }
               // alive exactly when T / tdiv, rounded up, is at most t_budget: T <= t_budget * tdiv
               if (T > t_budget(hh, lo.c2, supp, rem) * sp.tdiv) alive = false;
               else {
-                if (!sp.lite) {
+                if (!lite) {
                   uint32_t needs = pneeds;
                   const uint32_t keepc = (pbw & BW_CUTS) ? hw >> 8 : 0u;
-                  const CutStop cst{cutlow && sp.have_table, lo.low, lo.idx, T, hh, supp, rem};
-                  c2 = cx_bound<NQ>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts);
-                  bw = (needs << 8 & ~BW_CUTS) | (sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
+                  const CutStop cst{cutlow && (STD || sp.have_table), lo.low, lo.idx, T, hh, supp, rem};
+                  c2 = cx_bound<NQ, STD>(s, le, sp, scx, scsrc, keepc, small, cst, needs, n_cuts);
+                  bw = (needs << 8 & ~BW_CUTS) | (STD || sp.ncuts <= BW_MAXCUTS ? BW_CUTS : 0u) | BW_TUNK;
                 }
                 const int tmax = t_budget(hh, c2, supp, rem) * sp.tdiv;
                 if (T > tmax) alive = false;
@@ -412,7 +428,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                   alive = true;
                 } else if (!texact) {
                   n_t++;
-                  if (NQ + k <= 16) {
+                  if (STD || NQ + k <= 16) {
                     // the f = 0 part, then the flip-pair passes (odd first) while the lower bound leaves the child
                     // alive: at T bound T it is alive exactly when T <= tmax
                     uint32_t np = 0;
@@ -431,7 +447,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
                       const uint64_t sib = gballot<GS>(tcl == tc && T > lim) & todo;
                       if (sib) {
                         todo &= ~sib;
-                        n_pre += (uint32_t)__popcll(sib);
+                        settled += (uint32_t)__popcll(sib);
                       }
                     }
                   }
@@ -441,11 +457,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               if (alive && texact && T < (int)BW_TUNK) bw = (bw & ~BW_TUNK) | (uint32_t)T;
             }
             if (alive && keep) {
-              n_keys++;
               if constexpr (NQ == 3) {
                 int image = 0;
                 key = class_key3(s, k, lane, spos, tb.kt.adm, cjm, image);
-                if (sp.ncuts <= BW_IMAGE_CUTS) bw |= (uint32_t)image << BW_IMAGE;
+                if (STD || sp.ncuts <= BW_IMAGE_CUTS) bw |= (uint32_t)image << BW_IMAGE;
               } else {
                 key = class_key<NQ>(s, k, le, sp);
               }
@@ -455,36 +470,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
           }
         }
       }
-      const uint64_t me = 1ull << g;
-      if (stt == ST_ALIVE) alivem |= me;
-      if (stt == ST_FOUND) foundm |= me;
-      if (stt == ST_OVF) ovfm |= me;
-      if (stt == ST_ALIVE && keep && le == 0) { a.keys[pl * G + g] = key; a.info[pl * G + g] = bw; }
+      if (stt == ST_ALIVE) {
+        alivem |= 1ull << g;
+        if (keep && le == 0) { a.keys[pl * G + g] = key; a.info[pl * G + g] = bw; }
+      } else if (stt != ST_DEAD) {
+        rarem |= 1ull << g;
+        if (le == 0) {
+          a.status[pl * G + g] = stt;
+          atomicAdd(&tl[stt], 1u);
+          if (stt == ST_FOUND) atomicMin(&icnt[(size_t)inst * IC_N + IC_FIRST], (unsigned long long)((a.off + pl) * G + g));
+        }
+      }
     }
     // the children's status, one candidate per lane, and their tallies
     for (int b0 = 0; b0 < G; b0 += GS) {
       const int g = b0 + le;
-      if (g < G && ((range >> g) & 1))
-        a.status[pl * G + g] = (w2m >> g) & 1      ? ST_W2
-                               : (w3m >> g) & 1    ? ST_W3
-                               : (alivem >> g) & 1 ? (keep ? ST_ALIVE : ST_LAST)
-                               : (foundm >> g) & 1 ? ST_FOUND
-                               : (ovfm >> g) & 1   ? ST_OVF
-                                                   : ST_DEAD;
+      const bool mine = g >= gbeg && g < gend && !((rarem >> g) & 1);
+      const int st_w = NQ == 3 ? wst : (w2m >> g) & 1 ? ST_W2 : (w3m >> g) & 1 ? ST_W3 : ST_DEAD;
+      if (mine) a.status[pl * G + g] = (uint8_t)((alivem >> g) & 1 ? (keep ? ST_ALIVE : ST_LAST) : st_w);
     }
-    n_eval += (uint32_t)__popcll(evalm);
+    const uint32_t nal = (uint32_t)__popcll(alivem), nrare = (uint32_t)__popcll(rarem);
+    n_eval += nev;
+    n_pre += settled;
+    if (!lite && bounds) n_cheap += nev - settled - nrare;
+    if (keep) n_keys += nal;
     if (le == 0) {
-      if (w2m) atomicAdd(&tl[ST_W2], (uint32_t)__popcll(w2m));
-      if (w3m) atomicAdd(&tl[ST_W3], (uint32_t)__popcll(w3m));
-      if (alivem) atomicAdd(&tl[ST_ALIVE], (uint32_t)__popcll(alivem));
-      const uint64_t dead = evalm & ~(alivem | foundm | ovfm);
-      if (dead) atomicAdd(&tl[ST_DEAD], (uint32_t)__popcll(dead));
-      if (ovfm) atomicAdd(&tl[ST_OVF], (uint32_t)__popcll(ovfm));
-      if (foundm) {
-        atomicAdd(&tl[ST_FOUND], (uint32_t)__popcll(foundm));
-        atomicMin(&icnt[(size_t)inst * IC_N + IC_FIRST],
-                  (unsigned long long)((a.off + pl) * G + __ffsll((long long)foundm) - 1));
-      }
+      if (nw2) atomicAdd(&tl[ST_W2], nw2);
+      if (nw3) atomicAdd(&tl[ST_W3], nw3);
+      if (nal) atomicAdd(&tl[ST_ALIVE], nal);
+      if (const uint32_t dead = nev - nal - nrare) atomicAdd(&tl[ST_DEAD], dead);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -897,6 +911,8 @@ struct BInst {
   bool live = false;
   long long nodes = 0;
   double growth = 0;           // the last level's distinct / parents (0: not known yet)
+  int k = 0;                   // the root's sqrt2 exponent and largest coefficient
+  uint32_t coef = 0;
   double t0 = 0;
 };
 struct Pending {               // a search waiting to join the frontier as a root
@@ -975,6 +991,8 @@ struct chz_ctx {
   double k_stage[6] = {};       // expansion stage counts: residuals, structural bounds, cut ranks, T bounds, keys,
                                 // T-bound passes
   double avg_terms = 1;         // nonzero terms per inverse column, averaged over the candidates
+  bool std_spec = false;        // what the specialised expansion asks of a spec
+  int max_ik = 0;               // the largest sqrt2 exponent of a gate
   bool goal_skip = false;       // every candidate has a goal pre-image: the found-level skip is exact
   // per-level memory planning (chz_batch_set_budget): searches in frontier order; with a budget, a level expands
   // the longest prefix of them whose planned bytes fit, and the rest wait, carried to the next frontier unexpanded
@@ -1284,6 +1302,38 @@ static void prune_tree(chz_ctx *c) {
   }
 }
 
+// Whether the expansion of this frontier's next level may run as the specialised kernel: the spec is one of its kind
+// (std_spec), and by the searches' own roots no parent's coefficients reach 2^28 or the limit of an overflowing child (a
+// sum of two terms at most doubles them), nor any child's exponent the T bound's 16 bits
+static bool std_level(const chz_ctx *c) {
+  if (!c->std_spec) return false;
+  for (const BInst &b : c->binst) {
+    if (!b.live) continue;
+    const int room = b.t + 1;                     // gates from the root to this level's children
+    if (room > 24 || ((uint64_t)b.coef << room) >= std::min<uint64_t>(1u << 28, c->ks.maglim)) return false;
+    // a parent's exponent exceeds the root's by at most a gate's own each; alive, it is within the budget left
+    const int kp = std::min(b.k + b.t * c->max_ik, b.t ? b.depth - b.t : b.k);
+    if (c->ks.n + kp + c->max_ik > 16) return false;
+  }
+  return true;
+}
+template <int NQ> static void launch_level(chz_ctx *c, int var, bool spec, dim3 grid, hipStream_t s, const ExpandArgs &ea, long long m) {
+  const KSpec &ks = c->ks;
+  if constexpr (NQ > 1)
+    if (spec) {
+      switch (var) {
+        case 0: hipLaunchKernelGGL((k_level<NQ, 4, true>), grid, dim3(256), 0, s, ks, ea, m); return;
+        case 2: hipLaunchKernelGGL((k_level<NQ, 6, true>), grid, dim3(256), 0, s, ks, ea, m); return;
+        default: hipLaunchKernelGGL((k_level<NQ, 5, true>), grid, dim3(256), 0, s, ks, ea, m); return;
+      }
+    }
+  switch (var) {
+    case 0: hipLaunchKernelGGL((k_level<NQ, 4, false>), grid, dim3(256), 0, s, ks, ea, m); break;
+    case 2: hipLaunchKernelGGL((k_level<NQ, 6, false>), grid, dim3(256), 0, s, ks, ea, m); break;
+    default: hipLaunchKernelGGL((k_level<NQ, 5, false>), grid, dim3(256), 0, s, ks, ea, m); break;
+  }
+}
+
 // A level of one chunk from its expansion's statuses to the kept survivors' ranks without the host: survivors, sort, exact
 // dedupe, kept ranks, launched for ncc children (dncc: their number on the device) and reading the sizes that come out
 // on the way from the counters.  The buffers hold ncc entries.
@@ -1366,6 +1416,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   const long long mx = ncap + (long long)c->pending.size();
   level_room<NQ>(c, nxt, ncap, mx, tp, tg);
   const chz_ctx::Sched sc = c->sched[STEP_BUCKET];
+  const bool spec = std_level(c);
   const uint32_t *pinst = c->finst[cur].p;
   const std::vector<uintptr_t> key = {
       (uintptr_t)c->res[cur].p, (uintptr_t)c->pk[cur].p, (uintptr_t)c->g1[cur].p, (uintptr_t)c->g2[cur].p,
@@ -1375,7 +1426,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->runs.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
       (uintptr_t)c->sv[0].p, (uintptr_t)c->sv[1].p, (uintptr_t)c->hist.p, (uintptr_t)c->scan_tmp.p,
       (uintptr_t)c->gflag.p, (uintptr_t)ns, (uintptr_t)sc.var, (uintptr_t)sc.cap,
-      (uintptr_t)sc.tw};
+      (uintptr_t)sc.tw, (uintptr_t)spec};
   chz_ctx::StepGraph &sg = c->sgraph[cur];
   if (!sg.exec || sg.key != key) {
     if (sg.exec) { HIPCHK(hipGraphExecDestroy(sg.exec)); sg.exec = nullptr; }
@@ -1389,11 +1440,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
                   c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
                   c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cap * G + CPW - 1) / CPW, sc.cap));
-    switch (sc.var) {
-      case 0: hipLaunchKernelGGL((k_level<NQ, 4>), grid, dim3(256), 0, s, ks, ea, cap); break;
-      case 2: hipLaunchKernelGGL((k_level<NQ, 6>), grid, dim3(256), 0, s, ks, ea, cap); break;
-      default: hipLaunchKernelGGL((k_level<NQ, 5>), grid, dim3(256), 0, s, ks, ea, cap); break;
-    }
+    launch_level<NQ>(c, sc.var, spec, grid, s, ea, cap);
     level_tail<NQ>(c, cur, ncap, dncc, nullptr, false, s);
     hipError_t e = hipGetLastError();
     const hipError_t ec = hipStreamEndCapture(s, &graph);
@@ -1531,6 +1578,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   // children of the level, with one synchronisation and one copy at the end
   once = !c->tuning && !c->gt_filter && c->opts.dedupe && c->pending.empty() && ma == m && ma <= chunk && ma * G * E * 16 <= ONCE_BYTES;
   const long long maxcc = std::min<long long>(chunk, std::max<long long>(ma, 1)) * G;
+  const bool spec = std_level(c);
   if (once) level_room<NQ>(c, nxt, maxcc, maxcc, tp, tg);
 
   c->status.need(maxcc);
@@ -1559,11 +1607,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       HIPCHK(hipEventRecord(te0, c->stream));
     }
     c->ev.begin(K_EXPAND, c->stream);
-    switch (sc.var) {
-      case 0: hipLaunchKernelGGL((k_level<NQ, 4>), grid, dim3(256), 0, c->stream, ks, ea, cm); break;
-      case 2: hipLaunchKernelGGL((k_level<NQ, 6>), grid, dim3(256), 0, c->stream, ks, ea, cm); break;
-      default: hipLaunchKernelGGL((k_level<NQ, 5>), grid, dim3(256), 0, c->stream, ks, ea, cm); break;
-    }
+    launch_level<NQ>(c, sc.var, spec, grid, c->stream, ea, cm);
     c->ev.end(c->stream);
     if (c->tuning) {
       HIPCHK(hipEventRecord(te1, c->stream));
@@ -2031,13 +2075,6 @@ static void upload_spec(chz_ctx *c) {
       }
     }
   }
-  // Montgomery images of w^i: w = 3^((p-1)/8) mod p, times 2^32
-  auto mulm = [](uint64_t a, uint64_t b) { return (a * b) % P_MOD; };
-  uint64_t w = 1, b = 3, e = (P_MOD - 1) / 8;
-  while (e) { if (e & 1) w = mulm(w, b); b = mulm(b, b); e >>= 1; }
-  const uint64_t R = (1ull << 32) % P_MOD;
-  uint64_t wp = 1;
-  for (int i = 0; i < 4; i++) { k.wm[i] = (uint32_t)mulm(wp, R); wp = mulm(wp, w); }
   k.gates = c->d_gates; k.bad2 = c->d_bad2; k.bad3 = c->d_bad3; k.goal = c->d_goal; k.cxtable = c->d_cx;
   k.goalnz = 0;
   for (int i = 0; i < N * N; i++) {
@@ -2051,6 +2088,14 @@ static void upload_spec(chz_ctx *c) {
   for (int y = 0; y < k.nsym && y < 16; y++) k.cjm |= (uint32_t)(c->grp.conj[y] != 0) << y;
   std::vector<SpecTabs> tabs(1);
   build_level_tabs(tabs[0], dg, k, c->grp, s);
+  c->max_ik = 0;
+  bool two_terms = true;
+  for (int g = 0; g < G; g++) {
+    c->max_ik = std::max(c->max_ik, dg[g].ik);
+    two_terms = two_terms && (tabs[0].level.head[g].w & 1u);
+  }
+  c->std_spec = s.standard && !s.lite && k.pre && k.cut1 && k.ncuts == (k.n == 3 ? 3 : 1) && k.n > 1 && k.have_table &&
+                k.cxlds && k.cx_mono && two_terms;
   c->ktab.need(sizeof(SpecTabs));
   chz::copy_sync(c->ktab.p, tabs.data(), sizeof(SpecTabs), hipMemcpyHostToDevice, c->stream);
   k.ktab = (const uint4 *)c->ktab.p;
@@ -2104,7 +2149,9 @@ static int batch_add_parsed(chz_ctx *c, const HostSpec &hs, int depth, int tag) 
   b.t0 = now_s();
   Pending q;
   q.inst = bi;
-  q.k = hs.tk;
+  q.k = b.k = hs.tk;
+  for (const Zq &z : hs.target)
+    for (long long v : {(long long)z.a, (long long)z.b, (long long)z.c, (long long)z.d}) b.coef = std::max(b.coef, (uint32_t)std::llabs(v));
   q.U.resize(E);
   for (int i = 0; i < E; i++) {
     const Zq &z = hs.target[i];

@@ -254,27 +254,31 @@ constexpr int BW_IMAGE = 24, BW_IMAGE_CUTS = 5;
 // others are ranked here.  On return `needs` holds this matrix's packed needs.
 // The cx table is read from the expansion kernel's LDS copy `cxl` when it fits (sp.cxlds): the global table sits
 // behind a vector load on every child's dependency chain.
-__device__ __forceinline__ int cx_at(const KSpec &sp, const uint8_t *cxl, int idx) {
-  return sp.cxlds ? (int)cxl[idx] : sp.cxtable[idx];
+// STD (here and below): the spec is one the expansion's specialised kernel takes (std_spec)
+template <bool STD> __device__ __forceinline__ int cx_at(const KSpec &sp, const uint8_t *cxl, int idx) {
+  return STD || sp.cxlds ? (int)cxl[idx] : sp.cxtable[idx];
 }
+template <int NQ, bool STD> __device__ __forceinline__ int n_cuts_of(const KSpec &sp) { return STD ? (NQ == 3 ? 3 : 1) : sp.ncuts; }
 
 // The least a child's cuts can need, from its parent's packed needs: each need drops by at most the gate's per-cut delta
 // (operator-Schmidt ranks multiply; 7: by any amount).  low: the needs, packed; idx: their place in the cx table; c2: the
 // cut bound there, a lower bound on the child's since the table is non-decreasing in every need.
 struct CutLow { uint32_t low; int idx, c2; };
+template <int NQ, bool STD>
 __device__ __forceinline__ CutLow cut_low(const KSpec &sp, const uint8_t *cxl, uint32_t pneeds, uint32_t cdel) {
   CutLow o{0, 0, 0};
   int mult = 1, mx = 0;
-  for (int i = 0; i < sp.ncuts; i++) {
+#pragma unroll
+  for (int i = 0; i < n_cuts_of<NQ, STD>(sp); i++) {
     const int dl = (int)((cdel >> (3 * i)) & 7u);
     int nd = (int)((pneeds >> (3 * i)) & 7u) - dl;
     nd = dl == 7 || nd < 0 ? 0 : nd;
     o.low |= (uint32_t)nd << (3 * i);
     o.idx += nd * mult;
-    mult *= sp.rad[i];
+    mult *= STD ? 3 : sp.rad[i];
     if (nd > mx) mx = nd;
   }
-  o.c2 = sp.have_table ? cx_at(sp, cxl, o.idx) : mx;
+  o.c2 = STD || sp.have_table ? cx_at<STD>(sp, cxl, o.idx) : mx;
   return o;
 }
 
@@ -305,9 +309,9 @@ template <int NQ> __device__ __forceinline__ int cut_need1(uint32_t v, int le) {
 }
 
 // need of cut i of a matrix with the F_p image fp
-template <int NQ> __device__ __forceinline__ int cut_need(uint32_t fp, int le, const KSpec &sp, const uint8_t *csrc, int i) {
+template <int NQ, bool STD> __device__ __forceinline__ int cut_need(uint32_t fp, int le, const KSpec &sp, const uint8_t *csrc, int i) {
   constexpr int GS = 1 << (2 * NQ);
-  if (sp.cut1) return cut_need1<NQ>((uint32_t)__shfl(fp, (int)csrc[i * GS + le], GS), le);
+  if (STD || sp.cut1) return cut_need1<NQ>((uint32_t)__shfl(fp, (int)csrc[i * GS + le], GS), le);
   const int rad = sp.rad[i], sa = sp.cutsize[i];
   const int R = 1 << (2 * sa);
   int stop = R;
@@ -319,34 +323,36 @@ template <int NQ> __device__ __forceinline__ int cut_need(uint32_t fp, int le, c
   return need > rad - 1 ? rad - 1 : need;
 }
 
-template <int NQ> __device__ __forceinline__ int cx_bound(int4 s, int le, const KSpec &sp, const uint8_t *cxl,
+template <int NQ, bool STD> __device__ __forceinline__ int cx_bound(int4 s, int le, const KSpec &sp, const uint8_t *cxl,
                                                           const uint8_t *csrc, uint32_t keepc, bool small, const CutStop &st,
                                                           uint32_t &needs, uint32_t &ranks) {
   uint32_t fp = 0;
   bool have_fp = false;
+  const int nc = n_cuts_of<NQ, STD>(sp);
   int idx = 0, mult = 1, mx = 0, lo = st.lo;
   uint32_t out = 0;
-  int todo = sp.ncuts - __popc(keepc & ((1u << sp.ncuts) - 1));
-  for (int i = 0; i < sp.ncuts; i++) {
+  int todo = nc - __popc(keepc & ((1u << nc) - 1));
+#pragma unroll 1
+  for (int i = 0; i < nc; i++) {
     int need;
     if ((keepc >> i) & 1) need = (int)((needs >> (3 * i)) & 7u);
     else {
-      if (!have_fp) { fp = small ? fp_of_small(s, sp.wm) : fp_of(s, sp.wm); have_fp = true; }
-      need = cut_need<NQ>(fp, le, sp, csrc, i);
+      if (!have_fp) { fp = STD || small ? fp_of_small(s) : fp_of(s); have_fp = true; }
+      need = cut_need<NQ, STD>(fp, le, sp, csrc, i);
       ranks++;
       if (st.on && --todo > 0) {
         lo += (need - (int)((st.low >> (3 * i)) & 7u)) * mult;
-        const int c = wuni<NQ>(cx_at(sp, cxl, lo));
+        const int c = wuni<NQ>(cx_at<STD>(sp, cxl, lo));
         if (st.T > t_budget(st.h, c, st.supp, st.rem) * sp.tdiv) return c;
       }
     }
     if (i < BW_MAXCUTS) out |= (uint32_t)need << (3 * i);
     idx += need * mult;
-    mult *= sp.cut1 ? 3 : sp.rad[i];
+    mult *= STD || sp.cut1 ? 3 : sp.rad[i];
     if (need > mx) mx = need;
   }
   needs = out;
-  return sp.have_table ? wuni<NQ>(cx_at(sp, cxl, idx)) : mx;
+  return STD || sp.have_table ? wuni<NQ>(cx_at<STD>(sp, cxl, idx)) : mx;
 }
 
 // T lower bound: max over Pauli pairs of 2(n+k) - v(X_ab), all X_ab by one 2-D Walsh-Hadamard transform
