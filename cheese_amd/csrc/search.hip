@@ -59,6 +59,7 @@ struct ExpandArgs {
   uint64_t *keys;           // [ncc] class keys of kept children
   uint32_t *info;           // [ncc] bound words of kept children
   const uint32_t *pb;       // parents' bound words
+  const uint64_t *tm;       // parents' T columns (k_tcols; n = 3, specialised kernel)
   unsigned long long *stage;  // NSTRIPE stripes of the stage counts (ST_N each)
   const uint32_t *pinst;    // instance slot of every parent of the level (null: one instance, slot 0)
   const int *rem;           // per slot: gate budget left after this level's gate (depth - t)
@@ -90,6 +91,7 @@ struct LevelTabs {
   // (the exponent is read off the parent exactly), 24-31 1 + the T-bound class; y: DevGate::cdel; z: DevGate::ik;
   // w: bit 0 the terms above form its children, 1 a permutation of unit entries, 8-23 DevGate::cutloc
   uint4 head[MAXG];
+  uint64_t keep_cols[MAXG];        // n = 3: the parent's columns that a child keeps as one of its own (gate_columns)
   KeyTab kt;                       // n = 3: the class key's choice of symmetries
   uint8_t spos[16 * 64];           // n = 3: position of entry e under symmetry y (y * 64 + e)
   uint8_t scx[CXL_MAX];            // the cx table when it fits (KSpec::cxlds)
@@ -100,6 +102,7 @@ struct LevelTabs {
 struct SpecTabs {
   LevelTabs level;
   uint16_t sdesc[MAXG * 64];
+  uint8_t col_src[MAXG * 64];      // n = 3: gate_columns' src (255: none)
 };
 static_assert(sizeof(LevelTabs) % 16 == 0, "LevelTabs is copied as uint4");
 
@@ -215,6 +218,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const int4 S = a.res[pi * E + le];
     const int pk = wuni<NQ>(a.pk[pi]), g1 = wuni<NQ>((int)a.g1[pi]), g2 = wuni<NQ>((int)a.g2[pi]);
     const uint32_t pbw = (uint32_t)wuni<NQ>((int)a.pb[pi]);
+    const uint64_t tcols = STD && NQ == 3 ? (uint64_t)wuni64<NQ>((long long)a.tm[pi]) : 0ull;
     const uint32_t mag = STD ? 0u : zmag(S);
     const bool small = STD || gall<GS>(mag < (1u << 28));
     // A search whose circuit is found at this level ends with it: its parents without a goal child (no
@@ -261,6 +265,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     uint64_t w2m = 0, w3m = 0, dm = 0;
     int lim = 1 << 30, tcl = -1;                 // n = 3: candidate `lane`'s largest T bound by these bounds; its T class
     CutLow cl{0, 0, 0};                          // n = 3: candidate `lane`'s least cut needs
+    int tlo = 0;                                 // and least T bound
     // window cuts of every candidate of this parent, one candidate per lane, as two bit masks: the candidate
     // loop then tests bits instead of waiting on a table load per child
     for (int b0 = 0; b0 < G; b0 += GS) {
@@ -276,11 +281,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
       if ((pre || (NQ == 3 && cutlow)) && g < G) {
         const uint4 hd = tb.head[g];
         const CutLow lo = cutlow ? cut_low<NQ, STD>(sp, scx, pneeds, hd.y) : CutLow{0, 0, 0};
-        if constexpr (NQ == 3) cl = lo;
+        const int td = (int)(hd.x & 255u), Tp = (int)(pbw & BW_TUNK);
+        // The T bound is the largest exponent of the columns of the residual's Pauli transfer matrix.  A column that the
+        // gate leaves alone (a T on qubit q: those without X on q) and that attains the parent's bound is the child's
+        // too, so the bound cannot fall: 25.9 of 33.7 million T bounds of the budget-14 proof were evaluated to find that
+        // it had not
+        int T = tparent && td != 255 && Tp > td ? Tp - td : 0;
+        if constexpr (NQ == 3) {
+          cl = lo;
+          if (STD && tparent && (tcols & tb.keep_cols[g])) T = Tp;
+          tlo = T;
+        }
         if (pre) {
           const uint32_t w = hd.x;
-          const int td = (int)(w & 255u), Tp = (int)(pbw & BW_TUNK);
-          const int T = tparent && td != 255 && Tp > td ? Tp - td : 0;
           const int gm = (int)((w >> 8) & 7u), hq = he >> (__ffs(gm) - 1);
           const int kd = (w >> 16) & 1u ? pk + 1 - (hq & 1) - ((hq >> 4) & 1) : pk - (int)((w >> 11) & 31u), h = kd > 0 ? kd : 0;
           const int l = t_budget(h, lo.c2, __popc(pq & ~gm), rem) * sp.tdiv;
@@ -403,7 +416,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
               const int tcv = tcached ? (int)((tc_val >> (8 * tc)) & 0xff) : 0;
               const bool tcex = tcached && ((tc_ex >> tc) & 1);
               const bool tknown = (tpar && tdel == 0) || tcex;
-              const int Tbr = tpar ? (Tp > tdel ? Tp - tdel : 0) : 0;
+              const int Tbr = STD && NQ == 3 && cutlow ? (int)gget<GS>((uint32_t)tlo, g) : tpar ? (Tp > tdel ? Tp - tdel : 0) : 0;
               int T = tcex ? tcv : (Tbr > tcv ? Tbr : tcv);    // exact if tknown, else a lower bound
               bool texact = tknown;
               CutLow lo{0, 0, 0};
@@ -760,6 +773,9 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
   }
 }
 
+// T columns of a frontier node: the columns of its residual's Pauli transfer matrix (Paulis, X bits then Z bits) known to
+// attain its T bound, 0 when none is known.  The gather takes them from the parent where the gate only permutes columns, or
+// where the bound is the parent's; k_tcols forms those of the others.
 struct GatherArgs {
   const uint32_t *kidx;           // kept survivor ranks, in order
   long long nk;
@@ -788,7 +804,7 @@ struct GatherArgs {
 // It is bound by memory (1 KB read and written per node at n = 3): 11.2 million nodes of the Toffoli budget-14 proof take
 // 5.9 ms, 4.9 at the rate of a large copy; 11.3 with gate tables and goal pre-images read from global memory per node.
 template <int NQ>
-__global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
+__global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a, const uint32_t *pb, const uint64_t *tm, uint64_t *tm_next) {
   constexpr int N = 1 << NQ, E = N * N, GS = E, CPW = 64 / GS;
   const int lane = threadIdx.x & 63, le = lane & (GS - 1), slot = lane / GS;
   const long long wave = wave_index();
@@ -797,6 +813,9 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
   const int tn = a.tn;
   __shared__ __align__(16) ChildTab ct;
   load_child_tab(ct, sp);
+  __shared__ __align__(16) uint8_t col_src[NQ == 3 ? MAXG * 64 : 16];
+  if (NQ == 3 && tm)
+    for (int i = threadIdx.x; i < sp.G * 4; i += blockDim.x) ((uint4 *)col_src)[i] = ((const uint4 *)((const SpecTabs *)sp.ktab)->col_src)[i];
   __syncthreads();
   // goal pre-images, one candidate per lane (n = 3: every candidate)
   const int xgk = NQ == 3 && a.gflag && lane < sp.G ? sp.xgk[lane] : -1;
@@ -805,6 +824,7 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
   for (long long tb = wave * tn; tb < nk; tb += nwaves * tn) {
     const long long pl = tb + lane;
     uint32_t pi_l = 0, bw_l = 0;
+    uint64_t tm_l = 0;             // the parent's T columns, where they say something of the node's
     int g_l = 0, gp_l = 255, pk_l = 0;
     if (lane < tn && pl < nk) {
       const uint32_t kid = a.kidx[pl];
@@ -814,6 +834,8 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
       bw_l = a.surv_bw[kid] & bwkeep;
       gp_l = a.g1[pi_l];
       pk_l = a.pk[pi_l];
+      if (NQ == 3 && tm && !((pb[pi_l] ^ bw_l) & BW_TUNK) && (bw_l & BW_TUNK) != BW_TUNK) tm_l = tm[pi_l];
+      if (NQ == 3 && !tm && tm_next) tm_next[pl] = 0;     // no node has any yet
       a.g1_next[pl] = (uint8_t)g_l;
       a.g2_next[pl] = (uint8_t)gp_l;
       a.tree_par[pl] = pi_l;
@@ -864,11 +886,99 @@ __global__ __launch_bounds__(256) void k_gather(KSpec sp, GatherArgs a) {
           }
         }
       }
+      if (NQ == 3 && tm) {
+        const uint64_t pt = gget64<64>(tm_l, src);
+        const uint8_t from = pt ? col_src[g * 64 + lane] : (uint8_t)255;
+        const uint64_t t = gballot<64>(from < 64 && ((pt >> (from & 63)) & 1));
+        if (le == 0) tm_next[p] = t;
+      }
       if (le == 0) {
         a.pk_next[p] = k;
         a.pb_next[p] = bwp | (adj ? BW_GOAL : 0u);
         if (adj) a.gflag[a.pinst ? a.pinst[pi] : 0u] = 1u;
       }
+    }
+  }
+}
+
+// T columns of the nodes of a frontier that have none and whose T bound is known (n = 3; n + k <= 16), unless no T gate can
+// follow in the budget or the search ends at the next level: one pass of the
+// bound's transform, the one whose parity its valuation v has, and per column the bit that makes it v.  Only Paulis with
+// an X part on the residual's left count (flip pairs f >= 8): there the bit that the pairs leave out is one of the rows, and
+// the columns' bits are the low three of the transform's index.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_tcols(KSpec sp, const int4 *res, const int *pk, const uint32_t *pb,
+                                                                                    const uint32_t *inst, const int *rem, const uint32_t *gflag,
+                                                                                    uint64_t *tm, long long n) {
+  constexpr int NQ = 3, H = 32;
+  __shared__ __align__(1024) uint4 stage[2 * TS_STRIDE];
+  const int lane = threadIdx.x & 63;
+  const TStage st{(char *)stage, (threadIdx.x & ~63u) << 4};
+  const int f = lane == 0 ? 1 : lane, j = 31 - __clz(f);
+  uint32_t vb[2 * NQ - 1];
+#pragma unroll
+  for (int b = 0; b < 2 * NQ - 1; b++) vb[b] = (b >= j ? 32u : 16u) << b;
+  const uint32_t fo = (uint32_t)f << 4;
+  const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
+  // 16 nodes a wave and turn: with 64, a frontier of some ten thousand nodes left most of the chip idle
+  for (long long t0 = wave_index() * 16; t0 < n; t0 += nwaves * 16) {
+    int v_l = 0;
+    if (lane < 16 && t0 + lane < n && tm[t0 + lane] == 0) {
+      const uint32_t bw = pb[t0 + lane], nd = (bw & BW_NEEDS) >> 8;
+      const int T = (int)(bw & BW_TUNK), k = pk[t0 + lane];
+      if (T != (int)BW_TUNK && T > 0 && (bw & BW_CUTS) && NQ + k <= 16) {
+        const int c2 = sp.cxtable[(nd & 7u) + 3 * ((nd >> 3) & 7u) + 9 * ((nd >> 6) & 7u)];
+        const uint32_t i = inst[t0 + lane];
+        if (!(gflag && gflag[i]) && t_budget(k, c2, 0, rem[i] - 1) * sp.tdiv >= T - 1) v_l = 2 * (NQ + k) - T;
+      }
+    }
+    uint64_t todo = gballot<64>(v_l > 0);
+    while (todo) {
+      const int x = __ffsll((long long)todo) - 1;
+      todo &= todo - 1;
+      const int v = (int)gget<64>((uint32_t)v_l, x), pass = v & 1, m = (v - 2 + pass) >> 1;
+      const int4 s = res[(t0 + x) * 64 + lane];
+      __builtin_amdgcn_wave_barrier();
+      t_stage_x<NQ>(st, s, lane);
+      t_stage_p<NQ>(st, s, lane, pass);
+      __builtin_amdgcn_wave_barrier();
+      uint32_t at = st.group;
+      asm volatile("" : "+v"(at));
+      u16x2 q[H];
+#pragma unroll
+      for (int t = 0; t < H; t++) {
+        if (t) at ^= vb[t & 1 ? 0 : t & 2 ? 1 : t & 4 ? 2 : t & 8 ? 3 : 4];
+        const uint2 xv = *(const uint2 *)(st.lds + 16 * TS_STRIDE + (at ^ fo));
+        const uint4 mm = *(const uint4 *)(st.lds + at);
+        const u16x2 x01 = as16(xv.x), x23 = as16(xv.y);
+        q[t ^ (t >> 1)] = x01.xx * as16(mm.x) + x01.yy * as16(mm.y) + x23.xx * as16(mm.z) + x23.yy * as16(mm.w);
+      }
+#pragma unroll
+      for (int h = 1; h < H / 2; h <<= 1)
+#pragma unroll
+        for (int i = 0; i < H; i++)
+          if (!(i & h)) {
+            const u16x2 a = q[i], b = q[i | h];
+            q[i] = a + b;
+            q[i | h] = a - b;
+          }
+      // (the last step as in t_bound16s: no value has a bit below m, so bit m says that one of the column's attains it)
+      uint64_t cols = 0;
+#pragma unroll
+      for (int z = 0; z < 8; z++) {
+        uint32_t o = 0;
+#pragma unroll
+        for (int i = z; i < H / 2; i += 8) {
+          const uint32_t a = bits(q[i]), b = bits(q[i | H / 2]);
+          o |= (a ^ b) | ((a & b) << 1 & 0xfffefffeu);
+        }
+        uint64_t on = gballot<64>(((o | o >> 16) >> m) & 1u) & ~0xffull;
+        on |= on >> 32;
+        on |= on >> 16;
+        on |= on >> 8;
+        cols |= (on & 0xffull) << (8 * z);
+      }
+      if (lane == 0) tm[t0 + x] = cols;
+      __builtin_amdgcn_wave_barrier();
     }
   }
 }
@@ -943,6 +1053,7 @@ struct chz_ctx {
   chz::DBuf<int> pk[2];
   chz::DBuf<uint8_t> g1[2], g2[2];
   chz::DBuf<uint32_t> pb[2];        // bound words (T bound, cut needs) of the frontier's nodes
+  chz::DBuf<uint64_t> tm[2];        // their T columns (3 qubits, specialised expansion)
   std::vector<uint32_t *> tree_par;
   std::vector<uint8_t *> tree_gate;
   // per-level work arrays
@@ -991,6 +1102,8 @@ struct chz_ctx {
   double k_stage[6] = {};       // expansion stage counts: residuals, structural bounds, cut ranks, T bounds, keys,
                                 // T-bound passes
   double avg_terms = 1;         // nonzero terms per inverse column, averaged over the candidates
+  bool tcols = false;           // 3 qubits and std_spec: the frontier carries T columns
+  bool cols_on = false;         // some node of it may have any
   bool std_spec = false;        // what the specialised expansion asks of a spec
   int max_ik = 0;               // the largest sqrt2 exponent of a gate
   bool goal_skip = false;       // every candidate has a goal pre-image: the found-level skip is exact
@@ -1187,6 +1300,7 @@ struct RootArgs {
   int *pk;
   uint8_t *g1, *g2, *tg;
   uint32_t *finst, *pb, *tp;
+  uint64_t *tm;              // or null
   uint32_t *gflag;           // goal flags of ns slots to clear (a frontier of roots only), or null
   int ns;
 };
@@ -1200,6 +1314,7 @@ template <int E> __global__ void k_put_roots(RootArgs a) {
     a.finst[x] = (uint32_t)a.slot[i];
     a.pb[x] = BW_TUNK;
     a.tp[x] = NO_PARENT;
+    if (a.tm) a.tm[x] = 0;
   }
   if (a.gflag)
     for (long long i = i0; i < a.ns; i += stride) a.gflag[i] = 0u;
@@ -1221,7 +1336,8 @@ template <int NQ> static void append_roots(chz_ctx *c, int nxt, long long distin
     slot[i] = c->binst[q.inst].slot;
   }
   const RootArgs ra{u, k, slot, nr, distinct, c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tg,
-                    c->finst[nxt].p, c->pb[nxt].p, tp, c->m ? nullptr : c->gflag.p, c->nslots};
+                    c->finst[nxt].p, c->pb[nxt].p, tp, c->tcols ? c->tm[nxt].p : nullptr,
+                    c->m ? nullptr : c->gflag.p, c->nslots};
   hipLaunchKernelGGL(k_put_roots<E>, dim3(grid_for(nr * E / 64 + 1, 1024)), dim3(256), 0, c->stream, ra);
   HIPCHK(hipGetLastError());
   for (long long i = 0; i < nr; i++) {
@@ -1380,6 +1496,7 @@ static void level_room(chz_ctx *c, int nxt, long long ncc, long long mx, uint32_
   c->scan_tmp.need((size_t)nbS * 256 / SC_TILE + 4);
   c->res[nxt].need((size_t)mx * E); c->pk[nxt].need(mx); c->g1[nxt].need(mx); c->g2[nxt].need(mx);
   c->pb[nxt].need(mx); c->finst[nxt].need(mx);
+  if (c->tcols) c->tm[nxt].need(mx);
   tree_alloc(c, mx, tp, tg);
 }
 
@@ -1403,6 +1520,11 @@ constexpr bool kStepGraphs = true;
 // Levels launched for all their children at once (below): their next frontier's room, E entries a child, is bounded by
 // this many bytes (64K children of 3 qubits, 256K of 2)
 constexpr long long ONCE_BYTES = 64ll << 20;
+// Which frontiers k_tcols looks at: below some ten thousand nodes the expansion is as long as its longest chain, T bounds or
+// not, and searches with few gates left have few T bounds to save (24 searches of up to 10 gates in a batch, with every
+// frontier of 4K nodes looked at: 9.57 -> 10.05 ms; of 32K, and 6 gates left: 9.6)
+constexpr long long TCOLS_MIN = 32768;
+constexpr int TCOLS_LEFT = 6;
 constexpr int STEP_BUCKET = 10;    // the schedule of the 1,024-parent bucket drives the captured expansion
 
 template <int NQ>
@@ -1420,7 +1542,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   const uint32_t *pinst = c->finst[cur].p;
   const std::vector<uintptr_t> key = {
       (uintptr_t)c->res[cur].p, (uintptr_t)c->pk[cur].p, (uintptr_t)c->g1[cur].p, (uintptr_t)c->g2[cur].p,
-      (uintptr_t)c->pb[cur].p, (uintptr_t)pinst, (uintptr_t)c->status.p, (uintptr_t)c->keys.p, (uintptr_t)c->info.p,
+      (uintptr_t)c->pb[cur].p, (uintptr_t)c->tm[cur].p, (uintptr_t)pinst, (uintptr_t)c->status.p, (uintptr_t)c->keys.p, (uintptr_t)c->info.p,
       (uintptr_t)c->cnt, (uintptr_t)c->d_rem, (uintptr_t)c->d_keepi, (uintptr_t)c->icnt,
       (uintptr_t)c->bcount.p, (uintptr_t)c->surv_o.p, (uintptr_t)c->surv_key.p, (uintptr_t)c->surv_bw.p,
       (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->runs.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
@@ -1437,7 +1559,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
     std::lock_guard<std::recursive_mutex> capture_lock(capture_mu());
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, 0, ncap, 0, 0,
-                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
+                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
                   c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cap * G + CPW - 1) / CPW, sc.cap));
     launch_level<NQ>(c, sc.var, spec, grid, s, ea, cap);
@@ -1463,7 +1585,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
                       c->surv_bw.p, c->pb[nxt].p, c->cnt + C_KEPT, c->goal_skip ? c->gflag.p : nullptr, CPW};
   HIPCHK(hipMemsetAsync(c->gflag.p, 0, (size_t)ns * 4, c->stream));   // the graph's expansion has read them
   c->ev.begin(K_GATHER, c->stream);
-  hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((ncap + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga);
+  hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((ncap + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga, c->pb[cur].p, c->cols_on ? c->tm[cur].p : nullptr, c->tcols ? c->tm[nxt].p : nullptr);
   c->ev.end(c->stream);
   HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -1482,10 +1604,12 @@ template <int NQ> static void batch_step(chz_ctx *c) {
   const int G = ks.G;
   if (c->m == 0 && c->pending.empty()) return;
   if (c->m == 0) {   // a frontier of roots only
+    c->cols_on = false;
     const long long nr = (long long)c->pending.size();
     const int nxt = c->cur ^ 1;
     c->res[nxt].need(nr * E); c->pk[nxt].need(nr); c->g1[nxt].need(nr); c->g2[nxt].need(nr); c->finst[nxt].need(nr);
     c->pb[nxt].need(nr);
+    if (c->tcols) c->tm[nxt].need(nr);
     uint32_t *tp = nullptr;
     uint8_t *tg = nullptr;
     tree_alloc(c, nr, tp, tg);
@@ -1597,7 +1721,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     const chz_ctx::Sched sc = c->tuning ? c->force : c->sched[bucket];
     const int gsplit = (int)std::max<long long>(1, std::min<long long>(G, ((long long)sc.tw * CPW + cm - 1) / cm));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, off, ncc, 0, 0,
-                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
+                  c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
                   c->icnt, slot_stripes(ns), ns * IC_N, gsplit, nullptr, 0, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cm * gsplit + CPW - 1) / CPW, sc.cap));
     hipEvent_t te0 = nullptr, te1 = nullptr;
@@ -1637,7 +1761,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
                         c->res[nxt].p, c->pk[nxt].p, c->g1[nxt].p, c->g2[nxt].p, tp, tg, pinst, c->finst[nxt].p,
                         c->surv_bw.p, c->pb[nxt].p, c->cnt + C_KEPT, c->goal_skip ? c->gflag.p : nullptr, CPW};
     c->ev.begin(K_GATHER, c->stream);
-    hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((maxcc / 4 + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga);
+    hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((maxcc / 4 + CPW - 1) / CPW)), dim3(256), 0, c->stream, ks, ga, c->pb[cur].p, c->cols_on ? c->tm[cur].p : nullptr, c->tcols ? c->tm[nxt].p : nullptr);
     c->ev.end(c->stream);
     if (!alone) {
       hipLaunchKernelGGL(k_slot_bounds, dim3(grid_for(maxcc / 256 + 1, 256)), dim3(256), 0, c->stream, c->finst[nxt].p, maxcc,
@@ -1719,6 +1843,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     if (!gathered) {
       c->res[nxt].need((size_t)mn * E); c->pk[nxt].need(mn); c->g1[nxt].need(mn); c->g2[nxt].need(mn);
       c->pb[nxt].need(mn);
+      if (c->tcols) c->tm[nxt].need(mn);
       c->finst[nxt].need(mn);
       tree_alloc(c, mn, tp, tg);
     }
@@ -1729,9 +1854,16 @@ template <int NQ> static void batch_step(chz_ctx *c) {
                           gather_tile<NQ>(distinct)};
       c->ev.begin(K_GATHER, c->stream);
       hipLaunchKernelGGL(k_gather<NQ>, dim3(grid_for((distinct + ga.tn - 1) / ga.tn)), dim3(256), 0, c->stream, ks,
-                         ga);
+                         ga, c->pb[cur].p, c->cols_on ? c->tm[cur].p : nullptr, c->tcols ? c->tm[nxt].p : nullptr);
       c->ev.end(c->stream);
       c->k_work[K_GATHER] += (double)distinct * (E * 16.0 * 2.0 + 16.0);
+      int left = 0;                 // the most gates a search has left after this level
+      for (const BInst &b : c->binst) if (b.live) left = std::max(left, b.depth - (b.t + 1));
+      if (c->tcols && distinct >= TCOLS_MIN && left >= TCOLS_LEFT) {
+        c->cols_on = true;
+        hipLaunchKernelGGL(k_tcols, dim3(grid_for(distinct / 16 + 1, 4096)), dim3(256), 0, c->stream, ks, c->res[nxt].p, c->pk[nxt].p,
+                           c->pb[nxt].p, c->finst[nxt].p, c->d_rem, c->goal_skip ? c->gflag.p : nullptr, c->tm[nxt].p, distinct);
+      }
     }
     const bool single = c->pending.empty() && chz_batch_live(c) == 1;
     if (c->gt_filter && distinct)   // a table build keeps every level, resident, with its classes' keys
@@ -1747,6 +1879,8 @@ template <int NQ> static void batch_step(chz_ctx *c) {
                             c->stream));
       HIPCHK(hipMemcpyAsync(c->pb[nxt].p + distinct, c->pb[cur].p + ma, (size_t)ncarry * 4, hipMemcpyDeviceToDevice,
                             c->stream));
+      if (c->tcols)
+        HIPCHK(hipMemcpyAsync(c->tm[nxt].p + distinct, c->tm[cur].p + ma, (size_t)ncarry * 8, hipMemcpyDeviceToDevice, c->stream));
       HIPCHK(hipMemcpyAsync(c->finst[nxt].p + distinct, c->finst[cur].p + ma, (size_t)ncarry * 4,
                             hipMemcpyDeviceToDevice, c->stream));
       hipLaunchKernelGGL(k_carry_tree, dim3(grid_for(ncarry / 64 + 1)), dim3(256), 0, c->stream, tp + distinct,
@@ -2096,6 +2230,17 @@ static void upload_spec(chz_ctx *c) {
   }
   c->std_spec = s.standard && !s.lite && k.pre && k.cut1 && k.ncuts == (k.n == 3 ? 3 : 1) && k.n > 1 && k.have_table &&
                 k.cxlds && k.cx_mono && two_terms;
+  c->tcols = c->std_spec && k.n == 3;
+  std::memset(tabs[0].col_src, 255, sizeof tabs[0].col_src);
+  for (int g = 0; c->tcols && g < G; g++) {
+    std::vector<int> src;
+    gate_columns(s.gates[g], 3, src);
+    for (int b = 0; b < 64; b++)
+      if (src[b] >= 0) {
+        tabs[0].col_src[g * 64 + b] = (uint8_t)src[b];
+        tabs[0].level.keep_cols[g] |= 1ull << src[b];
+      }
+  }
   c->ktab.need(sizeof(SpecTabs));
   chz::copy_sync(c->ktab.p, tabs.data(), sizeof(SpecTabs), hipMemcpyHostToDevice, c->stream);
   k.ktab = (const uint4 *)c->ktab.p;
@@ -2508,7 +2653,7 @@ void chz_close(chz_ctx *c) {
   chz::free_tree(c);
   for (int b = 0; b < 2; b++) {
     c->res[b].release(); c->pk[b].release(); c->g1[b].release(); c->g2[b].release();
-    c->pb[b].release();
+    c->pb[b].release(); c->tm[b].release();
     c->sk[b].release(); c->sv[b].release();
   }
   c->finst[0].release(); c->finst[1].release(); c->ctl.release(); c->gflag.release();

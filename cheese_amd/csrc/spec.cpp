@@ -317,6 +317,58 @@ int gate_ptm_sde(const HostGate &g) {
   return sde;
 }
 
+void gate_columns(const HostGate &g, int n, std::vector<int> &src) {
+  const int L = 1 << g.nq;
+  src.assign((size_t)1 << (2 * n), -1);
+  const std::vector<Zq> &M = g.inv;
+  if ((int)M.size() != L * L) return;
+  std::vector<Zq> MB(L * L), C(L * L);
+  std::vector<int> loc(L * L, -1);               // the gate's own qubits: ax | az << nq, or -1
+  for (int bx = 0; bx < L; bx++)
+    for (int bz = 0; bz < L; bz++) {
+      for (int r = 0; r < L; r++)                // M B, as in gate_ptm_sde
+        for (int c = 0; c < L; c++) {
+          Zq v = M[r * L + (c ^ bx)];
+          if (__builtin_popcount(bz & c) & 1) v = {-v.a, -v.b, -v.c, -v.d};
+          MB[r * L + c] = v;
+        }
+      for (int r = 0; r < L; r++)
+        for (int c = 0; c < L; c++) {
+          Zq acc{0, 0, 0, 0};
+          for (int j = 0; j < L; j++) {
+            const Zq t = zq_mul(MB[r * L + j], zq_conj(M[c * L + j]));
+            acc = {acc.a + t.a, acc.b + t.b, acc.c + t.c, acc.d + t.d};
+          }
+          C[r * L + c] = acc;
+        }
+      int hits = 0;
+      for (int ax = 0; ax < L; ax++)
+        for (int az = 0; az < L; az++) {
+          Zq tr{0, 0, 0, 0};
+          for (int c = 0; c < L; c++) {
+            Zq v = C[(c ^ ax) * L + c];
+            if (__builtin_popcount(az & c) & 1) v = {-v.a, -v.b, -v.c, -v.d};
+            tr = {tr.a + v.a, tr.b + v.b, tr.c + v.c, tr.d + v.d};
+          }
+          if (zq_zero(tr)) continue;
+          hits++;
+          loc[bx | bz << g.nq] = ax | az << g.nq;
+        }
+      if (hits != 1) loc[bx | bz << g.nq] = -1;
+    }
+  for (int b = 0; b < 1 << (2 * n); b++) {
+    int l = 0;
+    for (int j = 0; j < g.nq; j++) l |= ((b >> g.q[j]) & 1) << j | ((b >> (n + g.q[j])) & 1) << (g.nq + j);
+    if (loc[l] < 0) continue;
+    int out = b;
+    for (int j = 0; j < g.nq; j++) {
+      out &= ~(1 << g.q[j] | 1 << (n + g.q[j]));
+      out |= ((loc[l] >> j) & 1) << g.q[j] | ((loc[l] >> (g.nq + j)) & 1) << (n + g.q[j]);
+    }
+    src[b] = out;
+  }
+}
+
 bool gate_is_clifford(const HostGate &g) { return gate_ptm_sde(g) == 0; }
 
 bool same_t_bound(const HostGate &a, const HostGate &b) {

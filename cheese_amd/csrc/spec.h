@@ -65,6 +65,10 @@ bool same_gate_set(const HostSpec &a, const HostSpec &b);
 
 // exact: the gate maps every Pauli operator to a multiple of a Pauli operator under conjugation
 bool gate_is_clifford(const HostGate &g);
+// Where the columns of a child's Pauli transfer matrix come from: src[b], for Pauli b of n qubits (bit q: X on qubit q, bit
+// n + q: Z), is the parent's column that is the child's column b up to sign (g^-1 P_b g = +-P_src), or -1 where it is a sum
+// of several
+void gate_columns(const HostGate &g, int n, std::vector<int> &src);
 // largest sqrt2-denominator exponent of the gate's Pauli transfer matrix (0: Clifford; 1: T), -1 if malformed
 int gate_ptm_sde(const HostGate &g);
 // operator-Schmidt rank over F_p of the gate across cut mask A (1 when all its qubits are on one side)

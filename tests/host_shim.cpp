@@ -51,3 +51,15 @@ extern "C" int shim_goal_skip(const char *spec, long len, long long scale) {
   std::vector<char> have;
   return chz::goal_preimages(s, X, have) ? 1 : 0;
 }
+
+// gate_columns of candidate g over the spec's qubits: 4^n sources (-1: a sum of several)
+extern "C" int shim_gate_columns(const char *spec, long len, int g, int *out, int cap) {
+  chz::HostSpec s;
+  std::string err;
+  if (chz::parse_spec(std::string(spec, (size_t)len), s, err) || g < 0 || g >= s.G()) return -1;
+  std::vector<int> src;
+  chz::gate_columns(s.gates[g], s.n, src);
+  if (cap < (int)src.size()) return -1;
+  for (size_t b = 0; b < src.size(); b++) out[b] = src[b];
+  return (int)src.size();
+}

@@ -195,3 +195,33 @@ def test_zdown_halves_in_32_bits():
             assert s == (a + c) // 2 and d == (c - a) // 2 and lo <= s <= hi and lo <= d <= hi, (a, c)
             n += 1
     assert n > 100000
+
+
+@pytest.mark.parametrize("n", [2, 3])
+def test_gate_columns_are_the_conjugated_paulis(shim, n):
+    """for every candidate of the default gate set and every Pauli b, g^-1 P_b g is the named Pauli up to sign, or a
+    sum of several exactly where none is named"""
+    import numpy as np
+    skel = W.skeleton(n)
+    spec = W.spec_from_skeleton(skel, W.unitary(n, []), 5).encode()
+    w = np.exp(1j * np.pi / 4)
+    N = 1 << n
+    paulis = []
+    for b in range(4 ** n):
+        x, z = b & (N - 1), b >> n
+        P = np.zeros((N, N), dtype=complex)
+        for c in range(N):
+            P[c ^ x, c] = (-1) ** bin(z & c).count("1")
+        paulis.append(P)
+    for g, name in enumerate(ln.split()[0] for ln in skel.splitlines() if ln.startswith("L_")):
+        parts = name.split("_")
+        gate, qs = parts[1], [int(q) for q in parts[2:]]
+        k, U = W.unitary(n, [(gate, qs)])
+        M = np.array([[sum(v * w ** i for i, v in enumerate(e)) for e in row] for row in U]) / np.sqrt(2) ** k
+        out = (ctypes.c_int * (4 ** n))()
+        assert shim.shim_gate_columns(spec, len(spec), g, out, 4 ** n) == 4 ** n
+        for b in range(4 ** n):
+            C = M.conj().T @ paulis[b] @ M
+            weights = [abs(np.trace(P.conj().T @ C)) / N for P in paulis]
+            hits = [i for i, v in enumerate(weights) if v > 1e-9]
+            assert list(out)[b] == (hits[0] if len(hits) == 1 else -1), (gate, qs, b)
