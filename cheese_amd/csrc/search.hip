@@ -31,7 +31,7 @@ namespace chz {
 // stage counts of the expansion's work model
 // C_M, C_NCC: the level's parents and children, written by the host with the level's control upload (read by the
 // kernels of a captured level step, whose launches are sized for a capacity)
-enum { C_W2 = 0, C_W3, C_DEAD, C_FOUND, C_ALIVE, C_OVF, C_NEEDT, C_FIRST, C_RUNS, C_REPOVF, C_KEPT, C_EVAL, C_SURV,
+enum { C_W2 = 0, C_W3, C_DEAD, C_FOUND, C_ALIVE, C_OVF, C_NEEDT, C_FIRST, C_REPOVF, C_KEPT, C_EVAL, C_SURV,
        C_CHEAP, C_CUTS, C_KEYS, C_TPASS, C_PRE, C_M, C_NCC, C_N };
 // per-instance counters of one level (a batch carries several searches that share the spec's gate set)
 enum { IC_W2 = 0, IC_W3, IC_DEAD, IC_FOUND, IC_ALIVE, IC_OVF, IC_FIRST, IC_N };
@@ -626,7 +626,6 @@ struct DedupeArgs {
   long long n;
   const uint64_t *surv_o, *surv_key;
   const uint32_t *surv_bw;
-  const uint32_t *runs;
   const int4 *res;                // parents' residuals
   const int *pk;
   uint8_t *kept;
@@ -672,34 +671,47 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
   const int grp = (threadIdx.x >> 6) * CPW + slot;
   const long long wave = wave_index();
   const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
-  const long long nruns = (long long)a.cnt[C_RUNS];
   const long long n = dev_n(a.n, a.nd);
   const uint64_t G = (uint64_t)sp.G;
-  for (long long base = wave * CPW; base < nruns; base += nwaves * CPW) {
-    const long long ri = base + slot;
-    if (ri >= nruns) continue;
-    const long long i0 = a.runs[ri];
-    const uint32_t key = a.k[i0];
-    int nrep = 0;
-    // a run is almost always one class: its members are each rebuilt once and compared with the first
-    // representative, of which (and of the second) an image stays in LDS.  A member's smallest image is known from its
-    // class key, so one comparison settles it where trying the group's elements in turn took six or seven; its
-    // entries come straight from its parent in global memory, the next member's on the way while it is compared.
-    // (The 22.4 million survivors of the Toffoli budget-14 proof: 20.4 ms with the members' parents staged in LDS,
-    // gate tables in global memory and the elements tried in turn, 12.3 here.)
+  constexpr uint64_t ALL = GS == 64 ? ~0ull : (1ull << GS) - 1;
+  // A lane group takes up to GS sorted positions at a time and deduplicates the runs of equal prefixes that start there, lane
+  // le holding position le's rank, child, key, parent exponent and slot: the chain of five dependent loads from a run to
+  // its members' parents is waited for once a tile, and each member then waits on one load (its parent's residual), issued
+  // while the member before it is compared, be it of another run.  (One run at a time, from a list of the runs: the
+  // budget-14 proof's dedupe 20.4 ms under the tracer, here 15.0.)
+  // A run is almost always one class: its members are each rebuilt once and compared with the first representative, of which
+  // (and of the second) an image stays in LDS.  A member's smallest image is known from its class key, so one comparison
+  // settles it where trying the group's elements in turn took six or seven; its entries come straight from its parent in
+  // global memory.  (With the members' parents staged in LDS, gate tables in global memory and the elements tried in
+  // turn it took another 8 ms.)
+  // Smaller tiles where there are not enough positions for all groups: a small level's dedupe is as long as its longest chain.
+  int tn = 4;
+  while (tn < GS && tn * nwaves * CPW < n) tn <<= 1;
+  for (long long t0 = (wave * CPW + slot) * tn; t0 < n; t0 += nwaves * CPW * tn) {
+    long long j0 = t0;
+    uint32_t key = 0;             // of the run that crosses the tile's end, once it is walked
+    bool crossing = false;
+    int nrep = 0, head = -1;
     int ck0 = 0, ck1 = 0;
-    // members in chunks of GS: lane le loads member j0 + le's rank, child, key, parent exponent and slot at once,
-    // so each member then waits on one load (its parent's residual), issued while the member before it is
-    // compared
-    for (long long j0 = i0; j0 < n; j0 += GS) {
+    for (;;) {
       const long long jj = j0 + le;
-      const bool in = jj < n && a.k[jj] == key;
-      const uint64_t inb = gballot<GS>(in);
-      const int nm = ~inb ? __ffsll((long long)~inb) - 1 : GS;     // members are contiguous from j0
+      const bool valid = jj < n && (crossing || le < tn);
+      const uint32_t kj = valid ? a.k[jj] : 0u;
+      uint64_t heads = 0, left, over = 0;       // over: the run that the tile's last position shares with the next tile
+      bool in;
+      if (!crossing) {
+        const bool first = valid && (jj == 0 || a.k[jj - 1] != kj), more = valid && jj + 1 < n && a.k[jj + 1] == kj;
+        heads = gballot<GS>(first);
+        const uint64_t cont = gballot<GS>(more);
+        if (!heads) break;                      // the tile lies within a run of an earlier one
+        const int h0 = __ffsll((long long)heads) - 1;
+        if ((cont >> (tn - 1)) & 1) over = ALL & ~((1ull << (63 - __clzll((long long)heads))) - 1);
+        in = le >= h0 && !((over >> le) & 1) && (more || !first) && valid;
+      } else in = valid && kj == key;
       uint32_t m_rank = 0, m_inst = 0, m_img = 0;
       uint64_t m_o = 0, m_key = 0;
       int m_pk = 0;
-      if (le < nm) {
+      if (in) {
         m_rank = a.v[jj];
         m_o = a.surv_o[m_rank];
         m_key = a.surv_key[m_rank];
@@ -708,26 +720,30 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
         m_pk = a.pk[pi];
         m_inst = a.pinst ? a.pinst[pi] : 0u;
       }
+      const uint64_t inb = gballot<GS>(in);
+      left = inb;
+      if (!crossing) {
+        // runs of two: only members that share their whole key are looked at (the sort brings together what agrees in
+        // part of it)
+        const uint64_t up = (uint64_t)(uint32_t)__shfl_down((int)(m_key >> 32), 1, GS) << 32 | (uint32_t)__shfl_down((int)m_key, 1, GS);
+        const uint64_t eq = gballot<GS>(in && m_key == up);
+        const uint64_t two = heads & inb & ~(heads >> 1) & (heads >> 2 | ~(inb >> 2));
+        const uint64_t apart = two & ~eq;
+        left &= ~(apart | apart << 1);
+      }
       auto terms = [&](int q) {
         const uint64_t o = gget64<GS>(m_o, q);
         return child_terms<NQ>(a.res + (long long)(o / G) * E, ct.desc[(int)(o % G) * 64 + le], le);
       };
-      // a run that ends in this chunk: only members that share their whole key with another one are looked at (the sort
-      // brings together what agrees in part of it)
-      uint64_t left = nm < 64 ? (1ull << nm) - 1 : ~0ull;
-      if (j0 == i0 && nm < GS) {
-        uint64_t shared = 0;
-        for (int q = 0; q < nm; q++) {
-          const uint64_t same = gballot<GS>(le < nm && m_key == gget64<GS>(m_key, q));
-          if (same & (same - 1)) shared |= 1ull << q;
-        }
-        left = shared;
-      }
       ChildTerms next{};
       if (left) next = terms(__ffsll((long long)left) - 1);
       while (left) {
         const int q = __ffsll((long long)left) - 1;
         left &= left - 1;
+        if (!crossing) {
+          const int h = 63 - __clzll((long long)(heads & ((2ull << q) - 1)));
+          if (h != head) { head = h; nrep = 0; }
+        }
         const uint32_t rank = gget<GS>(m_rank, q), inst = gget<GS>(m_inst, q);
         const uint64_t o = gget64<GS>(m_o, q), key64 = gget64<GS>(m_key, q);
         const int pk = (int)gget<GS>((uint32_t)m_pk, q), img = (int)gget<GS>(m_img, q);
@@ -768,7 +784,15 @@ void k_dedupe_runs(KSpec sp, DedupeArgs a) {
         } else if (le == 0) atomicAdd(&a.cnt[C_REPOVF], 1ull);
         __builtin_amdgcn_wave_barrier();
       }
-      if (nm < GS) break;      // the run ended inside this chunk
+      if (!crossing) {
+        if (!over) break;
+        crossing = true;                        // from its head, GS members at a time
+        nrep = 0;
+        const int h = __ffsll((long long)over) - 1;
+        j0 = t0 + h;
+        key = a.k[j0];
+      } else if (inb == ALL) j0 += GS;
+      else break;
     }
   }
 }
@@ -1061,7 +1085,7 @@ struct chz_ctx {
   chz::DBuf<uint64_t> keys, surv_o, surv_key;
   chz::DBuf<uint32_t> info, surv_bw;
   chz::DBuf<unsigned long long> bcount, hist;
-  chz::DBuf<uint32_t> sk[2], sv[2], runs, kidx;
+  chz::DBuf<uint32_t> sk[2], sv[2], kidx;
   // batch state: searches, frontier instance slots, per-slot device arrays, queued events
   std::vector<chz::BInst> binst;
   std::vector<chz::Pending> pending;
@@ -1456,7 +1480,6 @@ template <int NQ> static void launch_level(chz_ctx *c, int var, bool spec, dim3 
 template <int NQ>
 static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long long *dncc, uint32_t *gflag, bool timed,
                        hipStream_t s) {
-  constexpr int CPW = 64 >> (2 * NQ);
   const unsigned long long *nd = c->cnt + C_SURV;
   const uint32_t *pinst = c->finst[cur].p;
   const AliveOut ao{c->keys.p, c->info.p, 0, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
@@ -1471,11 +1494,9 @@ static void level_tail(chz_ctx *c, int cur, long long ncc, const unsigned long l
   begin(K_DEDUPE);
   const ActiveArgs aa{c->icnt, slot_stripes(c->nslots), c->nslots, c->ks.G, c->surv_o.p, pinst};
   hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(ncc / 256 + 1, 256)), dim3(256), 0, s, c->kept.p, ncc, nd, aa, gflag);
-  hipLaunchKernelGGL(k_run_starts, dim3(grid_for(ncc / (64 * RH_ITEMS) + 1)), dim3(256), 0, s, c->sk[0].p, ncc, c->runs.p,
-                     c->cnt + C_RUNS, nd);
-  const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncc, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p, c->res[cur].p,
+  const DedupeArgs da{c->sk[0].p, c->sv[0].p, ncc, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->res[cur].p,
                       c->pk[cur].p, c->kept.p, c->cnt, pinst, nd};
-  hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncc / CPW / 8 + 1, 1024)), dim3(256), 0, s, c->ks, da);
+  hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(ncc / 16 + 1, 2048)), dim3(256), 0, s, c->ks, da);
   end();
   begin(K_COMPACT);
   compact_kept(c, ncc, nd, s);
@@ -1490,7 +1511,7 @@ static void level_room(chz_ctx *c, int nxt, long long ncc, long long mx, uint32_
   c->status.need(ncc); c->keys.need(ncc); c->info.need(ncc);
   c->bcount.need(nbA + 1);
   c->surv_o.need(ncc); c->surv_key.need(ncc); c->surv_bw.need(ncc);
-  c->kept.need(ncc); c->kidx.need(ncc); c->runs.need(ncc);
+  c->kept.need(ncc); c->kidx.need(ncc);
   for (int b = 0; b < 2; b++) { c->sk[b].need(ncc); c->sv[b].need(ncc); }
   c->hist.need((size_t)nbS * 256 + 1);
   c->scan_tmp.need((size_t)nbS * 256 / SC_TILE + 4);
@@ -1503,7 +1524,7 @@ static void level_room(chz_ctx *c, int nxt, long long ncc, long long mx, uint32_
 // Captured level step for levels of at most STEP_CAP parents: expansion, survivor compaction, radix sort, exact
 // dedupe, the searches' continue flags and the kept compaction, in one graph built once per frontier parity with
 // launches sized for the capacity; every kernel reads the level's sizes from the counters the host uploads
-// (C_M, C_NCC) and those the step produces (C_SURV, C_RUNS, the kept total).  The graph holds no memset node.  It
+// (C_M, C_NCC) and those the step produces (C_SURV, C_KEPT).  The graph holds no memset node.  It
 // is rebuilt when a buffer address, the slot count or the schedule it was captured with changes.  The gather runs
 // after it as an ordinary launch (its tree level differs every step), then the level synchronises once.
 constexpr long long STEP_CAP = 1024;
@@ -1545,7 +1566,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       (uintptr_t)c->pb[cur].p, (uintptr_t)c->tm[cur].p, (uintptr_t)pinst, (uintptr_t)c->status.p, (uintptr_t)c->keys.p, (uintptr_t)c->info.p,
       (uintptr_t)c->cnt, (uintptr_t)c->d_rem, (uintptr_t)c->d_keepi, (uintptr_t)c->icnt,
       (uintptr_t)c->bcount.p, (uintptr_t)c->surv_o.p, (uintptr_t)c->surv_key.p, (uintptr_t)c->surv_bw.p,
-      (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->runs.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
+      (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
       (uintptr_t)c->sv[0].p, (uintptr_t)c->sv[1].p, (uintptr_t)c->hist.p, (uintptr_t)c->scan_tmp.p,
       (uintptr_t)c->gflag.p, (uintptr_t)ns, (uintptr_t)sc.var, (uintptr_t)sc.cap,
       (uintptr_t)sc.tw, (uintptr_t)spec};
@@ -1798,7 +1819,6 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     const ActiveArgs aa{c->icnt, slot_stripes(ns), ns, G, c->surv_o.p, pinst};
     gflag_clear = true;
     if (c->opts.dedupe && nsurv > 1) {
-      c->runs.need(nsurv);
       c->ev.begin(K_SORT, c->stream);
       sort_survivors(c, nsurv, nullptr, c->stream);
       c->ev.end(c->stream);
@@ -1806,11 +1826,9 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       c->ev.begin(K_DEDUPE, c->stream);
       hipLaunchKernelGGL(k_fill_kept, dim3(grid_for(nsurv / 256 + 1)), dim3(256), 0, c->stream, c->kept.p, nsurv,
                          nullptr, aa, c->gflag.p);
-      hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nsurv / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream,
-                         c->sk[0].p, nsurv, c->runs.p, c->cnt + C_RUNS, nullptr);
-      const DedupeArgs da{c->sk[0].p, c->sv[0].p, nsurv, c->surv_o.p, c->surv_key.p, c->surv_bw.p, c->runs.p,
+      const DedupeArgs da{c->sk[0].p, c->sv[0].p, nsurv, c->surv_o.p, c->surv_key.p, c->surv_bw.p,
                           c->res[cur].p, c->pk[cur].p, c->kept.p, c->cnt, pinst, nullptr};
-      hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(nsurv / CPW + 1, 4096)), dim3(256), 0, c->stream, ks, da);
+      hipLaunchKernelGGL(k_dedupe_runs<NQ>, dim3(grid_for(nsurv / 4 + 1, 4096)), dim3(256), 0, c->stream, ks, da);
       c->ev.end(c->stream);
       c->k_work[K_DEDUPE] += (double)nsurv * 9.0;
     } else {
@@ -2664,7 +2682,7 @@ void chz_close(chz_ctx *c) {
   for (auto &g : c->sgraph) if (g.exec) { (void)hipGraphExecDestroy(g.exec); g.exec = nullptr; }
   c->status.release(); c->kept.release(); c->keys.release(); c->surv_o.release(); c->surv_key.release();
   c->surv_bw.release();
-  c->info.release(); c->bcount.release(); c->hist.release(); c->runs.release(); c->kidx.release();
+  c->info.release(); c->bcount.release(); c->hist.release(); c->kidx.release();
   c->spec_blob.release();
   c->ktab.release();
   if (c->gt) { c->gt->release(); delete c->gt; c->gt = nullptr; }
