@@ -253,12 +253,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     // (every coefficient's parity agrees); it falls by no more than one
     int he = 0;                                  // bits q, 4 + q: the first, the second holds for qubit q
     if (pre) {
-      const uint64_t ba = gballot<GS>(S.x & 1), bb = gballot<GS>(S.y & 1), bc = gballot<GS>(S.z & 1), bd = gballot<GS>(S.w & 1);
+      // per lane the parities of a, b, c, d (bits 2-5) and of a + c, b + d (bits 0-1), compared with the paired column's: 50
+      // scalar instructions a parent fewer than by masks of ballots
+      const uint32_t par = (S.x & 1u) | (S.y & 1u) << 1 | (S.z & 1u) << 2 | (S.w & 1u) << 3;
+      const uint32_t w = par << 2 | ((par ^ par >> 2) & 3u);
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
-        auto differ = [&](uint64_t m) { return (m ^ (m >> (1 << q))) & pair_mask<NQ>(q); };
-        if (!(differ(ba ^ bc) | differ(bb ^ bd))) he |= 1 << q;
-        if (!(differ(ba) | differ(bb) | differ(bc) | differ(bd))) he |= 16 << q;
+        const uint32_t d = w ^ (NQ == 3 ? wave_xor32(w, 1 << q) : (uint32_t)__shfl_xor((int)w, 1 << q, GS));
+        if (!gany<GS>(d & 3u)) he |= 1 << q;
+        if (!gany<GS>(d & 0x3cu)) he |= 16 << q;
       }
     }
     const int pq = !lite ? support_mask<NQ>(S, le, gballot<GS>(!zzero(S)), N - 1) : 0;

@@ -160,15 +160,6 @@ template <int NQ> __host__ __device__ constexpr uint64_t offdiag_mask(int q) {
   return m;
 }
 
-// lanes whose column has bit q clear, as a group-local mask
-template <int NQ> __host__ __device__ constexpr uint64_t pair_mask(int q) {
-  constexpr int N = 1 << NQ, GS = N * N;
-  uint64_t m = 0;
-  for (int le = 0; le < GS; le++)
-    if (!((le >> q) & 1)) m |= 1ull << le;
-  return m;
-}
-
 // qubits the matrix acts on non-trivially (src/cheese.cu:305-319), as a mask; b = group ballot of the nonzero
 // entries.  A nonzero entry off the qubit's diagonal blocks settles that qubit without comparing blocks.
 // Only the qubits in `ask` are looked at: a gate leaves the others as trivial or not as they were in the parent.
