@@ -245,8 +245,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     // of 5.71 million children past the windows still form one (3.12 without the T siblings below).  Only where no child
     // can overflow (which would be reported) and the goal's own bounds are 0 (a goal child is never over its budget).
     // On the budget-14 proof the expansion takes 111 ms instead of 139.  Where a parent's candidates are split over
-    // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.
-    const bool pre = gsplit <= PRE_SPLIT && (STD || (sp.pre && gall<GS>(mag <= sp.maglim)));
+    // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.  Roots (no gate
+    // before them) form every residual: a target keeps its exponent as written, and where sqrt2 divides all of its entries
+    // a child's can be lower by more than the gate takes.
+    const bool pre = g1 != 255 && gsplit <= PRE_SPLIT && (STD || (sp.pre && gall<GS>(mag <= sp.maglim)));
     const bool tparent = (pbw & BW_TUNK) != BW_TUNK;
     // H on qubit q pairs the columns c and c ^ 2^q as their sum and difference over sqrt2: the exponent rises by one,
     // less one if sqrt2 divides every sum (the parities of a + c and b + d agree in each pair), less another if 2 does
