@@ -1242,9 +1242,11 @@ static void sort_survivors(chz_ctx *c, long long n, const unsigned long long *nd
   HIPCHK(radix_sort_pairs(c->sk[0].p, c->sv[0].p, c->sk[1].p, c->sv[1].p, n, c->hist.p, c->scan_tmp.p, s, nd, passes));
 }
 
-// the survivors of the level's only chunk, in order, their number in C_SURV
+// the survivors of the level's only chunk, in order, their number in C_SURV.  (A gate set without candidates has no
+// children: nothing is launched, since an empty grid is an error that the thread's next hipGetLastError would return.)
 static void compact_alive(chz_ctx *c, const FlagAlive &fa, long long ncc, const AliveOut &ao, const unsigned long long *dncc,
                           hipStream_t s) {
+  if (ncc == 0) return;
   const long long nb = (ncc + CT_TILE - 1) / CT_TILE;
   if (nb > 1)
     hipLaunchKernelGGL(k_flag_count<FlagAlive>, dim3((unsigned)nb), dim3(CT_THREADS), 0, s, fa, ncc, c->bcount.p, dncc);
@@ -1254,6 +1256,7 @@ static void compact_alive(chz_ctx *c, const FlagAlive &fa, long long ncc, const 
 
 // the kept survivors' ranks in kidx, their number in C_KEPT
 static void compact_kept(chz_ctx *c, long long n, const unsigned long long *nd, hipStream_t s) {
+  if (n == 0) return;
   const long long nb = (n + CT_TILE - 1) / CT_TILE;
   const FlagKept fk{c->kept.p};
   if (nb == 1) {
@@ -1764,7 +1767,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
       c->tune_ev.push_back({bucket, {te0, te1}});
     }
     const long long nb = (ncc + CT_TILE - 1) / CT_TILE;
-    if (once) break;
+    if (once || ncc == 0) break;
     const FlagAlive fa{c->status.p};
     const AliveOut ao{c->keys.p, c->info.p, off * G, c->surv_o.p, c->surv_key.p, c->surv_bw.p};
     c->ev.begin(K_COMPACT, c->stream);
