@@ -1152,6 +1152,14 @@ struct chz_tc {
   chz::DBuf<uint8_t> keep, hit, fresh;
   chz::DBuf<unsigned long long> cnt, bcount, hist, tmp, mask, moff;
   chz::DBuf<int> flags;
+  // all of them back to the block cache (the stream has synchronised)
+  void release_work() {
+    ckeys.release();
+    for (auto *b : {&sk[0], &sk[1], &sv[0], &sv[1], &runs, &list, &list2, &link, &inv}) b->release();
+    for (auto *b : {&keep, &hit, &fresh}) b->release();
+    for (auto *b : {&cnt, &bcount, &hist, &tmp, &mask, &moff}) b->release();
+    flags.release();
+  }
   // measurement
   chz::EventLog ev;
   long k_launch[tcn::F_N] = {};
@@ -1859,11 +1867,7 @@ void chz_tc_free(chz_tc *c) {
   c->tab.release();
   void *ps[] = {c->d_anti, c->d_plus, c->d_coef, c->d_rv, c->d_rw, c->d_limbs, c->d_troot_fp, c->d_hkey, c->d_hval};
   for (void *p : ps) chz::dev_free(p);
-  c->ckeys.release();
-  for (int i = 0; i < 2; i++) { c->sk[i].release(); c->sv[i].release(); }
-  c->runs.release(); c->list.release(); c->list2.release();
-  c->keep.release(); c->hit.release(); c->fresh.release();
-  c->cnt.release(); c->bcount.release(); c->hist.release(); c->tmp.release(); c->flags.release();
+  c->release_work();
   c->ev.destroy();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
