@@ -155,6 +155,26 @@ struct DevPool {
 };
 inline DevPool &dev_pool() { static DevPool *p = new DevPool(); return *p; }   // never destroyed: no frees at exit
 
+// the outgrown blocks of a context whose stream has synchronised
+inline void settle(Retired &list) {
+  for (auto &b : list) dev_pool().put(b.first, b.second);
+  list.clear();
+}
+
+// A block for the calling context.  The blocks its buffers outgrew are memory too: where the device has none left, they are
+// given back, after a synchronisation, and the cache is asked again.
+inline void *block_get(size_t bytes, size_t &got) {
+  Retired *list = owner_stream() ? retire_list() : nullptr;
+  if (!list || list->empty()) return dev_pool().get(bytes, got);
+  try {
+    return dev_pool().get(bytes, got);
+  } catch (DeviceError &) {
+    HIPCHK(sync_owner());
+    settle(*list);
+    return dev_pool().get(bytes, got);
+  }
+}
+
 // untyped blocks from the cache for code that frees by pointer; dev_free requires that no queued kernel still
 // uses the block (synchronise first)
 struct LiveBlocks {
@@ -164,7 +184,7 @@ struct LiveBlocks {
 inline LiveBlocks &live_blocks() { static LiveBlocks *l = new LiveBlocks(); return *l; }
 inline void *dev_alloc(size_t bytes) {
   size_t got = 0;
-  void *p = dev_pool().get(std::max<size_t>(bytes, 1), got);
+  void *p = block_get(std::max<size_t>(bytes, 1), got);
   std::lock_guard<std::mutex> g(live_blocks().mu);
   live_blocks().sizes[p] = got;
   return p;
@@ -186,12 +206,6 @@ inline void dev_free(void *p) {
   dev_pool().put(p, got);
 }
 
-// the outgrown blocks of a context whose stream has synchronised
-inline void settle(Retired &list) {
-  for (auto &b : list) dev_pool().put(b.first, b.second);
-  list.clear();
-}
-
 template <typename T> struct DBuf {     // grow-only device array on the block cache
   T *p = nullptr;
   size_t cap = 0, bytes = 0;
@@ -199,19 +213,10 @@ template <typename T> struct DBuf {     // grow-only device array on the block c
     if (n <= cap) return;
     const size_t c = std::max<size_t>(std::max<size_t>(n, cap + cap / 2), 1);
     size_t got = 0;
-    T *np = nullptr;
-    Retired *list = owner_stream() ? retire_list() : nullptr;
-    try {
-      np = (T *)dev_pool().get(c * sizeof(T), got);
-    } catch (DeviceError &) {
-      if (!list || list->empty()) throw;
-      HIPCHK(sync_owner());                 // the outgrown blocks are memory too
-      settle(*list);
-      np = (T *)dev_pool().get(c * sizeof(T), got);
-    }
+    T *np = (T *)block_get(c * sizeof(T), got);
     if (p) {
       // kernels already queued may still read the old block
-      if (list) list->push_back({p, bytes});
+      if (Retired *list = owner_stream() ? retire_list() : nullptr) list->push_back({p, bytes});
       else {
         HIPCHK(sync_owner());
         dev_pool().put(p, bytes);

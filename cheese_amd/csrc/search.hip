@@ -1174,7 +1174,7 @@ static void tree_alloc(chz_ctx *c, long long n, uint32_t *&tp, uint8_t *&tg) {
     }
   if (!blk) {
     size_t got = 0;
-    blk = dev_pool().get(need + need / 4 + 256, got);
+    blk = block_get(need + need / 4 + 256, got);
     c->tree_blocks[blk] = got;
   }
   tp = (uint32_t *)blk;
@@ -1618,6 +1618,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   c->ev.end(c->stream);
   HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  settle(c->retired);
   fold_counters(hc, ns);
   c->ev.flush(c->k_ms, c->k_launch);
   if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
@@ -1854,6 +1855,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     c->ev.end(c->stream);
     HIPCHK(hipMemcpyAsync(hc, c->cnt, C_N * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    settle(c->retired);
     if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
     distinct = (long long)hc[C_KEPT];
   }

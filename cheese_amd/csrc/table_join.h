@@ -49,6 +49,7 @@ static std::vector<Zq> identity_entries(int n) {
 // ends every search of the context's batch without a result (the table or join answered instead)
 static void batch_clear(chz_ctx *c) {
   HIPCHK(hipStreamSynchronize(c->stream));
+  settle(c->retired);
   for (BInst &b : c->binst) b.live = false;
   c->pending.clear();
   c->events.clear();
