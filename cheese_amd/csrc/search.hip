@@ -2216,6 +2216,7 @@ static void upload_spec(chz_ctx *c) {
     const Zq &z = s.goal[i];
     if (z.a != (i / N == i % N) || z.b || z.c || z.d) k.pre = 0;
   }
+  if (k.have_table && s.cxtable[0] != 0) k.pre = 0;     // the goal needs no cut, but its cut bound is not 0
   // a cut bound from lowered needs is a lower bound only if the table never decreases when a need grows
   k.cx_mono = 1;
   k.ncx = (int)s.cxtable.size();
