@@ -501,7 +501,7 @@ static thread_local std::string g_err;
 }  // namespace chz_cl
 
 namespace chz_cl {
-constexpr long long kQueryScratch = 1ll << 20;      // most words of one chz_cliff_query_words_noalloc call
+constexpr long long kQueryWords = 1ll << 20;      // most words of one chz_cliff_query_words_noalloc call
 }
 
 struct chz_cliff {
@@ -680,14 +680,14 @@ int chz_cliff_query_words(chz_cliff *c, const uint8_t *letters, const long long 
   return 0;
 }
 
-// chz_cliff_query_words with device buffers and no allocation, at most kQueryScratch words per call; the kernel goes on
+// chz_cliff_query_words with device buffers and no allocation, at most kQueryWords words per call; the kernel goes on
 // `stream` (NULL: the table's own stream, synchronised before returning).
 int chz_cliff_query_words_noalloc(chz_cliff *c, const uint8_t *d_letters, const long long *d_offs, long long nq,
                                   int *d_dist, void *stream) {
   if (nq < 0 || (nq > 0 && (!d_letters || !d_offs || !d_dist))) { chz_cl::g_err = "bad arguments"; return 3; }
-  if (nq > chz_cl::kQueryScratch) {
+  if (nq > chz_cl::kQueryWords) {
     chz_cl::g_err = "chz_cliff_query_words_noalloc: " + std::to_string(nq) + " words exceed the scratch capacity of " +
-                    std::to_string(chz_cl::kQueryScratch);
+                    std::to_string(chz_cl::kQueryWords);
     return 4;
   }
   if (nq == 0) return 0;

@@ -86,24 +86,11 @@ constexpr int DPP_QXOR1 = 0xB1, DPP_QXOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_M
 template <int CTRL> __device__ __forceinline__ uint32_t dpp32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
 }
-// all-reduce over the wave of a commutative operation: each step pairs every lane with one of another group whose
-// lanes already agree (quads, then 8, 16 and 32 lanes), so the pairing need not be a lane xor
-template <typename Op> __device__ __forceinline__ uint32_t wave_reduce32(uint32_t v, Op op) {
-  v = op(v, dpp32<DPP_QXOR1>(v));
-  v = op(v, dpp32<DPP_QXOR2>(v));
-  v = op(v, dpp32<DPP_HALF_MIRROR>(v));
-  v = op(v, dpp32<DPP_MIRROR>(v));
-  // v_permlane16_swap(v, v) returns rows (0, 0, 2, 2) and (1, 1, 3, 3) of v; v_permlane32_swap(v, v) the halves
-  // (0, 0) and (1, 1)
-  const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = op(p[0], p[1]);
-  const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return op(q[0], q[1]);
-}
-
-// The same for an operation with identity 0, as a wave-uniform value: two row broadcasts instead of the swaps leave the
-// total in lane 63 (six vector instructions and a readlane, where the all-reduce and a readfirstlane take thirteen).
-// row_bcast15 brings lane 15 of a row to the next one, here to rows 1 and 3, row_bcast31 lane 31 to rows 2 and 3.
+// A wave's total of a commutative operation with identity 0, as a wave-uniform value: each step pairs every lane with one of
+// another group whose lanes already agree (quads, then 8 and 16 lanes), so the pairing need not be a lane xor, and two row
+// broadcasts leave the total in lane 63 (six vector instructions and a readlane, where an all-reduce by permlane swaps and a
+// readfirstlane took thirteen).  row_bcast15 brings lane 15 of a row to the next one, here to rows 1 and 3, row_bcast31 lane
+// 31 to rows 2 and 3.
 template <typename Op> __device__ __forceinline__ uint32_t wave_total32(uint32_t v, Op op) {
   v = op(v, dpp32<DPP_QXOR1>(v));
   v = op(v, dpp32<DPP_QXOR2>(v));

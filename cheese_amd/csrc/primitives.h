@@ -308,7 +308,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_hist(const uint32_t *keys,
 }
 
 // this block's tile of (key, value) pairs placed from base[d], the first output position of digit d for the tile
-// (shared; advanced as the rounds go)
+// (shared)
 __device__ __forceinline__ void radix_scatter_tile(const uint32_t *kin, const uint32_t *vin, long long n, int shift,
                                                    unsigned long long *base, uint32_t *kout, uint32_t *vout) {
   constexpr int NW = RS_THREADS / 64;

@@ -53,14 +53,12 @@ struct ExpandArgs {
   const int *pk;            // parents' sqrt2 exponents
   const uint8_t *g1, *g2;   // parents' last / second-to-last gates (255: none)
   long long off;            // first parent of the chunk (index in the level)
-  long long ncc;            // children in the chunk
-  int t, keep;
-  uint8_t *status;          // [ncc]
-  uint64_t *keys;           // [ncc] class keys of kept children
-  uint32_t *info;           // [ncc] bound words of kept children
+  uint8_t *status;          // per child of the chunk
+  uint64_t *keys;           // class keys of kept children
+  uint32_t *info;           // bound words of kept children
   const uint32_t *pb;       // parents' bound words
   const uint64_t *tm;       // parents' T columns (k_tcols; n = 3, specialised kernel)
-  unsigned long long *stage;  // NSTRIPE stripes of the stage counts (ST_N each)
+  unsigned long long *stage;  // NSTRIPE stripes of the stage counts (SG_N each)
   const uint32_t *pinst;    // instance slot of every parent of the level (null: one instance, slot 0)
   const int *rem;           // per slot: gate budget left after this level's gate (depth - t)
   const uint8_t *keepi;     // per slot: this level's survivors become parents (t < depth)
@@ -1128,9 +1126,10 @@ struct chz_ctx {
   chz::EventLog ev;
   long k_launch[chz::K_NFAM] = {};
   double k_ms[chz::K_NFAM] = {}, k_work[chz::K_NFAM] = {};
-  double k_stage[6] = {};       // expansion stage counts: residuals, structural bounds, cut ranks, T bounds, keys,
-                                // T-bound passes
+  double k_stage[6] = {};       // expansion stage counts: children past the windows, structural bounds, cut ranks, T bounds,
+                                // keys, T-bound passes
   double avg_terms = 1;         // nonzero terms per inverse column, averaged over the candidates
+  double avg_qubits = 1;        // qubits per candidate
   bool tcols = false;           // 3 qubits and std_spec: the frontier carries T columns
   bool cols_on = false;         // some node of it may have any
   bool std_spec = false;        // what the specialised expansion asks of a spec
@@ -1181,34 +1180,34 @@ static void tree_alloc(chz_ctx *c, long long n, uint32_t *&tp, uint8_t *&tg) {
   tg = (uint8_t *)(tp + std::max<long long>(n, 1));
 }
 
-// Lane operations of the T bound as implemented.  The f = 0 part (32-bit): per entry 12 for |S|^2 = r + y sqrt2
-// and 2 per transform stage for each of r and y.  One flip-pair pass (16-bit, two to a packed lane operation): for
-// each of the 4^n - 1 flip pairs, half of E/2 Z[w] products (16 multiplies + 12 adds), of a (2n-1)-stage
-// transform of E/2 four-coefficient entries and of 6 operations per entry for the final combination.
+// Lane operations of the T bound as implemented, two 16-bit operations to a packed one.  The f = 0 part: per entry 14 16-bit
+// operations for |S|^2 = r + y sqrt2 and 1 for each of r and y per transform stage.  One flip-pair pass: for each of the
+// 4^n - 1 flip pairs, half of E/2 Z[w] products (8 multiplies and 6 adds of 16 bits), a (2n - 2)-stage transform of E/2
+// two-coefficient entries, and in place of the last stage 3 operations for every two of them.
 static double t_f0_ops(int nq) {
   const double E = (double)(1 << (2 * nq));
-  return E * 12 + 2 * nq * E * 2;
+  return E * 7 + 2 * nq * E;
 }
 static double t_pass_ops(int nq) {
   const double E = (double)(1 << (2 * nq)), H = E / 2;
-  return (E - 1) * (H * 28 + (2 * nq - 1) * H * 4 + H * 6) / 2 / 2;
+  return (E - 1) * H * (7 + (2 * nq - 2) + 1.5);
 }
 
 // Algorithmic integer operations of one level's expansion, by stage, in 32-bit lane operations (two 16-bit
-// operations of the packed T transform count as one):
-//   residual: per entry, 8 per nonzero term of the gate's inverse column (4 coefficient rotations, 4 adds), plus
-//             6 for the sqrt2-divisibility test and 4 for the goal comparison;
-//   structural bounds: per entry 4 for the nonzero test, 5 per qubit for the support comparison;
-//   cut rank: per entry 30 for the F_p image (4 Montgomery products and reductions) and 14 per elimination
-//             step (2 Montgomery products, 1 modular subtraction), stop = 3 steps;
+// operations of the packed T transform count as one); what is done for a parent as a whole is not counted:
+//   residual (of the children that form one): per entry, 8 per nonzero term of the gate's inverse column (4 coefficients
+//             turned, 4 adds), plus 6 for the sqrt2-divisibility test and 4 for the goal comparison;
+//   structural bounds: per entry 4 for the nonzero test, 5 per qubit of the gate for the support comparison;
+//   cut rank: per entry 14 per elimination step (2 products, 1 modular subtraction and reduction), two steps, and a third
+//             of the F_p image, which a child's ranks share (4 products and one reduction, 9);
 //   T bound: t_f0_ops per evaluation, t_pass_ops per flip-pair pass it ran;
-//   class key: per entry 20 per entry hash (2), 22 per symmetry (mix and 64-bit add).
+//   class key: per entry 9 for each of the two entry hashes; n = 3: 3 sums that choose the symmetries (7 steps and 2 to
+//             form a share each) and one image (6 for the summand, two sums), n < 3: every image.
 static double expand_ops(const chz_ctx *c, int nq, const unsigned long long *hc) {
   const double E = (double)(1 << (2 * nq));
-  const double child = E * (8.0 * c->avg_terms + 10.0), cheap = E * (4.0 + 5.0 * nq), cut = E * (30.0 + 3 * 14.0);
-  // class key per lane: two 32-bit entry hashes (about 16 ops each), then per symmetry one slot summand (a 24-bit
-  // and two 32-bit products with their shifts and xors, 13 ops) and its two-word share of the 64-bit sums
-  const double key = E * (2 * 16.0 + 15.0 * c->ks.nsym);
+  const double child = E * (8.0 * c->avg_terms + 10.0), cheap = E * (4.0 + 5.0 * c->avg_qubits), cut = E * (2 * 14.0 + 3.0);
+  const double image = 6.0 + 2.0 * (nq == 3 ? 7 : 2 * nq);
+  const double key = E * (2 * 9.0 + (nq == 3 ? 3 * 9.0 + image : image * c->ks.nsym));
   return (double)(hc[C_EVAL] - hc[C_PRE]) * child + (double)hc[C_CHEAP] * cheap + (double)hc[C_CUTS] * cut +
          (double)hc[C_NEEDT] * t_f0_ops(nq) + (double)hc[C_TPASS] * t_pass_ops(nq) + (double)hc[C_KEYS] * key;
 }
@@ -1587,7 +1586,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
     // no device-wide or allocating HIP call from another thread while this stream is captured (capture_mu)
     std::lock_guard<std::recursive_mutex> capture_lock(capture_mu());
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, 0, ncap, 0, 0,
+    ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, 0,
                   c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
                   c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cap * G + CPW - 1) / CPW, sc.cap));
@@ -1750,7 +1749,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     const int bucket = std::min(31, 63 - __builtin_clzll((unsigned long long)cm));
     const chz_ctx::Sched sc = c->tuning ? c->force : c->sched[bucket];
     const int gsplit = (int)std::max<long long>(1, std::min<long long>(G, ((long long)sc.tw * CPW + cm - 1) / cm));
-    ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, off, ncc, 0, 0,
+    ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, off,
                   c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
                   c->icnt, slot_stripes(ns), ns * IC_N, gsplit, nullptr, 0, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cm * gsplit + CPW - 1) / CPW, sc.cap));
@@ -2092,7 +2091,7 @@ static void upload_spec(chz_ctx *c) {
   const HostSpec &s = c->hs;
   const int N = s.N(), G = s.G();
   std::vector<DevGate> dg(G);
-  double terms = 0, columns = 0;
+  double terms = 0, columns = 0, qubits = 0;
   for (int g = 0; g < G; g++) {
     const HostGate &h = s.gates[g];
     DevGate &d = dg[g];
@@ -2122,6 +2121,7 @@ static void upload_spec(chz_ctx *c) {
     d.tdel = sde >= 0 && sde < 255 ? sde : 255;
     for (const Zq &z : h.inv) terms += (z.a | z.b | z.c | z.d) != 0;
     columns += d.L;
+    qubits += h.nq;
     d.cutloc = 0;
     d.cdel = 0;
     if ((int)s.cutmask.size() <= BW_MAXCUTS)
@@ -2134,6 +2134,7 @@ static void upload_spec(chz_ctx *c) {
       }
   }
   c->avg_terms = columns > 0 ? terms / columns : 1.0;
+  c->avg_qubits = G > 0 ? qubits / G : 1.0;
   // T-bound classes: non-Clifford candidates whose children always have equal T bounds (same_t_bound), so a
   // parent's expansion computes the bound once per class
   {
@@ -2533,7 +2534,7 @@ long long chz_batch_frontier(chz_ctx *c, long long max, long long stride, int *p
       uint32_t w = 0, slot = 0;
       chz::copy_sync(&w, c->pb[c->cur].p + j, 4, hipMemcpyDeviceToHost, c->stream);
       chz::copy_sync(&slot, c->finst[c->cur].p + j, 4, hipMemcpyDeviceToHost, c->stream);
-      // the node's gates from its root: the tree walked up from the current level, as walk_circuit does
+      // the node's gates from its root: the tree walked up from the current level, as walk_circuits does
       seq.clear();
       uint32_t i = (uint32_t)j;
       for (int s = c->gstep; s >= 0 && c->tree_par[s]; s--) {
