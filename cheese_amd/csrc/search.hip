@@ -67,6 +67,7 @@ struct ExpandArgs {
   int gsplit;               // a parent's candidates are split among this many lane groups (small levels)
   const unsigned long long *npd;   // parents read on the device (captured step; gsplit then from tw), or null
   int tw;                   // candidate-split threshold in waves (with npd)
+  int psplit;               // lane groups per parent up to which children are settled from the parent's bounds (pre_split)
   const uint32_t *gflag;    // per slot: some parent of the level has a goal child (null: not tracked)
 };
 
@@ -243,10 +244,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     // of 5.71 million children past the windows still form one (3.12 without the T siblings below).  Only where no child
     // can overflow (which would be reported) and the goal's own bounds are 0 (a goal child is never over its budget).
     // On the budget-14 proof the expansion takes 111 ms instead of 139.  Where a parent's candidates are split over
-    // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.  Roots (no gate
-    // before them) form every residual: a target keeps its exponent as written, and where sqrt2 divides all of its entries
-    // a child's can be lower by more than the gate takes.
-    const bool pre = g1 != 255 && gsplit <= PRE_SPLIT && (STD || (sp.pre && gall<GS>(mag <= sp.maglim)));
+    // many lane groups each of them would repeat this, which took small levels 5 % longer: PRE_SPLIT.  A parent whose
+    // entries sqrt2 divides has children of lower exponents yet; only a root can be one, since a target keeps its exponent
+    // as written, and the level of such a root forms every residual (pre_split).
+    const bool pre = gsplit <= a.psplit && (STD || (sp.pre && gall<GS>(mag <= sp.maglim)));
     const bool tparent = (pbw & BW_TUNK) != BW_TUNK;
     // H on qubit q pairs the columns c and c ^ 2^q as their sum and difference over sqrt2: the exponent rises by one,
     // less one if sqrt2 divides every sum (the parities of a + c and b + d agree in each pair), less another if 2 does
@@ -1050,6 +1051,7 @@ struct BInst {
   double growth = 0;           // the last level's distinct / parents (0: not known yet)
   int k = 0;                   // the root's sqrt2 exponent and largest coefficient
   uint32_t coef = 0;
+  bool reducible = false;      // sqrt2 divides the root's entries below its exponent
   double t0 = 0;
 };
 struct Pending {               // a search waiting to join the frontier as a root
@@ -1464,6 +1466,12 @@ static bool std_level(const chz_ctx *c) {
   }
   return true;
 }
+// Lane groups per parent up to which this frontier's children are settled from their parents' bounds: none beside a root that
+// sqrt2 divides
+static int pre_split(const chz_ctx *c) {
+  for (const BInst &b : c->binst) if (b.live && b.t == 0 && b.reducible) return 0;
+  return PRE_SPLIT;
+}
 template <int NQ> static void launch_level(chz_ctx *c, int var, bool spec, dim3 grid, hipStream_t s, const ExpandArgs &ea, long long m) {
   const KSpec &ks = c->ks;
   if constexpr (NQ > 1)
@@ -1567,6 +1575,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   level_room<NQ>(c, nxt, ncap, mx, tp, tg);
   const chz_ctx::Sched sc = c->sched[STEP_BUCKET];
   const bool spec = std_level(c);
+  const int psplit = pre_split(c);
   const uint32_t *pinst = c->finst[cur].p;
   const std::vector<uintptr_t> key = {
       (uintptr_t)c->res[cur].p, (uintptr_t)c->pk[cur].p, (uintptr_t)c->g1[cur].p, (uintptr_t)c->g2[cur].p,
@@ -1576,7 +1585,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
       (uintptr_t)c->kept.p, (uintptr_t)c->kidx.p, (uintptr_t)c->sk[0].p, (uintptr_t)c->sk[1].p,
       (uintptr_t)c->sv[0].p, (uintptr_t)c->sv[1].p, (uintptr_t)c->hist.p, (uintptr_t)c->scan_tmp.p,
       (uintptr_t)c->gflag.p, (uintptr_t)ns, (uintptr_t)sc.var, (uintptr_t)sc.cap,
-      (uintptr_t)sc.tw, (uintptr_t)spec};
+      (uintptr_t)sc.tw, (uintptr_t)spec, (uintptr_t)psplit};
   chz_ctx::StepGraph &sg = c->sgraph[cur];
   if (!sg.exec || sg.key != key) {
     if (sg.exec) { HIPCHK(hipGraphExecDestroy(sg.exec)); sg.exec = nullptr; }
@@ -1588,7 +1597,7 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
     HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, 0,
                   c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
-                  c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, c->goal_skip ? c->gflag.p : nullptr};
+                  c->icnt, slot_stripes(ns), ns * IC_N, 1, dm, sc.tw, psplit, c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cap * G + CPW - 1) / CPW, sc.cap));
     launch_level<NQ>(c, sc.var, spec, grid, s, ea, cap);
     level_tail<NQ>(c, cur, ncap, dncc, nullptr, false, s);
@@ -1617,7 +1626,11 @@ static void step_graph(chz_ctx *c, int cur, long long m, const unsigned long lon
   c->ev.end(c->stream);
   HIPCHK(hipMemcpyAsync(hc, c->cnt, counter_words(ns) * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  settle(c->retired);
+  // what a large level before this one outgrew; the few megabytes that small levels outgrow wait for the next large one, since
+  // giving blocks back waits for a capture that another engine has open
+  size_t held = 0;
+  for (const auto &b : c->retired) held += b.second;
+  if (held > (size_t)ONCE_BYTES) settle(c->retired);
   fold_counters(hc, ns);
   c->ev.flush(c->k_ms, c->k_launch);
   if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
@@ -1751,7 +1764,7 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     const int gsplit = (int)std::max<long long>(1, std::min<long long>(G, ((long long)sc.tw * CPW + cm - 1) / cm));
     ExpandArgs ea{c->res[cur].p, c->pk[cur].p, c->g1[cur].p, c->g2[cur].p, off,
                   c->status.p, c->keys.p, c->info.p, c->pb[cur].p, c->tm[cur].p, c->stage, pinst, c->d_rem, c->d_keepi,
-                  c->icnt, slot_stripes(ns), ns * IC_N, gsplit, nullptr, 0, c->goal_skip ? c->gflag.p : nullptr};
+                  c->icnt, slot_stripes(ns), ns * IC_N, gsplit, nullptr, 0, pre_split(c), c->goal_skip ? c->gflag.p : nullptr};
     const dim3 grid(grid_for((cm * gsplit + CPW - 1) / CPW, sc.cap));
     hipEvent_t te0 = nullptr, te1 = nullptr;
     if (c->tuning) {
@@ -2325,8 +2338,11 @@ static int batch_add_parsed(chz_ctx *c, const HostSpec &hs, int depth, int tag) 
   Pending q;
   q.inst = bi;
   q.k = b.k = hs.tk;
-  for (const Zq &z : hs.target)
+  b.reducible = hs.tk > 0;
+  for (const Zq &z : hs.target) {
     for (long long v : {(long long)z.a, (long long)z.b, (long long)z.c, (long long)z.d}) b.coef = std::max(b.coef, (uint32_t)std::llabs(v));
+    b.reducible = b.reducible && !((z.a - z.c) & 1) && !((z.b - z.d) & 1);
+  }
   q.U.resize(E);
   for (int i = 0; i < E; i++) {
     const Zq &z = hs.target[i];
