@@ -1867,7 +1867,6 @@ template <int NQ> static void batch_step(chz_ctx *c) {
     c->ev.end(c->stream);
     HIPCHK(hipMemcpyAsync(hc, c->cnt, C_N * 8, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    settle(c->retired);
     if (hc[C_REPOVF]) { set_err("a dedupe run holds more distinct classes than its buffer"); throw DeviceError(); }
     distinct = (long long)hc[C_KEPT];
   }
