@@ -461,6 +461,10 @@ constexpr uint32_t NO_NODE = 0xffffffffu;
 // matrices built in LDS) are left undone.  Measured there: comparisons 1.30 million -> 219 thousand, k_dedupe 68.9
 // -> 12.0 ms, k_keys 7.9 -> 6.7 ms, this kernel 0.2 ms.  A marked child always has an equal child of smaller index,
 // so the smallest child of a coset is never marked.
+// Growths of fewer than MARK_MIN children are left unmarked: the eight launches and the synchronisation took longer than what
+// they saved (1-qubit tables of depth 3 1.35 -> 1.19 ms, 2-qubit searches of 16 targets 1.27 -> 1.21; with the line at 200K
+// instead of 20K children 3-qubit tables of depth 3 take 2.56 ms instead of 1.95).
+constexpr long long MARK_MIN = 1 << 14;
 struct MarkArgs {
   const uint64_t *anti;
   const uint32_t *cmap;        // the level before: node of the level that holds child k * G + p - 1, or NO_NODE
@@ -1366,7 +1370,7 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
     c->ev.end(c->stream);
   }
   // where every child went, for the marks of the next growth
-  if (!last && nn) {
+  if (!last && nn * G >= MARK_MIN) {
     L.cmap = dalloc<uint32_t>(nc);
     L.cmap_np = np;
     hipLaunchKernelGGL(k_fill_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, L.cmap, nc, NO_NODE);
