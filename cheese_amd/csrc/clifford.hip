@@ -166,6 +166,18 @@ template <int NQ> struct Num {
       if ((d >> i) & 1) m = ((m >> (1 << i)) & L[i]) | ((m & L[i]) << (1 << i));
     return m;
   }
+  // place of the bit of m that r others lie below (halving; one by one, samples of the 3-qubit group took 38 us a call)
+  __host__ __device__ static uint32_t nth_bit(uint64_t m, uint32_t r) {
+    uint32_t at = 0;
+#pragma unroll
+    for (int w = 1 << (M - 1); w; w >>= 1) {
+      const uint32_t c = (uint32_t)__builtin_popcountll(m >> at & ((1ull << w) - 1));
+      const bool up = r >= c;
+      r -= up ? c : 0u;
+      at += up ? (uint32_t)w : 0u;
+    }
+    return at;
+  }
   // the tableau whose k-th chosen row is choice r[k], row i signed by bit i of s
   __host__ __device__ static uint64_t tableau(const uint32_t (&r)[M], uint32_t s) {
     uint64_t an[M], span = 1, T = 0;
@@ -176,12 +188,7 @@ template <int NQ> struct Num {
 #pragma unroll
       for (int j = 0; j < k; j++) m &= (M - 1 - j) == row + NQ ? an[j] : ~an[j];
       if (k < NQ) m &= ~span;
-      for (uint32_t c = r[k]; c; c--) m &= m - 1;
-#ifdef __HIP_DEVICE_COMPILE__
-      const uint32_t v = (uint32_t)__ffsll((long long)m) - 1;
-#else
-      const uint32_t v = (uint32_t)__builtin_ctzll(m);
-#endif
+      const uint32_t v = nth_bit(m, r[k]);
       an[k] = anti(v);
       if (k < NQ) span |= shift(span, v);
       T |= (uint64_t)(v | ((s >> row) & 1) << M) << (row * (M + 1));
@@ -532,7 +539,8 @@ const char *chz_cliff_last_error(void) { return chz_cl::g_err.c_str(); }
 template <int NQ> static int cliff_fill(chz_cliff *c) {
   using namespace chz_cl;
   constexpr long long C = Num<NQ>::matrices();
-  constexpr int MAXD = 15;                            // four planes
+  constexpr int MAXD = NQ == 1 ? 3 : NQ == 2 ? 9 : 13;    // the group's largest distance (its order is checked below)
+  static_assert(MAXD < 16, "four planes");
   long long slots = 64;
   while (slots < 2 * C) slots <<= 1;
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -560,7 +568,7 @@ template <int NQ> static int cliff_fill(chz_cliff *c) {
   hipLaunchKernelGGL(k_matrices<NQ>, grid, blockd, 0, c->stream, c->key, c->T.slot, c->T.smask);
   hipLaunchKernelGGL(k_neighbours<NQ>, grid, blockd, 0, c->stream, c->T, c->key, nb);
   hipLaunchKernelGGL(k_root, dim3(1), dim3(64), 0, c->stream, c->T, identity(NQ), front[0], seen, cnt);
-  // every level is queued at once: one after the last finds the level before it empty and ends
+  // every level is queued at once
   for (int d = 1; d <= MAXD; d++) {
     const BfsArgs a{c->key, nb, front[(d - 1) & 1], front[d & 1], seen, (ulonglong2 *)(blk + o_pl), blk + o_min, cnt, d};
     hipLaunchKernelGGL(k_bfs<NQ>, grid, blockd, 0, c->stream, a);
