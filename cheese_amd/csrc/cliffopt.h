@@ -45,7 +45,7 @@ int read_cliff_job(const char *text, size_t len, CliffJob &J, std::string &err) 
 template <int NQ> int cliff_opt(chz_cliff *c, const CliffJob &J, int beam, double t0, char *out, size_t cap) {
   using chz_cl::Cand;
   using Num = chz_cl::Num<NQ>;
-const int n = NQ, t = (int)J.tq.size();
+  const int n = NQ, t = (int)J.tq.size();
   std::vector<uint64_t> D(t + 1);                             // segment tableaux
   for (int j = 0; j <= t; j++) {
     uint64_t X = chz_cl::identity(n);
@@ -65,25 +65,31 @@ const int n = NQ, t = (int)J.tq.size();
   struct Places { std::vector<uint32_t> zs; uint32_t *zpos = nullptr; chz_cl::PlaceMat *pm = nullptr; long long nm = 0; };
   std::vector<Places> places(n);
   constexpr int grid = 256;             // blocks of a beam step
-  uint64_t *d_left = (uint64_t *)dalloc(chz_cl::TOPK * 8);
-  int *d_cost = (int *)dalloc(chz_cl::TOPK * 4);
-  unsigned int *d_hist = (unsigned int *)dalloc(256 * 4);
-  unsigned long long *d_top = (unsigned long long *)dalloc((size_t)grid * chz_cl::TOPK * 8);
-  if (!d_left || !d_cost || !d_hist || !d_top) { chz_cl::g_err = "device memory"; return 5; }
+  constexpr long long nbs = (Num::Z_ALL + CT_TILE - 1) / CT_TILE, nbu = (Num::Z_SYM + CT_TILE - 1) / CT_TILE;
+  // the arrays whose sizes do not depend on the job, one block (an allocation each: 0.04 ms more for a 2-qubit job)
+  size_t fixed = 0;
+  auto part = [&](size_t bytes) { const size_t at = fixed; fixed += (bytes + 255) & ~(size_t)255; return at; };
+  const size_t o_left = part(chz_cl::TOPK * 8), o_cost = part(chz_cl::TOPK * 4), o_hist = part(256 * 4),
+               o_top = part((size_t)grid * chz_cl::TOPK * 8), o_bc = part((nbs + 1) * 8), o_bu = part((nbu + 1) * 8),
+               o_tmp = part((nbs / SC_TILE + 8) * 8), o_zs = part((size_t)Num::Z_ALL * 4), o_zu = part((size_t)Num::Z_SYM * 4),
+               o_zpos = part((size_t)Num::Z_ALL * 4 * n);
+  uint8_t *const blk = (uint8_t *)dalloc(fixed);
+  if (!blk) { chz_cl::g_err = "device memory"; return 5; }
+  uint64_t *const d_left = (uint64_t *)(blk + o_left);
+  int *const d_cost = (int *)(blk + o_cost);
+  unsigned int *const d_hist = (unsigned int *)(blk + o_hist);
+  unsigned long long *const d_top = (unsigned long long *)(blk + o_top);
   long long most = 0;                   // rows of a step per state
   {
-    const long long nbs = (Num::Z_ALL + CT_TILE - 1) / CT_TILE, nbu = (Num::Z_SYM + CT_TILE - 1) / CT_TILE;
-    unsigned long long *bc = (unsigned long long *)dalloc((nbs + 1) * 8), *bu = (unsigned long long *)dalloc((nbu + 1) * 8);
-    unsigned long long *tmp = (unsigned long long *)dalloc((nbs / SC_TILE + 8) * 8);
-    uint32_t *zs = (uint32_t *)dalloc((size_t)Num::Z_ALL * 4), *zu = (uint32_t *)dalloc((size_t)Num::Z_SYM * 4);
-    if (!bc || !bu || !tmp || !zs || !zu) { chz_cl::g_err = "device memory"; return 5; }
+    unsigned long long *const bc = (unsigned long long *)(blk + o_bc), *const bu = (unsigned long long *)(blk + o_bu);
+    unsigned long long *const tmp = (unsigned long long *)(blk + o_tmp);
+    uint32_t *const zs = (uint32_t *)(blk + o_zs), *const zu = (uint32_t *)(blk + o_zu);
     for (int q = 0; q < n; q++) {
       if (std::find(J.tq.begin(), J.tq.end(), q) == J.tq.end()) continue;
       Places &P = places[q];
       const chz_cl::FlagZs<NQ> fs{q};
       const chz_cl::FlagZ<NQ> fu{q};
-      P.zpos = (uint32_t *)dalloc((size_t)Num::Z_ALL * 4);
-      if (!P.zpos) { chz_cl::g_err = "device memory"; return 5; }
+      P.zpos = (uint32_t *)(blk + o_zpos) + (size_t)q * Num::Z_ALL;
       hipLaunchKernelGGL(k_flag_count<chz_cl::FlagZs<NQ>>, dim3((unsigned)nbs), dim3(CT_THREADS), 0, c->stream, fs,
                          (long long)Num::Z_ALL, bc);
       CLCHK(scan_excl(bc, nbs, tmp, c->stream));
@@ -162,8 +168,7 @@ const int n = NQ, t = (int)J.tq.size();
   // the final segment after each kept state; the best total, first in state order
   int best = 0, bestv = 1 << 30;
   if (t > 0) {
-    int *d_fin = (int *)dalloc(chz_cl::TOPK * 4);
-    if (!d_fin) { chz_cl::g_err = "device memory"; return 5; }
+    int *const d_fin = d_cost;          // (the last step has read its costs)
     CLCHK(hipMemcpyAsync(d_left, hK.data(), hK.size() * 8, hipMemcpyHostToDevice, c->stream));
     hipLaunchKernelGGL(chz_cl::k_beam_final, dim3(((int)hK.size() + 63) / 64), dim3(64), 0, c->stream, c->T, n, d_left,
                        (int)hK.size(), D[t], d_fin);
