@@ -192,7 +192,7 @@ def random_circuits(n=32):
 
 
 def clifford_table(T, wall, nq=100000):
-    """C4: the whole 3-qubit Clifford group tabulated on the GPU (BFS into the HBM hash table), then 1e5 seeded
+    """C4: the whole 3-qubit Clifford group tabulated on the GPU (symplectic matrices x sign vectors), then 1e5 seeded
     random words of 5..40 gates answered in one batched launch"""
     from cheese_amd import clifford
     entries = T.digest()[1]
@@ -396,7 +396,8 @@ def main():
                      "work": "algorithmic 32-bit integer lane ops: stage counts x per-stage ops (residual, "
                              "structural bounds, cut ranks, T bound: its f = 0 part per evaluation and each "
                              "flip-pair pass it ran at two 16-bit ops per lane op, class keys)",
-                     "stages_per_step": {k: v // a.steps for k, v in stages.items()},
+                     "stages_per_step": {("past_windows" if k == "residuals" else k): v // a.steps
+                                         for k, v in stages.items()},
                      "valu_busy_profiled": valu_busy},
         "kernel_launches_per_step": {k: v["launches"] / a.steps for k, v in kstats.items() if v["launches"]},
         "autotune": {b: [v["waves_per_eu"], v["grid_cap"], v["split_waves"]] for b, v in tuned.items()} if tuned else None,
