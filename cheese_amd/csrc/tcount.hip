@@ -444,7 +444,7 @@ struct DedupeArgs {
   const unsigned long long *nruns;
   const uint64_t *keys;
   uint8_t *keep;               // by child; cleared for every child whose coset an earlier child holds
-  uint32_t *link;              // by child; set to that earlier child
+  uint32_t *link;              // by child; set to that earlier child (null: not asked for)
   int *flags;                  // bit 1: a run held more than DMAXREP distinct cosets
   unsigned long long *stat;    // [0] children visited in runs, [1] exact comparisons, [2] duplicates
 };
@@ -471,7 +471,7 @@ struct MarkArgs {
   long long np;                // parents of the level before
   const uint32_t *inv;         // node of the level -> its place among this growth's parents (null: the same)
   unsigned long long *mask;    // per parent of this growth (zero at the start)
-  uint32_t *link;              // by child: itself, or an equal child of smaller index
+  uint32_t *link;              // by child: itself, or an equal child of smaller index (null: not asked for)
   int G;
 };
 
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(64) void k_mark(MarkArgs a) {
       if (lane >= p && x != NO_NODE && !((a.anti[p - 1] >> q) & 1)) {
         const uint32_t c1 = x * (uint32_t)G + (uint32_t)(p - 1), c2 = y * (uint32_t)G + (uint32_t)(q - 1);
         const bool first = c1 < c2;
-        atomicMin(&a.link[first ? c2 : c1], first ? c1 : c2);
+        if (a.link) atomicMin(&a.link[first ? c2 : c1], first ? c1 : c2);
         atomicOr(&a.mask[first ? y : x], 1ull << (first ? q - 1 : p - 1));
       }
     }
@@ -565,7 +565,10 @@ template <int NQ> __global__ __launch_bounds__(64) void k_dedupe(DedupeArgs a) {
       n_vis++;
       if (dup) {
         n_dup++;
-        if (lane == 0) { a.keep[ch] = 0; a.link[ch] = first; }
+        if (lane == 0) {
+          a.keep[ch] = 0;
+          if (a.link) a.link[ch] = first;
+        }
       } else if (nrep < DMAXREP) {
         if (lane == 0) rep[nrep] = ch;
         nrep++;
@@ -754,7 +757,10 @@ template <int NQ> __global__ __launch_bounds__(64) void k_pairs(PairArgs a) {
     __builtin_amdgcn_wave_barrier();
     if (equal) {
       n_dup++;
-      if (lane == 0) { a.keep[ch] = 0; a.link[ch] = first; }
+      if (lane == 0) {
+        a.keep[ch] = 0;
+        if (a.link) a.link[ch] = first;
+      }
     } else if (lane == 0) {
       a.runs[atomicAdd(a.nruns, 1ull)] = (uint32_t)s;
     }
@@ -1257,9 +1263,13 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
   HIPCHK(hipMemsetAsync(c->flags.p, 0, sizeof(int), c->stream));
 
   // duplicates by commutation, from the growth before
-  c->link.need(nc);
+  uint32_t *link = nullptr;                   // (the last growth, which has the most children, needs none)
+  if (!last) {
+    c->link.need(nc);
+    link = c->link.p;
+  }
   c->cnt.need(6);                             // runs, visited, compared, duplicates; run members; runs left open
-  hipLaunchKernelGGL(k_iota_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, c->link.p, nc);
+  if (link) hipLaunchKernelGGL(k_iota_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, link, nc);
   hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, c->cnt.p, 6ll, 0ull);
   const bool marks = L.cmap != nullptr && np > 0;
   long long nu = nc;                          // children not marked
@@ -1274,7 +1284,7 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
       hipLaunchKernelGGL(k_fill_u32, dim3(gridt(L.count[t])), dim3(256), 0, c->stream, c->inv.p, L.count[t], NO_NODE);
       hipLaunchKernelGGL(k_invert, dim3(gridt(np)), dim3(256), 0, c->stream, plist, np, c->inv.p);
     }
-    MarkArgs ma{c->d_anti, L.cmap, L.cmap_np, plist ? c->inv.p : nullptr, c->mask.p, c->link.p, G};
+    MarkArgs ma{c->d_anti, L.cmap, L.cmap_np, plist ? c->inv.p : nullptr, c->mask.p, link, G};
     hipLaunchKernelGGL(k_mark, dim3(grid1(L.cmap_np)), dim3(64), 0, c->stream, ma);
     hipLaunchKernelGGL(k_unmarked, dim3(gridt(np)), dim3(256), 0, c->stream, c->mask.p, np, G, c->moff.p);
     HIPCHK(scan_excl(c->moff.p, np, c->tmp.p, c->stream));
@@ -1310,14 +1320,14 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
     hipLaunchKernelGGL(k_run_members, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p,
                        nu, c->sk[1].p, c->cnt.p + 4);
     PairArgs pa{R, F.mat[t], L.inst[t], plist, c->sk[0].p, c->sv[0].p, nu, c->sk[1].p, c->cnt.p + 4, c->ckeys.p,
-                c->keep.p, c->link.p, c->runs.p, c->cnt.p + 5, c->cnt.p};
+                c->keep.p, link, c->runs.p, c->cnt.p + 5, c->cnt.p};
     hipLaunchKernelGGL(k_pairs<NQ>, dim3(grid1(nu / 2 + 1, 16384)), dim3(64), 0, c->stream, pa);
   } else {
     hipLaunchKernelGGL(k_run_starts, dim3(grid_for(nu / (64 * RH_ITEMS) + 1)), dim3(256), 0, c->stream, c->sk[0].p,
                        nu, c->runs.p, c->cnt.p, nullptr);
   }
   // blocks read the number of runs on the device
-  DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nu, c->runs.p, c->cnt.p + (F.mat[t] ? 5 : 0), c->ckeys.p, c->keep.p, c->link.p,
+  DedupeArgs da{R, F, t, plist, c->sk[0].p, c->sv[0].p, nu, c->runs.p, c->cnt.p + (F.mat[t] ? 5 : 0), c->ckeys.p, c->keep.p, link,
                 c->flags.p, c->cnt.p + 1};
   hipLaunchKernelGGL(k_dedupe<NQ>, dim3(grid1(nu / 2 + 1, F.mat[t] ? 512 : 8192)), dim3(64), 0, c->stream, da);
   c->ev.end(c->stream);
@@ -1375,7 +1385,7 @@ static GrowOut grow(chz_tc *c, Levels &L, int t, const uint32_t *plist, long lon
     L.cmap_np = np;
     hipLaunchKernelGGL(k_fill_u32, dim3(gridt(nc)), dim3(256), 0, c->stream, L.cmap, nc, NO_NODE);
     hipLaunchKernelGGL(k_invert, dim3(gridt(nn)), dim3(256), 0, c->stream, c->list.p, nn, L.cmap);
-    hipLaunchKernelGGL(k_resolve, dim3(gridt(nc)), dim3(256), 0, c->stream, c->link.p, nc, L.cmap);
+    hipLaunchKernelGGL(k_resolve, dim3(gridt(nc)), dim3(256), 0, c->stream, link, nc, L.cmap);
   }
   HIPCHK(hipMemcpyAsync(&out.flags, c->flags.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   unsigned long long st[4] = {0, 0, 0, 0};
